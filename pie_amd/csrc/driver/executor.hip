@@ -571,14 +571,27 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     auto grouped = tiled ? pie_hip_moe_grouped_gemm_tiled : pie_hip_moe_grouped_gemm;
     auto wptr = [&](const Linear& l) { return tiled ? l.data_tiled : l.data; };
     auto sptr = [&](const Linear& l) { return tiled && l.scale_tiled ? l.scale_tiled : l.scale; };
-    if (w.wgu.kind == Quant::Bf16 && w.wdown.kind == Quant::Bf16 && H % 64 == 0 && Ie % 64 == 0 && grouped_in_blocks(N * K, E)) {
+    // many routes per expert (a prompt's tokens): blocks of an expert's routes on the tiled GEMM, which takes quantised
+    // weights row-major (widths and groups that the passes refuse stay refused)
+    const int unit = w.wgu.kind == Quant::Bf16 ? 64 : w.wgu.kind == Quant::Int4b8 ? 512 : 256;
+    const bool fits = H % unit == 0 && Ie % unit == 0 && (w.wgu.kind != Quant::Int4b8 || w.wgu.group >= 128);
+    bool done = false;
+    if (grouped_in_blocks(N * K, E, w.wgu.kind != Quant::Bf16)) {
         auto blocks = [&](const Linear& l, const uint16_t* act, const int32_t* rows, uint16_t* y, int rows_out, int cols, int epilogue) {
-            PIE_KERNEL(pie_hip_moe_grouped_gemm_mfma(act, rows, moe_offsets_, E, N * K, wptr(l), l.data_bytes() / E, y, rows_out, cols,
-                                                     epilogue, tiled ? 1 : 0, nullptr, 0, s));
+            const bool tm = tiled && l.kind == Quant::Bf16;
+            return pie_hip_moe_grouped_gemm_mfma_fmt(fmt, act, rows, moe_offsets_, E, N * K, tm ? l.data_tiled : l.data,
+                                                     l.data_bytes() / E, l.scale, l.scale_bytes() / E, sbf, l.group, y, rows_out,
+                                                     cols, epilogue, tm ? 1 : 0, nullptr, 0, s);
         };
-        blocks(w.wgu, xn_, moe_route_token_, act_, 2 * Ie, H, PIE_HIP_EPI_SWIGLU);
-        blocks(w.wdown, act_, nullptr, moe_y_, H, Ie, PIE_HIP_EPI_NONE);
-    } else {
+        const int st = fits ? blocks(w.wgu, xn_, moe_route_token_, act_, 2 * Ie, H, PIE_HIP_EPI_SWIGLU) : PIE_HIP_ERR_UNSUPPORTED;
+        if (st == PIE_HIP_OK) {
+            PIE_KERNEL(blocks(w.wdown, act_, nullptr, moe_y_, H, Ie, PIE_HIP_EPI_NONE));
+            done = true;
+        } else if (st != PIE_HIP_ERR_UNSUPPORTED) {
+            PIE_KERNEL(st);
+        }
+    }
+    if (!done) {
         PIE_KERNEL(grouped(fmt, xn_, moe_route_token_, moe_offsets_, E, hint, wptr(w.wgu),
                            w.wgu.data_bytes() / E, sptr(w.wgu), w.wgu.scale_bytes() / E, sbf, w.wgu.group,
                            act_, 2 * Ie, H, 1, s));

@@ -26,9 +26,9 @@
 //   * activations are the MFMA A operand, weights the B operand: an accumulator lane holds one
 //     weight row n (column of y) for four consecutive activation rows, so row scales are
 //     per-lane scalars and the SwiGLU partner (gate_i, up_i interleaved) is the neighbour lane.
-// Grouped form (the experts of a mixture, bf16): a block finds its problem from the route offsets — row
+// Grouped form (the experts of a mixture): a block finds its problem from the route offsets — row
 // blocks are numbered through all problems, no problem's rows share a block with another's — and gathers
-// its activation rows; weights may be in the tile-major order of the skinny kernels, of which a transfer
+// its activation rows; bf16 weights may be in the tile-major order of the skinny kernels, of which a transfer
 // takes the same 16-byte granules from other places.
 #include "common.hip.h"
 
@@ -57,11 +57,11 @@ struct GemmArgs {
     int pointwise;        // PIE_HIP_EPI_RELU2 and above: applied to the sum (0: nothing)
     PieHipGlu glu = kPlainGlu;   // swiglu
     float* partial;   // split-K: fp32 [gridDim.z][M][N] partial sums (row scale applied), else null
-    // grouped: rows offsets[p] .. offsets[p + 1] of y belong to problem p (of `problems`), whose weights start
-    // w_stride bytes after the one before; act_rows: the activation row of each (null: the same row)
+    // grouped: rows offsets[p] .. offsets[p + 1] of y belong to problem p (of `problems`), whose weights (scales)
+    // start w_stride (scale_stride) bytes after the one before; act_rows: the activation row of each (null: the same row)
     const int32_t* offsets;
     const int32_t* act_rows;
-    size_t w_stride;
+    size_t w_stride, scale_stride;
     int problems, tiled;
 };
 
@@ -240,7 +240,7 @@ struct Shape {
 };
 
 template <class SH>
-__global__ __launch_bounds__(SH::kNW* kWave) void gemm_mfma_kernel(const GemmArgs a) {
+__global__ __launch_bounds__(SH::kNW* kWave) void gemm_mfma_kernel(GemmArgs a) {
     constexpr int MT = SH::kMT, NW = SH::kNW;
     constexpr int TPR = NW / 2;                  // threads that share a staged weight row
     using F = typename SH::Format::template Staged<TPR>;
@@ -259,7 +259,10 @@ __global__ __launch_bounds__(SH::kNW* kWave) void gemm_mfma_kernel(const GemmArg
     int M = a.M, m0 = blockIdx.y * BMv, problem = 0;
     if constexpr (SH::kGrouped)
         if (!grouped_place(a.offsets, a.problems, BMv, blockIdx.y, lane, problem, m0, M)) return;
-    const unsigned char* w = a.w + (SH::kGrouped ? static_cast<size_t>(problem) * a.w_stride : 0);
+    if constexpr (SH::kGrouped) {
+        a.w += static_cast<size_t>(problem) * a.w_stride;
+        if constexpr (!F::kDirect) a.scale += static_cast<size_t>(problem) * a.scale_stride;
+    }
     const int wstep = SH::kGrouped && a.tiled ? 16 : 1;   // values between a granule and the one a k-value further, per k-value
     // split-K: block z owns the K steps [kbeg, kbeg + nk) (the host makes every share non-empty)
     const int nk_all = K / BK;
@@ -287,7 +290,7 @@ __global__ __launch_bounds__(SH::kNW* kWave) void gemm_mfma_kernel(const GemmArg
             const size_t at = SH::kGrouped && a.tiled
                                   ? ((static_cast<size_t>(n >> 4) * (K >> 5) + (g >> 2)) * 64 + (g & 3) * 16 + (n & 15)) * 8
                                   : static_cast<size_t>(n) * K + g * 8;
-            bptr[u] = reinterpret_cast<const uint16_t*>(w) + at;
+            bptr[u] = reinterpret_cast<const uint16_t*>(a.w) + at;
         }
     }
     auto issue_direct = [&](int kt) {
@@ -600,11 +603,12 @@ int gemm_entry(int format, const uint16_t* act_bf16, const void* weight, const v
     }
 }
 
-template <int MT>
-int launch_grouped(const GemmArgs& a, int routes, hipStream_t stream) {
+template <class F, int MT>
+int launch_grouped_mt(const GemmArgs& a, int routes, hipStream_t stream) {
     constexpr int NW = 8, BMv = 16 * MT * (NW / 2);
-    using SH = Shape<GBf16, MT, NW, true>;
-    constexpr size_t smem = static_cast<size_t>(kStages) * (BMv * (BK / 8) + kTileVecs) * sizeof(u32x4_t);
+    using SH = Shape<F, MT, NW, true>;
+    constexpr size_t smem = (static_cast<size_t>(kStages) * BMv * (BK / 8) +
+                             static_cast<size_t>(F::kDirect ? kStages : 2) * kTileVecs) * sizeof(u32x4_t);
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mfma_kernel<SH>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
@@ -614,45 +618,75 @@ int launch_grouped(const GemmArgs& a, int routes, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_mfma_kernel<SH>), dim3((a.N + BN - 1) / BN, blocks), dim3(NW * kWave), smem, stream, a);
     return launch_status();
 }
+template <class F>
+int launch_grouped(const GemmArgs& a, int routes, int block_rows, hipStream_t stream) {
+    switch (block_rows) {
+        case 64: return launch_grouped_mt<F, 1>(a, routes, stream);
+        case 128: return launch_grouped_mt<F, 2>(a, routes, stream);
+        case 256: return launch_grouped_mt<F, 4>(a, routes, stream);
+        default: return PIE_HIP_ERR_UNSUPPORTED;
+    }
+}
 }  // namespace
 }  // namespace pie_hip
 
-extern "C" int pie_hip_moe_grouped_gemm_mfma(const uint16_t* act_bf16, const int32_t* route_act_rows, const int32_t* expert_offsets,
-                                             int num_experts, int num_routes, const void* weights_bf16, size_t weight_stride_bytes,
-                                             uint16_t* y_bf16, int N, int K, int epilogue, int tiled, const PieHipGlu* glu,
-                                             int block_rows, void* stream) {
+extern "C" int pie_hip_moe_grouped_gemm_mfma_fmt(int format, const uint16_t* act_bf16, const int32_t* route_act_rows,
+                                                 const int32_t* expert_offsets, int num_experts, int num_routes,
+                                                 const void* weights, size_t weight_stride_bytes, const void* scales,
+                                                 size_t scale_stride_bytes, int scale_is_bf16, int group_size, uint16_t* y_bf16,
+                                                 int N, int K, int epilogue, int tiled, const PieHipGlu* glu, int block_rows,
+                                                 void* stream) {
     using namespace pie_hip;
-    if (!act_bf16 || !expert_offsets || !weights_bf16 || !y_bf16 || num_experts <= 0 || num_routes <= 0 || N <= 0 || K <= 0 ||
-        !glu_ok(glu, epilogue))
+    if (!act_bf16 || !expert_offsets || !weights || !y_bf16 || num_experts <= 0 || num_routes <= 0 || N <= 0 || K <= 0 ||
+        (format != PIE_HIP_FMT_BF16 && !scales) || !glu_ok(glu, epilogue))
         return PIE_HIP_ERR_INVALID;
     GemmArgs a{};
     a.swiglu = epilogue == PIE_HIP_EPI_SWIGLU ? 1 : 0;
     a.pointwise = pointwise_code(epilogue);
     if (a.swiglu && N % 2 != 0) return PIE_HIP_ERR_INVALID;
-    if (K % BK != 0 || (tiled && N % 16 != 0)) return PIE_HIP_ERR_UNSUPPORTED;
+    if (K % BK != 0 || (tiled && (N % 16 != 0 || format != PIE_HIP_FMT_BF16))) return PIE_HIP_ERR_UNSUPPORTED;
+    if (format == PIE_HIP_FMT_INT4B8) {
+        if (group_size < 32 || (group_size & (group_size - 1)) != 0 || K % group_size != 0) return PIE_HIP_ERR_UNSUPPORTED;
+        a.g_shift = __builtin_ctz(static_cast<unsigned>(group_size));
+    }
     a.act = act_bf16;
     a.act_rows = route_act_rows;
     a.offsets = expert_offsets;
     a.problems = num_experts;
-    a.w = static_cast<const unsigned char*>(weights_bf16);
+    a.w = static_cast<const unsigned char*>(weights);
     a.w_stride = weight_stride_bytes;
+    a.scale = static_cast<const unsigned char*>(scales);
+    a.scale_stride = scale_stride_bytes;
+    a.scale_is_bf16 = scale_is_bf16;
     a.tiled = tiled ? 1 : 0;
     a.y = y_bf16;
     a.M = num_routes;
     a.N = N;
     a.K = K;
     if (glu) a.glu = *glu;
-    // (64 experts of 3072 x 4096, routes per expert 16 / 64 / 256: 295 / 367 / 985 us in blocks of 64, 310 / 324 / 746 of
-    // 128, 377 / 412 / 679 of 256; passes of 16 rows: 390 / 1161 / 4300)
+    // (64 bf16 experts of 3072 x 4096, routes per expert 16 / 64 / 256: 295 / 367 / 985 us in blocks of 64, 310 / 324 / 746
+    // of 128, 377 / 412 / 679 of 256; passes of 16 rows: 390 / 1161 / 4300)
+    // (128 fp8 experts of 1536 x 2048, routes per expert 24 / 64 / 88 / 128 / 192 / 512: 100 / 153 / 195 / 279 / - / - us in blocks
+    // of 64, 123 / 138 / 152 / 216 / 325 / 647 of 128, 242 / 281 / 282 / 288 / 311 / 708 of 256; of 2048 x 768 128 throughout)
     const int each = num_routes / num_experts;
-    if (block_rows == 0) block_rows = each < 48 ? 64 : each < 112 ? 128 : 256;
+    if (block_rows == 0) block_rows = each < 48 ? 64 : each < 112 || format != PIE_HIP_FMT_BF16 ? 128 : 256;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    switch (block_rows) {
-        case 64: return launch_grouped<1>(a, num_routes, st);
-        case 128: return launch_grouped<2>(a, num_routes, st);
-        case 256: return launch_grouped<4>(a, num_routes, st);
-        default: return PIE_HIP_ERR_UNSUPPORTED;
+    switch (format) {
+        case PIE_HIP_FMT_INT4B8: return launch_grouped<GInt4>(a, num_routes, block_rows, st);
+        case PIE_HIP_FMT_INT8: return launch_grouped<GInt8>(a, num_routes, block_rows, st);
+        case PIE_HIP_FMT_FP8: return launch_grouped<GFp8>(a, num_routes, block_rows, st);
+        case PIE_HIP_FMT_BF16: return launch_grouped<GBf16>(a, num_routes, block_rows, st);
+        default: return PIE_HIP_ERR_INVALID;
     }
+}
+
+extern "C" int pie_hip_moe_grouped_gemm_mfma(const uint16_t* act_bf16, const int32_t* route_act_rows, const int32_t* expert_offsets,
+                                             int num_experts, int num_routes, const void* weights_bf16, size_t weight_stride_bytes,
+                                             uint16_t* y_bf16, int N, int K, int epilogue, int tiled, const PieHipGlu* glu,
+                                             int block_rows, void* stream) {
+    return pie_hip_moe_grouped_gemm_mfma_fmt(PIE_HIP_FMT_BF16, act_bf16, route_act_rows, expert_offsets, num_experts, num_routes,
+                                             weights_bf16, weight_stride_bytes, nullptr, 0, 0, 0, y_bf16, N, K, epilogue, tiled, glu,
+                                             block_rows, stream);
 }
 
 extern "C" int pie_hip_gemm_mfma(int format, const uint16_t* act_bf16, const void* weight,

@@ -439,8 +439,9 @@ def moe_grouped_gemm(act: torch.Tensor, route_act_rows: Optional[torch.Tensor],
                      scales: Optional[torch.Tensor], N: int, K: int, rows_hint: int,
                      group_size: int = 0, swiglu: bool = False,
                      y: Optional[torch.Tensor] = None, num_routes: Optional[int] = None,
-                     tiled: bool = False) -> torch.Tensor:
-    """One skinny GEMM per expert in a single launch.  `weights` is [E, N, K] in the format's
+                     tiled: bool = False, block_rows: Optional[int] = None) -> torch.Tensor:
+    """One skinny GEMM per expert in a single launch (block_rows given: the tiled GEMM over blocks of that many
+    routes, 0 for the library's choice).  `weights` is [E, N, K] in the format's
     element type (int4b8: [E, N, K/8] words), `scales` [E, N] (int4b8: [E, N, K/G]);
     `expert_offsets` int32 [E+1] are the first route row of each expert (routes sorted by expert);
     `route_act_rows` int32 [routes] names each route's activation row (None: route r reads
@@ -468,6 +469,12 @@ def moe_grouped_gemm(act: torch.Tensor, route_act_rows: Optional[torch.Tensor],
     wstride = weights[0].numel() * weights.element_size()
     sstride = 0 if scales is None else scales[0].numel() * scales.element_size()
     scale_is_bf16 = int(scales is not None and scales.dtype == torch.bfloat16)
+    if block_rows is not None:
+        _check(kernels().pie_hip_moe_grouped_gemm_mfma_fmt(
+            FMT[kind], _ptr(act), _ptr(route_act_rows), _ptr(expert_offsets), E, routes, _ptr(weights), C.c_size_t(wstride),
+            _ptr(scales), C.c_size_t(sstride), scale_is_bf16, group_size, _ptr(y), N, K, int(swiglu), int(tiled), None,
+            block_rows, _stream()), "pie_hip_moe_grouped_gemm_mfma_fmt")
+        return y
     fn = kernels().pie_hip_moe_grouped_gemm_tiled if tiled else kernels().pie_hip_moe_grouped_gemm
     st = fn(
         FMT[kind], _ptr(act), _ptr(route_act_rows), _ptr(expert_offsets), E, int(rows_hint),

@@ -236,3 +236,44 @@ def test_expert_block_at_c5_full_routing_through_the_tile_major_kernels(gpu, ora
     tok = st["rtok"].cpu().numpy()
     want = oracle.f32_to_bf16(oracle.fp8_decode(gu_q[expert_of, :, cols[tok]]) * gu_s[expert_of])
     assert np.array_equal(oracle.bf16_to_f32(g), oracle.bf16_to_f32(want))
+
+
+@pytest.mark.parametrize("fmt,K,G", [("fp8", 768, 0), ("int8", 256, 0), ("int4b8", 512, 128), ("fp8", 256, 0)])
+@pytest.mark.parametrize("block_rows", [0, 64, 128, 256])
+def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_rows):
+    """The tiled grouped GEMM over quantised experts against the row-major passes of 16 rows: experts without routes, with
+    one, with a block and one more; columns off the tile, gathered rows, row scales of both types, SwiGLU.  Both sum the
+    same exact bf16 products in fp32, in other orders: a sum of K products differs by at most 2 K 2^-24 of the sum of their
+    magnitudes, a rounded result by that and half a bf16 step (2^-8) each."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(541 + K + block_rows)
+    counts = [0, 1, 63, 64, 65, 129, 0, 257, 17]
+    E, N, T = len(counts), 144, 96
+    routes = sum(counts)
+    offs = dev(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), gpu)
+    rows = dev(rng.integers(0, T, routes).astype(np.int32), gpu)
+    act = dev(oracle.f32_to_bf16(rng.standard_normal((T, K)).astype(np.float32)), gpu, torch.bfloat16)
+    if fmt == "int4b8":
+        w = dev(rng.integers(-2**31, 2**31, (E, N, K // 8)).astype(np.int32), gpu)
+        scale = dev(oracle.f32_to_bf16(rng.uniform(0.005, 0.02, (E, N, K // G)).astype(np.float32)), gpu, torch.bfloat16)
+        size = float(8 * 0.02)
+    else:
+        w = dev(rng.integers(-128, 128, (E, N, K)).astype(np.int8) if fmt == "int8"
+                else rng.integers(0, 0x70, (E, N, K)).astype(np.uint8) | (rng.integers(0, 2, (E, N, K)) << 7).astype(np.uint8), gpu)
+        scale = dev(rng.uniform(0.001, 0.004, (E, N)).astype(np.float32), gpu)
+        if K == 768:
+            scale = scale.bfloat16()
+        size = 0.004 * (128 if fmt == "int8" else 256)
+    bound = K * 4.0 * size * 2 * K * 2.0 ** -24      # |act| < 4 but for one value in 16 000, whose share is far below the slack
+    for swiglu in (False, True):
+        args = (act, rows, offs, fmt, w, scale, N, K, 257, G, swiglu)
+        want = ops.moe_grouped_gemm(*args).float()
+        got = ops.moe_grouped_gemm(*args, block_rows=block_rows).float()
+        if swiglu:   # (the gate's rounding moves the result by a step of each factor)
+            assert torch.all((got - want).abs() <= 4 * 2.0 ** -8 * want.abs() + 2.0 ** -6 * want.abs().amax())
+        else:
+            assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + bound)
+    assert torch.equal(ops.moe_grouped_gemm(act[rows.long()].contiguous(), None, offs, fmt, w, scale, N, K, 257, G, block_rows=block_rows),
+                       ops.moe_grouped_gemm(act, rows, offs, fmt, w, scale, N, K, 257, G, block_rows=block_rows))
