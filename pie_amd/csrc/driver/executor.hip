@@ -729,39 +729,47 @@ void Executor::body(int N, int S, int max_kv_len) {
                 merged_into_wo = true;
             }
         }
-        if (merged_into_wo) {
-        } else if (kvq_attn && n_tiles_ > 0 && !masked_) {
+        // rows [r.row, r.row + r.rows) one by one
+        auto attend_rows = [&](const RowRun& r) {
+            const size_t at = static_cast<size_t>(r.row) * hq * d;
+            if (masked_) {   // (the whole batch)
+                const auto* bitmap = static_cast<const uint16_t*>(mask_bitmap_.ptr);
+                if (kvq_attn)
+                    PIE_KERNEL(pie_hip_attn_rows_paged_kvq_masked(kv_format_, q_, k_pool_[l], v_pool_[l], ksc, vsc, attn_, nullptr,
+                                                                  pages, row_begin, row_len, bitmap, mask_stride_, N, hq, hk, d,
+                                                                  page_size_, -1.f, max_kv_len, attn_ws_, attn_ws_bytes_, s));
+                else
+                    PIE_KERNEL(pie_hip_attn_rows_paged_masked(q_, kat, vat, attn_, nullptr, pages, row_begin, row_len, bitmap,
+                                                              mask_stride_, N, hq, hk, d, page_size_, -1.f, max_kv_len, attn_ws_,
+                                                              attn_ws_bytes_, s));
+                return;
+            }
+            const uint32_t* begin = row_begin + r.row;
+            const int32_t* len = row_len + r.row;
+            if (kvq_attn || r.uniform)
+                PIE_KERNEL((r.uniform ? pie_hip_attn_rows_paged_kvq_uniform : pie_hip_attn_rows_paged_kvq)(
+                    kvq_attn ? kv_format_ : PIE_HIP_KV_BF16, q_ + at, kvq_attn ? k_pool_[l] : kat, kvq_attn ? v_pool_[l] : vat,
+                    kvq_attn ? ksc : nullptr, kvq_attn ? vsc : nullptr, attn_ + at, nullptr, pages, begin, len, r.rows, hq, hk, d,
+                    page_size_, -1.f, r.max_len, attn_ws_, attn_ws_bytes_, s));
+            else
+                PIE_KERNEL(pie_hip_attn_rows_paged(q_ + at, kat, vat, attn_ + at, nullptr, pages, begin, len, r.rows, hq, hk, d,
+                                                   page_size_, -1.f, r.max_len, attn_ws_, attn_ws_bytes_, s));
+        };
+        if (!merged_into_wo && n_tiles_ > 0) {
             const auto* td = static_cast<const int32_t*>(tile_in_dev_.ptr);
-            PIE_KERNEL(pie_hip_attn_prefill_tiles_kvq(kv_format_, q_, k_pool_[l], v_pool_[l], ksc, vsc, attn_,
-                                                      pages, row_begin, row_len, td, td + n_tiles_, n_tiles_,
+            if (kvq_attn)
+                PIE_KERNEL(pie_hip_attn_prefill_tiles_kvq(kv_format_, q_, k_pool_[l], v_pool_[l], ksc, vsc, attn_,
+                                                          pages, row_begin, row_len, td, td + n_tiles_, n_tiles_,
+                                                          tile_rows_, hq, hk, d, page_size_, -1.f, s));
+            else
+                PIE_KERNEL(pie_hip_attn_prefill_tiles(q_, kat, vat, attn_, pages, row_begin, row_len, td, td + n_tiles_, n_tiles_,
                                                       tile_rows_, hq, hk, d, page_size_, -1.f, s));
-        } else if (kvq_attn && masked_) {
-            PIE_KERNEL(pie_hip_attn_rows_paged_kvq_masked(
-                kv_format_, q_, k_pool_[l], v_pool_[l], ksc, vsc, attn_, nullptr, pages, row_begin, row_len,
-                static_cast<const uint16_t*>(mask_bitmap_.ptr), mask_stride_, N, hq, hk, d, page_size_, -1.f,
-                max_kv_len, attn_ws_, attn_ws_bytes_, s));
-        } else if (kvq_attn) {
-            PIE_KERNEL((uniform_rows_ ? pie_hip_attn_rows_paged_kvq_uniform : pie_hip_attn_rows_paged_kvq)(
-                kv_format_, q_, k_pool_[l], v_pool_[l], ksc, vsc, attn_, nullptr, pages, row_begin, row_len, N, hq,
-                hk, d, page_size_, -1.f, max_kv_len, attn_ws_, attn_ws_bytes_, s));
-        } else if (n_tiles_ > 0) {
-            const auto* td = static_cast<const int32_t*>(tile_in_dev_.ptr);
-            PIE_KERNEL(pie_hip_attn_prefill_tiles(q_, kat, vat, attn_, pages, row_begin,
-                                                  row_len, td, td + n_tiles_, n_tiles_, tile_rows_, hq,
-                                                  hk, d, page_size_, -1.f, s));
-        } else if (masked_) {
-            PIE_KERNEL(pie_hip_attn_rows_paged_masked(
-                q_, kat, vat, attn_, nullptr, pages, row_begin, row_len,
-                static_cast<const uint16_t*>(mask_bitmap_.ptr), mask_stride_, N, hq, hk, d, page_size_,
-                -1.f, max_kv_len, attn_ws_, attn_ws_bytes_, s));
-        } else if (uniform_rows_) {
-            PIE_KERNEL(pie_hip_attn_rows_paged_kvq_uniform(PIE_HIP_KV_BF16, q_, kat, vat, nullptr, nullptr, attn_,
-                                                           nullptr, pages, row_begin, row_len, N, hq, hk, d,
-                                                           page_size_, -1.f, max_kv_len, attn_ws_, attn_ws_bytes_, s));
+        }
+        if (merged_into_wo) {
+        } else if (pure_decode_) {   // (max_kv_len: the bucket a graph is captured for)
+            attend_rows({0, N, max_kv_len, uniform_rows_});
         } else {
-            PIE_KERNEL(pie_hip_attn_rows_paged(q_, kat, vat, attn_, nullptr, pages,
-                                               row_begin, row_len, N, hq, hk, d, page_size_, -1.f,
-                                               max_kv_len, attn_ws_, attn_ws_bytes_, s));
+            for (const RowRun& r : runs_) attend_rows(r);
         }
         if (!merged_into_wo)
         linear_fused(w.wo, attn_, nullptr, m.rms_eps, x_, N, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
@@ -841,21 +849,100 @@ float pcg32_first_uniform(uint64_t seed) {
 
 }  // namespace
 
-// Prefill-shaped batches (every request brings at least 8 query rows, no custom masks) run
-// their attention on the matrix cores: rows are cut into tiles of consecutive rows of one
-// request.  Batches with single-row requests keep the per-row kernel, whose split-K spreads a
-// long context over the machine.
+// Rows of which the longest context is within an eighth of the mean: their attention launch may plan one round of
+// equally long blocks.
+bool Executor::evenly_long(const BatchPlan& plan, int row, int rows) {
+    if (rows < 2) return false;
+    long long total = 0;
+    int longest = 0;
+    for (int i = row; i < row + rows; ++i) {
+        total += plan.row_kv_len[i];
+        longest = std::max(longest, plan.row_kv_len[i]);
+    }
+    return 8LL * longest * rows <= 9 * total;
+}
+
+// Which rows' attention runs as tiles of consecutive rows of one request (on the matrix cores, a block per tile and
+// kv head that walks the keys once for all its rows) and which row by row (split keys, every row reading its own).
+// Decoded tokens run row by row; a portion of a prompt takes tiles where they cost less.  Microseconds, measured (one
+// portion of 8 .. 1024 rows behind 0 .. 8192 keys; 32 query heads over 8 and 4 kv heads of 128, over 8 of 64): row by
+// row 6 + the bytes of every row's keys and values at 12 TB/s (they come from the caches); as tiles 6 + 1.0 (heads of
+// 64: 0.7) per step of 32 keys of the longest, or 1.5 per step and resident slot once 512 blocks are more than
+// one round.  The two meet at about 90 rows (8 kv heads of 128).  335 rows behind 512 keys beside 23 decoded
+// tokens over 700 - 1200: 156 us per layer when all ran row by row, 62 since (tiles 34, single tokens 27).
 void Executor::prepare_tiles(const BatchPlan& plan) {
     n_tiles_ = 0;
+    runs_.clear();
     const ModelConfig& m = model_.cfg();
+    const bool uniform_heads = m.head_dim == 64 || m.head_dim == 128;
     int cap = pie_hip_attn_prefill_tile_rows(m.q_heads, m.kv_heads);
-    if (cap <= 0 || masked_ || page_size_ % 16 != 0 || (m.head_dim != 64 && m.head_dim != 128)) return;
-    long long blocks = 0;
-    for (int r = 0; r < plan.R; ++r) {
-        const int n = plan.qo_indptr[r + 1] - plan.qo_indptr[r];
-        if (n < 8) return;
-        blocks += static_cast<long long>((n + cap - 1) / cap) * m.kv_heads;
+    const double step_us = m.head_dim == 64 ? 0.7 : 1.0;
+    const double key_us = 4.0 * m.kv_heads * m.head_dim / 12e6;
+    // the tiled requests of a choice: those of at least 8 rows over at most `most` keys
+    auto tiled = [&](int r, int most) {
+        const int q0 = plan.qo_indptr[r], q1 = plan.qo_indptr[r + 1];
+        return q1 - q0 >= 8 && plan.row_kv_len[q1 - 1] <= most;
+    };
+    auto runs_of = [&](int most) {   // the other rows, in runs of neighbours
+        std::vector<RowRun> runs;
+        for (int r = 0; r < plan.R; ++r) {
+            const int q0 = plan.qo_indptr[r], q1 = plan.qo_indptr[r + 1];
+            if (q0 == q1 || tiled(r, most)) continue;
+            if (runs.empty() || runs.back().row + runs.back().rows != q0) runs.push_back({q0, 0, 0, false});
+            runs.back().rows += q1 - q0;
+            for (int i = q0; i < q1; ++i) runs.back().max_len = std::max(runs.back().max_len, plan.row_kv_len[i]);
+        }
+        return runs;
+    };
+    auto cost = [&](int most) {
+        double rows_us = 0.0;
+        long long blocks = 0, block_steps = 0;
+        int steps = 0;
+        for (int r = 0; r < plan.R; ++r) {
+            const int q0 = plan.qo_indptr[r], q1 = plan.qo_indptr[r + 1], n = q1 - q0;
+            if (n == 0) continue;
+            const int last = plan.row_kv_len[q1 - 1];
+            if (tiled(r, most)) {
+                const int tiles = (2 * n + cap - 1) / cap;
+                steps = std::max(steps, (last + 31) / 32);
+                blocks += static_cast<long long>(tiles) * m.kv_heads;
+                block_steps += static_cast<long long>(tiles) * m.kv_heads * ((last - n / 2 + 31) / 32);
+            } else {
+                rows_us += key_us * n * (last - 0.5 * (n - 1));
+            }
+        }
+        return (rows_us > 0.0 ? 6.0 + rows_us : 0.0) +
+               (blocks ? 6.0 + step_us * std::max<double>(steps, 1.5 * block_steps / 512.0) : 0.0);
+    };
+    constexpr int kNone = -1, kAll = 0x7FFFFFFF;
+    int most = kNone;
+    if (cap > 0 && !masked_ && !plan.pure_decode && page_size_ % 16 == 0 && uniform_heads) {
+        // every portion; those that alone would gain, and shorter ones, which ride along; none
+        int gain = kNone;
+        for (int r = 0; r < plan.R; ++r) {
+            const int n = plan.qo_indptr[r + 1] - plan.qo_indptr[r];
+            if (n < 8) continue;
+            const int last = plan.row_kv_len[plan.qo_indptr[r + 1] - 1];
+            if (key_us * n * (last - 0.5 * (n - 1)) > step_us * ((last + 31) / 32)) gain = std::max(gain, last);
+        }
+        double best = cost(kNone);
+        for (int cand : {gain, kAll}) {
+            const double c = cost(cand);
+            if (c < best && runs_of(cand).size() <= 2) {   // (a launch per run and layer)
+                best = c;
+                most = cand;
+            }
+        }
     }
+    if (most != kNone) runs_ = runs_of(most);
+    else runs_.push_back({0, plan.N, plan.max_kv_len, false});
+    for (RowRun& run : runs_) run.uniform = !plan.pure_decode && evenly_long(plan, run.row, run.rows);
+    if (most == kNone) return;
+    long long blocks = 0;
+    for (int r = 0; r < plan.R; ++r)
+        if (tiled(r, most))
+            blocks += static_cast<long long>((plan.qo_indptr[r + 1] - plan.qo_indptr[r] + cap - 1) / cap) * m.kv_heads;
+    if (blocks == 0) return;
     // fewer than three full-size blocks per CU: halve the tiles (measured on a causal prompt of
     // 2048 tokens, 512 full-size blocks: 110 -> 100 us; of 3072 tokens, 768 blocks: 169 -> 179)
     if (blocks < 768) cap /= 2;
@@ -864,7 +951,7 @@ void Executor::prepare_tiles(const BatchPlan& plan) {
     // last would run on alone.
     std::vector<std::pair<int32_t, int32_t>> tiles;   // (first row, rows)
     for (int r = 0; r < plan.R; ++r)
-        for (int t0 = plan.qo_indptr[r]; t0 < plan.qo_indptr[r + 1]; t0 += cap)
+        for (int t0 = plan.qo_indptr[r]; tiled(r, most) && t0 < plan.qo_indptr[r + 1]; t0 += cap)
             tiles.emplace_back(t0, std::min(cap, plan.qo_indptr[r + 1] - t0));
     std::stable_sort(tiles.begin(), tiles.end(), [&](const auto& a, const auto& b) {
         return plan.row_kv_len[a.first + a.second - 1] > plan.row_kv_len[b.first + b.second - 1];
@@ -1139,18 +1226,9 @@ void Executor::forward(const BatchPlan& plan, std::vector<uint32_t>& tokens_out,
 
     t0 = clk::now();
     n_page_refs_ = static_cast<int>(plan.page_indices.size());
-    // A decode batch whose longest context is within an eighth of the mean: the attention launch
-    // may then plan one round of equally long blocks (a graph is captured per answer).
-    uniform_rows_ = false;
-    if (plan.pure_decode && N >= 2 && !masked_) {
-        long long total = 0;
-        int longest = 0;
-        for (int i = 0; i < N; ++i) {
-            total += plan.row_kv_len[i];
-            longest = std::max(longest, plan.row_kv_len[i]);
-        }
-        uniform_rows_ = 8LL * longest * N <= 9 * total;
-    }
+    // (a graph is captured per answer)
+    pure_decode_ = plan.pure_decode;
+    uniform_rows_ = plan.pure_decode && !masked_ && evenly_long(plan, 0, N);
     // (4-bit blocks: the page expansion's extent changes from step to step, so no graph)
     const bool use_graph = cfg_.runtime.use_graphs && plan.pure_decode && !samp_gather_in_body_ && !masked_ &&
                            kv_format_ != PIE_HIP_KV_FP4_BLOCK;

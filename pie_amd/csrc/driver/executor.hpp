@@ -140,6 +140,7 @@ class Executor {
     void grow_outputs(size_t slots);
     void prepare_masks(const BatchPlan& plan);
     void prepare_tiles(const BatchPlan& plan);
+    static bool evenly_long(const BatchPlan& plan, int row, int rows);
     void prepare_samplers(const BatchPlan& plan);
     void enqueue_samplers();
     void collect_samplers(const BatchPlan& plan, SampleOutputs& out);
@@ -240,7 +241,13 @@ class Executor {
         void ensure(size_t bytes);
         void release();
     };
-    // query-row tiles of the current forward for the matrix-core prefill attention (0 = per-row kernel)
+    // query-row tiles of the current forward for the matrix-core prefill attention, and the runs of rows that
+    // take the per-row kernel
+    struct RowRun {
+        int row, rows, max_len;
+        bool uniform;   // about equally long
+    };
+    std::vector<RowRun> runs_;
     Growable tile_in_host_, tile_in_dev_;
     int n_tiles_ = 0, tile_rows_ = 0;
     // keys and values projected out of cached latents (the longest portion so far)
@@ -306,7 +313,8 @@ class Executor {
     std::vector<int32_t> rs_last_, rs_host_last_;   // the last of them
 
     std::map<std::tuple<int, int, int, int>, hipGraphExec_t> graphs_;   // (rows, sampling slots, context bucket, rows equally long)
-    bool uniform_rows_ = false;   // this step's rows are about equally long (decode batches)
+    bool pure_decode_ = false;    // this step has one row per request and no masks
+    bool uniform_rows_ = false;   // and its rows are about equally long
     int last_logit_rows_ = 0;
 };
 

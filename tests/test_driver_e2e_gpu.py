@@ -907,3 +907,59 @@ def test_start_up_kernel_measurement_keeps_results_within_rounding(gpu, oracle):
     a, b = outs
     assert a.shape == b.shape and cosine(a, b) > 0.9995
     assert np.max(np.abs(a - b)) <= 0.05 * np.max(np.abs(b)) + 1e-3
+
+
+@pytest.mark.parametrize("lens", [
+    # (cached tokens, tokens of this batch) per request; 32 query heads over 8 kv heads of 64: portions from about 130 rows
+    # on take tiles, single tokens and short portions the row kernel
+    [(20, 1), (37, 1), (48, 201)],             # decoded tokens ahead of a portion: one run of rows
+    [(20, 1), (0, 150), (33, 3), (64, 1)],     # on both sides of it: two
+    [(16, 1), (0, 140), (20, 1), (0, 7), (0, 170), (31, 1)],   # three runs: all row by row
+    [(0, 130), (0, 9), (47, 180)],             # portions only, a short one riding along
+    [(0, 16), (3, 17)],                        # portions only, too short for tiles
+])
+@pytest.mark.parametrize("kv", ["auto", "fp8_per_token_head"])
+def test_portions_beside_decoded_tokens(gpu, oracle, lens, kv):
+    """The rows a batch splits into tiles and single rows give what the same requests give alone, row by row: the same
+    values in other orders of summation (bf16 activations: cosine >= 0.9999)."""
+    from pie_amd import driver as drvmod
+
+    kw = dict(quant="bf16", q_heads=32, kv_heads=8, head_dim=64, hidden=256, intermediate=512, vocab=512, total_pages=256,
+              max_forward_tokens=512, kv_cache_dtype=kv, tune_linears=False)
+    rng = np.random.default_rng(sum(n for _, n in lens))
+    with drvmod.Driver(toml_config(**kw)) as d:
+        def frame(parts, samples):
+            """(first page, cached, tokens) per request; `samples`: sampled places per request"""
+            tok, pos, pages, ptr, last, qo = [], [], [], [0], [], [0]
+            for page, held, t in parts:
+                npg = -(-(held + len(t)) // 16)
+                tok += list(t)
+                pos += range(held, held + len(t))
+                pages += range(page, page + npg)
+                ptr.append(len(pages))
+                last.append(held + len(t) - (npg - 1) * 16)
+                qo.append(len(tok))
+            flat = [i for s in samples for i in s]
+            indptr = np.concatenate([[0], np.cumsum([len(s) for s in samples])])
+            return drvmod.ForwardFrame(tok, pos, pages, ptr, last, qo, sampling_indices=flat, sampling_indptr=indptr)
+
+        def logits(f):
+            assert d.forward(f).num_requests == len(f.frame.payload.forward.qo_indptr.ptr[:f.frame.payload.forward.qo_indptr.len]) - 1
+            return oracle.bf16_to_f32(d.export_tensor("debug.logits", np.uint16).reshape(-1, 512))
+
+        parts, at = [], 0
+        for held, n in lens:
+            if held:
+                d.forward(frame([(at, 0, rng.integers(0, 512, held))], [[held - 1]]))
+            parts.append((at, held, rng.integers(0, 512, n)))
+            at += -(-(held + n) // 16)
+        samples = [sorted({0, n // 2, n - 1}) for _, n in lens]
+        got = logits(frame(parts, samples))
+        row = 0
+        for (page, held, t), places in zip(parts, samples):
+            for p in places:   # alone, and cut so that no portion is long enough for tiles
+                for a in range(0, p, 7):
+                    d.forward(frame([(page, held + a, t[a:min(a + 7, p)])], [[0]]))
+                want = logits(frame([(page, held + p, t[p:p + 1])], [[0]]))[0]
+                assert cosine(got[row], want) >= 0.9999, (page, held, len(t), p)
+                row += 1
