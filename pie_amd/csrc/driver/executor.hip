@@ -866,9 +866,9 @@ bool Executor::evenly_long(const BatchPlan& plan, int row, int rows) {
 // kv head that walks the keys once for all its rows) and which row by row (split keys, every row reading its own).
 // Decoded tokens run row by row; a portion of a prompt takes tiles where they cost less.  Microseconds, measured (one
 // portion of 8 .. 1024 rows behind 0 .. 8192 keys; 32 query heads over 8 and 4 kv heads of 128, over 8 of 64): row by
-// row 6 + the bytes of every row's keys and values at 12 TB/s (they come from the caches); as tiles 6 + 1.0 (heads of
+// row 6 + the bytes of every row's keys and values at 12 TB/s (they come from the caches); as tiles 4.5 + 1.0 (heads of
 // 64: 0.7) per step of 32 keys of the longest, or 1.5 per step and resident slot once 512 blocks are more than
-// one round.  The two meet at about 90 rows (8 kv heads of 128).  335 rows behind 512 keys beside 23 decoded
+// one round.  The two meet at about 90 rows of a new prompt (8 kv heads of 128), 128 (8 of 64).  335 rows behind 512 keys beside 23 decoded
 // tokens over 700 - 1200: 156 us per layer when all ran row by row, 62 since (tiles 34, single tokens 27).
 void Executor::prepare_tiles(const BatchPlan& plan) {
     n_tiles_ = 0;
@@ -912,7 +912,7 @@ void Executor::prepare_tiles(const BatchPlan& plan) {
             }
         }
         return (rows_us > 0.0 ? 6.0 + rows_us : 0.0) +
-               (blocks ? 6.0 + step_us * std::max<double>(steps, 1.5 * block_steps / 512.0) : 0.0);
+               (blocks ? 4.5 + step_us * std::max<double>(steps, 1.5 * block_steps / 512.0) : 0.0);
     };
     constexpr int kNone = -1, kAll = 0x7FFFFFFF;
     int most = kNone;
