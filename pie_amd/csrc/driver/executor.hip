@@ -59,7 +59,10 @@ int fmt_code(Quant q) {
 // the tiles fit the machine (512 resident blocks).  Split-K tiled GEMM: the steps of one share
 // (+3 of prologue) at 1.06 / 1.36 us with two blocks per CU, per round of 512 blocks, plus ~15 us
 // for the second kernel and the partials.
-enum class GemmPath { Skinny, Tiled, TiledSplitK };
+// More than 128 rows: the tiled GEMM's two forms say themselves what they take (pie_hip_gemm_mfma_us); over 40 shapes of 160 -
+// 4096 rows in three formats the choice loses 0.5 % against the fastest of the three each time.
+enum class GemmPath { Skinny, Tiled, TiledSplitK, Wide };
+bool tile_major(const Linear& w) { return w.data_tiled && (w.kind != Quant::Int4b8 || w.scale_tiled); }
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
     const int passes = (M + 15) / 16;
@@ -68,17 +71,29 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     const int wpasses = M > 32 ? (M + 31) / 32 : passes;
     int p2 = 1;
     while (p2 < wpasses) p2 <<= 1;
-    // (past eight passes the machine is full: the cost grows in proportion)
+    // (past eight passes the machine is full: the cost grows in proportion, in powers of two up to 32, 17 - 31 passes a
+    // fifth worse than 32)
     const double wave_form = (M > 32 ? 1.38 : 1.0) *
-                             (p2 <= 8 ? 1.0 + 0.52 * (p2 - 1) : (1.0 + 0.52 * 7) * wpasses / 8.0);
+                             (p2 <= 8 ? 1.0 + 0.52 * (p2 - 1)
+                                      : (1.0 + 0.52 * 7) * 0.9 * (p2 <= 32 ? p2 : wpasses) / 8.0 * (p2 == 32 && wpasses < 32 ? 1.2 : 1.0));
+    // (prompts' passes are bound by the products and the decoding, not by the weights' width)
+    const double bytes = M > 128 && w.kind != Quant::Bf16 ? (w.kind == Quant::Int8 ? 0.63 : 0.5) * w.N * static_cast<double>(w.K)
+                                                          : static_cast<double>(w.data_bytes());
     const double skinny = w.data_tiled
-                              ? 5.0 + static_cast<double>(w.data_bytes()) / 3.8e6 * wave_form
+                              ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * wave_form
                               : 5.0 + static_cast<double>(w.data_bytes()) / 2.8e6 * (1.0 + 0.85 * (passes - 1));
+    if (M > 128) {
+        const int fmt = fmt_code(w.kind);
+        const double rows = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
+        const double blocks = tile_major(w) ? pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes) : rows;
+        if (skinny < blocks) return GemmPath::Skinny;
+        return blocks < rows ? GemmPath::Wide : GemmPath::Tiled;
+    }
     const int steps = w.K / 64;
-    const double tiles = static_cast<double>((w.N + 127) / 128) * (M <= 64 ? 1 : (M + 127) / 128);
+    const double tiles = static_cast<double>((w.N + 127) / 128);
     const double tiled = 2.0 + steps * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, tiles / 512.0);
     double split = 1e30;
-    const size_t need = M <= 128 ? pie_hip_gemm_mfma_workspace_bytes(M, w.N, w.K) : 0;
+    const size_t need = pie_hip_gemm_mfma_workspace_bytes(M, w.N, w.K);
     if (need && need <= ws_bytes) {
         const int shares = static_cast<int>(need / (static_cast<size_t>(M) * w.N * sizeof(float)));
         const int per = (steps + shares - 1) / shares;
@@ -89,7 +104,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
 }
 
 // The fitted cost model's kernel for M rows of `w`: 0 GEMV, 1 skinny GEMM, 2 tiled GEMM, 3 tiled GEMM
-// in K shares.  Two to four rows: the GEMV pays its dot products once per row, the skinny GEMM over
+// in K shares, 4 tiled GEMM over the tile-major copy.  Two to four rows: the GEMV pays its dot products once per row, the skinny GEMM over
 // the tile-major copy does not but needs the norm as its own launch (~4.8 us).  Costs fitted to
 // the 8B shapes decide (decode steps of 2 / 3 / 4 rows over 512-token contexts: 1.91 / 2.46 /
 // 2.79 ms with the GEMV everywhere, 2.01 / 2.08 / 2.14 ms with the skinny GEMM everywhere);
@@ -103,7 +118,7 @@ int model_route(const Linear& w, int M, bool has_norm, size_t ws_bytes) {
         if (t_gemv <= t_skinny) return 0;
     }
     const GemmPath p = pick_gemm(w, M, ws_bytes);
-    return p == GemmPath::Skinny ? 1 : p == GemmPath::Tiled ? 2 : 3;
+    return p == GemmPath::Skinny ? 1 : p == GemmPath::Tiled ? 2 : p == GemmPath::TiledSplitK ? 3 : 4;
 }
 
 // (PIE_GEMV_MAX_ROWS = n: rows up to n take the GEMV, more the skinny GEMM, whatever the costs say)
@@ -165,11 +180,18 @@ bool linear_fused(const Linear& w, const uint16_t* act, const uint16_t* norm_w, 
         const GemmPath path = tuned == 1   ? GemmPath::Skinny
                               : tuned == 2 ? GemmPath::Tiled
                               : tuned == 3 ? GemmPath::TiledSplitK
+                              : tuned == 4 ? GemmPath::Wide
                                            : pick_gemm(w, M, gemm_ws_bytes);   // (forced row limit, GEMV refusal)
+        if (path == GemmPath::Wide) {
+            const int sw = pie_hip_gemm_mfma_tiled(fmt, a, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, sbf, w.group, y, M,
+                                                   w.N, w.K, beta, swiglu, glu, gemm_ws, gemm_ws_bytes, s);
+            if (sw == PIE_HIP_OK) return true;
+            if (sw != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sw);
+        }
         if (path != GemmPath::Skinny) {
             // the tiled GEMM (weights dequantised to bf16 while staged), in K shares for a
             // decode batch whose output has few tiles
-            const bool split = path == GemmPath::TiledSplitK;
+            const bool split = path == GemmPath::TiledSplitK || M > 128;
             const int sg = pie_hip_gemm_mfma_glu(fmt, a, w.data, w.scale, sbf, w.group, y, M, w.N, w.K, beta, swiglu, glu,
                                                  split ? gemm_ws : nullptr, split ? gemm_ws_bytes : 0, s);
             if (sg == PIE_HIP_OK) return true;
@@ -285,13 +307,15 @@ void Executor::alloc_uniform() {
         for (size_t i = 0; i < T; ++i) iota[i] = static_cast<int64_t>(i);
         PIE_HIP_CHECK(hipMemcpy(iota_slots_, iota.data(), T * sizeof(int64_t), hipMemcpyHostToDevice));
     }
-    // fp32 partials of the split-K GEMM for decode batches of up to 128 rows (dense layers)
+    // fp32 partials of the split-K GEMM for decode batches of up to 128 rows (dense layers); prompts' K shares are at most two
+    // planes of 2048 x 4096
     if (!model_.layers.empty()) {
         const LayerWeights& l0 = model_.layers[0];
         for (const Linear* w : {&l0.wqkv, &l0.wo, &l0.wgu, &l0.wdown})
             for (int rows : {64, 128})
                 if (w->data && w->K % 64 == 0)
                     gemm_ws_bytes_ = std::max(gemm_ws_bytes_, pie_hip_gemm_mfma_workspace_bytes(rows, w->N, w->K));
+        if (T > 128) gemm_ws_bytes_ = size_t(64) << 20;
         gemm_ws_bytes_ = std::min<size_t>(gemm_ws_bytes_, size_t(64) << 20);
         if (gemm_ws_bytes_) PIE_HIP_CHECK(hipMalloc(&gemm_ws_, gemm_ws_bytes_));
     }

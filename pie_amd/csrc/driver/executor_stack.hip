@@ -159,6 +159,7 @@ void Executor::alloc_stack() {
             for (int rows : {64, 128})
                 if (!m.f32() && w->data && w->K % 64 == 0)
                     gemm_ws_bytes_ = std::max(gemm_ws_bytes_, pie_hip_gemm_mfma_workspace_bytes(rows, w->N, w->K));
+    if (T > 128 && gemm_ws_bytes_) gemm_ws_bytes_ = size_t(64) << 20;
     gemm_ws_bytes_ = std::min<size_t>(gemm_ws_bytes_, size_t(64) << 20);
     if (gemm_ws_bytes_) PIE_HIP_CHECK(hipMalloc(&gemm_ws_, gemm_ws_bytes_));
     // partial results of the attentions' splits: a plan with more than one split has at most 512 (tile,

@@ -30,7 +30,7 @@
 // blocks are numbered through all problems, no problem's rows share a block with another's — and gathers
 // its activation rows; bf16 weights may be in the tile-major order of the skinny kernels, of which a transfer
 // takes the same 16-byte granules from other places.
-#include "common.hip.h"
+#include "gemm_args.hip.h"
 
 #include <type_traits>
 
@@ -47,23 +47,6 @@ constexpr int kStages = 3;
 constexpr int kMaxMT = 8;   // 16-row activation tiles per wave, at most
 
 #define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
-
-struct GemmArgs {
-    const uint16_t* act;
-    const unsigned char* w;
-    const unsigned char* scale;
-    uint16_t* y;
-    int M, N, K, g_shift, beta, swiglu, scale_is_bf16;
-    int pointwise;        // PIE_HIP_EPI_RELU2 and above: applied to the sum (0: nothing)
-    PieHipGlu glu = kPlainGlu;   // swiglu
-    float* partial;   // split-K: fp32 [gridDim.z][M][N] partial sums (row scale applied), else null
-    // grouped: rows offsets[p] .. offsets[p + 1] of y belong to problem p (of `problems`), whose weights (scales)
-    // start w_stride (scale_stride) bytes after the one before; act_rows: the activation row of each (null: the same row)
-    const int32_t* offsets;
-    const int32_t* act_rows;
-    size_t w_stride, scale_stride;
-    int problems, tiled;
-};
 
 // The problem and the rows [m0, m1) of block row `t` when problems are cut into blocks of `rows` rows one after
 // another; false behind the last.  Every lane of the wave calls it and gets the same answer.
@@ -581,6 +564,11 @@ int gemm_entry(int format, const uint16_t* act_bf16, const void* weight, const v
         if (group_size < 32 || (group_size & (group_size - 1)) != 0 || K % group_size != 0)
             return PIE_HIP_ERR_UNSUPPORTED;
         a.g_shift = __builtin_ctz(static_cast<unsigned>(group_size));
+    }
+    // prompts over bf16 weights: the wide form where it is the faster one
+    if (format == PIE_HIP_FMT_BF16 && M > 128 && gemm_wide_us(format, M, N, K, 0, workspace ? workspace_bytes : 0) < gemm_tiles_us(format, M, N, K)) {
+        const int sw = launch_gemm_wide(format, a, 0, workspace, workspace_bytes, st);
+        if (sw != PIE_HIP_ERR_UNSUPPORTED) return sw;   // (activations or weights off a 16-byte boundary)
     }
     const int splits = workspace ? splitk_shares(M, N, K) : 1;
     if (splits > 1) {

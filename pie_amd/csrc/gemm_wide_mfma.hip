@@ -1,0 +1,599 @@
+// Tiled weight-only GEMM for prompts: y[M, N] = epilogue( act[M, K] · W[N, K]^T ), the same contract and rounding as
+// the kernel of gemm_mfma.hip, in blocks of 256 rows x 256 (or 128) columns.
+//
+// The tiles of gemm_mfma.hip (four waves to a SIMD pair, each reading operands, decoding and multiplying in turn) kept the
+// matrix pipe busy for less than half the time: a wave issues a vector instruction every eight cycles, the decoding of
+// int4 weights takes as many of those as half the MFMAs' time, and every step ended in a wait for all transfers.  Here:
+//   - eight waves, two to a SIMD, the second four one barrier behind the first: one wave's operand reads and transfers run
+//     beside the other's MFMAs; a wave's tile of 128 x 64 needs 24 reads of 16 bytes per 64 MFMAs;
+//   - the weights are the MFMAs' first operand, so that a lane ends with four neighbouring columns and stores 8 bytes;
+//   - weights are decoded between the MFMAs, one vector per phase, from the tile-major copy;
+//   - transfers into LDS run one to two steps ahead and no wait drains them;
+//   - a chiplet's blocks are neighbours (the row blocks of a column block share its weights in one L2).
+// What bounds it now: at 256 columns the matrix pipe and the decoding that shares its issue slots (int4: 1.4 us a step of 64
+// k-values for a block alone, 1.6 with the chip full, where the MFMAs take 0.9 at 2.4 GHz), at 128 the LDS reads.
+// Before / after, us (int4, fp8, bf16):
+//   2048 x 28672 x 4096   546 / 436,  519 / 425,  476 / 410      2048 x 4096 x 14336   245 / 214,  231 / 201,  202 / 190
+//   1024 x 28672 x 4096   302 / 229,  275 / 224,  295 / 206       489 x 4096 x 14336    84 /  71,   93 /  68,   97 /  64
+//   1319 x 16384 x 2048   125 / 110,  119 / 109,  114 /  98      1024 x 6144 x 4096     71 /  61,   70 /  59,   60 /  53
+// (the fourth in K shares; int4 and fp8 there against the skinny GEMM).
+#include "gemm_args.hip.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace pie_hip {
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
+constexpr int kRows = 256, kStepK = 64, kWaves = 8;
+constexpr int kActVecs = kRows * kStepK / 8;   // 16-byte vectors of an activation stage
+
+#define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
+// s_waitcnt lgkmcnt(0) alone and vmcnt(n) alone, n < 16 (gfx9 encoding).  The no-op keeps the compiler's own wait for a
+// value loaded before from being merged into this one: merged, it counts transfers into LDS as unordered and waits for all.
+#define PIE_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
+#define PIE_WAIT_VM(n)                              \
+    do {                                            \
+        __builtin_amdgcn_sched_barrier(0);          \
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (n));   \
+        asm volatile("s_nop 0");                    \
+        __builtin_amdgcn_sched_barrier(0);          \
+    } while (0)
+
+// ---- what a thread stages of a step's weights: V (32 or 16) of them, loaded from the tile-major copy (blocks of 1 KiB, 16 rows
+// by 64 bytes, lane 16 q + j its bytes 16 q .. 16 q + 15 of row j), as V / 8 16-byte vectors of bf16; wave w takes the
+// tiles of 16 rows from w V / 16 on.  (Row-major, a wave's load touches 32 rows' cache lines for 32 bytes each and took
+// the address unit longer than the MFMAs of a phase.) -----------------------------------------------------------------
+template <int V>
+struct WInt4T {   // a block is 128 values deep, a step half of it
+    static constexpr bool kDirect = false, kRowScale = false;
+    static constexpr int kLoads = 2, kDepth = 128;
+    struct Raw {
+        uint32_t v[V / 8];
+        uint16_t gs;
+    };
+    static __device__ __forceinline__ int tile(int wv, int lane, int) { return V == 32 ? 2 * wv + (lane >> 5) : wv; }
+    static __device__ __forceinline__ int granule(int lane, int v) { return V == 32 ? ((lane >> 4) & 1) * 4 + v : (lane >> 4) * 2 + v; }
+    // bytes of the thread's first value in a step's half block, of its row's first scale
+    static __device__ __forceinline__ uint32_t offset(int lane) {
+        return V == 32 ? (lane & 31) * 16 : ((lane >> 5) * 16 + (lane & 15)) * 16 + ((lane >> 4) & 1) * 8;
+    }
+    static __device__ __forceinline__ Raw load(const GemmArgs& a, const uint32_t* first, uint32_t scales, int k) {
+        Raw r;
+        const unsigned char* p = a.w + static_cast<size_t>(k >> 7) * 1024 + ((k >> 6) & 1) * 512 + first[0];
+        if constexpr (V == 32) {
+            const u32x4_t t = *reinterpret_cast<const u32x4_t*>(p);
+            r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
+        } else {
+            const u32x2_t t = *reinterpret_cast<const u32x2_t*>(p);
+            r.v[0] = t.x; r.v[1] = t.y;
+        }
+        r.gs = *reinterpret_cast<const uint16_t*>(a.scale + static_cast<size_t>(k >> a.g_shift) * 32 + scales);
+        return r;
+    }
+    // (nibble - 8) * scale: the even nibbles become the fp16 pairs 1024 + n, the odd ones (where they are) 1024 + 16 n, and
+    // one mixed-precision fma takes a half straight to the fp32 product.  Exact in fp32, so one rounding to bf16.  (A word's
+    // pairs are its codes in order, see pie_hip_repack_mfma_tiles_int4.)
+    static __device__ __forceinline__ u32x4_t decode(const Raw& r, int s, uint32_t k1024) {
+        const float gs = bf16_bits_to_f32(r.gs);
+        const float scale[2] = {gs, 0.0625f * gs}, off[2] = {-1032.f * gs, -72.f * gs};
+        u32x4_t o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f16x2_t pr = __builtin_bit_cast(f16x2_t, and_or(j < 2 ? r.v[s] : r.v[s] >> 8, j & 1 ? 0x00F000F0u : 0x000F000Fu, k1024));
+            o[j] = pack_bf16x2(fmaf(static_cast<float>(pr.x), scale[j & 1], off[j & 1]), fmaf(static_cast<float>(pr.y), scale[j & 1], off[j & 1]));
+        }
+        return o;
+    }
+};
+template <int V, int KVF>
+struct WByteT {   // a block is a step deep
+    static constexpr bool kDirect = false, kRowScale = true;
+    static constexpr int kLoads = V / 16, kDepth = 64;
+    struct Raw {
+        u32x4_t v[V / 16];
+    };
+    static __device__ __forceinline__ int tile(int wv, int, int v) { return V == 32 ? 2 * wv + (v >> 1) : wv; }
+    static __device__ __forceinline__ int granule(int lane, int v) { return (lane >> 4) * 2 + (v & 1); }
+    static __device__ __forceinline__ uint32_t offset(int lane) { return lane * 16; }
+    static __device__ __forceinline__ Raw load(const GemmArgs& a, const uint32_t* first, uint32_t, int k) {
+        Raw r;
+#pragma unroll
+        for (int i = 0; i < V / 16; ++i) r.v[i] = *reinterpret_cast<const u32x4_t*>(a.w + static_cast<size_t>(k >> 6) * 1024 + first[i]);
+        return r;
+    }
+    static __device__ __forceinline__ u32x4_t decode(const Raw& r, int s, uint32_t) {
+        return kv_decode_bf16<KVF>(u32x2_t{r.v[s >> 1][2 * (s & 1)], r.v[s >> 1][2 * (s & 1) + 1]});
+    }
+};
+struct WBf16T {   // row-major, moved without registers
+    static constexpr bool kDirect = true, kRowScale = false;
+    static constexpr int kLoads = 0, kDepth = 64;
+    struct Raw {};
+    static __device__ __forceinline__ int tile(int, int, int) { return 0; }
+    static __device__ __forceinline__ int granule(int, int) { return 0; }
+    static __device__ __forceinline__ uint32_t offset(int) { return 0; }
+    static __device__ __forceinline__ Raw load(const GemmArgs&, const uint32_t*, uint32_t, int) { return {}; }
+    static __device__ __forceinline__ u32x4_t decode(const Raw&, int, uint32_t) { return u32x4_t{0u, 0u, 0u, 0u}; }
+};
+struct WInt4 {
+    template <int V> using Staged = WInt4T<V>;
+};
+struct WFp8 {
+    template <int V> using Staged = WByteT<V, kKvFp8>;
+};
+struct WInt8 {
+    template <int V> using Staged = WByteT<V, kKvInt8>;
+};
+struct WBf16 {
+    template <int V> using Staged = WBf16T;
+};
+
+// position of granule g of tile row r (in 16-byte vectors)
+__device__ __forceinline__ int swz(int r, int g) { return r * 8 + (g ^ ((r >> 1) & 7)); }
+
+// The epilogue of row m, columns n .. n + 3 (those below N; n is a multiple of 4): SwiGLU over (gate, up) pairs rounded to
+// bf16 first, or a pointwise function and the residual.
+__device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, float* v) {
+    const int N = a.N, nout = a.swiglu ? N / 2 : N;
+    const bool whole = N % 4 == 0 && a.aligned;   // one 8- (SwiGLU: 4-) byte store
+    if (a.swiglu) {
+        uint16_t o[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            float g = v[2 * r], u = v[2 * r + 1];
+            if (a.glu.bias) {
+                g += a.glu.bias[min(n + 2 * r, N - 1)];
+                u += a.glu.bias[min(n + 2 * r + 1, N - 1)];
+            }
+            g = bf16_bits_to_f32(f32_to_bf16_bits(g));
+            u = bf16_bits_to_f32(f32_to_bf16_bits(u));
+            o[r] = f32_to_bf16_bits(glu_value(g, u, a.glu));
+        }
+        uint16_t* p = a.y + static_cast<size_t>(m) * nout + n / 2;
+        if (whole) {
+            *reinterpret_cast<uint32_t*>(p) = o[0] | static_cast<uint32_t>(o[1]) << 16;
+        } else {
+            p[0] = o[0];
+            if (n + 2 < N) p[1] = o[1];
+        }
+        return;
+    }
+    uint16_t* p = a.y + static_cast<size_t>(m) * nout + n;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = epilogue_pointwise<true>(v[r], a.pointwise);
+    if (whole) {
+        if (a.beta) {
+            const u32x2_t old = *reinterpret_cast<const u32x2_t*>(p);
+            v[0] += bf16_lo(old.x);
+            v[1] += bf16_hi(old.x);
+            v[2] += bf16_lo(old.y);
+            v[3] += bf16_hi(old.y);
+        }
+        *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else {
+        for (int r = 0; r < 4 && n + r < N; ++r) {
+            if (a.beta) v[r] += bf16_bits_to_f32(p[r]);
+            p[r] = f32_to_bf16_bits(v[r]);
+        }
+    }
+}
+
+template <class FMT, int COLS>
+struct Wide {
+    static constexpr int kVals = COLS / 8;          // weights a thread stages per step
+    using F = typename FMT::template Staged<kVals>;
+    static constexpr int kAH = COLS / 128;          // halves of 64 rows of a wave's tile: 128 x 64 or 64 x 64 outputs
+    static constexpr int kWn = COLS / 64;           // waves along the columns
+    static constexpr int kStages = COLS == 256 ? 2 : 3;
+    static constexpr int kColVecs = COLS * kStepK / 8;
+    static constexpr int kColStages = kStages;
+    static constexpr size_t kSmem = (static_cast<size_t>(kStages) * kActVecs + static_cast<size_t>(kColStages) * kColVecs) * 16;
+};
+
+template <class FMT, int COLS>
+__global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmArgs a, int first_col, int row_blocks, int per_xcd, int tiles) {
+    using W = Wide<FMT, COLS>;
+    using F = typename W::F;
+    constexpr int AH = W::kAH, S = W::kStages;
+    extern __shared__ __align__(16) unsigned char smem[];
+    u32x4_t* lds_a = reinterpret_cast<u32x4_t*>(smem);
+    u32x4_t* lds_b = lds_a + S * kActVecs;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int j = lane & 15, q = lane >> 4;
+    const int wm = wv / W::kWn, wn = wv % W::kWn;
+    // blocks go to the XCDs in turn: each XCD's are neighbours, the row blocks of a column block side by side
+    const int tile = static_cast<int>(blockIdx.x & 7) * per_xcd + static_cast<int>(blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int m0 = tile % row_blocks * kRows, n0 = first_col + tile / row_blocks * COLS;
+    const int M = a.M, N = a.N, K = a.K;
+    const int nk_all = K / kStepK;
+    const int per_split = (nk_all + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
+    const int kbeg = blockIdx.z * per_split;
+    const int nk = min(per_split, nk_all - kbeg);
+
+    // direct transfers: a chunk (1 KiB) is eight tile rows; lane p lands at position p of it, which holds granule
+    // (p % 8) ^ key(row).  With 256 columns a tile's rows move in halves, those that a wave's phases read together: activations
+    // 0 - 63 and 64 - 127 of either half of the waves, columns 0 - 31 and 32 - 63 of every wave's 64.
+    constexpr int AC = 4, BC = F::kDirect ? COLS / 64 : 0;   // chunks per wave
+    uint32_t aoff[4], boff[4];   // bytes (the launcher checked that they fit); half h, chunk u at 2h + u
+    int arow[4], brow[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        arow[u] = AH == 2 ? (u & 1) * 128 + (u >> 1) * 64 + wv * 8 : (u * kWaves + wv) * 8;
+        brow[u] = AH == 2 ? ((u & 1) * 2 + (wv >> 2)) * 64 + (u >> 1) * 32 + (wv & 3) * 8 : (u * kWaves + wv) * 8;
+        const int ar = arow[u] + (lane >> 3), br = brow[u] + (lane >> 3);
+        aoff[u] = static_cast<uint32_t>(min(m0 + ar, M - 1)) * (2u * K) + ((lane & 7) ^ ((ar >> 1) & 7)) * 16;
+        if (u < BC) boff[u] = static_cast<uint32_t>(min(n0 + br, N - 1)) * (2u * K) + ((lane & 7) ^ ((br >> 1) & 7)) * 16;
+    }
+    // chunks [u0, u1) of step kt's activations (bf16 weights)
+    auto issue_a = [&](int kt, int stage, int u0, int u1) {
+        const unsigned char* p = reinterpret_cast<const unsigned char*>(a.act) + static_cast<size_t>(kbeg + min(kt, nk - 1)) * (kStepK * 2);
+#pragma unroll
+        for (int u = u0; u < u1; ++u)
+            __builtin_amdgcn_global_load_lds(p + aoff[u], PIE_LDS_PTR(lds_a + stage * kActVecs + arow[u] * 8), 16, 0, 0);
+    };
+    auto issue_b = [&](int kt, int stage, int u0, int u1) {
+        const unsigned char* p = a.w + static_cast<size_t>(kbeg + min(kt, nk - 1)) * (kStepK * 2);
+#pragma unroll
+        for (int u = u0; u < u1 && u < BC; ++u)
+            __builtin_amdgcn_global_load_lds(p + boff[u], PIE_LDS_PTR(lds_b + stage * W::kColVecs + brow[u] * 8), 16, 0, 0);
+    };
+    // quantised weights: the thread's tiles (at most two) in bytes of the first block, its rows' scales
+    constexpr int VPT = W::kVals / 8;   // 16-byte vectors of bf16
+    uint32_t w_first[2], s_first = 0;
+    if constexpr (!F::kDirect) {
+        const int last = (N + 15) / 16 - 1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            w_first[i] = static_cast<uint32_t>(min(n0 / 16 + F::tile(wv, lane, 2 * i), last)) * (K / F::kDepth * 1024u) + F::offset(lane);
+        s_first = (static_cast<uint32_t>(min(n0 / 16 + F::tile(wv, lane, 0), last)) * (K >> a.g_shift) * 16u + j) * 2u;
+    }
+    auto load_w = [&](int kt) { return F::load(a, w_first, s_first, (kbeg + min(kt, nk - 1)) * kStepK); };
+
+    uint32_t magic = 0x64006400u;   // (1024, 1024) as an fp16 pair, opaque to the compiler
+    asm volatile("" : "+v"(magic));
+    auto store_w = [&](const typename F::Raw& r, int stage, int v) {
+        if constexpr (!F::kDirect) lds_b[stage * W::kColVecs + swz(F::tile(wv, lane, v) * 16 + j, F::granule(lane, v))] = F::decode(r, v, magic);
+    };
+
+    f32x4_t acc[4 * AH][4];
+#pragma unroll
+    for (int t = 0; t < 4 * AH; ++t)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) acc[t][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    // quantised weights: registers hold S steps, which are decoded one vector per phase
+    typename F::Raw rr[S];
+#define PIE_FENCE() __builtin_amdgcn_sched_barrier(0)
+#define PIE_MEET()                         \
+    do {                                   \
+        PIE_FENCE();                       \
+        asm volatile("" ::: "memory");     \
+        __builtin_amdgcn_s_barrier();      \
+        asm volatile("" ::: "memory");     \
+        PIE_FENCE();                       \
+    } while (0)
+#pragma unroll
+    for (int i = 0; i < S; ++i) rr[i] = load_w(i);
+    PIE_FENCE();
+    issue_a(0, 0, 0, 4);
+    issue_b(0, 0, 0, 4);
+    issue_a(1, 1, 0, AH == 2 ? 2 : 4);   // (in steady state a step's transfers begin in the second step before it)
+    issue_b(1, 1, 0, 4);
+    PIE_FENCE();
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) store_w(rr[0], 0, v);
+    PIE_FENCE();
+    rr[0] = load_w(S);
+    store_w(rr[1], 1, 0);
+    if constexpr (F::kDirect) PIE_WAIT_VM(AC / AH + BC);
+    else PIE_WAIT_VM(0);
+    PIE_WAIT_LGKM0();
+    PIE_MEET();
+    if (wv >= kWaves / 2) PIE_MEET();
+
+    bf16x8_t af[2][4], bf[2][2][2];   // [k half][row tile], [column half][k half][column tile]
+    const int key = j >> 1;
+    // (the operands of a phase's first eight MFMAs first: they start when those have arrived)
+    auto read_ab = [&](int a_stage, int a_half, int b_stage, int b_half) {   // a half of -1: not read
+        const u32x4_t* A = lds_a + a_stage * kActVecs + (wm * 64 * AH + max(a_half, 0) * 64 + j) * 8;
+        const u32x4_t* B = lds_b + b_stage * W::kColVecs + (wn * 64 + max(b_half, 0) * 32 + j) * 8;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int at = (ks * 4 + q) ^ key;
+            if (b_half >= 0) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) bf[b_half][ks][t] = __builtin_bit_cast(bf16x8_t, B[t * 128 + at]);
+            }
+            if (a_half >= 0) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) af[ks][t] = __builtin_bit_cast(bf16x8_t, A[t * 128 + at]);
+            }
+            PIE_FENCE();
+        }
+    };
+    // A phase's MFMAs.  Between them the wave decodes one vector of the weights `r` into the tile `w_stage`: a wave issues a
+    // vector instruction every eight cycles and an MFMA keeps the matrix pipe for sixteen, so one decode instruction behind
+    // each is free, while in the memory part the same instructions outlast the other wave's MFMAs.
+    auto multiply = [&](int ah, int bh, const typename F::Raw& r, int w_stage, int v) {
+        PIE_MEET();
+        __builtin_amdgcn_s_setprio(1);
+        store_w(r, w_stage, v);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+                    acc[ah * 4 + t][bh * 2 + n] =
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[bh][ks][n], af[ks][t], acc[ah * 4 + t][bh * 2 + n], 0, 0, 0);
+        if constexpr (!F::kDirect) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        PIE_MEET();
+    };
+    // One step of 64 k-values; `stage` = kt % S.  A step is 2 AH phases, each a memory part (operand reads, loads ahead) and
+    // 16 MFMAs, with a barrier behind either; the waves of the second half are one barrier behind, so that on every SIMD one
+    // wave's memory part runs beside the other's MFMAs.
+    // What a phase reads is overwritten no earlier than two phases later, when the waves behind have waited for their reads
+    // too, and what it reads was waited for by all waves a phase before; every wait leaves the transfers issued
+    // since in flight.  A step's weights are decoded from the last phase of the second step before it on.
+    constexpr int HA = 2, HB = F::kDirect ? 2 : 0, L = F::kLoads;   // vector-memory operations of a half tile, of the weights
+    auto step = [&](auto slot, int kt) {
+        constexpr int stage = decltype(slot)::value, next = (stage + 1) % S, after = (stage + 2) % S;
+        if constexpr (AH == 2) {
+            read_ab(stage, 0, stage, 0);
+            issue_a(kt + 1, next, 2, 4);
+            if constexpr (F::kDirect) PIE_WAIT_VM(2 * HA + 3 * HB);   // this step's second column half has landed
+            multiply(0, 0, rr[next], next, 1);
+            read_ab(0, -1, stage, 1);
+            PIE_WAIT_VM(2 * HA + 2 * HB + L);                         // and its second half of the rows
+            multiply(0, 1, rr[next], next, 2);
+            read_ab(stage, 1, 0, -1);
+            issue_a(kt + 2, stage, 0, 2);
+            issue_b(kt + 2, stage, 0, 2);
+            multiply(1, 1, rr[next], next, 3);
+            issue_b(kt + 2, stage, 2, 4);
+            PIE_WAIT_VM(2 * HA + 3 * HB);                             // step kt + 1's first halves, step kt + 2's weights
+            rr[next] = load_w(kt + 3);
+            PIE_WAIT_LGKM0();
+            multiply(1, 0, rr[stage], stage, 0);
+        } else {
+            read_ab(stage, 0, stage, 0);
+            issue_a(kt + 2, after, 0, 4);   // (last read in step kt - 1)
+            issue_b(kt + 2, after, 0, 4);
+            multiply(0, 0, rr[next], next, 1);
+            read_ab(0, -1, stage, 1);
+            PIE_WAIT_VM(AC + BC + L);   // step kt + 1's transfers
+            rr[next] = load_w(kt + 4);
+            PIE_WAIT_LGKM0();
+            multiply(0, 1, rr[after], after, 0);
+        }
+    };
+    int kt = 0;
+    for (; kt + S <= nk; kt += S) {
+        step(std::integral_constant<int, 0>{}, kt);
+        step(std::integral_constant<int, 1>{}, kt + 1);
+        if constexpr (S == 3) step(std::integral_constant<int, 2>{}, kt + 2);
+    }
+    if (kt < nk) step(std::integral_constant<int, 0>{}, kt);
+    if (S == 3 && kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
+    if (wv < kWaves / 2) PIE_MEET();
+    __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the block ends)
+
+    // ---- epilogue: a lane holds four neighbouring columns of one row per tile ----
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        const int n = n0 + wn * 64 + nt * 16 + 4 * q;
+        if (n >= N) continue;
+        float rs[4];
+        if constexpr (F::kRowScale) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int c = min(n + r, N - 1);
+                rs[r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[c])
+                                        : reinterpret_cast<const float*>(a.scale)[c];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4 * AH; ++t) {
+            const int m = m0 + wm * 64 * AH + t * 16 + j;
+            if (m >= M) continue;
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = F::kRowScale ? acc[t][nt][r] * rs[r] : acc[t][nt][r];
+            if (a.partial) {
+                float* p = a.partial + (static_cast<size_t>(blockIdx.z) * M + m) * N + n;
+                if (N % 4 == 0) *reinterpret_cast<f32x4_t*>(p) = f32x4_t{v[0], v[1], v[2], v[3]};
+                else
+                    for (int r = 0; r < 4 && n + r < N; ++r) p[r] = v[r];
+            } else {
+                wide_store(a, m, n, v);
+            }
+        }
+    }
+}
+
+// Sums the K shares' partials of four columns and applies the epilogue the kernel would have applied.
+__global__ __launch_bounds__(256) void wide_reduce_kernel(const GemmArgs a, int splits) {
+    const int N = a.N, quads = (N + 3) / 4;
+    const size_t idx = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= static_cast<size_t>(a.M) * quads) return;
+    const int m = static_cast<int>(idx / quads), n = static_cast<int>(idx % quads) * 4;
+    const size_t plane = static_cast<size_t>(a.M) * N;
+    const float* p = a.partial + static_cast<size_t>(m) * N + n;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < splits; ++z) {
+        if (N % 4 == 0) {
+            const f32x4_t t = *reinterpret_cast<const f32x4_t*>(p + z * plane);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += t[r];
+        } else {
+            for (int r = 0; r < 4 && n + r < N; ++r) v[r] += p[z * plane + r];
+        }
+    }
+    wide_store(a, m, n, v);
+}
+
+template <class F, int COLS>
+int launch(const GemmArgs& a, int first_col, int col_blocks, int splits, hipStream_t stream) {
+    using W = Wide<F, COLS>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<F, COLS>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(W::kSmem));
+    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+    const int rows = (a.M + kRows - 1) / kRows;
+    const int tiles = rows * col_blocks, per = (tiles + 7) / 8;
+    hipLaunchKernelGGL((gemm_wide_kernel<F, COLS>), dim3(8 * per, 1, splits), dim3(kWaves * kWave), W::kSmem, stream, a, first_col,
+                       rows, per, tiles);
+    return launch_status();
+}
+
+// What a launch takes, in microseconds: a round of up to one block per CU is `fixed` and, per step of 64 k-values, `step` for
+// a few blocks; `fixed_full` and `step_full` more when all 256 CUs have one (shared caches, stores, power), most of it only
+// when nearly all have.  Fitted to 160 - 4096 rows of 4096 x 14336, 28672 x 4096, 16384 x 2048 and 4096 x 4096 (within 7 %).
+struct Rate {
+    double fixed, step, fixed_full, step_full;
+};
+struct Rates {
+    Rate wide256, wide128;
+    double few, many, round, tall;   // the kernel of gemm_mfma.hip, per step: up to 256 blocks of 128 rows (few + many per
+                                     // 256), each 256 of more, each 256 blocks of 256 rows
+};
+constexpr Rates kRates[] = {
+    /* int4 */ {{14.0, 1.36, 8.0, 0.26}, {6.0, 0.76, 1.0, 0.15}, 0.58, 0.20, 0.64, 1.14},
+    /* int8 */ {{14.0, 1.31, 10.0, 0.22}, {7.0, 0.72, 2.0, 0.12}, 0.56, 0.20, 0.62, 1.10},
+    /* fp8 */ {{14.0, 1.31, 10.0, 0.20}, {7.0, 0.71, 2.0, 0.12}, 0.49, 0.17, 0.58, 1.08},
+    /* bf16 */ {{14.0, 0.90, 10.0, 0.43}, {6.0, 0.62, 1.0, 0.19}, 0.36, 0.21, 0.57, 0.98},
+};
+double launch_us(const Rate& r, long long blocks, int steps) {
+    const long long rounds = blocks / 256;
+    const double fill = static_cast<double>(blocks % 256) / 256.0, cube = fill * fill * fill;
+    return 3.0 + rounds * (r.fixed + r.fixed_full + steps * (r.step + r.step_full)) +
+           (fill > 0.0 ? r.fixed + cube * r.fixed_full + steps * (r.step + cube * r.step_full) : 0.0);
+}
+
+// How the wide form runs a shape: `first` blocks of 256 columns and the rest in blocks of 128, in `splits` shares of K.
+// Whole rounds of the larger block are the fastest; what is left over may fill the machine better in smaller ones (2048 rows of
+// 28672 columns: 896 blocks of 256 are 3.5 rounds, 457 us int4; 768 of them and 256 of 128 columns 437).  Few blocks over a long K run in shares that fill
+// one round, whose fp32 sums a second kernel adds in the order of K (160 rows of 4096 x 14336 int4: 32 blocks 175 us, in eight
+// shares 42).
+struct Plan {
+    int first = 0, splits = 1;
+    double us = 1e30;
+};
+Plan plan_of(const Rates& r, int M, int N, int K, size_t ws_bytes) {
+    const int rows = (M + kRows - 1) / kRows, steps = K / kStepK, c256 = (N + 255) / 256;
+    auto rest_of = [&](int first) { return (std::max(0, N - first * 256) + 127) / 128; };
+    Plan best;
+    const int whole = static_cast<int>(static_cast<long long>(rows) * c256 / 256 * 256 / rows);
+    for (int first : {0, whole, c256}) {
+        double us = 0.0;
+        if (first) us += launch_us(r.wide256, static_cast<long long>(rows) * first, steps);
+        if (rest_of(first)) us += launch_us(r.wide128, static_cast<long long>(rows) * rest_of(first), steps);
+        if (us < best.us) best = {first, 1, us};
+    }
+    const long long blocks = static_cast<long long>(rows) * rest_of(0);
+    for (int s = 2; s <= 8 && blocks * s <= 256 && steps / s >= 8; ++s) {
+        if (static_cast<long long>((steps + s - 1) / s) * (s - 1) + 4 > steps) continue;   // (the last share would be next to nothing)
+        const size_t bytes = static_cast<size_t>(s) * M * N * sizeof(float);
+        if (bytes > ws_bytes) break;
+        const double us = launch_us(r.wide128, blocks * s, (steps + s - 1) / s) + 3.0 + (0.9 * bytes + 2.0 * M * N) / 4e6;
+        if (us < best.us) best = {0, s, us};
+    }
+    return best;
+}
+bool fits(int format, int M, int N, int K, int group_size) {
+    if (K % (format == PIE_HIP_FMT_INT4B8 ? 128 : 64) != 0 || K < 4 * kStepK) return false;
+    if (format == PIE_HIP_FMT_INT4B8 && (group_size < 64 || (group_size & (group_size - 1)) != 0 || K % group_size != 0)) return false;
+    return 2ll * M * K <= 0xFFFFFFFFll && 2ll * (N + 15) * K <= 0xFFFFFFFFll && (M + 255ll) / 256 * ((N + 127ll) / 128) < 0x0FFFFFFF;
+}
+
+template <class F>
+int run(GemmArgs a, const Plan& p, float* ws, hipStream_t stream) {
+    int st = PIE_HIP_OK;
+    a.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+    if (p.splits > 1) a.partial = ws;
+    if (p.first) st = launch<F, 256>(a, 0, p.first, 1, stream);
+    const int rest = (std::max(0, a.N - p.first * 256) + 127) / 128;
+    if (st == PIE_HIP_OK && rest) st = launch<F, 128>(a, p.first * 256, rest, p.splits, stream);
+    if (st != PIE_HIP_OK || p.splits == 1) return st;
+    const size_t quads = static_cast<size_t>(a.M) * ((a.N + 3) / 4);
+    hipLaunchKernelGGL(wide_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, a, p.splits);
+    return launch_status();
+}
+
+}  // namespace
+
+double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
+    return fits(format, M, N, K, group_size) ? plan_of(kRates[format], M, N, K, ws_bytes).us : 1e30;
+}
+// (the choice between its two heights is launch_gemm's)
+double gemm_tiles_us(int format, int M, int N, int K) {
+    const Rates& r = kRates[format];
+    const long long cols = (N + 127) / 128, low = cols * ((M + 127) / 128), high = cols * ((M + 255) / 256);
+    const long long low_rounds = (low + 255) / 256, high_rounds = (high + 255) / 256;
+    const double steps = K / kStepK;
+    if (1.85 * static_cast<double>(high_rounds) < static_cast<double>(low_rounds)) return high_rounds * (5.0 + steps * r.tall);
+    return 5.0 + steps * (low <= 256 ? r.few + r.many * static_cast<double>(low) / 256.0 : r.round * static_cast<double>(low_rounds));
+}
+
+int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {
+    if (!fits(format, a.M, a.N, a.K, group_size) || reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16)
+        return PIE_HIP_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(ws) % 16) ws = nullptr;
+    const Plan p = plan_of(kRates[format], a.M, a.N, a.K, ws ? ws_bytes : 0);
+    switch (format) {
+        case PIE_HIP_FMT_INT4B8: return run<WInt4>(a, p, static_cast<float*>(ws), stream);
+        case PIE_HIP_FMT_INT8: return run<WInt8>(a, p, static_cast<float*>(ws), stream);
+        case PIE_HIP_FMT_FP8: return run<WFp8>(a, p, static_cast<float*>(ws), stream);
+        case PIE_HIP_FMT_BF16: return run<WBf16>(a, p, static_cast<float*>(ws), stream);
+        default: return PIE_HIP_ERR_INVALID;
+    }
+}
+
+}  // namespace pie_hip
+
+extern "C" float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes) {
+    if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return 1e30f;
+    const double tiles = pie_hip::gemm_tiles_us(format, M, N, K);
+    const double wide = tiled || format == PIE_HIP_FMT_BF16 ? pie_hip::gemm_wide_us(format, M, N, K, group_size, workspace_bytes) : 1e30;
+    return static_cast<float>(std::min(tiles, wide));
+}
+
+extern "C" int pie_hip_gemm_mfma_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale, int scale_is_bf16,
+                                       int group_size, uint16_t* y_bf16, int M, int N, int K, int beta, int epilogue,
+                                       const PieHipGlu* glu, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace pie_hip;
+    if (!glu_ok(glu, epilogue)) return PIE_HIP_ERR_INVALID;
+    if (!act_bf16 || !weight || !y_bf16 || M <= 0 || N <= 0 || K <= 0) return PIE_HIP_ERR_INVALID;
+    if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || (format != PIE_HIP_FMT_BF16 && !scale)) return PIE_HIP_ERR_INVALID;
+    const int pointwise = pointwise_code(epilogue), swiglu = epilogue == PIE_HIP_EPI_SWIGLU ? 1 : 0;
+    if ((swiglu && N % 2 != 0) || ((swiglu || pointwise) && beta)) return PIE_HIP_ERR_INVALID;
+    if (format != PIE_HIP_FMT_BF16 && N % 16 != 0) return PIE_HIP_ERR_UNSUPPORTED;   // (there is no tile-major copy)
+    GemmArgs a{};
+    a.act = act_bf16;
+    a.w = static_cast<const unsigned char*>(weight);
+    a.scale = static_cast<const unsigned char*>(scale);
+    a.y = y_bf16;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.beta = beta;
+    a.swiglu = swiglu;
+    a.pointwise = pointwise;
+    if (glu) a.glu = *glu;
+    a.scale_is_bf16 = scale_is_bf16;
+    if (format == PIE_HIP_FMT_INT4B8 && group_size > 0) a.g_shift = __builtin_ctz(static_cast<unsigned>(group_size));
+    return launch_gemm_wide(format, a, group_size, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}

@@ -606,6 +606,38 @@ def gemm_mfma(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None
     return y
 
 
+def gemm_mfma_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
+                    rule: Optional[Glu] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The GEMM of prompts in blocks of 256 rows, over a row-major bf16 weight or a tile-major quantised one
+    (`repack_mfma_tiles`); with a workspace few blocks over a long K run in shares of K."""
+    _dev(act, torch.bfloat16, "act")
+    M, K = act.shape
+    kind = w.kind.removesuffix("+tiled")
+    if K != w.K or (kind == w.kind) != (kind == "bf16"):
+        raise KernelError("act K != weight K, or not the order the kernel reads")
+    n_out = w.N // 2 if epilogue == 1 else w.N
+    if y is None:
+        if beta:
+            raise KernelError("beta=1 needs an existing y")
+        y = torch.empty((M, n_out), dtype=torch.bfloat16, device=act.device)
+    _dev(y, torch.bfloat16, "y")
+    if tuple(y.shape) != (M, n_out):
+        raise KernelError("y shape mismatch")
+    scale_is_bf16 = int(w.scale is not None and w.scale.dtype == torch.bfloat16)
+    st = kernels().pie_hip_gemm_mfma_tiled(FMT[kind], _ptr(act), _ptr(w.data), _ptr(w.scale), scale_is_bf16, w.group_size, _ptr(y),
+                                           M, w.N, K, beta, epilogue, None if rule is None else C.byref(rule), _ptr(workspace),
+                                           C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream())
+    _check(st, "pie_hip_gemm_mfma_tiled")
+    return y
+
+
+def gemm_mfma_us(kind: str, M: int, N: int, K: int, group: int, tiled: bool, workspace_bytes: int = 0) -> float:
+    """Estimated microseconds of the tiled GEMMs over more than 128 rows."""
+    lib = kernels()
+    lib.pie_hip_gemm_mfma_us.restype = C.c_float
+    return float(lib.pie_hip_gemm_mfma_us(FMT[kind], M, N, K, group, int(tiled), C.c_size_t(workspace_bytes)))
+
+
 def gemm_mfma_workspace_bytes(M: int, N: int, K: int) -> int:
     lib = kernels()
     lib.pie_hip_gemm_mfma_workspace_bytes.restype = C.c_size_t

@@ -143,3 +143,88 @@ def test_gemm_split_k_beta_swiglu_one_hot(gpu, oracle, kind):
     fused = bits(ops.gemm_mfma(xg, wi, swiglu=True, split_k=True))
     unfused = bits(ops.swiglu_bf16(ops.gemm_mfma(xg, w, split_k=True)))
     assert np.array_equal(fused, unfused)
+
+
+# one row, the edges of the 256-row and 128-column blocks, step counts that leave 0 - 2 behind the unrolled loops, enough
+# blocks for 256 columns, whole rounds of those and a rest of 128 columns
+WIDE = [(1, 16, 256), (255, 144, 320), (257, 272, 448), (300, 16656, 256), (600, 23056, 384)]
+
+
+def wide_case(oracle, gpu, kind, M, N, K, seed):
+    import torch
+    from pie_amd import ops
+
+    K = (K + 127) // 128 * 128 if kind == "int4b8" else K
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    rng = np.random.default_rng(seed)
+    _, mk = make_weight(oracle, rng, kind, N, K, G=64 if K % 256 else 128)
+    w = mk(gpu)
+    return torch.randn(M, K, generator=g, device=gpu).to(torch.bfloat16), w, w if kind == "bf16" else ops.repack_mfma_tiles(w)
+
+
+def assert_near_exact(got, act, w, ref=None):
+    """bf16 rounding of a sum whose fp32 error is bounded by K terms' worth of half-ulps."""
+    import torch
+    x, wd = act.double(), w.data.reshape(w.N, w.K).double()
+    ref = x @ wd.T if ref is None else ref
+    assert torch.isfinite(got).all()
+    assert ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + w.K * 2.0 ** -23 * (x.abs() @ wd.abs().T)).all()
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("M,N,K", WIDE)
+def test_wide_blocks_equal_the_tiles(gpu, oracle, kind, M, N, K):
+    """Blocks of 256 rows: the same products summed in the same order as the 128-row tiles (bf16, which takes either by
+    its rule: the exact sums)."""
+    import torch
+    from pie_amd import ops
+
+    act, w, t = wide_case(oracle, gpu, kind, M, N, K, 700 + M)
+    got = ops.gemm_mfma_tiled(act, t)
+    if kind == "bf16":
+        assert_near_exact(got, act, w)
+        assert torch.equal(ops.gemm_mfma_tiled(act, w, y=torch.ones_like(got), beta=1),
+                           ops.gemm_mfma(act, w, y=torch.ones_like(got), beta=1))
+    else:
+        assert torch.equal(got, ops.gemm_mfma(act, w))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_wide_epilogues_and_shares(gpu, oracle, kind):
+    import torch
+    from pie_amd import ops
+
+    act, w, t = wide_case(oracle, gpu, kind, 257, 272, 2048, 720)
+    y0 = torch.randn(257, 272, device=gpu).to(torch.bfloat16)
+    ws = torch.empty(16 << 20, dtype=torch.uint8, device=gpu)
+    plain = ops.gemm_mfma(act, w)
+    assert torch.equal(ops.gemm_mfma_tiled(act, t), plain)
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, y=y0.clone(), beta=1), ops.gemm_mfma(act, w, y=y0.clone(), beta=1))
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=ops.GELU), ops.gemm_mfma(act, w, swiglu=ops.GELU))
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1), ops.gemm_mfma(act, w, swiglu=True))
+    if kind == "bf16":
+        bias = torch.randn(272, device=gpu)
+        rule = ops.glu(bias, 7.0, 1.702, 1.0)
+        assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1, rule=rule), ops.linear_glu("tiled", act, w.data, rule))
+    # in shares of K: at most a rounding apart from the sum in one piece (fp32 partials)
+    for beta in (0, 1):
+        ref = ops.gemm_mfma(act, w, y=y0.clone(), beta=1) if beta else plain
+        got = ops.gemm_mfma_tiled(act, t, y=y0.clone() if beta else None, beta=beta, workspace=ws)
+        assert (got.float() - ref.float()).abs().max() <= 2.0 ** -7 * float(ref.float().abs().max())
+        assert (got == ref).float().mean() > 0.98
+    pairs = ops.gemm_mfma_tiled(act, t, workspace=ws)   # (gate, up) columns side by side
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1, workspace=ws),
+                       ops.swiglu_bf16(torch.cat([pairs[:, 0::2], pairs[:, 1::2]], dim=1).contiguous()))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_wide_refusals(gpu, oracle, kind):
+    """Shapes the blocks do not take are refused, not misread."""
+    import torch
+    from pie_amd import ops
+
+    for M, N, K in [(256, 128, 192), (256, 128, 288)]:
+        act = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
+        _, mk = make_weight(oracle, np.random.default_rng(1), kind, N, K, G=32)
+        with pytest.raises(ops.KernelError):
+            ops.gemm_mfma_tiled(act, mk(gpu) if kind == "bf16" else ops.repack_mfma_tiles(mk(gpu)))
