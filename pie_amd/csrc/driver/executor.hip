@@ -77,7 +77,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
                              (p2 <= 8 ? 1.0 + 0.52 * (p2 - 1)
                                       : (1.0 + 0.52 * 7) * 0.9 * (p2 <= 32 ? p2 : wpasses) / 8.0 * (p2 == 32 && wpasses < 32 ? 1.2 : 1.0));
     // (prompts' passes are bound by the products and the decoding, not by the weights' width)
-    const double bytes = M > 128 && w.kind != Quant::Bf16 ? (w.kind == Quant::Int8 ? 0.63 : 0.5) * w.N * static_cast<double>(w.K)
+    const double bytes = M > 128 && w.kind != Quant::Bf16 ? (w.kind == Quant::Int8 ? 0.63 : w.kind == Quant::Fp8 ? 0.57 : 0.5) * w.N * static_cast<double>(w.K)
                                                           : static_cast<double>(w.data_bytes());
     const double skinny = w.data_tiled
                               ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * wave_form
@@ -595,14 +595,14 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     auto grouped = tiled ? pie_hip_moe_grouped_gemm_tiled : pie_hip_moe_grouped_gemm;
     auto wptr = [&](const Linear& l) { return tiled ? l.data_tiled : l.data; };
     auto sptr = [&](const Linear& l) { return tiled && l.scale_tiled ? l.scale_tiled : l.scale; };
-    // many routes per expert (a prompt's tokens): blocks of an expert's routes on the tiled GEMM, which takes quantised
-    // weights row-major (widths and groups that the passes refuse stay refused)
+    // many routes per expert (a prompt's tokens): blocks of an expert's routes on the tiled GEMM, which takes int4 weights
+    // row-major (widths and groups that the passes refuse stay refused)
     const int unit = w.wgu.kind == Quant::Bf16 ? 64 : w.wgu.kind == Quant::Int4b8 ? 512 : 256;
     const bool fits = H % unit == 0 && Ie % unit == 0 && (w.wgu.kind != Quant::Int4b8 || w.wgu.group >= 128);
     bool done = false;
     if (grouped_in_blocks(N * K, E, w.wgu.kind != Quant::Bf16)) {
         auto blocks = [&](const Linear& l, const uint16_t* act, const int32_t* rows, uint16_t* y, int rows_out, int cols, int epilogue) {
-            const bool tm = tiled && l.kind == Quant::Bf16;
+            const bool tm = tiled && l.kind != Quant::Int4b8;
             return pie_hip_moe_grouped_gemm_mfma_fmt(fmt, act, rows, moe_offsets_, E, N * K, tm ? l.data_tiled : l.data,
                                                      l.data_bytes() / E, l.scale, l.scale_bytes() / E, sbf, l.group, y, rows_out,
                                                      cols, epilogue, tm ? 1 : 0, nullptr, 0, s);

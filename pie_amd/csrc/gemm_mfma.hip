@@ -48,34 +48,6 @@ constexpr int kMaxMT = 8;   // 16-row activation tiles per wave, at most
 
 #define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
-// The problem and the rows [m0, m1) of block row `t` when problems are cut into blocks of `rows` rows one after
-// another; false behind the last.  Every lane of the wave calls it and gets the same answer.
-__device__ __forceinline__ bool grouped_place(const int32_t* __restrict__ offsets, int problems, int rows, int t, int lane,
-                                              int& p, int& m0, int& m1) {
-    int before = 0;
-    for (int base = 0; base < problems; base += kWave) {
-        const int e = base + lane;
-        const int lo = e < problems ? offsets[e] : 0, hi = e < problems ? offsets[e + 1] : 0;
-        const int n = (hi - lo + rows - 1) / rows;
-        int sum = n;
-#pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-            const int o = __shfl_up(sum, d);
-            if (lane >= d) sum += o;
-        }
-        const unsigned long long past = __ballot(before + sum > t);
-        if (past) {
-            const int at = __ffsll(past) - 1;
-            p = __builtin_amdgcn_readfirstlane(base + at);
-            m0 = __builtin_amdgcn_readfirstlane(__shfl(lo, at) + (t - before - __shfl(sum - n, at)) * rows);
-            m1 = __builtin_amdgcn_readfirstlane(__shfl(hi, at));
-            return true;
-        }
-        before += __shfl(sum, kWave - 1);
-    }
-    return false;
-}
-
 __device__ __forceinline__ uint32_t pack_trunc(float lo, float hi) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
@@ -632,7 +604,9 @@ extern "C" int pie_hip_moe_grouped_gemm_mfma_fmt(int format, const uint16_t* act
     a.swiglu = epilogue == PIE_HIP_EPI_SWIGLU ? 1 : 0;
     a.pointwise = pointwise_code(epilogue);
     if (a.swiglu && N % 2 != 0) return PIE_HIP_ERR_INVALID;
-    if (K % BK != 0 || (tiled && (N % 16 != 0 || format != PIE_HIP_FMT_BF16))) return PIE_HIP_ERR_UNSUPPORTED;
+    const bool bytes = format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8;
+    if (K % BK != 0 || (tiled && (N % 16 != 0 || (format != PIE_HIP_FMT_BF16 && !(bytes && (block_rows == 0 || block_rows == 128))))))
+        return PIE_HIP_ERR_UNSUPPORTED;
     if (format == PIE_HIP_FMT_INT4B8) {
         if (group_size < 32 || (group_size & (group_size - 1)) != 0 || K % group_size != 0) return PIE_HIP_ERR_UNSUPPORTED;
         a.g_shift = __builtin_ctz(static_cast<unsigned>(group_size));
@@ -652,6 +626,7 @@ extern "C" int pie_hip_moe_grouped_gemm_mfma_fmt(int format, const uint16_t* act
     a.N = N;
     a.K = K;
     if (glu) a.glu = *glu;
+    if (tiled && bytes) return launch_gemm_experts(format, a, num_routes, static_cast<hipStream_t>(stream));
     // (64 bf16 experts of 3072 x 4096, routes per expert 16 / 64 / 256: 295 / 367 / 985 us in blocks of 64, 310 / 324 / 746
     // of 128, 377 / 412 / 679 of 256; passes of 16 rows: 390 / 1161 / 4300)
     // (128 fp8 experts of 1536 x 2048, routes per expert 24 / 64 / 88 / 128 / 192 / 512: 100 / 153 / 195 / 279 / - / - us in blocks

@@ -38,9 +38,19 @@ constexpr int kActVecs = kRows * kStepK / 8;   // 16-byte vectors of an activati
 #define PIE_WAIT_VM(n)                              \
     do {                                            \
         __builtin_amdgcn_sched_barrier(0);          \
-        __builtin_amdgcn_s_waitcnt(0x0F70 | (n));   \
+        __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14)); \
         asm volatile("s_nop 0");                    \
         __builtin_amdgcn_sched_barrier(0);          \
+    } while (0)
+
+#define PIE_FENCE() __builtin_amdgcn_sched_barrier(0)
+#define PIE_MEET()                         \
+    do {                                   \
+        PIE_FENCE();                       \
+        asm volatile("" ::: "memory");     \
+        __builtin_amdgcn_s_barrier();      \
+        asm volatile("" ::: "memory");     \
+        PIE_FENCE();                       \
     } while (0)
 
 // ---- what a thread stages of a step's weights: V (32 or 16) of them, loaded from the tile-major copy (blocks of 1 KiB, 16 rows
@@ -269,15 +279,6 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
 
     // quantised weights: registers hold S steps, which are decoded one vector per phase
     typename F::Raw rr[S];
-#define PIE_FENCE() __builtin_amdgcn_sched_barrier(0)
-#define PIE_MEET()                         \
-    do {                                   \
-        PIE_FENCE();                       \
-        asm volatile("" ::: "memory");     \
-        __builtin_amdgcn_s_barrier();      \
-        asm volatile("" ::: "memory");     \
-        PIE_FENCE();                       \
-    } while (0)
 #pragma unroll
     for (int i = 0; i < S; ++i) rr[i] = load_w(i);
     PIE_FENCE();
@@ -425,6 +426,173 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
     }
 }
 
+// ---- experts: the rows of a problem gathered by route, one-byte weights, blocks of 128 rows x 64 NG columns -------------
+// A hundred rows per expert make an expert's weights as many bytes as its products are time, and each is wanted by one
+// block only.  So weights do not pass through LDS: a wave owns 16 NG columns for all 128 rows, the tile-major copy gives it
+// the MFMAs' operand by plain loads, four steps ahead in registers, each decoded once.  The activations are shared in LDS,
+// four steps ahead too.  Two blocks of four waves to a CU, independent of one another: one's prologue, waits and stores
+// run beside the other's MFMAs.  NG = 3: 254 registers (four spill; two read the activations half as often again: 122 against
+// 116 us).  A row block's column blocks stay on one chiplet and share its activations there.
+// Bound by the weights at 82 routes per expert: 128 fp8 experts of 1536 x 2048 116 us (402 MB; the tiles through LDS 147, four
+// routes per expert 98), of 2048 x 768 83 (84): twelve steps, of which the prologue and the stores take as long again.
+constexpr int kExpertRows = 128;
+__device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
+    __builtin_amdgcn_global_load_lds(from, PIE_LDS_PTR(to), 16, 0, 0);
+}
+template <int KVF, int NG>
+__global__ __launch_bounds__(256, 2) void gemm_experts_kernel(GemmArgs a, int col_blocks) {
+    constexpr int S = 4;                        // steps of 64 k-values in flight: LDS stages, weight registers
+    constexpr int kVecs = kExpertRows * kStepK / 8;
+    extern __shared__ __align__(16) unsigned char smem[];
+    u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int j = lane & 15, q = lane >> 4;
+    const int at = static_cast<int>(blockIdx.x >> 3);
+    int problem, m0, M;
+    if (!grouped_place(a.offsets, a.problems, kExpertRows, at / col_blocks * 8 + static_cast<int>(blockIdx.x & 7), lane, problem, m0, M)) return;
+    const int N = a.N, K = a.K, nk = K / kStepK, T = (N + 15) / 16;
+    const int tile0 = (at % col_blocks * 4 + wv) * NG;
+    const unsigned char* w = a.w + static_cast<size_t>(problem) * a.w_stride;
+    const unsigned char* scale = a.scale + static_cast<size_t>(problem) * a.scale_stride;
+
+    // the weights first: they depend on the problem alone, the activations on the routes' rows too
+    uint32_t woff[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) woff[i] = static_cast<uint32_t>(min(tile0 + i, T - 1)) * (nk * 1024u) + lane * 16u;
+    u32x4_t raw[S][NG];
+    auto load_w = [&](int kt, int slot) __attribute__((always_inline)) {
+        const unsigned char* pw = w + static_cast<size_t>(min(kt, nk - 1)) * 1024;
+#pragma unroll
+        for (int i = 0; i < NG; ++i) raw[slot][i] = *reinterpret_cast<const u32x4_t*>(pw + woff[i]);
+        PIE_FENCE();
+    };
+    const unsigned char* aptr[4];
+    int arow[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        arow[u] = min(m0 + (u * 4 + wv) * 8 + (lane >> 3), M - 1);
+        if (a.act_rows) arow[u] = a.act_rows[arow[u]];
+    }
+    PIE_FENCE();
+#pragma unroll
+    for (int i = 0; i < S; ++i) load_w(i, i);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        aptr[u] = reinterpret_cast<const unsigned char*>(a.act) + static_cast<size_t>(arow[u]) * (2u * K) +
+                  ((lane & 7) ^ ((((u * 4 + wv) * 8 + (lane >> 3)) >> 1) & 7)) * 16;
+    auto issue_a = [&](int kt, int stage) __attribute__((always_inline)) {
+        const size_t k = static_cast<size_t>(min(kt, nk - 1)) * (kStepK * 2);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) to_lds(aptr[u] + k, lds + stage * kVecs + (u * 4 + wv) * 64);
+        PIE_FENCE();
+    };
+    bf16x8_t af[2][4], bw[2][NG];   // [phase & 1][row tile], [k half][column tile]
+    const int key = j >> 1;
+    auto read_a = [&](int stage, int s, int rh, int to) __attribute__((always_inline)) {
+        const u32x4_t* A = lds + stage * kVecs + (rh * 64 + j) * 8 + ((2 * q + s) ^ key);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) af[to][t] = __builtin_bit_cast(bf16x8_t, A[t * 128]);
+    };
+    auto decode = [&](const u32x4_t& r, int s) __attribute__((always_inline)) {
+        return __builtin_bit_cast(bf16x8_t, kv_decode_bf16<KVF>(u32x2_t{r[2 * s], r[2 * s + 1]}));
+    };
+    f32x4_t acc[8][NG];
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int n = 0; n < NG; ++n) acc[t][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int i = 0; i < S; ++i) issue_a(i, i);
+    constexpr int kOps = 4 + NG;
+    PIE_WAIT_VM(3 * 4);
+    PIE_MEET();
+    read_a(0, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) bw[0][i] = decode(raw[0][i], 0);
+    auto mfmas = [&](int s, int rh) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int n = 0; n < NG; ++n)
+                acc[rh * 4 + t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[s][n], af[rh][t], acc[rh * 4 + t][n], 0, 0, 0);
+    };
+    auto order = [&]() __attribute__((always_inline)) {   // the reads ahead between the first MFMAs, the decoding between all
+#pragma unroll
+        for (int u = 0; u < 4 * NG; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (u < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+        }
+        PIE_FENCE();
+    };
+    auto step = [&](auto slot, int kt) __attribute__((always_inline)) {
+        constexpr int cur = decltype(slot)::value, next = (cur + 1) % S;
+        PIE_FENCE();
+        read_a(cur, 0, 1, 1);
+#pragma unroll
+        for (int i = 0; i < NG / 2; ++i) bw[1][i] = decode(raw[cur][i], 1);
+        mfmas(0, 0);
+        order();
+        read_a(cur, 1, 0, 0);
+#pragma unroll
+        for (int i = NG / 2; i < NG; ++i) bw[1][i] = decode(raw[cur][i], 1);
+        mfmas(0, 1);
+        order();
+        // step kt + 1 has come
+        if (kt < 2) PIE_WAIT_VM(2 * 4);
+        else PIE_WAIT_VM(2 * kOps);
+        read_a(cur, 1, 1, 1);
+#pragma unroll
+        for (int i = 0; i < NG / 2; ++i) bw[0][i] = decode(raw[next][i], 0);
+        mfmas(1, 0);
+        order();
+        PIE_WAIT_LGKM0();
+        PIE_MEET();
+        read_a(next, 0, 0, 0);
+        PIE_FENCE();
+        issue_a(kt + S, cur);
+        load_w(kt + S, cur);
+#pragma unroll
+        for (int i = NG / 2; i < NG; ++i) bw[0][i] = decode(raw[next][i], 0);
+        mfmas(1, 1);
+        order();
+    };
+    int kt = 0;
+    for (; kt + S <= nk; kt += S) {
+        step(std::integral_constant<int, 0>{}, kt);
+        step(std::integral_constant<int, 1>{}, kt + 1);
+        step(std::integral_constant<int, 2>{}, kt + 2);
+        step(std::integral_constant<int, 3>{}, kt + 3);
+    }
+    if (kt < nk) step(std::integral_constant<int, 0>{}, kt);
+    if (kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
+    if (kt + 2 < nk) step(std::integral_constant<int, 2>{}, kt + 2);
+    __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the block ends)
+
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const int n = (tile0 + i) * 16 + 4 * q;
+        if (n >= N) continue;
+        float rs[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = min(n + r, N - 1);
+            rs[r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(scale)[c]) : reinterpret_cast<const float*>(scale)[c];
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int m = m0 + t * 16 + j;
+            if (m >= M) continue;
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = acc[t][i][r] * rs[r];
+            wide_store(a, m, n, v);
+        }
+    }
+}
+
 // Sums the K shares' partials of four columns and applies the epilogue the kernel would have applied.
 __global__ __launch_bounds__(256) void wide_reduce_kernel(const GemmArgs a, int splits) {
     const int N = a.N, quads = (N + 3) / 4;
@@ -471,9 +639,9 @@ struct Rates {
                                      // 256), each 256 of more, each 256 blocks of 256 rows
 };
 constexpr Rates kRates[] = {
-    /* int4 */ {{14.0, 1.36, 8.0, 0.26}, {6.0, 0.76, 1.0, 0.15}, 0.58, 0.20, 0.64, 1.14},
-    /* int8 */ {{14.0, 1.31, 10.0, 0.22}, {7.0, 0.72, 2.0, 0.12}, 0.56, 0.20, 0.62, 1.10},
-    /* fp8 */ {{14.0, 1.31, 10.0, 0.20}, {7.0, 0.71, 2.0, 0.12}, 0.49, 0.17, 0.58, 1.08},
+    /* int4 */ {{14.0, 1.36, 8.0, 0.26}, {6.0, 0.76, 1.0, 0.15}, 0.57, 0.20, 0.64, 1.14},
+    /* int8 */ {{14.0, 1.31, 10.0, 0.22}, {7.0, 0.72, 2.0, 0.12}, 0.54, 0.20, 0.62, 1.10},
+    /* fp8 */ {{14.0, 1.31, 10.0, 0.20}, {7.0, 0.71, 2.0, 0.12}, 0.47, 0.17, 0.58, 1.08},
     /* bf16 */ {{14.0, 0.90, 10.0, 0.43}, {6.0, 0.62, 1.0, 0.19}, 0.36, 0.21, 0.57, 0.98},
 };
 double launch_us(const Rate& r, long long blocks, int steps) {
@@ -513,6 +681,20 @@ Plan plan_of(const Rates& r, int M, int N, int K, size_t ws_bytes) {
     }
     return best;
 }
+template <int KVF>
+int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
+    constexpr int NG = 3;
+    constexpr size_t smem = 4 * static_cast<size_t>(kExpertRows) * kStepK * 2;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_experts_kernel<KVF, NG>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+    const int cols = (a.N + 64 * NG - 1) / (64 * NG);
+    const long long rows = routes / kExpertRows + std::min(routes, a.problems);   // (no cut of the routes into problems makes more)
+    const long long blocks = (rows + 7) / 8 * 8 * cols;
+    if (blocks > 0x7FFFFFFF) return PIE_HIP_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL((gemm_experts_kernel<KVF, NG>), dim3(static_cast<unsigned>(blocks)), dim3(256), smem, stream, a, cols);
+    return launch_status();
+}
 bool fits(int format, int M, int N, int K, int group_size) {
     if (K % (format == PIE_HIP_FMT_INT4B8 ? 128 : 64) != 0 || K < 4 * kStepK) return false;
     if (format == PIE_HIP_FMT_INT4B8 && (group_size < 64 || (group_size & (group_size - 1)) != 0 || K % group_size != 0)) return false;
@@ -545,7 +727,7 @@ double gemm_tiles_us(int format, int M, int N, int K) {
     const long long low_rounds = (low + 255) / 256, high_rounds = (high + 255) / 256;
     const double steps = K / kStepK;
     if (1.85 * static_cast<double>(high_rounds) < static_cast<double>(low_rounds)) return high_rounds * (5.0 + steps * r.tall);
-    return 5.0 + steps * (low <= 256 ? r.few + r.many * static_cast<double>(low) / 256.0 : r.round * static_cast<double>(low_rounds));
+    return (format == PIE_HIP_FMT_BF16 ? 9.0 : 7.0) + steps * (low <= 256 ? r.few + r.many * static_cast<double>(low) / 256.0 : r.round * static_cast<double>(low_rounds));
 }
 
 int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {
@@ -560,6 +742,17 @@ int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, si
         case PIE_HIP_FMT_BF16: return run<WBf16>(a, p, static_cast<float*>(ws), stream);
         default: return PIE_HIP_ERR_INVALID;
     }
+}
+
+int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t stream) {
+    GemmArgs b = a;
+    b.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+    if (a.K % kStepK != 0 || a.N % 16 != 0 || static_cast<long long>(a.N) * a.K > 0xFFFFFFFFll ||
+        reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16 || a.w_stride % 16)
+        return PIE_HIP_ERR_UNSUPPORTED;
+    if (format == PIE_HIP_FMT_FP8) return launch_experts<kKvFp8>(b, routes, stream);
+    if (format == PIE_HIP_FMT_INT8) return launch_experts<kKvInt8>(b, routes, stream);
+    return PIE_HIP_ERR_UNSUPPORTED;
 }
 
 }  // namespace pie_hip

@@ -277,3 +277,36 @@ def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_row
             assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + bound)
     assert torch.equal(ops.moe_grouped_gemm(act[rows.long()].contiguous(), None, offs, fmt, w, scale, N, K, 257, G, block_rows=block_rows),
                        ops.moe_grouped_gemm(act, rows, offs, fmt, w, scale, N, K, 257, G, block_rows=block_rows))
+
+
+@pytest.mark.parametrize("fmt", ["fp8", "int8"])
+@pytest.mark.parametrize("N,K", [(144, 64), (192, 192), (400, 320), (16, 768)])
+def test_byte_experts_over_tile_major_weights(gpu, oracle, fmt, N, K):
+    """Blocks of 128 routes over the tile-major copy against those over row-major weights: an expert without routes, with one,
+    at the edges of a block, columns off the 192 of a block, one step of 64 k-values and remainders of the four in flight.
+    The same exact products in fp32, in another order: the bound of the test above."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(560 + N + K)
+    counts = [0, 1, 127, 128, 129, 0, 257, 17, 0]
+    E, T, routes = len(counts), 96, sum(counts)
+    offs = dev(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), gpu)
+    rows = dev(rng.integers(0, T, routes).astype(np.int32), gpu)
+    act = dev(oracle.f32_to_bf16(rng.standard_normal((T, K)).astype(np.float32)), gpu, torch.bfloat16)
+    w = dev(rng.integers(-128, 128, (E, N, K)).astype(np.int8) if fmt == "int8"
+            else rng.integers(0, 0x70, (E, N, K)).astype(np.uint8) | (rng.integers(0, 2, (E, N, K)) << 7).astype(np.uint8), gpu)
+    scale = dev(rng.uniform(0.001, 0.004, (E, N)).astype(np.float32), gpu)
+    if K == 192:
+        scale = scale.bfloat16()
+    t = ops.repack_mfma_tiles(ops.WeightView(fmt, w.reshape(E * N, K), scale.reshape(-1), 0, E * N, K)).data.reshape(E, N, K)
+    bound = K * 4.0 * 0.004 * (128 if fmt == "int8" else 256) * 2 * K * 2.0 ** -24
+    for swiglu in (False, True):
+        want = ops.moe_grouped_gemm(act, rows, offs, fmt, w, scale, N, K, 257, 0, swiglu, block_rows=128).float()
+        got = ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, swiglu, block_rows=0, tiled=True).float()
+        if swiglu:
+            assert torch.all((got - want).abs() <= 4 * 2.0 ** -8 * want.abs() + 2.0 ** -6 * want.abs().amax())
+        else:
+            assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + bound)
+    assert torch.equal(ops.moe_grouped_gemm(act[rows.long()].contiguous(), None, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True),
+                       ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True))
