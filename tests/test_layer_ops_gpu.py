@@ -96,6 +96,35 @@ def test_qkv_rope_kvwrite(gpu, oracle, hq, hk, d, interleaved, qknorm):
                           kp0.reshape(pages * ps, -1)[untouched])
 
 
+@pytest.mark.parametrize("hq,hk,d", [(3, 1, 16), (5, 2, 32), (32, 8, 64), (7, 1, 128), (3, 2, 1024)])
+@pytest.mark.parametrize("pairing", [0, 1, 2])
+@pytest.mark.parametrize("qknorm", [False, True])
+def test_qkv_rope_vectors_equal_elements(gpu, oracle, hq, hk, d, pairing, qknorm):
+    """The 16-byte form against the element form, which takes rows off a 16-byte boundary: the same expression per pair; with head
+    norms the squares are summed in another order, which moves a result by a bf16 step at most."""
+    import torch
+    from pie_amd import ops
+
+    g = torch.Generator(device=gpu).manual_seed(58 + hq + d)
+    N, pages, ps = 5, 2, 16
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu).to(torch.bfloat16)
+    packed = rnd(N, (hq + 2 * hk) * d)
+    shifted = torch.empty(packed.numel() + 1, dtype=torch.bfloat16, device=gpu)[1:].view_as(packed).copy_(packed)
+    tab = torch.rand(N, d, generator=g, device=gpu) * 2 - 1
+    slots = torch.tensor([3, -1, 0, 31, 7], device=gpu)
+    qw, kw = (rnd(d), rnd(d)) if qknorm else (None, None)
+    outs = []
+    for x in (packed, shifted):
+        kp, vp = torch.zeros(pages, ps, hk, d, dtype=torch.bfloat16, device=gpu), torch.zeros(pages, ps, hk, d, dtype=torch.bfloat16, device=gpu)
+        outs.append((ops.qkv_rope_kvwrite(x, kp, vp, tab, slots, hq, hk, d, pairing, qw, kw, 1e-6), kp, vp))
+    assert shifted.data_ptr() % 16 and torch.equal(outs[0][2], outs[1][2])
+    for got, want in zip(outs[0][:2], outs[1][:2]):
+        if qknorm:
+            assert ulp_diff(bits(got), bits(want)).max() <= 1
+        else:
+            assert torch.equal(got, want)
+
+
 def test_swiglu(gpu, oracle):
     import torch
     from pie_amd import ops
