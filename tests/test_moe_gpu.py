@@ -310,3 +310,20 @@ def test_byte_experts_over_tile_major_weights(gpu, oracle, fmt, N, K):
             assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + bound)
     assert torch.equal(ops.moe_grouped_gemm(act[rows.long()].contiguous(), None, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True),
                        ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True))
+
+
+@pytest.mark.parametrize("tokens", [1, 129, 2048, 2049])
+def test_sorted_layout_of_prompts(gpu, tokens):
+    """A block sorts up to 16384 routes out of its registers and more out of memory: either way each expert's routes are together,
+    between its offsets, and name their tokens."""
+    import torch
+    from pie_amd import ops
+
+    E, K = 128, 8
+    logits = torch.randn(tokens, E, generator=torch.Generator(device=gpu).manual_seed(570 + tokens), device=gpu).to(torch.bfloat16)
+    idx, _, offs, rtok, rpos = ops.moe_route(logits, K)
+    flat, pos = idx.reshape(-1).long(), rpos.reshape(-1).long()
+    assert torch.equal(pos.sort().values, torch.arange(tokens * K, device=gpu))
+    assert torch.equal(offs.long(), torch.cat([torch.zeros(1, dtype=torch.long, device=gpu), torch.bincount(flat, minlength=E).cumsum(0)]))
+    assert torch.all((pos >= offs.long()[flat]) & (pos < offs.long()[flat + 1]))
+    assert torch.equal(rtok.long()[pos], torch.arange(tokens * K, device=gpu) // K)
