@@ -15,8 +15,7 @@
 // rescale) is per lane and the probabilities leave the first product already in the register
 // layout the second one consumes — with the 32 keys of a step in the order
 // [4g..4g+3, 16+4g..16+4g+3] per 16-lane group g, which is the order V^T is laid out in LDS.
-// K rows are padded to 272 B and V^T rows to 80 B: every 16-byte operand read of 16 lanes
-// touches 64 distinct banks.  The next step's K/V are requested from HBM before the current
+// The next step's K/V are requested from HBM before the current
 // step is multiplied.  Probabilities enter the second product as a hi + lo pair of bf16 values
 // (fp32 accumulators), and the normaliser sums the unrounded values.
 #include "common.hip.h"
@@ -32,7 +31,29 @@ constexpr int kTileWaves = 4;
 constexpr int kTileThreads = kTileWaves * kWave;
 constexpr int kStepKeys = 32;
 constexpr int kBlockRows = 128;           // (token, head) rows per block
-constexpr int kVtStride = kStepKeys + 8;  // bf16 elements per V^T row (80 B)
+
+// LDS places, in elements.  An operand read takes 16 bytes per lane, and the lanes served together are 0 - 3, 12 - 15, 20 - 23 and
+// 24 - 27 (and so on): quarters of two neighbouring granules' rows, which have to fall into 16 different granules of the
+// banks.  K rows are padded by a granule, and rows 4 - 11 of 16 swap neighbouring granules.
+template <int D>
+__device__ __forceinline__ int k_at(int key, int c) { return key * (D + 8) + (c ^ ((key + 4) >> 3 & 1)) * 8; }
+// V^T rows are 64 bytes whose four granules change places by (row / 4) % 4 -> 0, 2, 3, 1; every 16 rows are padded by one, so that
+// the rows that neighbouring threads write differ too.
+__device__ __forceinline__ int vt_at(int row, int slot) {
+    const int r = row >> 2;
+    return row * kStepKeys + (row >> 4) * 8 + ((((slot >> 3) ^ (r & 1) << 1 ^ (r & 2) ^ (r & 2) >> 1) & 3) << 3 | (slot & 7));
+}
+
+// two buffers: a step's tiles are written while the previous step's are read, one barrier per step
+template <int D, bool Q8>
+struct TileLds {
+    alignas(16) uint16_t ks[2][kStepKeys * (D + 8)];
+    alignas(16) uint16_t vt[2][D * kStepKeys + D / 16 * 8];
+    alignas(16) float sc[2][Q8 ? 2 * kStepKeys : 4];   // K | V scales of a step
+};
+// ... or a group's accumulators, maxima and sums at the end
+template <int D, bool Q8>
+constexpr size_t kGroupBytes = sizeof(TileLds<D, Q8>) > (D / 16 + 1) * kTileThreads * 16 ? sizeof(TileLds<D, Q8>) : (D / 16 + 1) * kTileThreads * 16;
 
 // slot of key kappa (0..31) inside a V^T row
 __device__ __forceinline__ int vt_slot(int kappa) {
@@ -44,8 +65,16 @@ __device__ __forceinline__ int vt_slot(int kappa) {
 // KVF: one-byte pools (the codes become bf16 — exactly — on the way into the LDS tiles, one
 // 16-code piece per thread and matrix; the step's per-(token, kv head) scales sit in LDS and
 // multiply the scores (K) and the probabilities (V): float(code) * scale as in the row kernels).
-template <int D, int GQA, int QT, int KVF = kKvBf16>
-__global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
+// KP: groups of four waves that take a tile's steps in turn and meet at the end (in LDS, in fp32).  A block alone on its
+// CU is one wave per SIMD, which waits out every step's chain of products, exponentials and barrier: 1.25 us for 32 keys.
+// Up to 512 blocks of one 16-row tile per wave run in two groups: 358 rows behind 300 keys (32 heads over 8 of 128, 184
+// blocks) 25 -> 20 us, 128 behind 2000 67 -> 48, a prompt of 489 20.5 -> 17, of 1024 40 -> 34.  (Four groups: 20, 41, 18; at
+// 128 registers they spill.)
+// What bounds full launches: the vector unit and the matrix pipe, which overlap little (2048 rows: 158 instructions and 24 products
+// per wave and step, 80 us).  Before neighbouring threads took neighbouring pieces of a row, and with other LDS places,
+// LDS was busy two thirds of the time, over half of that with conflicts: 83 us.
+template <int D, int GQA, int QT, int KVF = kKvBf16, int KP = 1>
+__global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ k_pages_raw,
     const void* __restrict__ v_pages_raw, const float* __restrict__ k_scales,
     const float* __restrict__ v_scales, uint16_t* __restrict__ o,
@@ -56,7 +85,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
     constexpr int KS = D / 32;             // k steps of the first product
     constexpr int DT = D / 16;             // d tiles of the second product
     constexpr int LPR = D / 8;             // 16-byte pieces per K/V row
-    constexpr int KSTRIDE = D + 8;         // bf16 elements per K row in LDS
     constexpr bool Q8 = KVF != kKvBf16;
     constexpr int LPRQ = D / 16;           // 16-code pieces per one-byte row
     constexpr int PIECES = Q8 ? 1 : kStepKeys * LPR / kTileThreads;   // 16-byte pieces per thread per matrix
@@ -68,11 +96,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
     const unsigned char* v_bytes = static_cast<const unsigned char*>(v_pages_raw);
     // two LDS buffers: a step's tiles are written while the previous step's are read, one
     // barrier per step
-    __shared__ __attribute__((aligned(16))) float s_sc_all[2][Q8 ? 2 * kStepKeys : 1];   // K | V scales of a step
-
-    __shared__ __attribute__((aligned(16))) uint16_t Ks_all[2][kStepKeys * KSTRIDE];
-    __shared__ __attribute__((aligned(16))) uint16_t Vt_all[2][D * kVtStride];
-    __shared__ int s_kmax;
+    static_assert(KP == 1 || QT == 1, "the groups' results meet in the tiles' place");
+    using L = TileLds<D, Q8>;
+    extern __shared__ __align__(16) unsigned char smem[];
 
     // Blocks start in the order of their linear index: tile-major, the kv heads of a tile side by
     // side.  A caller that lists its tiles longest first therefore gets the long causal tiles
@@ -83,29 +109,30 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
     const int lin = blockIdx.y * gridDim.x + blockIdx.x;
     const int tile = lin / hk;
     const int kvh = lin - tile * hk;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+    const int part = KP == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kTileThreads);
+    const int tid = threadIdx.x & (kTileThreads - 1), lane = tid & (kWave - 1), wv = tid / kWave;
     const int l16 = lane & 15, g = lane >> 4;
     const int s0 = tile_start[tile], n_rows = tile_rows[tile];
     const uint32_t pg_lo = row_begin[s0];
+    L& lds = *reinterpret_cast<L*>(smem + part * kGroupBytes<D, Q8>);
 
-    if (tid == 0) s_kmax = 0;
-    __syncthreads();
-    if (tid < n_rows) atomicMax(&s_kmax, row_len[s0 + tid]);
-    __syncthreads();
-    const int kmax = s_kmax;
-
+    // (every wave finds the longest extent for itself: no barrier between the loads that lead to the first keys)
+    int longest = row_len[s0 + min(lane, max(n_rows, 1) - 1)];
+    if constexpr (TQ > kWave) longest = max(longest, row_len[s0 + min(lane + kWave, max(n_rows, 1) - 1)]);
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) longest = max(longest, __shfl_xor(longest, sh, kWave));
+    const int kmax = max(0, __builtin_amdgcn_readfirstlane(longest));
     // this lane's two query rows (one per 16-row tile of the wave)
-    int my_len[QT], my_row[QT], my_head[QT];
+    int my_len[QT];
     bf16x8_t qf[QT][KS];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int m = wv * 16 * QT + qt * 16 + l16;
         const int h = m / TQ, t = m % TQ;
         const bool valid = t < n_rows;
-        my_row[qt] = s0 + (valid ? t : 0);
-        my_head[qt] = kvh * GQA + h;
-        my_len[qt] = valid ? row_len[my_row[qt]] : 0;
-        const uint16_t* qp = q + (static_cast<size_t>(my_row[qt]) * hq + my_head[qt]) * D + 8 * g;
+        const int row = s0 + (valid ? t : 0);
+        my_len[qt] = valid ? row_len[row] : 0;
+        const uint16_t* qp = q + (static_cast<size_t>(row) * hq + kvh * GQA + h) * D + 8 * g;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             u32x4_t v = *reinterpret_cast<const u32x4_t*>(qp + 32 * ks);
@@ -124,26 +151,30 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
 
     // K/V staging: thread -> (key pair kp, 16-byte piece dc) so that two adjacent keys of one
     // piece meet in one thread (their V values pack into 4-byte LDS writes)
-    constexpr int PAIRS = kStepKeys / 2;
     constexpr int PF = 2;   // steps of K/V in flight
+    // from a group's step to its next: up to four steps the first group takes all (the meeting costs what sharing them saves, 128
+    // keys 8.1 us alone and 8.3 shared)
+    const bool shared = KP > 1 && kmax > 4 * kStepKeys;
+    const int advance = shared ? kStepKeys * KP : kStepKeys;
     u32x4_t kreg[PF][PIECES], vreg[PF][PIECES];
     float sreg[PF];   // one-byte pools: thread t < 32 holds the K scale of key t, t < 64 V's
     auto piece_of = [&](int u, int& key, int& dc) {
+        // (neighbouring threads take neighbouring pieces of a row: with neighbouring keys a wave's load touched 16 rows'
+        // lines for 64 bytes each, which kept the address unit busy for longer than the products took)
         if constexpr (Q8) {   // thread -> (key, 16-code piece); threads past the tile idle
-            key = tid % kStepKeys;
-            dc = tid / kStepKeys;
+            key = tid / LPRQ;
+            dc = tid % LPRQ;
             return;
         }
         if (PIECES == 1) {   // D = 64: one piece per thread
-            key = tid % kStepKeys;
-            dc = tid / kStepKeys;
+            key = tid / LPR;
+            dc = tid % LPR;
             return;
         }
         // pieces of one thread: (pair, dc) pairs p = tid + kTileThreads * (u / 2); key = 2 * pair + (u & 1)
         const int p = tid + kTileThreads * (u >> 1);
-        const int pair = p % PAIRS;
-        dc = p / PAIRS;
-        key = 2 * pair + (u & 1);
+        dc = p % LPR;
+        key = 2 * (p / LPR) + (u & 1);
     };
     // a 32-key step touches at most two pages (page_size % 16 == 0): their ids come through
     // scalar loads, so the vector-memory queue holds K/V loads only, in step order
@@ -168,7 +199,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
         if constexpr (Q8) {
             int key, dc;
             piece_of(0, key, dc);
-            if (dc < LPRQ) {
+            if (key < kStepKeys) {
                 const size_t off = token_head(key) * D + dc * 16;
                 kreg[slot][0] = *reinterpret_cast<const u32x4_t*>(k_bytes + off);
                 vreg[slot][0] = *reinterpret_cast<const u32x4_t*>(v_bytes + off);
@@ -176,6 +207,27 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
             if (tid < 2 * kStepKeys) {
                 const float* sp = tid < kStepKeys ? k_scales : v_scales;
                 sreg[slot] = sp ? sp[token_sc(tid % kStepKeys)] : 1.f;
+            }
+            return;
+        }
+        if (j0 + kStepKeys <= kmax) {
+            // a whole step: a key's place is its page's first token of the step plus the key, the same in both pages (a
+            // pair of keys is in one of them); 12 vector instructions where the general form below takes 40
+            const int in_a = pa_end - j0;
+            const size_t base_a = (static_cast<size_t>(pid_a) * ps + (ps - in_a)) * hk + kvh, base_b = (static_cast<size_t>(pid_b) * ps - in_a) * hk + kvh;
+#pragma unroll
+            for (int u = 0; u < PIECES; u += 2) {
+                int key, dc;
+                piece_of(u, key, dc);
+                const size_t off = ((key < in_a ? base_a : base_b) + static_cast<unsigned>(key * hk)) * D + dc * 8;
+                const uint16_t* kp = k_pages + off;
+                const uint16_t* vp = v_pages + off;
+                kreg[slot][u] = *reinterpret_cast<const u32x4_t*>(kp);
+                vreg[slot][u] = *reinterpret_cast<const u32x4_t*>(vp);
+                if constexpr (PIECES > 1) {
+                    kreg[slot][u + 1] = *reinterpret_cast<const u32x4_t*>(kp + hk * D);
+                    vreg[slot][u + 1] = *reinterpret_cast<const u32x4_t*>(vp + hk * D);
+                }
             }
             return;
         }
@@ -189,17 +241,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
         }
     };
     auto stage = [&](int slot) {   // register slot = LDS buffer
-        uint16_t* Ks = Ks_all[slot];
-        uint16_t* Vt = Vt_all[slot];
-        float* s_sc = s_sc_all[slot];
+        uint16_t* Ks = lds.ks[slot];
+        uint16_t* Vt = lds.vt[slot];
+        float* s_sc = lds.sc[slot];
         if constexpr (Q8) {
             int key, dc;
             piece_of(0, key, dc);
-            if (dc < LPRQ) {
+            if (key < kStepKeys) {
                 const u32x4_t kw = kreg[slot][0], vw = vreg[slot][0];
-                uint16_t* kd = &Ks[key * KSTRIDE + dc * 16];
-                *reinterpret_cast<u32x4_t*>(kd) = kv_decode_bf16<KVF>(u32x2_t{kw.x, kw.y});
-                *reinterpret_cast<u32x4_t*>(kd + 8) = kv_decode_bf16<KVF>(u32x2_t{kw.z, kw.w});
+                *reinterpret_cast<u32x4_t*>(&Ks[k_at<D>(key, 2 * dc)]) = kv_decode_bf16<KVF>(u32x2_t{kw.x, kw.y});
+                *reinterpret_cast<u32x4_t*>(&Ks[k_at<D>(key, 2 * dc + 1)]) = kv_decode_bf16<KVF>(u32x2_t{kw.z, kw.w});
                 const int col = vt_slot(key);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -207,7 +258,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
                     kv_decode_f32<KVF>(u32x2_t{vw[2 * h], vw[2 * h + 1]}, f);
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
-                        Vt[(dc * 16 + 8 * h + e) * kVtStride + col] = static_cast<uint16_t>(__float_as_uint(f[e]) >> 16);
+                        Vt[vt_at(dc * 16 + 8 * h + e, col)] = static_cast<uint16_t>(__float_as_uint(f[e]) >> 16);
                 }
             }
             if (tid < 2 * kStepKeys) s_sc[tid] = sreg[slot];
@@ -217,7 +268,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
         for (int u = 0; u < PIECES; ++u) {
             int key, dc;
             piece_of(u, key, dc);
-            *reinterpret_cast<u32x4_t*>(&Ks[key * KSTRIDE + dc * 8]) = kreg[slot][u];
+            *reinterpret_cast<u32x4_t*>(&Ks[k_at<D>(key, dc)]) = kreg[slot][u];
         }
 #pragma unroll
         for (int u = 0; u + 1 < PIECES || (PIECES == 1 && u == 0); u += 2) {
@@ -228,7 +279,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
                 const uint32_t w[4] = {vreg[slot][0].x, vreg[slot][0].y, vreg[slot][0].z, vreg[slot][0].w};
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    Vt[(dc * 8 + e) * kVtStride + col] = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
+                    Vt[vt_at(dc * 8 + e, col)] = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
             } else {
                 const uint32_t a[4] = {vreg[slot][u].x, vreg[slot][u].y, vreg[slot][u].z, vreg[slot][u].w};
                 const uint32_t b[4] = {vreg[slot][u + 1].x, vreg[slot][u + 1].y, vreg[slot][u + 1].z, vreg[slot][u + 1].w};
@@ -236,7 +287,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
                 for (int e = 0; e < 8; ++e) {
                     const uint32_t lo = (a[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
                     const uint32_t hi = (b[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-                    *reinterpret_cast<uint32_t*>(&Vt[(dc * 8 + e) * kVtStride + col]) = lo | (hi << 16);
+                    *reinterpret_cast<uint32_t*>(&Vt[vt_at(dc * 8 + e, col)]) = lo | (hi << 16);
                 }
             }
         }
@@ -256,11 +307,11 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
     // step first stages step j + 1 from the other register slot into the other buffer (whose
     // readers passed the last barrier), then refills that slot with step j + 3.
     auto step = [&](int slot, int j0) {
-        const uint16_t* Ks = Ks_all[slot];
-        const uint16_t* Vt = Vt_all[slot];
-        const float* s_sc = s_sc_all[slot];
-        if (j0 + kStepKeys < kmax) stage(slot ^ 1);
-        if (j0 + 3 * kStepKeys < kmax) issue(slot ^ 1, j0 + 3 * kStepKeys);   // (slot ^ 1 held step j + 1)
+        const uint16_t* Ks = lds.ks[slot];
+        const uint16_t* Vt = lds.vt[slot];
+        const float* s_sc = lds.sc[slot];
+        if (j0 + advance < kmax) stage(slot ^ 1);
+        if (j0 + 3 * advance < kmax) issue(slot ^ 1, j0 + 3 * advance);   // (slot ^ 1 held step j + 1)
         // (one-byte pools) the scales of this lane's keys 16nt + 4g + r
         f32x4_t ksc[2], vsc[2];
         if constexpr (Q8) {
@@ -281,7 +332,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt) {
                 const bf16x8_t kf = __builtin_bit_cast(
-                    bf16x8_t, *reinterpret_cast<const u32x4_t*>(&Ks[(16 * nt + l16) * KSTRIDE + 32 * ks + 8 * g]));
+                    bf16x8_t, *reinterpret_cast<const u32x4_t*>(&Ks[k_at<D>(16 * nt + l16, 4 * ks + g)]));
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt)
                     st[qt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qt][ks], st[qt][nt], 0, 0, 0);
@@ -350,24 +401,52 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
             const bf16x8_t vf = __builtin_bit_cast(
-                bf16x8_t, *reinterpret_cast<const u32x4_t*>(&Vt[(16 * dt + l16) * kVtStride + 8 * g]));
+                bf16x8_t, *reinterpret_cast<const u32x4_t*>(&Vt[vt_at(16 * dt + l16, 8 * g)]));
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
                 acc[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf_hi[qt], acc[qt][dt], 0, 0, 0);
                 acc[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf_lo[qt], acc[qt][dt], 0, 0, 0);
             }
         }
-        __syncthreads();   // step j + 1 is staged, step j read
     };
 
-    if (kmax > 0) issue(0, 0);
-    if (kmax > kStepKeys) issue(1, kStepKeys);
-    if (kmax > 0) stage(0);
-    if (kmax > 2 * kStepKeys) issue(0, 2 * kStepKeys);
+    const int first = KP == 1 || shared || part == 0 ? part * kStepKeys : kmax;
+    if (first < kmax) issue(0, first);
+    if (first + advance < kmax) issue(1, first + advance);
+    if (first < kmax) stage(0);
+    if (first + 2 * advance < kmax) issue(0, first + 2 * advance);
     __syncthreads();
-    for (int j0 = 0; j0 < kmax; j0 += PF * kStepKeys) {   // unrolled by PF: compile-time register slots
-        step(0, j0);
-        if (j0 + kStepKeys < kmax) step(1, j0 + kStepKeys);
+    for (int j0 = 0; j0 < kmax; j0 += PF * advance) {   // unrolled by PF: compile-time register slots
+        if (KP == 1 || first + j0 < kmax) step(0, first + j0);
+        __syncthreads();   // step j + 1 is staged, step j read
+        if (j0 + advance < kmax) {
+            if (KP == 1 || first + j0 + advance < kmax) step(1, first + j0 + advance);
+            __syncthreads();
+        }
+    }
+    if constexpr (KP > 1) {
+        // the other groups' accumulators, maxima and sums in their tiles' place; the first group adds them up
+        if (!shared && part > 0) return;
+        if (part > 0) {
+            f32x4_t* mine = reinterpret_cast<f32x4_t*>(&lds);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) mine[dt * kTileThreads + tid] = acc[0][dt];
+            mine[DT * kTileThreads + tid] = f32x4_t{mx[0], lsum[0], 0.f, 0.f};
+        }
+        if (shared) __syncthreads();
+        if (part > 0) return;
+        const float c = Q8 ? 1.f : scale_log2e;
+#pragma unroll
+        for (int other = 1; other < KP && shared; ++other) {
+            const f32x4_t* its = reinterpret_cast<const f32x4_t*>(smem + other * kGroupBytes<D, Q8>);
+            const f32x4_t st = its[DT * kTileThreads + tid];
+            const float m_new = fmaxf(mx[0], st[0]), safe = m_new == -INFINITY ? 0.f : m_new;
+            const float wa = __builtin_amdgcn_exp2f((mx[0] - safe) * c), wb = __builtin_amdgcn_exp2f((st[0] - safe) * c);
+            mx[0] = m_new;
+            lsum[0] = lsum[0] * wa + st[1] * wb;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[0][dt] = acc[0][dt] * wa + its[dt * kTileThreads + tid] * wb;
+        }
     }
 
     // normalise and store: this lane holds, for its query, d = 16 dt + 4 g + r
@@ -379,7 +458,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_prefill_tile_kernel(
         const int m = wv * 16 * QT + qt * 16 + l16;
         if (m % TQ >= n_rows) continue;
         const float inv = l > 0.f ? 1.0f / l : 0.f;
-        uint16_t* op = o + (static_cast<size_t>(my_row[qt]) * hq + my_head[qt]) * D + 4 * g;
+        uint16_t* op = o + (static_cast<size_t>(s0 + m % TQ) * hq + kvh * GQA + m / TQ) * D + 4 * g;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
             const f32x4_t a = acc[qt][dt];
@@ -395,25 +474,28 @@ int launch_tiles(int kv_format, const uint16_t* q, const void* k_pages, const vo
                  const uint32_t* page_indices, const uint32_t* row_begin, const int32_t* row_len,
                  const int32_t* tile_start, const int32_t* tile_rows, int num_tiles, int hq, int hk,
                  int ps, float scale, hipStream_t stream) {
-    const dim3 grid(num_tiles, hk);
     const float sl = scale * 1.4426950408889634f;
-    if (kv_format == PIE_HIP_KV_BF16)
-        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, kKvBf16>), grid, dim3(kTileThreads), 0, stream, q,
-                           k_pages, v_pages, k_scales, v_scales, o, page_indices, row_begin, row_len,
-                           tile_start, tile_rows, hq, hk, ps, sl);
-    else if (kv_format == PIE_HIP_KV_INT8_PER_TOKEN_HEAD)
-        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, kKvInt8>), grid, dim3(kTileThreads), 0, stream, q,
-                           k_pages, v_pages, k_scales, v_scales, o, page_indices, row_begin, row_len,
-                           tile_start, tile_rows, hq, hk, ps, sl);
-    else if (kv_format == PIE_HIP_KV_FP8_E5M2)
-        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, kKvBf8>), grid, dim3(kTileThreads), 0, stream, q,
-                           k_pages, v_pages, k_scales, v_scales, o, page_indices, row_begin, row_len,
-                           tile_start, tile_rows, hq, hk, ps, sl);
-    else
-        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, kKvFp8>), grid, dim3(kTileThreads), 0, stream, q,
-                           k_pages, v_pages, k_scales, v_scales, o, page_indices, row_begin, row_len,
-                           tile_start, tile_rows, hq, hk, ps, sl);
-    return launch_status();
+    auto run = [&](auto format, auto groups) {
+        constexpr int KVF = decltype(format)::value, KP = decltype(groups)::value;
+        constexpr size_t smem = KP * kGroupBytes<D, KVF != kKvBf16>;
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_tile_kernel<D, GQA, QT, KVF, KP>),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+        if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, KVF, KP>), dim3(num_tiles, hk), dim3(kTileThreads * KP), smem, stream, q,
+                           k_pages, v_pages, k_scales, v_scales, o, page_indices, row_begin, row_len, tile_start, tile_rows, hq, hk, ps, sl);
+        return launch_status();
+    };
+    auto grouped = [&](auto format) {
+        if constexpr (QT == 1) {
+            const long long blocks = static_cast<long long>(num_tiles) * hk;
+            if (blocks <= 512) return run(format, std::integral_constant<int, 2>{});
+        }
+        return run(format, std::integral_constant<int, 1>{});
+    };
+    if (kv_format == PIE_HIP_KV_BF16) return grouped(std::integral_constant<int, kKvBf16>{});
+    if (kv_format == PIE_HIP_KV_INT8_PER_TOKEN_HEAD) return grouped(std::integral_constant<int, kKvInt8>{});
+    if (kv_format == PIE_HIP_KV_FP8_E5M2) return grouped(std::integral_constant<int, kKvBf8>{});
+    return grouped(std::integral_constant<int, kKvFp8>{});
 }
 
 }  // namespace

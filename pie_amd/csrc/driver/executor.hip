@@ -980,6 +980,12 @@ void Executor::prepare_tiles(const BatchPlan& plan) {
     std::stable_sort(tiles.begin(), tiles.end(), [&](const auto& a, const auto& b) {
         return plan.row_kv_len[a.first + a.second - 1] > plan.row_kv_len[b.first + b.second - 1];
     });
+    // More blocks than run in two groups, one to a CU: every second round of 256 the other way round, so that the blocks that
+    // share a CU have about as many steps together as any others (a causal prompt of 2048 tokens, 32 heads over 8: 92 -> 83 us;
+    // 3000: 167 -> 156; 4096: 273 -> 256; of 1024, 512 blocks: 34 -> 40).
+    const size_t round = static_cast<size_t>(std::max(1, 256 / m.kv_heads));
+    for (size_t at = round; tiles.size() * m.kv_heads > 512 && at < tiles.size(); at += 2 * round)
+        std::reverse(tiles.begin() + at, tiles.begin() + std::min(at + round, tiles.size()));
     std::vector<int32_t> start, rows;
     for (const auto& tl : tiles) {
         start.push_back(tl.first);

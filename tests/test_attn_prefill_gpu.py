@@ -118,3 +118,39 @@ def test_tiles_over_one_byte_pools_match_the_oracle(gpu, oracle, fmt, hq, hk, d,
     assert np.all(err <= tol), f"worst {np.max(err / tol):.2f}x tol"
     want = oracle.bf16_to_f32(ref.view(torch.uint16).cpu().numpy()).astype(np.float64)
     assert np.all(np.abs(got - want) <= 2.0 ** -7 * np.maximum(np.abs(want), np.abs(got)) + 2e-4)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_many_tiles_equal_few(gpu, d):
+    """Above 512 blocks a block's waves walk all keys, up to there two groups of them take every other step and meet at the end:
+    the same weights and sums in another order, one bf16 rounding each (the bar of the first test, twice).  Extents on and beside
+    the steps of 32 keys, the second group without a key, tiles of one row."""
+    import torch
+    from pie_amd import ops
+
+    hq, hk, ps = 32, 8, 16
+    tr = ops.attn_prefill_tile_rows(hq, hk) // 2
+    ctx = [1, 31, 32, 33, 64, 65, 97, 128, 700]
+    pages = [-(-c // ps) for c in ctx]
+    first = np.concatenate([[0], np.cumsum(pages)])
+    row_begin = np.concatenate([np.full(c, f) for c, f in zip(ctx, first)]).astype(np.int32)
+    row_len = np.concatenate([np.arange(1, c + 1) for c in ctx]).astype(np.int32)
+    tiles, at = [], 0
+    for c in ctx:
+        tiles += [(at + t, min(tr, c - t)) for t in range(0, c, tr)]
+        at += c
+    assert len(tiles) * hk > 512
+    g = torch.Generator(device=gpu).manual_seed(63 + d)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu).to(torch.bfloat16)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    args = (rnd(at, hq, d), rnd(int(first[-1]), ps, hk, d), rnd(int(first[-1]), ps, hk, d),
+            torch.randperm(int(first[-1]), generator=g, device=gpu).int(), dev(row_begin), dev(row_len))
+    start, count = (dev(np.array(x, np.int32)) for x in zip(*tiles))
+    whole = ops.attention_prefill_tiles(*args, start, count, rows_per_tile=tr).float()
+    half = len(tiles) // 2
+    parts = torch.zeros_like(whole)
+    for sl in (slice(0, half), slice(half, None)):
+        o = ops.attention_prefill_tiles(*args, start[sl].contiguous(), count[sl].contiguous(), rows_per_tile=tr).float()
+        for s, n in zip(start[sl].tolist(), count[sl].tolist()):
+            parts[s:s + n] = o[s:s + n]
+    assert torch.all((whole - parts).abs() <= 2.0 ** -7 * torch.maximum(whole.abs(), parts.abs()) + 2e-4)
