@@ -99,6 +99,8 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const int per = (steps + shares - 1) / shares;
         split = 15.0 + (per + 3) * (M <= 64 ? 1.06 : 1.36) * std::ceil(tiles * shares / 512.0);
     }
+    const double columns = tile_major(w) ? pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, 0) : 1e30;
+    if (columns < std::min({skinny, split, tiled})) return GemmPath::Wide;
     if (split < skinny && split < tiled) return GemmPath::TiledSplitK;
     return tiled < skinny ? GemmPath::Tiled : GemmPath::Skinny;
 }
@@ -187,6 +189,7 @@ bool linear_fused(const Linear& w, const uint16_t* act, const uint16_t* norm_w, 
                                                    w.N, w.K, beta, swiglu, glu, gemm_ws, gemm_ws_bytes, s);
             if (sw == PIE_HIP_OK) return true;
             if (sw != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sw);
+            if (force >= 0) return false;
         }
         if (path != GemmPath::Skinny) {
             // the tiled GEMM (weights dequantised to bf16 while staged), in K shares for a
@@ -369,7 +372,7 @@ size_t Executor::scale_page_bytes() const {
 
 // Start-up measurement of the decoder linears' candidate kernels.  For every role (q|k|v, wo,
 // gate|up, down) and a ladder of row counts the GEMV (2-4 rows), the skinny GEMM and the tiled GEMM
-// (17-128 rows; in K shares where the workspace allows) run over the weights of successive layers
+// (17-128 rows; in K shares where the workspace allows; over the tile-major copy of one-byte weights) run over the weights of successive layers
 // (so that they come from HBM, as in a forward pass) on zeroed activations; the fastest goes into
 // every layer's table for the row counts up to the next rung.
 void Executor::tune_linears() {
@@ -444,7 +447,8 @@ void Executor::tune_linears() {
             int best = -1;
             double best_t = 1e30, model_t = 1e30;
             const int by_model = model_route(l0, M, r.norm != nullptr, gemm_ws_bytes_);
-            for (int cand = M <= 4 ? 0 : 1; cand <= (M <= 4 ? 1 : 3); ++cand) {
+            for (int cand = M <= 4 ? 0 : 1; cand <= (M <= 4 ? 1 : 4); ++cand) {
+                if (cand == 4 && by_model != 4) continue;   // (far slower where the model does not expect it)
                 if (cand == 3 && (M > 128 || pie_hip_gemm_mfma_workspace_bytes(M, l0.N, l0.K) == 0 ||
                                   pie_hip_gemm_mfma_workspace_bytes(M, l0.N, l0.K) > gemm_ws_bytes_))
                     continue;

@@ -439,19 +439,26 @@ constexpr int kExpertRows = 128;
 __device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
     __builtin_amdgcn_global_load_lds(from, PIE_LDS_PTR(to), 16, 0, 0);
 }
-template <int KVF, int NG>
-__global__ __launch_bounds__(256, 2) void gemm_experts_kernel(GemmArgs a, int col_blocks) {
-    constexpr int S = 4;                        // steps of 64 k-values in flight: LDS stages, weight registers
-    constexpr int kVecs = kExpertRows * kStepK / 8;
+// The same for one matrix and up to 128 rows (64 columns per block, two groups of waves that take the steps in turn and meet at the
+// end: a block is alone on its CU, and one wave per SIMD waits out every step's chain): 77 rows of 16384 x 2048 int8 16.7 us, fp8
+// 16.4 (128 x 128 tiles 27 and 26, passes of 32 rows 26 and 24; one group 18.4 and 17.7), 40 rows 13.7 and 11.3 (18.5 and 16.6).
+// RT row tiles of 16, NG column tiles per wave, S steps of 64 k-values in flight (LDS stages and weight registers).
+template <int KVF, int RT, int NG, int S, bool EXPERTS, int KP = 1>
+__global__ __launch_bounds__(256 * KP, 2) void gemm_columns_kernel(GemmArgs a, int col_blocks) {
+    constexpr int kRowsB = RT * 16, kVecs = kRowsB * kStepK / 8, HT = RT / 2, AC = RT / 2;   // a half's row tiles; chunks of eight rows per wave
     extern __shared__ __align__(16) unsigned char smem[];
-    u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem);
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int part = KP == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 256);
+    u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem) + part * S * kVecs;
+    const int tid = threadIdx.x & 255, lane = tid & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int j = lane & 15, q = lane >> 4;
-    const int at = static_cast<int>(blockIdx.x >> 3);
-    int problem, m0, M;
-    if (!grouped_place(a.offsets, a.problems, kExpertRows, at / col_blocks * 8 + static_cast<int>(blockIdx.x & 7), lane, problem, m0, M)) return;
-    const int N = a.N, K = a.K, nk = K / kStepK, T = (N + 15) / 16;
+    const int at = EXPERTS ? static_cast<int>(blockIdx.x >> 3) : static_cast<int>(blockIdx.x);
+    int problem = 0, m0 = 0, M = a.M;
+    if constexpr (EXPERTS)
+        if (!grouped_place(a.offsets, a.problems, kRowsB, at / col_blocks * 8 + static_cast<int>(blockIdx.x & 7), lane, problem, m0, M)) return;
+    const int N = a.N, K = a.K, nk_all = K / kStepK, T = (N + 15) / 16;
+    const int nk = (nk_all - part + KP - 1) / KP;   // this group's steps: part, part + KP, ..
+    auto place = [&](int kt) { return min(part + KP * min(kt, max(nk, 1) - 1), nk_all - 1); };   // (past them, or without any: a step again)
     const int tile0 = (at % col_blocks * 4 + wv) * NG;
     const unsigned char* w = a.w + static_cast<size_t>(problem) * a.w_stride;
     const unsigned char* scale = a.scale + static_cast<size_t>(problem) * a.scale_stride;
@@ -459,70 +466,70 @@ __global__ __launch_bounds__(256, 2) void gemm_experts_kernel(GemmArgs a, int co
     // the weights first: they depend on the problem alone, the activations on the routes' rows too
     uint32_t woff[NG];
 #pragma unroll
-    for (int i = 0; i < NG; ++i) woff[i] = static_cast<uint32_t>(min(tile0 + i, T - 1)) * (nk * 1024u) + lane * 16u;
+    for (int i = 0; i < NG; ++i) woff[i] = static_cast<uint32_t>(min(tile0 + i, T - 1)) * (nk_all * 1024u) + lane * 16u;
     u32x4_t raw[S][NG];
     auto load_w = [&](int kt, int slot) __attribute__((always_inline)) {
-        const unsigned char* pw = w + static_cast<size_t>(min(kt, nk - 1)) * 1024;
+        const unsigned char* pw = w + static_cast<size_t>(place(kt)) * 1024;
 #pragma unroll
         for (int i = 0; i < NG; ++i) raw[slot][i] = *reinterpret_cast<const u32x4_t*>(pw + woff[i]);
         PIE_FENCE();
     };
-    const unsigned char* aptr[4];
-    int arow[4];
+    const unsigned char* aptr[AC];
+    int arow[AC];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < AC; ++u) {
         arow[u] = min(m0 + (u * 4 + wv) * 8 + (lane >> 3), M - 1);
-        if (a.act_rows) arow[u] = a.act_rows[arow[u]];
+        if (EXPERTS && a.act_rows) arow[u] = a.act_rows[arow[u]];
     }
     PIE_FENCE();
 #pragma unroll
     for (int i = 0; i < S; ++i) load_w(i, i);
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < AC; ++u)
         aptr[u] = reinterpret_cast<const unsigned char*>(a.act) + static_cast<size_t>(arow[u]) * (2u * K) +
                   ((lane & 7) ^ ((((u * 4 + wv) * 8 + (lane >> 3)) >> 1) & 7)) * 16;
     auto issue_a = [&](int kt, int stage) __attribute__((always_inline)) {
-        const size_t k = static_cast<size_t>(min(kt, nk - 1)) * (kStepK * 2);
+        const size_t k = static_cast<size_t>(place(kt)) * (kStepK * 2);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) to_lds(aptr[u] + k, lds + stage * kVecs + (u * 4 + wv) * 64);
+        for (int u = 0; u < AC; ++u) to_lds(aptr[u] + k, lds + stage * kVecs + (u * 4 + wv) * 64);
         PIE_FENCE();
     };
-    bf16x8_t af[2][4], bw[2][NG];   // [phase & 1][row tile], [k half][column tile]
+    bf16x8_t af[2][HT], bw[2][NG];   // [phase & 1][row tile], [k half][column tile]
     const int key = j >> 1;
     auto read_a = [&](int stage, int s, int rh, int to) __attribute__((always_inline)) {
-        const u32x4_t* A = lds + stage * kVecs + (rh * 64 + j) * 8 + ((2 * q + s) ^ key);
+        const u32x4_t* A = lds + stage * kVecs + (rh * HT * 16 + j) * 8 + ((2 * q + s) ^ key);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) af[to][t] = __builtin_bit_cast(bf16x8_t, A[t * 128]);
+        for (int t = 0; t < HT; ++t) af[to][t] = __builtin_bit_cast(bf16x8_t, A[t * 128]);
     };
     auto decode = [&](const u32x4_t& r, int s) __attribute__((always_inline)) {
         return __builtin_bit_cast(bf16x8_t, kv_decode_bf16<KVF>(u32x2_t{r[2 * s], r[2 * s + 1]}));
     };
-    f32x4_t acc[8][NG];
+    f32x4_t acc[RT][NG];
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+    for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int n = 0; n < NG; ++n) acc[t][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
     for (int i = 0; i < S; ++i) issue_a(i, i);
-    constexpr int kOps = 4 + NG;
-    PIE_WAIT_VM(3 * 4);
+    constexpr int kOps = AC + NG;
+    PIE_WAIT_VM((S - 1) * AC);
     PIE_MEET();
     read_a(0, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < NG; ++i) bw[0][i] = decode(raw[0][i], 0);
     auto mfmas = [&](int s, int rh) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < HT; ++t)
 #pragma unroll
             for (int n = 0; n < NG; ++n)
-                acc[rh * 4 + t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[s][n], af[rh][t], acc[rh * 4 + t][n], 0, 0, 0);
+                acc[rh * HT + t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[s][n], af[rh][t], acc[rh * HT + t][n], 0, 0, 0);
     };
     auto order = [&]() __attribute__((always_inline)) {   // the reads ahead between the first MFMAs, the decoding between all
 #pragma unroll
-        for (int u = 0; u < 4 * NG; ++u) {
+        for (int u = 0; u < HT * NG; ++u) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (u < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (u < HT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
         }
         PIE_FENCE();
@@ -541,8 +548,8 @@ __global__ __launch_bounds__(256, 2) void gemm_experts_kernel(GemmArgs a, int co
         mfmas(0, 1);
         order();
         // step kt + 1 has come
-        if (kt < 2) PIE_WAIT_VM(2 * 4);
-        else PIE_WAIT_VM(2 * kOps);
+        if (kt < S - 2) PIE_WAIT_VM((S - 2) * AC);   // (of the first S the weights left first)
+        else PIE_WAIT_VM((S - 2) * kOps);
         read_a(cur, 1, 1, 1);
 #pragma unroll
         for (int i = 0; i < NG / 2; ++i) bw[0][i] = decode(raw[next][i], 0);
@@ -559,17 +566,37 @@ __global__ __launch_bounds__(256, 2) void gemm_experts_kernel(GemmArgs a, int co
         mfmas(1, 1);
         order();
     };
+    // (a group a step short of the others meets them all the same)
+    const int rounds = (nk_all + KP - 1) / KP;
+    auto steps = [&](int kt, auto whole) __attribute__((always_inline)) {
+        auto one = [&](auto slot) __attribute__((always_inline)) {
+            constexpr int i = decltype(slot)::value;
+            if (decltype(whole)::value || kt + i < nk) step(slot, kt + i);
+            else if (KP > 1 && kt + i < rounds) PIE_MEET();
+        };
+        one(std::integral_constant<int, 0>{});
+        one(std::integral_constant<int, 1>{});
+        one(std::integral_constant<int, 2>{});
+        one(std::integral_constant<int, 3>{});
+    };
+    static_assert(S == 4, "steps() is unrolled by hand");
     int kt = 0;
-    for (; kt + S <= nk; kt += S) {
-        step(std::integral_constant<int, 0>{}, kt);
-        step(std::integral_constant<int, 1>{}, kt + 1);
-        step(std::integral_constant<int, 2>{}, kt + 2);
-        step(std::integral_constant<int, 3>{}, kt + 3);
-    }
-    if (kt < nk) step(std::integral_constant<int, 0>{}, kt);
-    if (kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
-    if (kt + 2 < nk) step(std::integral_constant<int, 2>{}, kt + 2);
+    for (; kt + S <= nk_all / KP; kt += S) steps(kt, std::true_type{});
+    if (kt < rounds) steps(kt, std::false_type{});
     __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the block ends)
+    if constexpr (KP > 1) {   // the groups' sums meet in the activations' place
+        static_assert(NG == 1 && KP == 2 && RT * 256 <= S * kVecs, "");
+        __syncthreads();
+        f32x4_t* meet = reinterpret_cast<f32x4_t*>(smem);
+        if (part > 0) {
+#pragma unroll
+            for (int t = 0; t < RT; ++t) meet[t * 256 + tid] = acc[t][0];
+        }
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) acc[t][0] += meet[t * 256 + tid];
+    }
 
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
@@ -582,7 +609,7 @@ __global__ __launch_bounds__(256, 2) void gemm_experts_kernel(GemmArgs a, int co
             rs[r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(scale)[c]) : reinterpret_cast<const float*>(scale)[c];
         }
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
+        for (int t = 0; t < RT; ++t) {
             const int m = m0 + t * 16 + j;
             if (m >= M) continue;
             float v[4];
@@ -683,22 +710,52 @@ Plan plan_of(const Rates& r, int M, int N, int K, size_t ws_bytes) {
 }
 template <int KVF>
 int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
-    constexpr int NG = 3;
-    constexpr size_t smem = 4 * static_cast<size_t>(kExpertRows) * kStepK * 2;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_experts_kernel<KVF, NG>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+    constexpr int NG = 3, S = 4;
+    constexpr size_t smem = S * static_cast<size_t>(kExpertRows) * kStepK * 2;
+    constexpr auto kernel = &gemm_columns_kernel<KVF, kExpertRows / 16, NG, S, true>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
     const int cols = (a.N + 64 * NG - 1) / (64 * NG);
     const long long rows = routes / kExpertRows + std::min(routes, a.problems);   // (no cut of the routes into problems makes more)
     const long long blocks = (rows + 7) / 8 * 8 * cols;
     if (blocks > 0x7FFFFFFF) return PIE_HIP_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((gemm_experts_kernel<KVF, NG>), dim3(static_cast<unsigned>(blocks)), dim3(256), smem, stream, a, cols);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), smem, stream, a, cols);
     return launch_status();
+}
+template <int KVF, int RT>
+int launch_columns(const GemmArgs& a, hipStream_t stream) {
+    constexpr int S = 4, KP = 2;
+    constexpr size_t smem = KP * S * static_cast<size_t>(RT * 16) * kStepK * 2;
+    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, 1, S, false, KP>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+    const int cols = (a.N + 63) / 64;
+    hipLaunchKernelGGL(kernel, dim3(cols), dim3(256 * KP), smem, stream, a, cols);
+    return launch_status();
+}
+template <int KVF>
+int launch_columns(const GemmArgs& a, hipStream_t stream) {
+    return a.M <= 64 ? launch_columns<KVF, 4>(a, stream) : a.M <= 96 ? launch_columns<KVF, 6>(a, stream) : launch_columns<KVF, 8>(a, stream);
 }
 bool fits(int format, int M, int N, int K, int group_size) {
     if (K % (format == PIE_HIP_FMT_INT4B8 ? 128 : 64) != 0 || K < 4 * kStepK) return false;
     if (format == PIE_HIP_FMT_INT4B8 && (group_size < 64 || (group_size & (group_size - 1)) != 0 || K % group_size != 0)) return false;
     return 2ll * M * K <= 0xFFFFFFFFll && 2ll * (N + 15) * K <= 0xFFFFFFFFll && (M + 255ll) / 256 * ((N + 127ll) / 128) < 0x0FFFFFFF;
+}
+
+// up to 128 rows of one-byte weights
+bool columns_fit(int format, int M, int N, int K) {
+    return M <= 128 && (format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8) && K % kStepK == 0 && N % 16 == 0 &&
+           static_cast<long long>(N) * K <= 0xFFFFFFFFll;
+}
+// A round of blocks (one to a CU, two with 64 rows' LDS) takes 4 us and 0.27 - 0.5 a step (measured at 40 - 128 rows of
+// 16384, 5120 and 3072 x 2048 and 28672 x 4096).
+double columns_us(int format, int M, int N, int K) {
+    const int size = M <= 64 ? 0 : M <= 96 ? 1 : 2;
+    constexpr double kStepUs[2][3] = {{0.34, 0.40, 0.51}, {0.27, 0.39, 0.50}};
+    const long long blocks = (N + 63) / 64, slots = size == 0 ? 512 : 256;
+    const double crowd = size == 0 && blocks > 256 ? 1.6 : 1.0;
+    return 4.0 + static_cast<double>((blocks + slots - 1) / slots) * (K / kStepK) * kStepUs[format == PIE_HIP_FMT_FP8][size] * crowd;
 }
 
 template <class F>
@@ -718,6 +775,7 @@ int run(GemmArgs a, const Plan& p, float* ws, hipStream_t stream) {
 }  // namespace
 
 double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
+    if (columns_fit(format, M, N, K)) return columns_us(format, M, N, K);
     return fits(format, M, N, K, group_size) ? plan_of(kRates[format], M, N, K, ws_bytes).us : 1e30;
 }
 // (the choice between its two heights is launch_gemm's)
@@ -731,6 +789,11 @@ double gemm_tiles_us(int format, int M, int N, int K) {
 }
 
 int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {
+    if (columns_fit(format, a.M, a.N, a.K) && reinterpret_cast<uintptr_t>(a.act) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0) {
+        GemmArgs b = a;
+        b.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+        return format == PIE_HIP_FMT_FP8 ? launch_columns<kKvFp8>(b, stream) : launch_columns<kKvInt8>(b, stream);
+    }
     if (!fits(format, a.M, a.N, a.K, group_size) || reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16)
         return PIE_HIP_ERR_UNSUPPORTED;
     if (reinterpret_cast<uintptr_t>(ws) % 16) ws = nullptr;
@@ -759,7 +822,8 @@ int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t s
 
 extern "C" float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes) {
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return 1e30f;
-    const double tiles = pie_hip::gemm_tiles_us(format, M, N, K);
+    const double tiles = M > 128 ? pie_hip::gemm_tiles_us(format, M, N, K) : 1e30;
+    if (M <= 128 && !(tiled && pie_hip::columns_fit(format, M, N, K))) return 1e30f;
     const double wide = tiled || format == PIE_HIP_FMT_BF16 ? pie_hip::gemm_wide_us(format, M, N, K, group_size, workspace_bytes) : 1e30;
     return static_cast<float>(std::min(tiles, wide));
 }

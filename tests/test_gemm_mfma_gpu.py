@@ -145,9 +145,9 @@ def test_gemm_split_k_beta_swiglu_one_hot(gpu, oracle, kind):
     assert np.array_equal(fused, unfused)
 
 
-# one row, the edges of the 256-row and 128-column blocks, step counts that leave 0 - 2 behind the unrolled loops, enough
+# the fewest rows, the edges of the 256-row and 128-column blocks, step counts that leave 0 - 2 behind the unrolled loops, enough
 # blocks for 256 columns, whole rounds of those and a rest of 128 columns
-WIDE = [(1, 16, 256), (255, 144, 320), (257, 272, 448), (300, 16656, 256), (600, 23056, 384)]
+WIDE = [(129, 16, 256), (255, 144, 320), (257, 272, 448), (300, 16656, 256), (600, 23056, 384)]
 
 
 def wide_case(oracle, gpu, kind, M, N, K, seed):
@@ -228,3 +228,27 @@ def test_wide_refusals(gpu, oracle, kind):
         _, mk = make_weight(oracle, np.random.default_rng(1), kind, N, K, G=32)
         with pytest.raises(ops.KernelError):
             ops.gemm_mfma_tiled(act, mk(gpu) if kind == "bf16" else ops.repack_mfma_tiles(mk(gpu)))
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (17, 80, 128), (64, 208, 320), (65, 64, 448), (96, 144, 512), (97, 272, 576), (128, 64, 1088)])
+def test_columns_of_few_rows(gpu, oracle, kind, M, N, K):
+    """Up to 128 rows in blocks of 64 columns, against the exact sums: the edges of the three row counts, columns off a block, one
+    step of 64 k-values (the second group of waves has none), odd and even counts, remainders of the four in flight."""
+    import torch
+    from pie_amd import ops
+
+    act, w, t = wide_case(oracle, gpu, kind, M, N, K, 740 + M)
+    codes = w.data.double() if kind == "int8" else w.data.view(torch.float8_e4m3fn).double()
+    wd = codes.reshape(N, K) * w.scale.double().reshape(N, 1)
+    x = act.double()
+    bound = K * 2.0 ** -23 * (x.abs() @ wd.abs().T)
+    ref = x @ wd.T
+    got = ops.gemm_mfma_tiled(act, t).double()
+    assert torch.isfinite(got).all() and ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + bound).all()
+    y0 = torch.randn(M, N, device=gpu).to(torch.bfloat16)
+    got = ops.gemm_mfma_tiled(act, t, y=y0.clone(), beta=1).double()
+    assert ((got - ref - y0.double()).abs() <= 2.0 ** -8 * (ref + y0.double()).abs() + 2 * bound).all()
+    pairs = ops.gemm_mfma_tiled(act, t)
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1),
+                       ops.swiglu_bf16(torch.cat([pairs[:, 0::2], pairs[:, 1::2]], dim=1).contiguous()))
