@@ -267,7 +267,7 @@ int pie_hip_gemm_mfma_glu(int format, const uint16_t* act_bf16, const void* weig
  * (pie_hip_repack_mfma_tiles[_int4]; int4 scales from pie_hip_repack_scale_tiles; N % 16 == 0): K % 64 == 0 (int4: 128,
  * groups a power of two from 64 on), K >= 256, act and weight on 16-byte boundaries.  With a workspace (of any size) few
  * blocks over a long K run in shares of K.  Up to 128 rows of int8 or fp8 weights run in blocks of 64 columns, any
- * K % 64 == 0.  `epilogue` and `glu` as in pie_hip_gemm_mfma_glu. */
+ * K % 64 == 0; 17 to 48 rows of int4 weights (groups from 128 on) in blocks of 128, any K % 128 == 0.  `epilogue` and `glu` as in pie_hip_gemm_mfma_glu. */
 int pie_hip_gemm_mfma_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale,
                             int scale_is_bf16, int group_size, uint16_t* y_bf16, int M, int N, int K, int beta,
                             int epilogue, const PieHipGlu* glu, void* workspace, size_t workspace_bytes, void* stream);

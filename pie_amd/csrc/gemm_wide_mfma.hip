@@ -620,6 +620,182 @@ __global__ __launch_bounds__(256 * KP, 2) void gemm_columns_kernel(GemmArgs a, i
     }
 }
 
+// ---- 17 to 48 rows of int4 weights: the columns form with a scale group's products summed before they are scaled -------------
+// (The passes of 16 and 32 rows side by side read the weights once each, out of the L2 the second time, and that is what they
+// wait for: 40 rows of 28672 x 4096 29.8 us, here 24.2; 32 rows 23.0 and 20.9.  What bounds it: the vector unit and the matrix
+// pipe, 145 instructions and 36 products per wave and step, which overlap little: one group of waves with a block's scaling
+// spread over the next one's products 27.8.  64 rows need more registers than a wave has: 33.8 against 31.)
+// A wave's step is a tile-major block (16 columns x 128 k-values) of each of its NG tiles.  The codes enter the products as
+// 128 + n; what 136 times the activations' sum is too much leaves with a product against ones, once for all tiles.
+constexpr int kC4Step = 128, kC4Stages = 4, kC4Groups = 2;
+// places of a row's sixteen 16-byte granules: granule c at c ^ c4_key(row).  The lanes an LDS read serves together (0 - 3 and
+// 12 - 15 of one granule's rows, 4 - 11 of the next but three) find sixteen different places.
+__device__ __forceinline__ int c4_key(int row) { return (row & 15) < 4 ? row & 15 : (row & 15) < 12 ? (row & 15) + 4 : (row & 15) - 8; }
+
+template <int RT, int NG>
+__global__ __launch_bounds__(256 * kC4Groups, 2) void gemm_columns4_kernel(const GemmArgs a) {
+    constexpr int S = kC4Stages, KP = kC4Groups, kVecs = RT * 16 * (kC4Step / 8);
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int part_id = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 256);
+    u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem) + part_id * S * kVecs;
+    const int tid = threadIdx.x & 255, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int j = lane & 15, q = lane >> 4;
+    const int N = a.N, K = a.K, M = a.M, T = N / 16, nb = K / kC4Step;
+    const int nk = (nb - part_id + KP - 1) / KP;   // this group's steps
+    auto place = [&](int kt) { return min(part_id + KP * min(kt, max(nk, 1) - 1), nb - 1); };   // (past them, or without any: a step again)
+    const int tile0 = (static_cast<int>(blockIdx.x) * 4 + wv) * NG, groups = K >> a.g_shift, to_group = a.g_shift - 7;
+
+    uint32_t woff[NG], soff[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const uint32_t tile = min(tile0 + i, T - 1);
+        woff[i] = tile * (nb * 1024u) + lane * 16u;
+        soff[i] = tile * (groups * 32u) + q * 8u;
+    }
+    u32x4_t raw[S][NG];
+    u32x2_t gs[S][NG];
+    auto load_w = [&](int kt, int slot) __attribute__((always_inline)) {
+        const int b = place(kt);
+        const unsigned char* pw = a.w + static_cast<size_t>(b) * 1024;
+        const unsigned char* ps = a.scale + static_cast<size_t>(b >> to_group) * 32;
+#pragma unroll
+        for (int i = 0; i < NG; ++i) raw[slot][i] = *reinterpret_cast<const u32x4_t*>(pw + woff[i]);
+#pragma unroll
+        for (int i = 0; i < NG; ++i) gs[slot][i] = *reinterpret_cast<const u32x2_t*>(ps + soff[i]);
+        PIE_FENCE();
+    };
+    uint32_t aoff[RT];
+#pragma unroll
+    for (int u = 0; u < RT; ++u) {
+        const int r = (u * 4 + wv) * 4 + (lane >> 4);
+        aoff[u] = static_cast<uint32_t>(min(r, M - 1)) * (2u * K) + ((lane & 15) ^ c4_key(r)) * 16;
+    }
+    auto issue_a = [&](int kt, int stage) __attribute__((always_inline)) {
+        const unsigned char* pa = reinterpret_cast<const unsigned char*>(a.act) + static_cast<size_t>(place(kt)) * (kC4Step * 2);
+#pragma unroll
+        for (int u = 0; u < RT; ++u) to_lds(pa + aoff[u], lds + stage * kVecs + (u * 4 + wv) * 64);
+        PIE_FENCE();
+    };
+    const int key = c4_key(j);
+    bf16x8_t af[2][RT], bw[2][NG];
+    auto read_a = [&](int stage, int s, int to) __attribute__((always_inline)) {
+        const u32x4_t* A = lds + stage * kVecs + j * 16 + ((4 * q + s) ^ key);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) af[to][t] = __builtin_bit_cast(bf16x8_t, A[t * 256]);
+    };
+    uint32_t k128 = 0x43004300u;   // (128.0, 128.0) as a bf16 pair, opaque to the compiler
+    asm volatile("" : "+v"(k128));
+    auto decode = [&](const u32x4_t& r, int s) __attribute__((always_inline)) {
+        const uint32_t v = r[s];
+        return __builtin_bit_cast(bf16x8_t, u32x4_t{and_or(v, 0x000F000Fu, k128), and_or(v >> 4, 0x000F000Fu, k128),
+                                                    and_or(v >> 8, 0x000F000Fu, k128), and_or(v >> 12, 0x000F000Fu, k128)});
+    };
+    const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4_t{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t acc[RT][NG], sum[RT][NG], sx[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int i = 0; i < NG; ++i) acc[t][i] = zero;
+
+#pragma unroll
+    for (int i = 0; i < S; ++i) load_w(i, i);
+#pragma unroll
+    for (int i = 0; i < S; ++i) issue_a(i, i);
+    constexpr int kOps = RT + 2 * NG;
+    PIE_WAIT_VM((S - 1) * RT);
+    PIE_MEET();
+    read_a(0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) bw[0][i] = decode(raw[0][i], 0);
+    auto step = [&](auto slot, int kt) __attribute__((always_inline)) {
+        constexpr int cur = decltype(slot)::value, next = (cur + 1) % S;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            PIE_FENCE();
+            if (s < 3) {
+                read_a(cur, s + 1, (s + 1) & 1);
+#pragma unroll
+                for (int i = 0; i < NG; ++i) bw[(s + 1) & 1][i] = decode(raw[cur][i], s + 1);
+            } else {
+                // step kt + 1 has come (of the first S the weights left first)
+                if (kt < S - 2) PIE_WAIT_VM((S - 2) * RT);
+                else PIE_WAIT_VM((S - 2) * kOps);
+                PIE_WAIT_LGKM0();
+                PIE_MEET();
+                read_a(next, 0, 0);
+#pragma unroll
+                for (int i = 0; i < NG; ++i) bw[0][i] = decode(raw[next][i], 0);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                sx[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, af[s & 1][t], s ? sx[t] : zero, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < NG; ++i)
+                    sum[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[s & 1][i], af[s & 1][t], s ? sum[t][i] : zero, 0, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < RT * (NG + 1); ++u) {   // the reads ahead between the first products, the decoding between all
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (u < RT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            }
+        }
+        // (lane: row j, columns 4q .. 4q + 3 of a tile)
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            const float sc[4] = {bf16_lo(gs[cur][i].x), bf16_hi(gs[cur][i].x), bf16_lo(gs[cur][i].y), bf16_hi(gs[cur][i].y)};
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[t][i][r] = fmaf(sc[r], fmaf(-136.f, sx[t][r], sum[t][i][r]), acc[t][i][r]);
+        }
+        PIE_FENCE();
+        issue_a(kt + S, cur);
+        load_w(kt + S, cur);
+    };
+    const int rounds = (nb + KP - 1) / KP;
+    auto steps = [&](int kt, auto whole) __attribute__((always_inline)) {
+        auto one = [&](auto slot) __attribute__((always_inline)) {
+            constexpr int i = decltype(slot)::value;
+            if (decltype(whole)::value || kt + i < nk) step(slot, kt + i);
+            else if (kt + i < rounds) PIE_MEET();
+        };
+        one(std::integral_constant<int, 0>{});
+        one(std::integral_constant<int, 1>{});
+        one(std::integral_constant<int, 2>{});
+        one(std::integral_constant<int, 3>{});
+    };
+    int kt = 0;
+    for (; kt + S <= nb / KP; kt += S) steps(kt, std::true_type{});
+    if (kt < rounds) steps(kt, std::false_type{});
+    __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the sums take their place)
+    __syncthreads();
+    f32x4_t* meet = reinterpret_cast<f32x4_t*>(smem);
+    if (part_id > 0) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int i = 0; i < NG; ++i) meet[(t * NG + i) * 256 + tid] = acc[t][i];
+    }
+    __syncthreads();
+    if (part_id > 0) return;
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const int n = (tile0 + i) * 16 + 4 * q;
+        if (n >= N) continue;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int m = t * 16 + j;
+            if (m >= M) continue;
+            const f32x4_t o = acc[t][i] + meet[(t * NG + i) * 256 + tid];
+            float v[4] = {o[0], o[1], o[2], o[3]};
+            wide_store(a, m, n, v);
+        }
+    }
+}
+
 // Sums the K shares' partials of four columns and applies the epilogue the kernel would have applied.
 __global__ __launch_bounds__(256) void wide_reduce_kernel(const GemmArgs a, int splits) {
     const int N = a.N, quads = (N + 3) / 4;
@@ -743,14 +919,28 @@ bool fits(int format, int M, int N, int K, int group_size) {
     return 2ll * M * K <= 0xFFFFFFFFll && 2ll * (N + 15) * K <= 0xFFFFFFFFll && (M + 255ll) / 256 * ((N + 127ll) / 128) < 0x0FFFFFFF;
 }
 
-// up to 128 rows of one-byte weights
-bool columns_fit(int format, int M, int N, int K) {
-    return M <= 128 && (format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8) && K % kStepK == 0 && N % 16 == 0 &&
-           static_cast<long long>(N) * K <= 0xFFFFFFFFll;
+template <int RT>
+int launch_columns4(const GemmArgs& a, hipStream_t stream) {
+    constexpr int NG = 2;
+    constexpr size_t smem = kC4Groups * kC4Stages * static_cast<size_t>(RT * 16) * kC4Step * 2;
+    static_assert(static_cast<size_t>(RT) * NG * 256 * 16 <= smem, "the sums fit the activations' place");
+    constexpr auto kernel = &gemm_columns4_kernel<RT, NG>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernel, dim3((a.N + 64 * NG - 1) / (64 * NG)), dim3(256 * kC4Groups), smem, stream, a);
+    return launch_status();
+}
+// up to 128 rows of one-byte weights, 17 to 48 of int4 ones
+bool columns_fit(int format, int M, int N, int K, int group_size) {
+    if (N % 16 != 0 || static_cast<long long>(N) * K > 0xFFFFFFFFll) return false;
+    if (format == PIE_HIP_FMT_INT4B8)
+        return M > 16 && M <= 48 && K % kC4Step == 0 && group_size >= kC4Step && (group_size & (group_size - 1)) == 0 && K % group_size == 0;
+    return M <= 128 && (format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8) && K % kStepK == 0;
 }
 // A round of blocks (one to a CU, two with 64 rows' LDS) takes 4 us and 0.27 - 0.5 a step (measured at 40 - 128 rows of
 // 16384, 5120 and 3072 x 2048 and 28672 x 4096).
 double columns_us(int format, int M, int N, int K) {
+    if (format == PIE_HIP_FMT_INT4B8) return 4.0 + (N + 32767) / 32768 * (K / (2 * kC4Step)) * (M <= 32 ? 1.05 : 1.26);
     const int size = M <= 64 ? 0 : M <= 96 ? 1 : 2;
     constexpr double kStepUs[2][3] = {{0.34, 0.40, 0.51}, {0.27, 0.39, 0.50}};
     const long long blocks = (N + 63) / 64, slots = size == 0 ? 512 : 256;
@@ -775,7 +965,7 @@ int run(GemmArgs a, const Plan& p, float* ws, hipStream_t stream) {
 }  // namespace
 
 double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
-    if (columns_fit(format, M, N, K)) return columns_us(format, M, N, K);
+    if (columns_fit(format, M, N, K, group_size)) return columns_us(format, M, N, K);
     return fits(format, M, N, K, group_size) ? plan_of(kRates[format], M, N, K, ws_bytes).us : 1e30;
 }
 // (the choice between its two heights is launch_gemm's)
@@ -789,9 +979,10 @@ double gemm_tiles_us(int format, int M, int N, int K) {
 }
 
 int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {
-    if (columns_fit(format, a.M, a.N, a.K) && reinterpret_cast<uintptr_t>(a.act) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0) {
+    if (columns_fit(format, a.M, a.N, a.K, group_size) && reinterpret_cast<uintptr_t>(a.act) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0) {
         GemmArgs b = a;
         b.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+        if (format == PIE_HIP_FMT_INT4B8) return a.M <= 32 ? launch_columns4<2>(b, stream) : launch_columns4<3>(b, stream);
         return format == PIE_HIP_FMT_FP8 ? launch_columns<kKvFp8>(b, stream) : launch_columns<kKvInt8>(b, stream);
     }
     if (!fits(format, a.M, a.N, a.K, group_size) || reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16)
@@ -823,7 +1014,7 @@ int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t s
 extern "C" float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes) {
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return 1e30f;
     const double tiles = M > 128 ? pie_hip::gemm_tiles_us(format, M, N, K) : 1e30;
-    if (M <= 128 && !(tiled && pie_hip::columns_fit(format, M, N, K))) return 1e30f;
+    if (M <= 128 && !(tiled && pie_hip::columns_fit(format, M, N, K, group_size))) return 1e30f;
     const double wide = tiled || format == PIE_HIP_FMT_BF16 ? pie_hip::gemm_wide_us(format, M, N, K, group_size, workspace_bytes) : 1e30;
     return static_cast<float>(std::min(tiles, wide));
 }

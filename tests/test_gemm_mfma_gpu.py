@@ -252,3 +252,31 @@ def test_columns_of_few_rows(gpu, oracle, kind, M, N, K):
     pairs = ops.gemm_mfma_tiled(act, t)
     assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1),
                        ops.swiglu_bf16(torch.cat([pairs[:, 0::2], pairs[:, 1::2]], dim=1).contiguous()))
+
+
+@pytest.mark.parametrize("M,N,K,G", [(17, 16, 128, 128), (32, 144, 256, 256), (33, 272, 640, 128), (48, 128, 1024, 256), (40, 400, 1152, 128)])
+def test_columns_of_few_rows_int4(gpu, oracle, M, N, K, G):
+    """17 to 48 rows of int4 weights: the codes' products are summed exactly per group and scaled in fp32, so the exact sums with
+    the products' offset of 136 in the bound; columns off a block, one step of 128 k-values, odd counts, groups of two steps."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(760 + M)
+    wd, mk = make_weight(oracle, rng, "int4b8", N, K, G=G)
+    w = mk(gpu)
+    act = torch.randn(M, K, generator=torch.Generator(device=gpu).manual_seed(760 + M), device=gpu).to(torch.bfloat16)
+    t = ops.repack_mfma_tiles(w)
+    codes = np.stack([(wd["data"] >> (4 * i)) & 0xF for i in range(8)], axis=-1).reshape(N, K).astype(np.float64) - 8.0
+    scale = np.repeat(oracle.bf16_to_f32(wd["scale"]).astype(np.float64), G, axis=1)
+    wf = torch.from_numpy(codes * scale).to(gpu)
+    x = act.double()
+    ref = x @ wf.T
+    bound = K * 2.0 ** -23 * (x.abs() @ torch.from_numpy((np.abs(codes) + 272.0) * scale).to(gpu).T)
+    got = ops.gemm_mfma_tiled(act, t).double()
+    assert torch.isfinite(got).all() and ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + bound).all()
+    # and what those terms come to: as close to the exact sums as the passes of 16 and 32 rows are
+    if K % 512 == 0:
+        assert (got - ref).abs().mean() <= 1.02 * (ops.gemm_skinny(act, t).double() - ref).abs().mean()
+    pairs = ops.gemm_mfma_tiled(act, t)
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1),
+                       ops.swiglu_bf16(torch.cat([pairs[:, 0::2], pairs[:, 1::2]], dim=1).contiguous()))
