@@ -417,7 +417,8 @@ extern "C" int pie_hip_qkv_rope_kvwrite(const uint16_t* packed_qkv, uint16_t* q_
     const uintptr_t all = reinterpret_cast<uintptr_t>(packed_qkv) | reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(k_pages) |
                           reinterpret_cast<uintptr_t>(v_pages) | reinterpret_cast<uintptr_t>(q_norm_weight) |
                           reinterpret_cast<uintptr_t>(k_norm_weight) | reinterpret_cast<uintptr_t>(rope_table);
-    if (head_dim >= 16 && head_dim <= 1024 && (head_dim & (head_dim - 1)) == 0 && all % 16 == 0) {
+    // (64 tokens of 40 heads: 4.9 us in 16-byte accesses, 4.7 with a block per head; 381 of 48 5.2 and 5.9)
+    if (num_tokens > 128 && head_dim >= 16 && head_dim <= 1024 && (head_dim & (head_dim - 1)) == 0 && all % 16 == 0) {
         const int shift = __builtin_ctz(static_cast<unsigned>(head_dim)) - 4, heads = num_q_heads + 2 * num_kv_heads;
         const int threads = std::min(512, ((heads << shift) + 63) / 64 * 64);
         auto* kernel = interleaved == 0 ? qkv_rope_kvwrite_vec_kernel<0> : interleaved == 1 ? qkv_rope_kvwrite_vec_kernel<1> : qkv_rope_kvwrite_vec_kernel<2>;

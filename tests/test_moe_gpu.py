@@ -312,9 +312,9 @@ def test_byte_experts_over_tile_major_weights(gpu, oracle, fmt, N, K):
                        ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True))
 
 
-@pytest.mark.parametrize("tokens", [1, 129, 2048, 2049])
+@pytest.mark.parametrize("tokens", [128, 129, 2048, 2049])
 def test_sorted_layout_of_prompts(gpu, tokens):
-    """A block sorts up to 16384 routes out of its registers and more out of memory: either way each expert's routes are together,
+    """A block sorts 1025 to 16384 routes out of its registers, others out of memory: either way each expert's routes are together,
     between its offsets, and name their tokens."""
     import torch
     from pie_amd import ops
