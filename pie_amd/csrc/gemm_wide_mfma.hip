@@ -429,12 +429,11 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
 // ---- experts: the rows of a problem gathered by route, one-byte weights, blocks of 128 rows x 64 NG columns -------------
 // A hundred rows per expert make an expert's weights as many bytes as its products are time, and each is wanted by one
 // block only.  So weights do not pass through LDS: a wave owns 16 NG columns for all 128 rows, the tile-major copy gives it
-// the MFMAs' operand by plain loads, four steps ahead in registers, each decoded once.  The activations are shared in LDS,
-// four steps ahead too.  Two blocks of four waves to a CU, independent of one another: one's prologue, waits and stores
-// run beside the other's MFMAs.  NG = 3: 254 registers (four spill; two read the activations half as often again: 122 against
-// 116 us).  A row block's column blocks stay on one chiplet and share its activations there.
-// Bound by the weights at 82 routes per expert: 128 fp8 experts of 1536 x 2048 116 us (402 MB; the tiles through LDS 147, four
-// routes per expert 98), of 2048 x 768 83 (84): twelve steps, of which the prologue and the stores take as long again.
+// the MFMAs' operand by plain loads, three or four steps ahead in registers, each decoded once.  The activations are shared in LDS,
+// as far ahead.  Two or three blocks of four waves to a CU, independent of one another: one's prologue, waits and stores run
+// beside the other's MFMAs.  A row block's column blocks stay on one chiplet and share its activations there.
+// Bound by the weights: 128 fp8 experts of 1536 x 2048 at 82 routes 116 us (402 MB; the tiles through LDS 147, four routes per
+// expert 98), of 2048 x 768 74 (84 through LDS).
 constexpr int kExpertRows = 128;
 __device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
     __builtin_amdgcn_global_load_lds(from, PIE_LDS_PTR(to), 16, 0, 0);
@@ -444,7 +443,7 @@ __device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
 // 16.4 (128 x 128 tiles 27 and 26, passes of 32 rows 26 and 24; one group 18.4 and 17.7), 40 rows 13.7 and 11.3 (18.5 and 16.6).
 // RT row tiles of 16, NG column tiles per wave, S steps of 64 k-values in flight (LDS stages and weight registers).
 template <int KVF, int RT, int NG, int S, bool EXPERTS, int KP = 1>
-__global__ __launch_bounds__(256 * KP, 2) void gemm_columns_kernel(GemmArgs a, int col_blocks) {
+__global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(GemmArgs a, int col_blocks) {
     constexpr int kRowsB = RT * 16, kVecs = kRowsB * kStepK / 8, HT = RT / 2, AC = RT / 2;   // a half's row tiles; chunks of eight rows per wave
     extern __shared__ __align__(16) unsigned char smem[];
     const int part = KP == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 256);
@@ -577,9 +576,9 @@ __global__ __launch_bounds__(256 * KP, 2) void gemm_columns_kernel(GemmArgs a, i
         one(std::integral_constant<int, 0>{});
         one(std::integral_constant<int, 1>{});
         one(std::integral_constant<int, 2>{});
-        one(std::integral_constant<int, 3>{});
+        if constexpr (S > 3) one(std::integral_constant<int, 3>{});
     };
-    static_assert(S == 4, "steps() is unrolled by hand");
+    static_assert(S == 3 || S == 4, "steps() is unrolled by hand");
     int kt = 0;
     for (; kt + S <= nk_all / KP; kt += S) steps(kt, std::true_type{});
     if (kt < rounds) steps(kt, std::false_type{});
@@ -884,9 +883,8 @@ Plan plan_of(const Rates& r, int M, int N, int K, size_t ws_bytes) {
     }
     return best;
 }
-template <int KVF>
+template <int KVF, int NG, int S>
 int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
-    constexpr int NG = 3, S = 4;
     constexpr size_t smem = S * static_cast<size_t>(kExpertRows) * kStepK * 2;
     constexpr auto kernel = &gemm_columns_kernel<KVF, kExpertRows / 16, NG, S, true>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
@@ -1004,8 +1002,12 @@ int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t s
     if (a.K % kStepK != 0 || a.N % 16 != 0 || static_cast<long long>(a.N) * a.K > 0xFFFFFFFFll ||
         reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16 || a.w_stride % 16)
         return PIE_HIP_ERR_UNSUPPORTED;
-    if (format == PIE_HIP_FMT_FP8) return launch_experts<kKvFp8>(b, routes, stream);
-    if (format == PIE_HIP_FMT_INT8) return launch_experts<kKvInt8>(b, routes, stream);
+    // Three blocks of 128 columns to a CU hide one another's prologue, waits and stores better than two of 192, which read
+    // the activations less often: 128 fp8 experts of 1536 x 2048, 16 / 48 / 82 / 188 routes each 107 / 113 / 116 / 220 us against 101 / 109 /
+    // 121 / 230; of 2048 x 768, twelve steps, 59 / 64 / 74 / 152 against 63 / 75 / 82 / 167.
+    const bool wide = a.K > 1024 && routes < 64ll * a.problems;
+    if (format == PIE_HIP_FMT_FP8) return wide ? launch_experts<kKvFp8, 3, 4>(b, routes, stream) : launch_experts<kKvFp8, 2, 3>(b, routes, stream);
+    if (format == PIE_HIP_FMT_INT8) return wide ? launch_experts<kKvInt8, 3, 4>(b, routes, stream) : launch_experts<kKvInt8, 2, 3>(b, routes, stream);
     return PIE_HIP_ERR_UNSUPPORTED;
 }
 

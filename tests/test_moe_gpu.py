@@ -280,16 +280,16 @@ def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_row
 
 
 @pytest.mark.parametrize("fmt", ["fp8", "int8"])
-@pytest.mark.parametrize("N,K", [(144, 64), (192, 192), (400, 320), (16, 768)])
+@pytest.mark.parametrize("N,K", [(144, 64), (192, 192), (400, 320), (16, 768), (208, 1088)])
 def test_byte_experts_over_tile_major_weights(gpu, oracle, fmt, N, K):
     """Blocks of 128 routes over the tile-major copy against those over row-major weights: an expert without routes, with one,
-    at the edges of a block, columns off the 192 of a block, one step of 64 k-values and remainders of the four in flight.
+    at the edges of a block, columns off a block, one step of 64 k-values and remainders of those in flight (K above 1024 and few routes: the other block).
     The same exact products in fp32, in another order: the bound of the test above."""
     import torch
     from pie_amd import ops
 
     rng = np.random.default_rng(560 + N + K)
-    counts = [0, 1, 127, 128, 129, 0, 257, 17, 0]
+    counts = [0, 1, 127, 128, 129, 0, 257, 17, 0] + [0] * (4 if K > 1024 else 0)
     E, T, routes = len(counts), 96, sum(counts)
     offs = dev(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), gpu)
     rows = dev(rng.integers(0, T, routes).astype(np.int32), gpu)
