@@ -32,7 +32,7 @@ constexpr int kRows = 256, kStepK = 64, kWaves = 8;
 constexpr int kActVecs = kRows * kStepK / 8;   // 16-byte vectors of an activation stage
 
 #define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
-// s_waitcnt lgkmcnt(0) alone and vmcnt(n) alone, n < 16 (gfx9 encoding).  The no-op keeps the compiler's own wait for a
+// s_waitcnt lgkmcnt(0) alone and vmcnt(n) alone, n < 64 (gfx9 encoding).  The no-op keeps the compiler's own wait for a
 // value loaded before from being merged into this one: merged, it counts transfers into LDS as unordered and waits for all.
 #define PIE_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
 #define PIE_WAIT_VM(n)                              \
