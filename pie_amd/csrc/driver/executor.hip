@@ -71,25 +71,30 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     const int wpasses = M > 32 ? (M + 31) / 32 : passes;
     int p2 = 1;
     while (p2 < wpasses) p2 <<= 1;
-    // (past eight passes the machine is full: the cost grows in proportion, in powers of two up to 32, 17 - 31 passes a
-    // fifth worse than 32)
-    const double wave_form = (M > 32 ? 1.38 : 1.0) *
-                             (p2 <= 8 ? 1.0 + 0.52 * (p2 - 1)
-                                      : (1.0 + 0.52 * 7) * 0.9 * (p2 <= 32 ? p2 : wpasses) / 8.0 * (p2 == 32 && wpasses < 32 ? 1.2 : 1.0));
-    // (prompts' passes are bound by the products and the decoding, not by the weights' width)
-    const double bytes = M > 128 && w.kind != Quant::Bf16 ? (w.kind == Quant::Int8 ? 0.63 : w.kind == Quant::Fp8 ? 0.57 : 0.5) * w.N * static_cast<double>(w.K)
-                                                          : static_cast<double>(w.data_bytes());
-    const double skinny = w.data_tiled
-                              ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * wave_form
-                              : 5.0 + static_cast<double>(w.data_bytes()) / 2.8e6 * (1.0 + 0.85 * (passes - 1));
-    if (M > 128) {
-        const int fmt = fmt_code(w.kind);
-        const double rows = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
-        const double blocks = tile_major(w) ? pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes) : rows;
-        if (skinny < blocks) return GemmPath::Skinny;
-        return blocks < rows ? GemmPath::Wide : GemmPath::Tiled;
-    }
+    // (past eight passes the machine is full: the cost grows in proportion)
+    const double data = static_cast<double>(w.data_bytes());
+    const double wave_form = (M > 32 ? 1.38 : 1.0) * (p2 <= 8 ? 1.0 + 0.52 * (p2 - 1) : (1.0 + 0.52 * 7) * wpasses / 8.0);
+    const double skinny = w.data_tiled ? 5.0 + data / 3.8e6 * wave_form : 5.0 + data / 2.8e6 * (1.0 + 0.85 * (passes - 1));
     const int steps = w.K / 64;
+    if (M > 128) {
+        // Int4 weights: the skinny GEMM multiplies the codes and scales a group's sum in fp32, the blocks round every code times
+        // its scale to bf16 first, which takes a product's error from 0.0017 of its norm to 0.0022 (K of 4096, groups of 128).
+        // So int4 weights leave the skinny GEMM only where it is estimated slower than 128-row tiles, at 512 of them to a
+        // round: 28672 x 4096 at once, 6144 x 4096 from 481 rows on, 4096 x 4096 from 705, 4096 x 14336 from 769.  (At 381 rows of
+        // these skinny / wide blocks take 169 / 120, 45 / 42, 28 / 31 and 73 / 68 us.)
+        const double high = static_cast<double>((w.N + 127) / 128) * ((M + 127) / 128);
+        if (w.kind == Quant::Int4b8 && skinny <= 2.0 + steps * 0.68 * std::max(1.0, high / 512.0)) return GemmPath::Skinny;
+        // (prompts' passes cost in powers of two up to 32, 17 - 31 passes a fifth worse than 32, and are bound by the products and
+        // the decoding, not by the weights' width)
+        const double bytes = w.kind == Quant::Bf16 ? data : (w.kind == Quant::Int8 ? 0.63 : w.kind == Quant::Fp8 ? 0.57 : 0.5) * w.N * static_cast<double>(w.K);
+        const double prompt_form = p2 <= 8 ? wave_form : 1.38 * (1.0 + 0.52 * 7) * 0.9 * (p2 <= 32 ? p2 : wpasses) / 8.0 * (p2 == 32 && wpasses < 32 ? 1.2 : 1.0);
+        const double rows_us = w.data_tiled ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * prompt_form : skinny;
+        const int fmt = fmt_code(w.kind);
+        const double tiles = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
+        const double blocks = tile_major(w) ? pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes) : tiles;
+        if (rows_us < blocks) return GemmPath::Skinny;
+        return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
+    }
     const double tiles = static_cast<double>((w.N + 127) / 128);
     const double tiled = 2.0 + steps * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, tiles / 512.0);
     double split = 1e30;
@@ -1349,3 +1354,21 @@ void Executor::copy_pages_d2d(const uint32_t* srcs, const uint32_t* dsts, size_t
 }
 
 }  // namespace pie_hip_driver
+
+// Host-only hook on the rules that choose a linear's kernel, as pie_hip_driver_plan is on the planner: what a matrix [N, K] of
+// a storage format takes at M rows before any start-up measurement (0 GEMV, 1 skinny GEMM, 2 tiled GEMM, 3 tiled GEMM in
+// K shares, 4 tiled GEMM over the tile-major copy).
+extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, int K, int tile_major, size_t workspace_bytes) {
+    using namespace pie_hip_driver;
+    if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return -1;
+    constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
+    static_assert(PIE_HIP_FMT_INT4B8 == 0 && PIE_HIP_FMT_INT8 == 1 && PIE_HIP_FMT_FP8 == 2 && PIE_HIP_FMT_BF16 == 3, "");
+    Linear w;
+    w.kind = kinds[format];
+    w.N = N;
+    w.K = K;
+    w.group = group;
+    int there = 0;   // (only whether a copy is there counts)
+    if (tile_major) w.data_tiled = w.scale_tiled = &there;
+    return model_route(w, M, false, workspace_bytes);
+}

@@ -160,6 +160,8 @@ def lib() -> C.CDLL:
         l.pie_hip_driver_plan.restype = C.c_longlong
         l.pie_hip_driver_plan.argtypes = [C.POINTER(ForwardRequestDesc), C.c_int, C.c_int, C.c_void_p,
                                           C.c_void_p, C.c_size_t, C.c_char_p, C.c_size_t]
+        l.pie_hip_driver_linear_route.restype = C.c_int
+        l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
         l.pie_driver_hip_run_inproc.restype = C.c_int
         l.pie_driver_hip_run_inproc.argtypes = [C.c_int, C.POINTER(C.c_char_p), C.c_int, READY_FN,
                                                 C.c_void_p, InProcVTable]
@@ -456,3 +458,15 @@ def plan(frame: ForwardFrame, page_size: int, total_pages: int) -> dict:
     out.update(R=R2, N=N2, S=S, max_kv_len=int(tail[3]), pure_decode=bool(tail[4]),
                all_greedy=bool(tail[5]), has_user_masks=bool(tail[6]))
     return out
+
+
+LINEAR_ROUTES = ("gemv", "skinny", "tiled", "tiled in shares", "wide")
+
+
+def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: bool = True, workspace_bytes: int = 32 << 20) -> str:
+    """Host-only: the kernel the driver's rules give M rows of a matrix [N, K] of a storage format."""
+    code = ("int4b8", "int8", "fp8", "bf16").index(kind)
+    route = lib().pie_hip_driver_linear_route(code, group, M, N, K, int(tile_major), workspace_bytes)
+    if route < 0:
+        raise ValueError("linear_route")
+    return LINEAR_ROUTES[route]
