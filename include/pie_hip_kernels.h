@@ -310,7 +310,8 @@ int pie_hip_moe_grouped_gemm_mfma(const uint16_t* act_bf16, const int32_t* route
                                   uint16_t* y_bf16, int N, int K, int epilogue, int tiled, const PieHipGlu* glu,
                                   int block_rows, void* stream);
 /* The same over experts in any storage format, row-major (bf16, fp8 and int8 also tile-major; the latter two in blocks of
- * 128 routes); `scales` as in pie_hip_moe_grouped_gemm.  Int4 groups are powers of two from 32 on. */
+ * 128 routes); `scales` as in pie_hip_moe_grouped_gemm.  Int4 groups are powers of two from 32 on; each int4 code times its
+ * scale is rounded to bf16 (pie_hip_moe_grouped_gemm scales a group's sum in fp32). */
 int pie_hip_moe_grouped_gemm_mfma_fmt(int format, const uint16_t* act_bf16, const int32_t* route_act_rows,
                                       const int32_t* expert_offsets, int num_experts, int num_routes,
                                       const void* weights, size_t weight_stride_bytes, const void* scales,

@@ -604,17 +604,16 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     auto grouped = tiled ? pie_hip_moe_grouped_gemm_tiled : pie_hip_moe_grouped_gemm;
     auto wptr = [&](const Linear& l) { return tiled ? l.data_tiled : l.data; };
     auto sptr = [&](const Linear& l) { return tiled && l.scale_tiled ? l.scale_tiled : l.scale; };
-    // many routes per expert (a prompt's tokens): blocks of an expert's routes on the tiled GEMM, which takes int4 weights
-    // row-major (widths and groups that the passes refuse stay refused)
-    const int unit = w.wgu.kind == Quant::Bf16 ? 64 : w.wgu.kind == Quant::Int4b8 ? 512 : 256;
-    const bool fits = H % unit == 0 && Ie % unit == 0 && (w.wgu.kind != Quant::Int4b8 || w.wgu.group >= 128);
+    // many routes per expert (a prompt's tokens): blocks of an expert's routes on the tiled GEMM (widths that the passes
+    // refuse stay refused)
+    const int unit = w.wgu.kind == Quant::Bf16 ? 64 : 256;
+    const bool fits = H % unit == 0 && Ie % unit == 0;
     bool done = false;
-    if (grouped_in_blocks(N * K, E, w.wgu.kind != Quant::Bf16)) {
+    if (grouped_in_blocks(w.wgu.kind, N * K, E)) {
         auto blocks = [&](const Linear& l, const uint16_t* act, const int32_t* rows, uint16_t* y, int rows_out, int cols, int epilogue) {
-            const bool tm = tiled && l.kind != Quant::Int4b8;
-            return pie_hip_moe_grouped_gemm_mfma_fmt(fmt, act, rows, moe_offsets_, E, N * K, tm ? l.data_tiled : l.data,
-                                                     l.data_bytes() / E, l.scale, l.scale_bytes() / E, sbf, l.group, y, rows_out,
-                                                     cols, epilogue, tm ? 1 : 0, nullptr, 0, s);
+            return pie_hip_moe_grouped_gemm_mfma_fmt(fmt, act, rows, moe_offsets_, E, N * K, wptr(l), l.data_bytes() / E, l.scale,
+                                                     l.scale_bytes() / E, sbf, l.group, y, rows_out, cols, epilogue, tiled ? 1 : 0,
+                                                     nullptr, 0, s);
         };
         const int st = fits ? blocks(w.wgu, xn_, moe_route_token_, act_, 2 * Ie, H, PIE_HIP_EPI_SWIGLU) : PIE_HIP_ERR_UNSUPPORTED;
         if (st == PIE_HIP_OK) {
@@ -1371,4 +1370,13 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
     int there = 0;   // (only whether a copy is there counts)
     if (tile_major) w.data_tiled = w.scale_tiled = &there;
     return model_route(w, M, false, workspace_bytes);
+}
+
+// The same for a mixture's experts: whether `routes` over `experts` of a storage format run in blocks of an expert's routes (1)
+// or in passes of 16 (0).
+extern "C" int pie_hip_driver_experts_in_blocks(int format, long long routes, int experts) {
+    using namespace pie_hip_driver;
+    if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || routes <= 0 || experts <= 0) return -1;
+    constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
+    return Executor::grouped_in_blocks(kinds[format], routes, experts) ? 1 : 0;
 }

@@ -128,6 +128,17 @@ class Executor {
         return k ? k_pool_[layer] : v_pool_[layer];
     }
 
+    // From this many routes per expert on, blocks of routes beat passes of 16 over an expert's weights.  One-byte weights
+    // are decoded once per block and their tile-major passes are faster: 128 fp8 experts of 1536 x 2048 and 2048 x 768, both
+    // products, passes / blocks at 12, 16, 24, 32 and 88 routes per expert: 134 / 157, 154 / 155, 206 / 160, 256 / 164 and
+    // 605 / 240 us; over row-major weights 172 / 157, 203 / 161, 254 / 160, 312 / 173 and 697 / 240 (int8 at 12 and 16: 175 / 180,
+    // 212 / 175).  Int4 experts stay in passes, which scale a group's sum in fp32: the blocks round every code times its
+    // scale to bf16 (see pick_gemm).
+    static bool grouped_in_blocks(Quant kind, long long routes, int experts) {
+        return kind != Quant::Int4b8 && routes >= (kind == Quant::Bf16 ? kBlockRoutes : kByteBlockRoutes) * static_cast<long long>(experts);
+    }
+    static constexpr int kBlockRoutes = 12, kByteBlockRoutes = 16;
+
   private:
     // staged inputs: one pinned host block mirrored by one device block.  Layer stacks add the
     // rows' requests and the requests' row ranges and state slots.
@@ -145,14 +156,6 @@ class Executor {
     void enqueue_samplers();
     void collect_samplers(const BatchPlan& plan, SampleOutputs& out);
     void moe_block(const LayerWeights& w, int N, const uint16_t* next_norm, hipStream_t s);
-    // From this many routes per expert on, blocks of routes beat passes of 16 over an expert's weights.  Quantised weights
-    // are decoded once per block and their tile-major passes are faster: 128 fp8 experts of 1536 x 2048 and 2048 x 768, both
-    // products, passes / blocks at 12, 16, 24, 32 and 88 routes per expert: 134 / 157, 154 / 155, 206 / 160, 256 / 164 and
-    // 605 / 240 us.
-    static bool grouped_in_blocks(long long routes, int experts, bool quantised = false) {
-        return routes >= (quantised ? kQuantBlockRoutes : kBlockRoutes) * static_cast<long long>(experts);
-    }
-    static constexpr int kBlockRoutes = 12, kQuantBlockRoutes = 16;
     static constexpr int kFusedRouteRows = 256;   // batches up to this size take pie_hip_moe_norm_route
     static constexpr size_t kMergeProjMaxBytes = 64 * 1024;   // partial results a merging output projection reads per block
     bool xn_holds_next_norm_ = false;             // (while a forward is being enqueued) xn_ = the coming layer's normalised rows

@@ -399,7 +399,7 @@ void Executor::stack_mixture(const StackLayer& w, int N) {
         return;
     }
     const int hint = std::max(1, std::min(N, 2 * ((routes + E - 1) / E)));
-    const bool blocks = grouped_in_blocks(routes, E);
+    const bool blocks = grouped_in_blocks(Quant::Bf16, routes, E);
     auto grouped = [&](const Linear& l, const void* act, const int32_t* rows, void* y, int epilogue, const PieHipGlu* rule) {
         if (blocks) {
             PIE_KERNEL(pie_hip_moe_grouped_gemm_mfma(static_cast<const uint16_t*>(act), rows, stack_.route_offsets, E, routes,

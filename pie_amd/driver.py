@@ -162,6 +162,8 @@ def lib() -> C.CDLL:
                                           C.c_void_p, C.c_size_t, C.c_char_p, C.c_size_t]
         l.pie_hip_driver_linear_route.restype = C.c_int
         l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
+        l.pie_hip_driver_experts_in_blocks.restype = C.c_int
+        l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int]
         l.pie_driver_hip_run_inproc.restype = C.c_int
         l.pie_driver_hip_run_inproc.argtypes = [C.c_int, C.POINTER(C.c_char_p), C.c_int, READY_FN,
                                                 C.c_void_p, InProcVTable]
@@ -460,13 +462,18 @@ def plan(frame: ForwardFrame, page_size: int, total_pages: int) -> dict:
     return out
 
 
+_FORMATS = ("int4b8", "int8", "fp8", "bf16")
 LINEAR_ROUTES = ("gemv", "skinny", "tiled", "tiled in shares", "wide")
 
 
 def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: bool = True, workspace_bytes: int = 32 << 20) -> str:
     """Host-only: the kernel the driver's rules give M rows of a matrix [N, K] of a storage format."""
-    code = ("int4b8", "int8", "fp8", "bf16").index(kind)
-    route = lib().pie_hip_driver_linear_route(code, group, M, N, K, int(tile_major), workspace_bytes)
+    route = lib().pie_hip_driver_linear_route(_FORMATS.index(kind), group, M, N, K, int(tile_major), workspace_bytes)
     if route < 0:
         raise ValueError("linear_route")
     return LINEAR_ROUTES[route]
+
+
+def experts_in_blocks(kind: str, routes: int, experts: int) -> bool:
+    """Host-only: whether a mixture's routes run in blocks of an expert's routes (else in passes of 16)."""
+    return lib().pie_hip_driver_experts_in_blocks(_FORMATS.index(kind), routes, experts) == 1

@@ -46,3 +46,14 @@ def test_formats_whose_scales_wait_for_the_sum_take_the_blocks():
     assert drv.linear_route("int4b8", 2048, 28672, 4096, 128) == "wide"
     assert drv.linear_route("int4b8", 40, 28672, 4096, 128) == "wide"    # (its columns form: groups scaled in fp32)
     assert drv.linear_route("int4b8", 1, 4096, 4096, 128) == "gemv"
+
+
+@pytest.mark.parametrize("experts", [8, 128])
+def test_int4_experts_keep_fp32_scales(experts):
+    """The passes of 16 routes scale int4 groups in fp32, the blocks of routes round each code times its scale to bf16."""
+    from pie_amd import driver as drv
+
+    for each in (1, 15, 16, 17, 88, 500, 4096):
+        assert not drv.experts_in_blocks("int4b8", each * experts, experts)
+    for kind, first in (("fp8", 16), ("int8", 16), ("bf16", 12)):
+        assert [drv.experts_in_blocks(kind, n * experts, experts) for n in (first - 1, first, 500)] == [False, True, True]
