@@ -881,133 +881,25 @@ float pcg32_first_uniform(uint64_t seed) {
 
 }  // namespace
 
-// Rows of which the longest context is within an eighth of the mean: their attention launch may plan one round of
-// equally long blocks.
-bool Executor::evenly_long(const BatchPlan& plan, int row, int rows) {
-    if (rows < 2) return false;
-    long long total = 0;
-    int longest = 0;
-    for (int i = row; i < row + rows; ++i) {
-        total += plan.row_kv_len[i];
-        longest = std::max(longest, plan.row_kv_len[i]);
-    }
-    return 8LL * longest * rows <= 9 * total;
-}
-
-// Which rows' attention runs as tiles of consecutive rows of one request (on the matrix cores, a block per tile and
-// kv head that walks the keys once for all its rows) and which row by row (split keys, every row reading its own).
-// Decoded tokens run row by row; a portion of a prompt takes tiles where they cost less.  Microseconds, measured (one
-// portion of 8 .. 1024 rows behind 0 .. 8192 keys; 32 query heads over 8 and 4 kv heads of 128, over 8 of 64): row by
-// row 6 + the bytes of every row's keys and values at 12 TB/s (they come from the caches); as tiles 4.5 + 1.0 (heads of
-// 64: 0.7) per step of 32 keys of the longest, or 1.5 per step and resident slot once 512 blocks are more than
-// one round.  The two meet at about 90 rows of a new prompt (8 kv heads of 128), 128 (8 of 64).  335 rows behind 512 keys beside 23 decoded
-// tokens over 700 - 1200: 156 us per layer when all ran row by row, 62 since (tiles 34, single tokens 27).
+// Cuts the batch (attention_cut.hpp) and uploads its tiles.
 void Executor::prepare_tiles(const BatchPlan& plan) {
-    n_tiles_ = 0;
-    runs_.clear();
     const ModelConfig& m = model_.cfg();
-    const bool uniform_heads = m.head_dim == 64 || m.head_dim == 128;
-    int cap = pie_hip_attn_prefill_tile_rows(m.q_heads, m.kv_heads);
-    const double step_us = m.head_dim == 64 ? 0.7 : 1.0;
-    const double key_us = 4.0 * m.kv_heads * m.head_dim / 12e6;
-    // the tiled requests of a choice: those of at least 8 rows over at most `most` keys
-    auto tiled = [&](int r, int most) {
-        const int q0 = plan.qo_indptr[r], q1 = plan.qo_indptr[r + 1];
-        return q1 - q0 >= 8 && plan.row_kv_len[q1 - 1] <= most;
-    };
-    auto runs_of = [&](int most) {   // the other rows, in runs of neighbours
-        std::vector<RowRun> runs;
-        for (int r = 0; r < plan.R; ++r) {
-            const int q0 = plan.qo_indptr[r], q1 = plan.qo_indptr[r + 1];
-            if (q0 == q1 || tiled(r, most)) continue;
-            if (runs.empty() || runs.back().row + runs.back().rows != q0) runs.push_back({q0, 0, 0, false});
-            runs.back().rows += q1 - q0;
-            for (int i = q0; i < q1; ++i) runs.back().max_len = std::max(runs.back().max_len, plan.row_kv_len[i]);
-        }
-        return runs;
-    };
-    auto cost = [&](int most) {
-        double rows_us = 0.0;
-        long long blocks = 0, block_steps = 0;
-        int steps = 0;
-        for (int r = 0; r < plan.R; ++r) {
-            const int q0 = plan.qo_indptr[r], q1 = plan.qo_indptr[r + 1], n = q1 - q0;
-            if (n == 0) continue;
-            const int last = plan.row_kv_len[q1 - 1];
-            if (tiled(r, most)) {
-                const int tiles = (2 * n + cap - 1) / cap;
-                steps = std::max(steps, (last + 31) / 32);
-                blocks += static_cast<long long>(tiles) * m.kv_heads;
-                block_steps += static_cast<long long>(tiles) * m.kv_heads * ((last - n / 2 + 31) / 32);
-            } else {
-                rows_us += key_us * n * (last - 0.5 * (n - 1));
-            }
-        }
-        return (rows_us > 0.0 ? 6.0 + rows_us : 0.0) +
-               (blocks ? 4.5 + step_us * std::max<double>(steps, 1.5 * block_steps / 512.0) : 0.0);
-    };
-    constexpr int kNone = -1, kAll = 0x7FFFFFFF;
-    int most = kNone;
-    if (cap > 0 && !masked_ && !plan.pure_decode && page_size_ % 16 == 0 && uniform_heads) {
-        // every portion; those that alone would gain, and shorter ones, which ride along; none
-        int gain = kNone;
-        for (int r = 0; r < plan.R; ++r) {
-            const int n = plan.qo_indptr[r + 1] - plan.qo_indptr[r];
-            if (n < 8) continue;
-            const int last = plan.row_kv_len[plan.qo_indptr[r + 1] - 1];
-            if (key_us * n * (last - 0.5 * (n - 1)) > step_us * ((last + 31) / 32)) gain = std::max(gain, last);
-        }
-        double best = cost(kNone);
-        for (int cand : {gain, kAll}) {
-            const double c = cost(cand);
-            if (c < best && runs_of(cand).size() <= 2) {   // (a launch per run and layer)
-                best = c;
-                most = cand;
-            }
-        }
-    }
-    if (most != kNone) runs_ = runs_of(most);
-    else runs_.push_back({0, plan.N, plan.max_kv_len, false});
-    for (RowRun& run : runs_) run.uniform = !plan.pure_decode && evenly_long(plan, run.row, run.rows);
-    if (most == kNone) return;
-    long long blocks = 0;
-    for (int r = 0; r < plan.R; ++r)
-        if (tiled(r, most))
-            blocks += static_cast<long long>((plan.qo_indptr[r + 1] - plan.qo_indptr[r] + cap - 1) / cap) * m.kv_heads;
-    if (blocks == 0) return;
-    // fewer than three full-size blocks per CU: halve the tiles (measured on a causal prompt of
-    // 2048 tokens, 512 full-size blocks: 110 -> 100 us; of 3072 tokens, 768 blocks: 169 -> 179)
-    if (blocks < 768) cap /= 2;
-    tile_rows_ = cap;
-    // Longest first: the kernel starts its blocks in tile order, and a long causal tile started
-    // last would run on alone.
-    std::vector<std::pair<int32_t, int32_t>> tiles;   // (first row, rows)
-    for (int r = 0; r < plan.R; ++r)
-        for (int t0 = plan.qo_indptr[r]; tiled(r, most) && t0 < plan.qo_indptr[r + 1]; t0 += cap)
-            tiles.emplace_back(t0, std::min(cap, plan.qo_indptr[r + 1] - t0));
-    std::stable_sort(tiles.begin(), tiles.end(), [&](const auto& a, const auto& b) {
-        return plan.row_kv_len[a.first + a.second - 1] > plan.row_kv_len[b.first + b.second - 1];
-    });
-    // More blocks than run in two groups, one to a CU: every second round of 256 the other way round, so that the blocks that
-    // share a CU have about as many steps together as any others (a causal prompt of 2048 tokens, 32 heads over 8: 92 -> 83 us;
-    // 3000: 167 -> 156; 4096: 273 -> 256; of 1024, 512 blocks: 34 -> 40).
-    const size_t round = static_cast<size_t>(std::max(1, 256 / m.kv_heads));
-    for (size_t at = round; tiles.size() * m.kv_heads > 512 && at < tiles.size(); at += 2 * round)
-        std::reverse(tiles.begin() + at, tiles.begin() + std::min(at + round, tiles.size()));
-    std::vector<int32_t> start, rows;
-    for (const auto& tl : tiles) {
-        start.push_back(tl.first);
-        rows.push_back(tl.second);
-    }
-    const size_t n = start.size(), bytes = 8 * n;
+    const bool fits = !masked_ && !plan.pure_decode && page_size_ % 16 == 0 && (m.head_dim == 64 || m.head_dim == 128);
+    const AttentionCut cut = cut_attention(plan, m.kv_heads, m.head_dim, fits ? pie_hip_attn_prefill_tile_rows(m.q_heads, m.kv_heads) : 0);
+    runs_ = cut.runs;
+    tile_rows_ = cut.tile_rows;
+    n_tiles_ = static_cast<int>(cut.tiles.size());
+    if (n_tiles_ == 0) return;
+    const size_t n = cut.tiles.size(), bytes = 8 * n;
     tile_in_host_.pinned = true;
     tile_in_host_.ensure(bytes);
     tile_in_dev_.ensure(bytes);
     auto* h = static_cast<int32_t*>(tile_in_host_.ptr);
-    std::memcpy(h, start.data(), 4 * n);
-    std::memcpy(h + n, rows.data(), 4 * n);
+    for (size_t i = 0; i < n; ++i) {
+        h[i] = cut.tiles[i].first;
+        h[n + i] = cut.tiles[i].second;
+    }
     PIE_HIP_CHECK(hipMemcpyAsync(tile_in_dev_.ptr, h, bytes, hipMemcpyHostToDevice, stream_));
-    n_tiles_ = static_cast<int>(n);
 }
 
 // Custom attention masks: each row's BRLE runs become cumulative bounds, the device expands
@@ -1379,4 +1271,26 @@ extern "C" int pie_hip_driver_experts_in_blocks(int format, long long routes, in
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || routes <= 0 || experts <= 0) return -1;
     constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
     return Executor::grouped_in_blocks(kinds[format], routes, experts) ? 1 : 0;
+}
+
+// And for a batch's attention: the rows of request r are qo_indptr[r] .. qo_indptr[r + 1] (of R requests), row i sees
+// row_kv_len[i] keys.  out receives {tile height, tiles, runs}, (first row, rows) of each tile and (first row, rows, equally long) of each
+// run.  Returns the number of values, or -1 where they do not fit `cap`.
+extern "C" long long pie_hip_driver_attention_cut(const int* qo_indptr, int R, const int* row_kv_len, int q_heads, int kv_heads,
+                                                  int head_dim, int* out, size_t cap) {
+    using namespace pie_hip_driver;
+    if (!qo_indptr || !row_kv_len || !out || R <= 0 || q_heads <= 0 || kv_heads <= 0) return -1;
+    BatchPlan plan;
+    plan.R = R;
+    plan.N = qo_indptr[R];
+    plan.qo_indptr.assign(qo_indptr, qo_indptr + R + 1);
+    plan.row_kv_len.assign(row_kv_len, row_kv_len + plan.N);
+    plan.max_kv_len = plan.N ? *std::max_element(plan.row_kv_len.begin(), plan.row_kv_len.end()) : 0;
+    const AttentionCut cut = cut_attention(plan, kv_heads, head_dim, pie_hip_attn_prefill_tile_rows(q_heads, kv_heads));
+    std::vector<int> v = {cut.tile_rows, static_cast<int>(cut.tiles.size()), static_cast<int>(cut.runs.size())};
+    for (const auto& t : cut.tiles) v.insert(v.end(), {t.first, t.second});
+    for (const RowRun& r : cut.runs) v.insert(v.end(), {r.row, r.rows, r.uniform ? 1 : 0});
+    if (v.size() > cap) return -1;
+    std::copy(v.begin(), v.end(), out);
+    return static_cast<long long>(v.size());
 }

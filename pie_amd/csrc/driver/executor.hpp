@@ -46,6 +46,7 @@
 #include "config.hpp"
 #include "model.hpp"
 #include "pie_hip_kernels.h"
+#include "attention_cut.hpp"
 #include "planner.hpp"
 
 namespace pie_hip_driver {
@@ -151,7 +152,6 @@ class Executor {
     void grow_outputs(size_t slots);
     void prepare_masks(const BatchPlan& plan);
     void prepare_tiles(const BatchPlan& plan);
-    static bool evenly_long(const BatchPlan& plan, int row, int rows);
     void prepare_samplers(const BatchPlan& plan);
     void enqueue_samplers();
     void collect_samplers(const BatchPlan& plan, SampleOutputs& out);
@@ -246,10 +246,6 @@ class Executor {
     };
     // query-row tiles of the current forward for the matrix-core prefill attention, and the runs of rows that
     // take the per-row kernel
-    struct RowRun {
-        int row, rows, max_len;
-        bool uniform;   // about equally long
-    };
     std::vector<RowRun> runs_;
     Growable tile_in_host_, tile_in_dev_;
     int n_tiles_ = 0, tile_rows_ = 0;

@@ -164,6 +164,8 @@ def lib() -> C.CDLL:
         l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
         l.pie_hip_driver_experts_in_blocks.restype = C.c_int
         l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int]
+        l.pie_hip_driver_attention_cut.restype = C.c_longlong
+        l.pie_hip_driver_attention_cut.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_size_t]
         l.pie_driver_hip_run_inproc.restype = C.c_int
         l.pie_driver_hip_run_inproc.argtypes = [C.c_int, C.POINTER(C.c_char_p), C.c_int, READY_FN,
                                                 C.c_void_p, InProcVTable]
@@ -477,3 +479,18 @@ def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: 
 def experts_in_blocks(kind: str, routes: int, experts: int) -> bool:
     """Host-only: whether a mixture's routes run in blocks of an expert's routes (else in passes of 16)."""
     return lib().pie_hip_driver_experts_in_blocks(_FORMATS.index(kind), routes, experts) == 1
+
+
+def attention_cut(requests: Sequence[tuple], q_heads: int, kv_heads: int, head_dim: int) -> dict:
+    """Host-only: how the driver cuts a batch's attention.  requests: (cached tokens, tokens of this batch) each.  Returns the
+    tiles' height, the (first row, rows) of each tile and the (first row, rows, equally long) of each run of other rows."""
+    qo = np.concatenate([[0], np.cumsum([n for _, n in requests])]).astype(np.int32)
+    lens = np.concatenate([np.arange(h + 1, h + n + 1) for h, n in requests]).astype(np.int32)
+    out = np.zeros(16 + 5 * len(lens), np.int32)
+    n = lib().pie_hip_driver_attention_cut(qo.ctypes.data, len(requests), lens.ctypes.data, q_heads, kv_heads, head_dim,
+                                           out.ctypes.data, len(out))
+    if n < 0:
+        raise ValueError("attention_cut")
+    tiles, runs = int(out[1]), int(out[2])
+    return dict(tile_rows=int(out[0]), tiles=[tuple(t) for t in out[3:3 + 2 * tiles].reshape(-1, 2).tolist()],
+                runs=[(a, b, bool(c)) for a, b, c in out[3 + 2 * tiles:3 + 2 * tiles + 3 * runs].reshape(-1, 3).tolist()])

@@ -57,3 +57,75 @@ def test_int4_experts_keep_fp32_scales(experts):
         assert not drv.experts_in_blocks("int4b8", each * experts, experts)
     for kind, first in (("fp8", 16), ("int8", 16), ("bf16", 12)):
         assert [drv.experts_in_blocks(kind, n * experts, experts) for n in (first - 1, first, 500)] == [False, True, True]
+
+
+# microseconds of one layer's attention over a bf16 cache on an MI355X, row by row and as tiles: a portion of 32, 64, 112, 160 and 256
+# rows by (query heads, kv heads, head size) and cached tokens
+MEASURED_ROWS = (32, 64, 112, 160, 256)
+MEASURED = {
+    ((32, 8, 128), 0): [(4.4, 5.3), (5.1, 6.1), (9.6, 7.9), (14.4, 8.3), (22.1, 10.5)],
+    ((32, 8, 128), 256): [(7.5, 11.1), (11.1, 11.8), (19.7, 12.8), (25.0, 13.7), (37.5, 15.4)],
+    ((32, 8, 128), 1000): [(15.2, 26.5), (24.6, 27.0), (56.2, 27.4), (73.4, 28.6), (105.1, 30.3)],
+    ((32, 8, 128), 2000): [(23.7, 45.7), (40.5, 46.7), (86.6, 46.4), (116.2, 47.9), (164.1, 50.5)],
+    ((32, 4, 128), 0): [(5.0, 5.3), (5.4, 6.1), (7.0, 7.9), (11.3, 8.3), (14.8, 10.4)],
+    ((32, 4, 128), 256): [(8.2, 11.1), (8.7, 11.8), (12.6, 12.8), (19.4, 13.9), (24.4, 15.6)],
+    ((32, 4, 128), 1000): [(15.8, 26.2), (16.7, 26.7), (24.9, 27.6), (50.3, 28.5), (74.0, 30.1)],
+    ((32, 4, 128), 2000): [(20.1, 45.6), (25.2, 46.6), (40.7, 46.9), (82.0, 47.9), (111.7, 49.8)],
+    ((32, 8, 64), 0): [(3.4, 4.1), (3.7, 4.9), (6.0, 6.2), (7.5, 6.6), (12.7, 8.0)],
+    ((32, 8, 64), 256): [(5.2, 8.5), (7.0, 8.8), (11.3, 9.6), (14.0, 10.4), (21.2, 11.8)],
+    ((32, 8, 64), 1000): [(9.9, 20.4), (15.7, 20.8), (31.5, 21.1), (42.0, 22.2), (58.2, 23.3)],
+    ((32, 8, 64), 2000): [(15.4, 35.1), (25.8, 35.7), (47.9, 36.0), (60.4, 36.7), (89.7, 38.2)],
+}
+
+
+def taken(requests, heads):
+    """Indices of the requests whose rows are tiled; checks that every row is in one tile or one run, once."""
+    from pie_amd import driver as drv
+
+    cut = drv.attention_cut(requests, *heads)
+    first = np.concatenate([[0], np.cumsum([n for _, n in requests])])
+    seen, tiled = np.zeros(first[-1], int), set()
+    for a, n in cut["tiles"]:
+        r = int(np.searchsorted(first, a, side="right")) - 1
+        assert 0 < n <= cut["tile_rows"] and a + n <= first[r + 1]   # (one request's rows)
+        seen[a:a + n] += 1
+        tiled.add(r)
+    for a, n, _ in cut["runs"]:
+        seen[a:a + n] += 1
+    assert (seen == 1).all()
+    return sorted(tiled)
+
+
+def test_measured_portions_take_their_faster_form():
+    for (heads, history), times in MEASURED.items():
+        for n, (rows, tiles) in zip(MEASURED_ROWS, times):
+            us = tiles if taken([(history, n)], heads) else rows
+            assert us <= 1.08 * min(rows, tiles), (heads, history, n, us)
+
+
+@pytest.mark.parametrize("heads", [(32, 8, 128), (32, 4, 128), (32, 8, 64), (8, 8, 128), (16, 8, 128), (8, 2, 64), (32, 32, 128)])
+@pytest.mark.parametrize("history", [0, 60, 256, 1000, 2000, 8000])
+def test_longer_portions_do_not_fall_back_to_rows(heads, history):
+    """A portion takes tiles from some number of rows on, not here and there, and about where its rows fill a round of blocks."""
+    tiles = [bool(taken([(history, n)], heads)) for n in range(8, 800)]
+    first = tiles.index(True) + 8
+    assert all(tiles[first - 8:])
+    assert 512 < first * heads[1] <= 1024
+
+
+def test_portions_behind_a_context_beside_decoded_tokens_take_tiles():
+    decoded = [(700 + 40 * i, 1) for i in range(8)]
+    assert taken(decoded + [(2000, 100)], (32, 8, 128)) == [8]
+    assert taken(decoded + [(2000, 30)], (32, 8, 128)) == []
+    assert taken(decoded + [(0, 400), (0, 20)], (32, 8, 128)) == [8, 9]     # (the shorter one rides along)
+    assert taken([(0, 400), (4000, 16)], (32, 8, 128)) == [0]               # (and a few rows behind many keys do not)
+    assert taken([(900, 1)] * 64, (32, 8, 128)) == []
+    assert taken([(500, 60)] * 4, (32, 8, 64)) == [0, 1, 2, 3]
+
+
+@pytest.mark.parametrize("seed", range(8))
+def test_every_row_is_attended_once(seed):
+    rng = np.random.default_rng(300 + seed)
+    for _ in range(60):
+        requests = [(int(rng.integers(0, 3000)), int(1 if rng.random() < 0.5 else rng.integers(1, 300))) for _ in range(int(rng.integers(1, 20)))]
+        taken(requests, [(32, 8, 128), (32, 4, 128), (32, 8, 64), (32, 32, 128), (12, 2, 128), (14, 2, 64)][seed % 6])
