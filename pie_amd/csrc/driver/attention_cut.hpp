@@ -44,11 +44,14 @@ inline bool evenly_long(const BatchPlan& plan, int row, int rows) {
 // pools, whose decoding costs what their smaller size saves; 2178 points):
 //   row by row: 4.5, and per 512 blocks (row, kv head) of one round 0.0185 a key (from the caches; a decoded token's own keys come
 //     from memory, 2.6 as much); what goes beyond the first round costs 4 per 512 blocks more, and half a round's time once;
+//     every run of rows after the first costs 6 more (a launch of few blocks, behind the one before: a token over 500 - 900 keys 8 - 10);
 //   tiles: 4.2 + 0.67 per 32 keys of the longest, or 1.85 of that per step and slot once 512 blocks are more than one round.
 // (Heads of 64: 0.55 of the first, 0.57 per 32 keys.)  So a portion takes tiles about from where its rows fill a round, 512 blocks,
 // whatever is cached: 64 / 80 rows over 8 kv heads of 128 take, row by row and as tiles, 5.1 and 6.1 / 8.2 and 7.0 us without a context, 11.1
 // and 11.8 / 16.4 and 12.4 behind 256 keys, 40.5 and 46.7 / 70.1 and 46.1 behind 2000; over 4 kv heads 128 / 144 rows behind 2000 41.7 and 47.4 /
-// 74.9 and 47.3.  Over the 1500 points of single portions the rule is 1.2 % from the faster form on average, 5.4 % over the others.
+// 74.9 and 47.3.  20 decoded tokens over 800 keys, 500 rows, a token, 400 rows and a token take 105 row by row and 58 cut into three
+// runs beside tiles (over 4 kv heads 65 and 55); four times a token over 500 keys and 130 rows, and a token, 42 and 56.
+// Over the 1500 points of single portions the rule is 1.2 % from the faster form on average, over the others 5.3 %.
 inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_dim, int full_tile) {
     AttentionCut cut;
     const double size = head_dim == 64 ? 0.55 : 1.0;
@@ -70,7 +73,7 @@ inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_
         }
         return runs;
     };
-    auto by_rows_us = [&](int rows, double keys, int longest) {
+    auto by_rows_us = [&](int rows, double keys, int longest) {   // one run
         const double rounds = rows * static_cast<double>(kv_heads) / 512.0;
         return 4.5 + block_key_us * kv_heads * keys + (rounds > 1.0 ? 4.0 * size * (rounds - 1.0) + 0.5 * 512.0 * block_key_us * longest : 0.0);
     };
@@ -81,8 +84,13 @@ inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_
     auto tiles_us = [&](double steps, double block_steps) { return 4.2 + step_us * std::max(steps, 1.85 * block_steps / 512.0); };
     auto steps_of = [](double keys) { return keys / 32.0 + 0.5; };
     auto cost = [&](int most) {
-        double keys = 0.0, block_steps = 0.0, steps = 0.0;
-        int rows = 0, longest = 0;
+        double us = 0.0, keys = 0.0, block_steps = 0.0, steps = 0.0;
+        int rows = 0, longest = 0, runs = 0;
+        auto end_run = [&] {
+            if (rows) us += by_rows_us(rows, keys, longest) + (runs++ ? 6.0 : 0.0);
+            rows = longest = 0;
+            keys = 0.0;
+        };
         for (int r = 0; r < plan.R; ++r) {
             const int n = rows_of(r);
             if (n == 0) continue;
@@ -90,13 +98,15 @@ inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_
                 const int tiles = (2 * n + full_tile - 1) / full_tile;
                 steps = std::max(steps, steps_of(last_of(r)));
                 block_steps += tiles * kv_heads * steps_of(last_of(r) - 0.5 * n);
+                end_run();
             } else {
                 rows += n;
                 keys += keys_of(r);
                 longest = std::max(longest, last_of(r));
             }
         }
-        return (rows ? by_rows_us(rows, keys, longest) : 0.0) + (block_steps > 0.0 ? tiles_us(steps, block_steps) : 0.0);
+        end_run();
+        return us + (block_steps > 0.0 ? tiles_us(steps, block_steps) : 0.0);
     };
     constexpr int kNone = -1, kAll = 0x7FFFFFFF;
     int most = kNone;
@@ -109,7 +119,7 @@ inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_
         double best = cost(kNone);
         for (int cand : {gain, kAll}) {
             const double c = cost(cand);
-            if (c < best && runs_of(cand).size() <= 2) {   // (a launch per run and layer)
+            if (c < best) {
                 best = c;
                 most = cand;
             }
