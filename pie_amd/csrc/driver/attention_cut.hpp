@@ -37,13 +37,16 @@ inline bool evenly_long(const BatchPlan& plan, int row, int rows) {
 }
 
 // Decoded tokens run row by row; a portion of a prompt (8 rows or more) takes tiles where they cost less.  `full_tile`: the
-// rows of the kernel's larger tile, 0 where tiles cannot serve (masks, page and head sizes, decode batches).
+// rows of the kernel's larger tile, 0 where tiles cannot serve (masks, page and head sizes, decode batches); `one_byte`: the cache's
+// values.
 //
 // The costs, in microseconds, are fits to both kernels over portions of 8 - 512 rows behind 0 - 8000 keys, alone and beside 1 - 48
 // decoded tokens, and over several portions (32, 16 and 8 query heads over 8, 4 and 2 kv heads of 128 and 64, bf16 and one-byte
 // pools, whose decoding costs what their smaller size saves; 2178 points):
 //   row by row: 4.5, and per 512 blocks (row, kv head) of one round 0.0185 a key (from the caches; a decoded token's own keys come
 //     from memory, 2.6 as much); what goes beyond the first round costs 4 per 512 blocks more, and half a round's time once;
+//     a round over 3500 bf16 keys and more reads past the caches, 1.3 as much (64 rows over 8 kv heads behind 4000 keys 104, as tiles
+//     86; over a one-byte cache 88 and 91);
 //     every run of rows after the first costs 6 more (a launch of few blocks, behind the one before: a token over 500 - 900 keys 8 - 10);
 //   tiles: 4.2 + 0.67 per 32 keys of the longest, or 1.85 of that per step and slot once 512 blocks are more than one round.
 // (Heads of 64: 0.55 of the first, 0.57 per 32 keys.)  So a portion takes tiles about from where its rows fill a round, 512 blocks,
@@ -51,8 +54,8 @@ inline bool evenly_long(const BatchPlan& plan, int row, int rows) {
 // and 11.8 / 16.4 and 12.4 behind 256 keys, 40.5 and 46.7 / 70.1 and 46.1 behind 2000; over 4 kv heads 128 / 144 rows behind 2000 41.7 and 47.4 /
 // 74.9 and 47.3.  20 decoded tokens over 800 keys, 500 rows, a token, 400 rows and a token take 105 row by row and 58 cut into three
 // runs beside tiles (over 4 kv heads 65 and 55); four times a token over 500 keys and 130 rows, and a token, 42 and 56.
-// Over the 1500 points of single portions the rule is 1.2 % from the faster form on average, over the others 5.3 %.
-inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_dim, int full_tile) {
+// Over the 1500 points of single portions the rule is 1.1 % from the faster form on average, over the others 5.3 %.
+inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_dim, bool one_byte, int full_tile) {
     AttentionCut cut;
     const double size = head_dim == 64 ? 0.55 : 1.0;
     const double step_us = head_dim == 64 ? 0.57 : 0.67;
@@ -75,7 +78,8 @@ inline AttentionCut cut_attention(const BatchPlan& plan, int kv_heads, int head_
     };
     auto by_rows_us = [&](int rows, double keys, int longest) {   // one run
         const double rounds = rows * static_cast<double>(kv_heads) / 512.0;
-        return 4.5 + block_key_us * kv_heads * keys + (rounds > 1.0 ? 4.0 * size * (rounds - 1.0) + 0.5 * 512.0 * block_key_us * longest : 0.0);
+        const double far = !one_byte && rounds <= 1.0 && size * rounds * longest >= 3500.0 ? 1.3 : 1.0;
+        return 4.5 + far * block_key_us * kv_heads * keys + (rounds > 1.0 ? 4.0 * size * (rounds - 1.0) + 0.5 * 512.0 * block_key_us * longest : 0.0);
     };
     auto keys_of = [&](int r) {
         const int n = rows_of(r);

@@ -885,7 +885,8 @@ float pcg32_first_uniform(uint64_t seed) {
 void Executor::prepare_tiles(const BatchPlan& plan) {
     const ModelConfig& m = model_.cfg();
     const bool fits = !masked_ && !plan.pure_decode && page_size_ % 16 == 0 && (m.head_dim == 64 || m.head_dim == 128);
-    const AttentionCut cut = cut_attention(plan, m.kv_heads, m.head_dim, fits ? pie_hip_attn_prefill_tile_rows(m.q_heads, m.kv_heads) : 0);
+    const bool one_byte = kv_format_ != PIE_HIP_KV_BF16 && kv_format_ != PIE_HIP_KV_FP4_BLOCK;   // (4-bit pools are read as bf16)
+    const AttentionCut cut = cut_attention(plan, m.kv_heads, m.head_dim, one_byte, fits ? pie_hip_attn_prefill_tile_rows(m.q_heads, m.kv_heads) : 0);
     runs_ = cut.runs;
     tile_rows_ = cut.tile_rows;
     n_tiles_ = static_cast<int>(cut.tiles.size());
@@ -1277,7 +1278,7 @@ extern "C" int pie_hip_driver_experts_in_blocks(int format, long long routes, in
 // row_kv_len[i] keys.  out receives {tile height, tiles, runs}, (first row, rows) of each tile and (first row, rows, equally long) of each
 // run.  Returns the number of values, or -1 where they do not fit `cap`.
 extern "C" long long pie_hip_driver_attention_cut(const int* qo_indptr, int R, const int* row_kv_len, int q_heads, int kv_heads,
-                                                  int head_dim, int* out, size_t cap) {
+                                                  int head_dim, int one_byte, int* out, size_t cap) {
     using namespace pie_hip_driver;
     if (!qo_indptr || !row_kv_len || !out || R <= 0 || q_heads <= 0 || kv_heads <= 0) return -1;
     BatchPlan plan;
@@ -1286,7 +1287,7 @@ extern "C" long long pie_hip_driver_attention_cut(const int* qo_indptr, int R, c
     plan.qo_indptr.assign(qo_indptr, qo_indptr + R + 1);
     plan.row_kv_len.assign(row_kv_len, row_kv_len + plan.N);
     plan.max_kv_len = plan.N ? *std::max_element(plan.row_kv_len.begin(), plan.row_kv_len.end()) : 0;
-    const AttentionCut cut = cut_attention(plan, kv_heads, head_dim, pie_hip_attn_prefill_tile_rows(q_heads, kv_heads));
+    const AttentionCut cut = cut_attention(plan, kv_heads, head_dim, one_byte != 0, pie_hip_attn_prefill_tile_rows(q_heads, kv_heads));
     std::vector<int> v = {cut.tile_rows, static_cast<int>(cut.tiles.size()), static_cast<int>(cut.runs.size())};
     for (const auto& t : cut.tiles) v.insert(v.end(), {t.first, t.second});
     for (const RowRun& r : cut.runs) v.insert(v.end(), {r.row, r.rows, r.uniform ? 1 : 0});

@@ -165,7 +165,7 @@ def lib() -> C.CDLL:
         l.pie_hip_driver_experts_in_blocks.restype = C.c_int
         l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int]
         l.pie_hip_driver_attention_cut.restype = C.c_longlong
-        l.pie_hip_driver_attention_cut.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_size_t]
+        l.pie_hip_driver_attention_cut.argtypes = [C.c_void_p, C.c_int, C.c_void_p] + [C.c_int] * 4 + [C.c_void_p, C.c_size_t]
         l.pie_driver_hip_run_inproc.restype = C.c_int
         l.pie_driver_hip_run_inproc.argtypes = [C.c_int, C.POINTER(C.c_char_p), C.c_int, READY_FN,
                                                 C.c_void_p, InProcVTable]
@@ -481,13 +481,13 @@ def experts_in_blocks(kind: str, routes: int, experts: int) -> bool:
     return lib().pie_hip_driver_experts_in_blocks(_FORMATS.index(kind), routes, experts) == 1
 
 
-def attention_cut(requests: Sequence[tuple], q_heads: int, kv_heads: int, head_dim: int) -> dict:
+def attention_cut(requests: Sequence[tuple], q_heads: int, kv_heads: int, head_dim: int, one_byte: bool = False) -> dict:
     """Host-only: how the driver cuts a batch's attention.  requests: (cached tokens, tokens of this batch) each.  Returns the
     tiles' height, the (first row, rows) of each tile and the (first row, rows, equally long) of each run of other rows."""
     qo = np.concatenate([[0], np.cumsum([n for _, n in requests])]).astype(np.int32)
     lens = np.concatenate([np.arange(h + 1, h + n + 1) for h, n in requests]).astype(np.int32)
     out = np.zeros(16 + 5 * len(lens), np.int32)
-    n = lib().pie_hip_driver_attention_cut(qo.ctypes.data, len(requests), lens.ctypes.data, q_heads, kv_heads, head_dim,
+    n = lib().pie_hip_driver_attention_cut(qo.ctypes.data, len(requests), lens.ctypes.data, q_heads, kv_heads, head_dim, int(one_byte),
                                            out.ctypes.data, len(out))
     if n < 0:
         raise ValueError("attention_cut")
