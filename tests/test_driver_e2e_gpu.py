@@ -909,23 +909,27 @@ def test_start_up_kernel_measurement_keeps_results_within_rounding(gpu, oracle):
     assert np.max(np.abs(a - b)) <= 0.05 * np.max(np.abs(b)) + 1e-3
 
 
-@pytest.mark.parametrize("lens", [
-    # (cached tokens, tokens of this batch) per request; 32 query heads over 8 kv heads of 64: portions from about 130 rows
-    # on take tiles, single tokens and short portions the row kernel
-    [(20, 1), (37, 1), (48, 201)],             # decoded tokens ahead of a portion: one run of rows
-    [(20, 1), (0, 150), (33, 3), (64, 1)],     # on both sides of it: two
-    [(16, 1), (0, 140), (20, 1), (0, 7), (0, 170), (31, 1)],   # three runs: all row by row
-    [(0, 130), (0, 9), (47, 180)],             # portions only, a short one riding along
-    [(0, 16), (3, 17)],                        # portions only, too short for tiles
+@pytest.mark.parametrize("lens,tiled,runs", [
+    # (cached tokens, tokens of this batch) per request, the requests that take tiles and the runs of other rows
+    ([(20, 1), (37, 1), (48, 201)], [2], 1),                                            # decoded tokens ahead of a portion
+    ([(20, 1), (0, 400), (33, 3), (64, 1)], [1], 2),                                    # on both sides of it
+    ([(40, 1), (41, 1), (42, 1), (10, 300)], [3], 1),                                   # about equally long ones
+    ([(16, 1), (0, 400), (20, 1), (0, 390), (31, 1), (0, 7)], [1, 3], 3),               # and between two portions
+    ([(0, 130), (0, 9), (47, 180)], [0, 1, 2], 0),                                      # portions only, a short one riding along
+    ([(0, 16), (3, 17)], [], 1),                                                        # portions only, too short for tiles
+    ([(500, 1), (0, 130)] * 3 + [(400, 1)], [], 1),                                     # too short for so many runs
 ])
 @pytest.mark.parametrize("kv", ["auto", "fp8_per_token_head"])
-def test_portions_beside_decoded_tokens(gpu, oracle, lens, kv):
+def test_portions_beside_decoded_tokens(gpu, oracle, lens, tiled, runs, kv):
     """The rows a batch splits into tiles and single rows give what the same requests give alone, row by row: the same
     values in other orders of summation (bf16 activations: cosine >= 0.9999)."""
     from pie_amd import driver as drvmod
 
+    cut = drvmod.attention_cut(lens, 32, 8, 64, kv != "auto")
+    first = np.concatenate([[0], np.cumsum([n for _, n in lens])])
+    assert sorted({int(np.searchsorted(first, a, side="right")) - 1 for a, _ in cut["tiles"]}) == tiled and len(cut["runs"]) == runs
     kw = dict(quant="bf16", q_heads=32, kv_heads=8, head_dim=64, hidden=256, intermediate=512, vocab=512, total_pages=256,
-              max_forward_tokens=512, kv_cache_dtype=kv, tune_linears=False)
+              max_forward_tokens=1024, kv_cache_dtype=kv, tune_linears=False)
     rng = np.random.default_rng(sum(n for _, n in lens))
     with drvmod.Driver(toml_config(**kw)) as d:
         def frame(parts, samples):
