@@ -68,7 +68,8 @@ def test_tiles_match_oracle_and_row_kernel(gpu, oracle, hq, hk, d, ps, half):
 
 @pytest.mark.parametrize("fmt", ["fp8_e4m3", "int8_per_token_head", "fp8_per_token_head", "fp8_e5m2"])
 @pytest.mark.parametrize("hq,hk,d,ps", [(8, 2, 128, 16), (4, 4, 64, 16), (32, 8, 128, 32)])
-def test_tiles_over_one_byte_pools_match_the_oracle(gpu, oracle, fmt, hq, hk, d, ps):
+@pytest.mark.parametrize("half", [False, True])
+def test_tiles_over_one_byte_pools_match_the_oracle(gpu, oracle, fmt, hq, hk, d, ps, half):
     """The tile kernel over quantised pools against the oracle's attention over the dequantised
     values float(code) * scale (codes and scales written by the library's quantising write,
     itself bit-exact against the oracle's quantiser), to the bar of the bf16 pools; the per-row
@@ -80,7 +81,7 @@ def test_tiles_over_one_byte_pools_match_the_oracle(gpu, oracle, fmt, hq, hk, d,
     rng = np.random.default_rng(70 + hq + d)
     ctx = [200, 75, 33, 1]
     b = make_paged_batch(rng, ctx, hk, d, ps, f32_to_bf16=oracle.f32_to_bf16)
-    tr = ops.attn_prefill_tile_rows(hq, hk)
+    tr = ops.attn_prefill_tile_rows(hq, hk) // (2 if half else 1)
     chunks = [(120, 80), (0, 75), (0, 33), (0, 1)]
     row_begin, row_len, tile_start, tile_n = build_rows(b, ctx, chunks, tr)
     rows = len(row_begin)
@@ -120,17 +121,19 @@ def test_tiles_over_one_byte_pools_match_the_oracle(gpu, oracle, fmt, hq, hk, d,
     assert np.all(np.abs(got - want) <= 2.0 ** -7 * np.maximum(np.abs(want), np.abs(got)) + 2e-4)
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "fp8_per_token_head", "int8_per_token_head", "fp8_e5m2"])
 @pytest.mark.parametrize("d", [64, 128])
-def test_many_tiles_equal_few(gpu, d):
+def test_many_tiles_equal_few(gpu, d, fmt):
     """Above 512 blocks a block's waves walk all keys, up to there two groups of them take every other step and meet at the end:
     the same weights and sums in another order, one bf16 rounding each (the bar of the first test, twice).  Extents on and beside
-    the steps of 32 keys, the second group without a key, tiles of one row."""
+    the steps of 32 keys, tiles of one row; up to four steps, which one group takes alone, and beyond: the second group's last step
+    of one key, whole, and missing."""
     import torch
     from pie_amd import ops
 
     hq, hk, ps = 32, 8, 16
     tr = ops.attn_prefill_tile_rows(hq, hk) // 2
-    ctx = [1, 31, 32, 33, 64, 65, 97, 128, 700]
+    ctx = [1, 31, 32, 33, 64, 65, 97, 128, 129, 160, 161, 193, 700]
     pages = [-(-c // ps) for c in ctx]
     first = np.concatenate([[0], np.cumsum(pages)])
     row_begin = np.concatenate([np.full(c, f) for c, f in zip(ctx, first)]).astype(np.int32)
@@ -143,14 +146,25 @@ def test_many_tiles_equal_few(gpu, d):
     g = torch.Generator(device=gpu).manual_seed(63 + d)
     rnd = lambda *shape: torch.randn(*shape, generator=g, device=gpu).to(torch.bfloat16)
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
-    args = (rnd(at, hq, d), rnd(int(first[-1]), ps, hk, d), rnd(int(first[-1]), ps, hk, d),
-            torch.randperm(int(first[-1]), generator=g, device=gpu).int(), dev(row_begin), dev(row_len))
+    n = int(first[-1])
+    kp, vp = rnd(n, ps, hk, d), rnd(n, ps, hk, d)
+    ks = vs = None
+    if fmt != "bf16":
+        k_rows, v_rows = kp.reshape(-1, hk, d), vp.reshape(-1, hk, d)
+        kp, vp = (torch.zeros((n, ps, hk, d), dtype=torch.uint8, device=gpu) for _ in range(2))
+        if fmt != "fp8_e5m2":
+            ks, vs = (torch.ones((n, hk, ps), dtype=torch.float32, device=gpu) for _ in range(2))
+        ops.kv_write_quant(fmt, k_rows, v_rows, torch.arange(n * ps, device=gpu), kp, vp, ks, vs)
+    args = (fmt, rnd(at, hq, d), kp, vp, ks, vs, torch.randperm(n, generator=g, device=gpu).int(), dev(row_begin), dev(row_len))
     start, count = (dev(np.array(x, np.int32)) for x in zip(*tiles))
-    whole = ops.attention_prefill_tiles(*args, start, count, rows_per_tile=tr).float()
+    run = (lambda *tl: ops.attention_prefill_tiles_kvq(*args, *tl, rows_per_tile=tr)) if fmt != "bf16" else \
+        (lambda *tl: ops.attention_prefill_tiles(args[1], kp, vp, *args[6:], *tl, rows_per_tile=tr))
+    whole = run(start, count).float()
     half = len(tiles) // 2
+    assert (len(tiles) - half) * hk <= 512
     parts = torch.zeros_like(whole)
     for sl in (slice(0, half), slice(half, None)):
-        o = ops.attention_prefill_tiles(*args, start[sl].contiguous(), count[sl].contiguous(), rows_per_tile=tr).float()
-        for s, n in zip(start[sl].tolist(), count[sl].tolist()):
-            parts[s:s + n] = o[s:s + n]
+        o = run(start[sl].contiguous(), count[sl].contiguous()).float()
+        for a, m in zip(start[sl].tolist(), count[sl].tolist()):
+            parts[a:a + m] = o[a:a + m]
     assert torch.all((whole - parts).abs() <= 2.0 ** -7 * torch.maximum(whole.abs(), parts.abs()) + 2e-4)
