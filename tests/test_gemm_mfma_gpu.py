@@ -145,8 +145,8 @@ def test_gemm_split_k_beta_swiglu_one_hot(gpu, oracle, kind):
     assert np.array_equal(fused, unfused)
 
 
-# the fewest rows, the edges of the 256-row and 128-column blocks, step counts that leave 0 - 2 behind the unrolled loops, enough
-# blocks for 256 columns, whole rounds of those and a rest of 128 columns
+# the fewest rows, the edges of the 256-row and 128-column blocks, step counts that leave 0 - 2 behind the unrolled loops, many blocks
+# (of 128 columns, by the estimates; int8 and fp8 take the fourth in 256)
 WIDE = [(129, 16, 256), (255, 144, 320), (257, 272, 448), (300, 16656, 256), (600, 23056, 384)]
 
 
@@ -217,17 +217,69 @@ def test_wide_epilogues_and_shares(gpu, oracle, kind):
                        ops.swiglu_bf16(torch.cat([pairs[:, 0::2], pairs[:, 1::2]], dim=1).contiguous()))
 
 
+# Blocks of 256 columns, in all formats by the estimates: one round, the last block 144 columns wide and the last rows 44; 128 whole
+# columns of blocks (three rounds) and a rest of 128-column blocks behind them.  9 and 49 steps of 64 k-values (int4, whose steps are
+# pairs: 10 and 50).
 @pytest.mark.parametrize("kind", KINDS)
-def test_wide_refusals(gpu, oracle, kind):
-    """Shapes the blocks do not take are refused, not misread."""
+@pytest.mark.parametrize("M,N,K", [(300, 16528, 576), (1500, 32784, 3136)])
+def test_wide_blocks_of_256_columns(gpu, kind, M, N, K):
     import torch
     from pie_amd import ops
 
-    for M, N, K in [(256, 128, 192), (256, 128, 288)]:
-        act = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
-        _, mk = make_weight(oracle, np.random.default_rng(1), kind, N, K, G=32)
-        with pytest.raises(ops.KernelError):
-            ops.gemm_mfma_tiled(act, mk(gpu) if kind == "bf16" else ops.repack_mfma_tiles(mk(gpu)))
+    g = torch.Generator(device=gpu).manual_seed(730 + M)
+    rand = lambda lo, hi, *shape, dtype: torch.randint(lo, hi, shape, generator=g, device=gpu, dtype=dtype)
+    K = (K + 127) // 128 * 128 if kind == "int4b8" else K
+    if kind == "int4b8":
+        w = ops.int4b8_view(rand(-2**31, 2**31 - 1, N, K // 8, dtype=torch.int32), torch.rand(N, K // 128, generator=g, device=gpu).bfloat16(), 128)
+    elif kind == "bf16":
+        w = ops.WeightView("bf16", torch.randn(N, K, generator=g, device=gpu).bfloat16(), None, 0, N, K)
+    else:
+        codes = rand(-128, 128, N, K, dtype=torch.int8) if kind == "int8" else rand(0, 0x70, N, K, dtype=torch.uint8)
+        w = ops.WeightView(kind, codes, torch.rand(N, generator=g, device=gpu), 0, N, K)
+    t = w if kind == "bf16" else ops.repack_mfma_tiles(w)
+    act = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+    y0 = torch.randn(M, N, generator=g, device=gpu).bfloat16()
+    plain = ops.gemm_mfma_tiled(act, t)
+    summed = ops.gemm_mfma_tiled(act, t, y=y0.clone(), beta=1)
+    if kind == "bf16":
+        assert_near_exact(plain, act, w)
+        ref = plain.double() + y0.double()   # (the sum is rounded once, with the residual: a step of the plain result's rounding and its own)
+        assert ((summed.double() - ref).abs() <= 2.0 ** -8 * (plain.double().abs() + ref.abs())).all()
+        bias = torch.randn(N, generator=g, device=gpu)
+        rule = ops.glu(bias, 7.0, 1.702, 1.0)
+        assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1, rule=rule), ops.linear_glu("tiled", act, w.data, rule))
+    else:   # the same products summed in the same order
+        assert torch.equal(plain, ops.gemm_mfma(act, w))
+        assert torch.equal(summed, ops.gemm_mfma(act, w, y=y0.clone(), beta=1))
+        assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=ops.RELU2), ops.gemm_mfma(act, w, swiglu=ops.RELU2))
+    pairs = torch.cat([plain[:, 0::2], plain[:, 1::2]], dim=1).contiguous()
+    assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1), ops.swiglu_bf16(pairs))
+
+
+@pytest.mark.parametrize("kind,M,N,K,G", [
+    ("bf16", 256, 128, 192, 0), ("int8", 256, 128, 192, 0), ("fp8", 256, 128, 192, 0),        # K below four steps
+    ("int4b8", 256, 128, 128, 128),
+    ("bf16", 256, 128, 288, 0), ("int8", 256, 128, 288, 0), ("fp8", 256, 128, 288, 0),        # K off a step
+    ("int4b8", 256, 128, 320, 64),
+    ("int4b8", 256, 128, 256, 32), ("int4b8", 256, 128, 384, 96), ("int4b8", 40, 128, 256, 64),   # groups
+    ("int8", 256, 24, 256, 0), ("fp8", 64, 24, 256, 0), ("int4b8", 256, 24, 256, 128),        # columns without a tile-major copy
+])
+def test_wide_refusals(gpu, kind, M, N, K, G):
+    """Shapes the blocks do not take are refused by the call, not misread (and not by what prepares their weights).  40 rows of
+    groups of 64: the columns form does not take them, the blocks do."""
+    import torch
+    from pie_amd import ops
+
+    act = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
+    rows, words = -(-N // 256) * 256, K * 2   # (more than any reading of the shape could touch)
+    data = torch.zeros(rows * words, device=gpu, dtype=torch.uint8)
+    scale = torch.ones(rows * K, device=gpu, dtype=torch.bfloat16)
+    w = ops.WeightView(kind, data, None, 0, N, K) if kind == "bf16" else ops.WeightView(kind + "+tiled", data, scale, G, N, K)
+    if (M, K, G) == (40, 256, 64):
+        assert (ops.gemm_mfma_tiled(act, w) == 0).all()
+        return
+    with pytest.raises(ops.KernelError):
+        ops.gemm_mfma_tiled(act, w)
 
 
 @pytest.mark.parametrize("kind", ["int8", "fp8"])
