@@ -244,7 +244,8 @@ def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_row
     """The tiled grouped GEMM over quantised experts against the row-major passes of 16 rows: experts without routes, with
     one, with a block and one more; columns off the tile, gathered rows, row scales of both types, SwiGLU.  Both sum the
     same exact bf16 products in fp32, in other orders: a sum of K products differs by at most 2 K 2^-24 of the sum of their
-    magnitudes, a rounded result by that and half a bf16 step (2^-8) each."""
+    magnitudes, a rounded result by that and half a bf16 step (2^-8) each.  Int4: the passes scale a group's sum in fp32, the
+    blocks round every code times its scale to bf16, up to 2^-9 of each product more; the exact sums of either are checked."""
     import torch
     from pie_amd import ops
 
@@ -267,6 +268,8 @@ def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_row
             scale = scale.bfloat16()
         size = 0.004 * (128 if fmt == "int8" else 256)
     bound = K * 4.0 * size * 2 * K * 2.0 ** -24      # |act| < 4 but for one value in 16 000, whose share is far below the slack
+    if fmt == "int4b8":
+        bound += K * 4.0 * size * 2.0 ** -9
     for swiglu in (False, True):
         args = (act, rows, offs, fmt, w, scale, N, K, 257, G, swiglu)
         want = ops.moe_grouped_gemm(*args).float()
@@ -275,6 +278,18 @@ def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_row
             assert torch.all((got - want).abs() <= 4 * 2.0 ** -8 * want.abs() + 2.0 ** -6 * want.abs().amax())
         else:
             assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + bound)
+            if fmt == "int4b8":
+                codes = torch.stack([(w >> (4 * i)) & 0xF for i in range(8)], dim=-1).reshape(E, N, K).double() - 8.0
+                each = scale.double().repeat_interleave(G, dim=-1)
+                x = act.double()[rows.long()]
+                # (the passes' codes enter their products as 128 + n, 136 times the activations' sum leaves again)
+                for y, weights, offset in ((want, codes * each, 272.0), (got, (codes * each).bfloat16().double(), 0.0)):
+                    at = 0
+                    for e, n in enumerate(counts):
+                        ref = x[at:at + n] @ weights[e].T
+                        slack = K * 2.0 ** -23 * (x[at:at + n].abs() @ (weights[e].abs() + offset * each[e]).T)
+                        assert torch.all((y[at:at + n].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + slack)
+                        at += n
     assert torch.equal(ops.moe_grouped_gemm(act[rows.long()].contiguous(), None, offs, fmt, w, scale, N, K, 257, G, block_rows=block_rows),
                        ops.moe_grouped_gemm(act, rows, offs, fmt, w, scale, N, K, 257, G, block_rows=block_rows))
 
