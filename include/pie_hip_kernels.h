@@ -271,6 +271,9 @@ int pie_hip_gemm_mfma_glu(int format, const uint16_t* act_bf16, const void* weig
 int pie_hip_gemm_mfma_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale,
                             int scale_is_bf16, int group_size, uint16_t* y_bf16, int M, int N, int K, int beta,
                             int epilogue, const PieHipGlu* glu, void* workspace, size_t workspace_bytes, void* stream);
+/* Workspace with which pie_hip_gemm_mfma_tiled (and pie_hip_gemm_mfma over bf16 weights) may run any 129 to `most_rows` rows
+ * in the shares of K it would choose (0: none). */
+size_t pie_hip_gemm_mfma_tiled_workspace_bytes(int most_rows, int N, int K);
 /* Estimated microseconds of a tiled GEMM: over more than 128 rows the faster of pie_hip_gemm_mfma and, with a tile-major
  * copy (`tiled`) or bf16 weights, pie_hip_gemm_mfma_tiled; up to 128 rows the latter alone (1e30: not taken). */
 float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes);

@@ -315,16 +315,17 @@ void Executor::alloc_uniform() {
         for (size_t i = 0; i < T; ++i) iota[i] = static_cast<int64_t>(i);
         PIE_HIP_CHECK(hipMemcpy(iota_slots_, iota.data(), T * sizeof(int64_t), hipMemcpyHostToDevice));
     }
-    // fp32 partials of the split-K GEMM for decode batches of up to 128 rows (dense layers); prompts' K shares are at most two
-    // planes of 2048 x 4096
+    // fp32 partials of the split-K GEMM for decode batches of up to 128 rows (dense layers) and of prompts' K shares
     if (!model_.layers.empty()) {
         const LayerWeights& l0 = model_.layers[0];
         for (const Linear* w : {&l0.wqkv, &l0.wo, &l0.wgu, &l0.wdown})
             for (int rows : {64, 128})
                 if (w->data && w->K % 64 == 0)
                     gemm_ws_bytes_ = std::max(gemm_ws_bytes_, pie_hip_gemm_mfma_workspace_bytes(rows, w->N, w->K));
-        if (T > 128) gemm_ws_bytes_ = size_t(64) << 20;
         gemm_ws_bytes_ = std::min<size_t>(gemm_ws_bytes_, size_t(64) << 20);
+        for (const Linear* w : {&l0.wqkv, &l0.wo, &l0.router, m.num_experts ? &l0.wo : &l0.wgu, m.num_experts ? &l0.wo : &l0.wdown})
+            if (w->data)
+                gemm_ws_bytes_ = std::max(gemm_ws_bytes_, pie_hip_gemm_mfma_tiled_workspace_bytes(static_cast<int>(T), w->N, w->K));
         if (gemm_ws_bytes_) PIE_HIP_CHECK(hipMalloc(&gemm_ws_, gemm_ws_bytes_));
     }
 }

@@ -159,8 +159,12 @@ void Executor::alloc_stack() {
             for (int rows : {64, 128})
                 if (!m.f32() && w->data && w->K % 64 == 0)
                     gemm_ws_bytes_ = std::max(gemm_ws_bytes_, pie_hip_gemm_mfma_workspace_bytes(rows, w->N, w->K));
-    if (T > 128 && gemm_ws_bytes_) gemm_ws_bytes_ = size_t(64) << 20;
     gemm_ws_bytes_ = std::min<size_t>(gemm_ws_bytes_, size_t(64) << 20);
+    // prompts' K shares
+    for (StackLayer& l : model_.stack)
+        for (const Linear* w : {&l.w_in, &l.w_uq, &l.wo, &l.w_gate1, &l.w_gate2, l.spec.moe.experts ? &l.wo : &l.w_up, l.spec.moe.experts ? &l.wo : &l.w_down})
+            if (!m.f32() && w->data)
+                gemm_ws_bytes_ = std::max(gemm_ws_bytes_, pie_hip_gemm_mfma_tiled_workspace_bytes(static_cast<int>(T), w->N, w->K));
     if (gemm_ws_bytes_) PIE_HIP_CHECK(hipMalloc(&gemm_ws_, gemm_ws_bytes_));
     // partial results of the attentions' splits: a plan with more than one split has at most 512 (tile,
     // split) blocks of 32 (token, head) pairs (latent) or 16 heads (grouped)

@@ -883,6 +883,16 @@ Plan plan_of(const Rates& r, int M, int N, int K, size_t ws_bytes) {
     }
     return best;
 }
+// Most bytes the shares of any number of rows from 129 to `most_rows` can take: blocks * shares <= 256 bounds them by 32 MiB.
+size_t shares_bytes(int most_rows, int N, int K) {
+    const int steps = K / kStepK, cols = (N + 127) / 128;
+    size_t bytes = 0;
+    for (int rows = 1; most_rows > 128 && rows <= (most_rows + kRows - 1) / kRows && rows * cols <= 128; ++rows) {
+        const int s = std::min({8, 256 / (rows * cols), steps / 8});
+        if (s > 1) bytes = std::max(bytes, static_cast<size_t>(s) * std::min(most_rows, rows * kRows) * N * sizeof(float));
+    }
+    return bytes;
+}
 template <int KVF, int NG, int S>
 int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
     constexpr size_t smem = S * static_cast<size_t>(kExpertRows) * kStepK * 2;
@@ -1019,6 +1029,10 @@ extern "C" float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group
     if (M <= 128 && !(tiled && pie_hip::columns_fit(format, M, N, K, group_size))) return 1e30f;
     const double wide = tiled || format == PIE_HIP_FMT_BF16 ? pie_hip::gemm_wide_us(format, M, N, K, group_size, workspace_bytes) : 1e30;
     return static_cast<float>(std::min(tiles, wide));
+}
+
+extern "C" size_t pie_hip_gemm_mfma_tiled_workspace_bytes(int most_rows, int N, int K) {
+    return N > 0 && K > 0 ? pie_hip::shares_bytes(most_rows, N, K) : 0;
 }
 
 extern "C" int pie_hip_gemm_mfma_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale, int scale_is_bf16,

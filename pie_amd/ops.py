@@ -638,6 +638,12 @@ def gemm_mfma_us(kind: str, M: int, N: int, K: int, group: int, tiled: bool, wor
     return float(lib.pie_hip_gemm_mfma_us(FMT[kind], M, N, K, group, int(tiled), C.c_size_t(workspace_bytes)))
 
 
+def gemm_mfma_tiled_workspace_bytes(most_rows: int, N: int, K: int) -> int:
+    lib = kernels()
+    lib.pie_hip_gemm_mfma_tiled_workspace_bytes.restype = C.c_size_t
+    return int(lib.pie_hip_gemm_mfma_tiled_workspace_bytes(most_rows, N, K))
+
+
 def gemm_mfma_workspace_bytes(M: int, N: int, K: int) -> int:
     lib = kernels()
     lib.pie_hip_gemm_mfma_workspace_bytes.restype = C.c_size_t

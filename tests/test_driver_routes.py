@@ -59,6 +59,24 @@ def test_int4_experts_keep_fp32_scales(experts):
         assert [drv.experts_in_blocks(kind, n * experts, experts) for n in (first - 1, first, 500)] == [False, True, True]
 
 
+def test_workspace_of_shares_is_what_the_shares_take():
+    """With the bytes the library names no row count up to the limit is estimated slower than with all the memory there is, and
+    they are no more than 32 MiB, none where no shape takes shares."""
+    from pie_amd import ops
+
+    rng = np.random.default_rng(12)
+    assert ops.gemm_mfma_tiled_workspace_bytes(2048, 4096, 4096) == 32 << 20
+    assert ops.gemm_mfma_tiled_workspace_bytes(128, 4096, 4096) == 0          # (no prompts)
+    assert ops.gemm_mfma_tiled_workspace_bytes(4096, 28672, 4096) == 0        # (more than half a round of blocks in one row of them)
+    for _ in range(60):
+        top, N, K = int(rng.integers(129, 4097)), int(rng.integers(1, 1200)) * 16, int(rng.integers(4, 240)) * 64
+        named = ops.gemm_mfma_tiled_workspace_bytes(top, N, K)
+        assert named <= 32 << 20
+        for M in rng.integers(129, top + 1, 20):
+            for kind in ("int8", "bf16"):
+                assert ops.gemm_mfma_us(kind, int(M), N, K, 0, True, named) == ops.gemm_mfma_us(kind, int(M), N, K, 0, True, 1 << 40)
+
+
 # microseconds of one layer's attention over a bf16 cache on an MI355X, row by row and as tiles: a portion of 32, 64, 112, 160 and 256
 # rows by (query heads, kv heads, head size) and cached tokens
 MEASURED_ROWS = (32, 64, 112, 160, 256)
