@@ -60,7 +60,7 @@ int fmt_code(Quant q) {
 // (+3 of prologue) at 1.06 / 1.36 us with two blocks per CU, per round of 512 blocks, plus ~15 us
 // for the second kernel and the partials.
 // More than 128 rows: the tiled GEMM's two forms say themselves what they take (pie_hip_gemm_mfma_us); over 40 shapes of 160 -
-// 4096 rows in three formats the choice loses 0.5 % against the fastest of the three each time.
+// 4096 rows in three formats a choice by these estimates loses 0.5 % against the fastest of the three each time.
 enum class GemmPath { Skinny, Tiled, TiledSplitK, Wide };
 bool tile_major(const Linear& w) { return w.data_tiled && (w.kind != Quant::Int4b8 || w.scale_tiled); }
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
@@ -1277,22 +1277,28 @@ extern "C" int pie_hip_driver_experts_in_blocks(int format, long long routes, in
 
 // And for a batch's attention: the rows of request r are qo_indptr[r] .. qo_indptr[r + 1] (of R requests), row i sees
 // row_kv_len[i] keys.  out receives {tile height, tiles, runs}, (first row, rows) of each tile and (first row, rows, equally long) of each
-// run.  Returns the number of values, or -1 where they do not fit `cap`.
+// run.  Returns the number of values, or -1 where they do not fit `cap` or the lists make no batch.
 extern "C" long long pie_hip_driver_attention_cut(const int* qo_indptr, int R, const int* row_kv_len, int q_heads, int kv_heads,
                                                   int head_dim, int one_byte, int* out, size_t cap) {
     using namespace pie_hip_driver;
-    if (!qo_indptr || !row_kv_len || !out || R <= 0 || q_heads <= 0 || kv_heads <= 0) return -1;
-    BatchPlan plan;
-    plan.R = R;
-    plan.N = qo_indptr[R];
-    plan.qo_indptr.assign(qo_indptr, qo_indptr + R + 1);
-    plan.row_kv_len.assign(row_kv_len, row_kv_len + plan.N);
-    plan.max_kv_len = plan.N ? *std::max_element(plan.row_kv_len.begin(), plan.row_kv_len.end()) : 0;
-    const AttentionCut cut = cut_attention(plan, kv_heads, head_dim, one_byte != 0, pie_hip_attn_prefill_tile_rows(q_heads, kv_heads));
-    std::vector<int> v = {cut.tile_rows, static_cast<int>(cut.tiles.size()), static_cast<int>(cut.runs.size())};
-    for (const auto& t : cut.tiles) v.insert(v.end(), {t.first, t.second});
-    for (const RowRun& r : cut.runs) v.insert(v.end(), {r.row, r.rows, r.uniform ? 1 : 0});
-    if (v.size() > cap) return -1;
-    std::copy(v.begin(), v.end(), out);
-    return static_cast<long long>(v.size());
+    if (!qo_indptr || !row_kv_len || !out || R <= 0 || q_heads <= 0 || kv_heads <= 0 || qo_indptr[0] != 0) return -1;
+    for (int r = 0; r < R; ++r)
+        if (qo_indptr[r + 1] < qo_indptr[r]) return -1;
+    try {
+        BatchPlan plan;
+        plan.R = R;
+        plan.N = qo_indptr[R];
+        plan.qo_indptr.assign(qo_indptr, qo_indptr + R + 1);
+        plan.row_kv_len.assign(row_kv_len, row_kv_len + plan.N);
+        plan.max_kv_len = plan.N ? *std::max_element(plan.row_kv_len.begin(), plan.row_kv_len.end()) : 0;
+        const AttentionCut cut = cut_attention(plan, kv_heads, head_dim, one_byte != 0, pie_hip_attn_prefill_tile_rows(q_heads, kv_heads));
+        std::vector<int> v = {cut.tile_rows, static_cast<int>(cut.tiles.size()), static_cast<int>(cut.runs.size())};
+        for (const auto& t : cut.tiles) v.insert(v.end(), {t.first, t.second});
+        for (const RowRun& r : cut.runs) v.insert(v.end(), {r.row, r.rows, r.uniform ? 1 : 0});
+        if (v.size() > cap) return -1;
+        std::copy(v.begin(), v.end(), out);
+        return static_cast<long long>(v.size());
+    } catch (const std::exception&) {
+        return -1;
+    }
 }

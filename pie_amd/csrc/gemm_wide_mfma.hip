@@ -16,7 +16,8 @@
 //   2048 x 28672 x 4096   546 / 436,  519 / 425,  476 / 410      2048 x 4096 x 14336   245 / 214,  231 / 201,  202 / 190
 //   1024 x 28672 x 4096   302 / 229,  275 / 224,  295 / 206       489 x 4096 x 14336    84 /  71,   93 /  68,   97 /  64
 //   1319 x 16384 x 2048   125 / 110,  119 / 109,  114 /  98      1024 x 6144 x 4096     71 /  61,   70 /  59,   60 /  53
-// (the fourth in K shares; int4 and fp8 there against the skinny GEMM).
+// (the fourth in K shares; int4 and fp8 there against the skinny GEMM, which the driver's int4 prompts of such shapes keep:
+// these blocks round an int4 code times its scale to bf16, the skinny GEMM scales a group's sum in fp32).
 #include "gemm_args.hip.h"
 
 #include <algorithm>
