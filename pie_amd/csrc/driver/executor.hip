@@ -149,7 +149,7 @@ bool routes_to_gemv(const Linear& w, int M, bool has_norm, size_t ws_bytes) {
 // (norm as its own kernel into `norm_tmp`): the matrix-core skinny GEMM, which streams the
 // weights once per 16 rows, or the tiled matrix-core GEMM where its cost model wins; shapes those do
 // not take fall back to the GEMV path.
-// `force`: -1 = pick (the start-up measurement when there is one, else the cost model); 0..3 = that
+// `force`: -1 = pick (the start-up measurement when there is one, else the cost model); 0..4 = that
 // kernel whatever the costs (the tuner's own launches).  Returns false when a forced kernel does
 // not take the shape.
 }  // namespace
@@ -378,7 +378,7 @@ size_t Executor::scale_page_bytes() const {
 
 // Start-up measurement of the decoder linears' candidate kernels.  For every role (q|k|v, wo,
 // gate|up, down) and a ladder of row counts the GEMV (2-4 rows), the skinny GEMM and the tiled GEMM
-// (17-128 rows; in K shares where the workspace allows; over the tile-major copy of one-byte weights) run over the weights of successive layers
+// (17-128 rows; in K shares where the workspace allows; over the tile-major copy where the model expects that) run over the weights of successive layers
 // (so that they come from HBM, as in a forward pass) on zeroed activations; the fastest goes into
 // every layer's table for the row counts up to the next rung.
 void Executor::tune_linears() {
