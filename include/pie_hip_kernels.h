@@ -267,7 +267,8 @@ int pie_hip_gemm_mfma_glu(int format, const uint16_t* act_bf16, const void* weig
  * (pie_hip_repack_mfma_tiles[_int4]; int4 scales from pie_hip_repack_scale_tiles; N % 16 == 0): K % 64 == 0 (int4: 128,
  * groups a power of two from 64 on), K >= 256, act and weight on 16-byte boundaries.  With a workspace (of any size) few
  * blocks over a long K run in shares of K.  Up to 128 rows of int8 or fp8 weights run in blocks of 64 columns, any
- * K % 64 == 0; 17 to 48 rows of int4 weights (groups from 128 on) in blocks of 128, any K % 128 == 0.  `epilogue` and `glu` as in pie_hip_gemm_mfma_glu. */
+ * K % 64 == 0; 17 to 48 rows of int4 weights (groups from 128 on, any K % 128 == 0) are pie_hip_gemm_groups_tiled's.  `epilogue` and `glu` as
+ * in pie_hip_gemm_mfma_glu. */
 int pie_hip_gemm_mfma_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale,
                             int scale_is_bf16, int group_size, uint16_t* y_bf16, int M, int N, int K, int beta,
                             int epilogue, const PieHipGlu* glu, void* workspace, size_t workspace_bytes, void* stream);
@@ -277,6 +278,20 @@ size_t pie_hip_gemm_mfma_tiled_workspace_bytes(int most_rows, int N, int K);
 /* Estimated microseconds of a tiled GEMM: over more than 128 rows the faster of pie_hip_gemm_mfma and, with a tile-major
  * copy (`tiled`) or bf16 weights, pie_hip_gemm_mfma_tiled; up to 128 rows the latter alone (1e30: not taken). */
 float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes);
+
+/* pie_hip_gemm_skinny_tiled's arithmetic (int4b8 codes multiplied as they are, a group's sum scaled in fp32) in blocks of up to 64 rows x 128
+ * columns, over the tile-major copy: K % 128 == 0, N % 16 == 0, groups a power of two from 128 on, act and weight on 16-byte and scales
+ * on 8-byte boundaries.  With a workspace few blocks over a long K run in shares of K, as many as it holds of 4 M N bytes each.
+ * `epilogue` and `glu` as in pie_hip_gemm_mfma_glu; the estimate in microseconds (1e30: not taken). */
+int pie_hip_gemm_groups_tiled(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, uint16_t* y_bf16,
+                              int M, int N, int K, int beta, int epilogue, const PieHipGlu* glu, void* workspace,
+                              size_t workspace_bytes, void* stream);
+float pie_hip_gemm_groups_us(int M, int N, int K, int group_size, size_t workspace_bytes);
+/* pie_hip_qkv_rope_skinny_tiled in that form (q_out and the pools on 8-byte boundaries). */
+int pie_hip_qkv_rope_groups_tiled(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, int M, int K,
+                                  const float* rope_table, const int64_t* kv_slots, uint16_t* q_out, uint16_t* k_pages,
+                                  uint16_t* v_pages, int num_q_heads, int num_kv_heads, int head_dim, int pairing,
+                                  void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * MoE grouped weight-only GEMM: one skinny problem per expert in a single launch.

@@ -63,8 +63,11 @@ int fmt_code(Quant q) {
 // 4096 rows in three formats a choice by these estimates loses 0.5 % against the fastest of the three each time.
 enum class GemmPath { Skinny, Tiled, TiledSplitK, Wide };
 bool tile_major(const Linear& w) { return w.data_tiled && (w.kind != Quant::Int4b8 || w.scale_tiled); }
-GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
-    if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
+struct Skinny {
+    int p2, wpasses;        // passes of the wave-private form, and as the power of two they cost
+    double wave_form, us;
+};
+Skinny skinny_cost(const Linear& w, int M) {
     const int passes = (M + 15) / 16;
     // the wave-private form runs its passes side by side: cost steps at powers of two; above 32
     // rows a pass covers 32 rows and costs 1.38 of a 16-row one
@@ -74,12 +77,24 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     // (past eight passes the machine is full: the cost grows in proportion)
     const double data = static_cast<double>(w.data_bytes());
     const double wave_form = (M > 32 ? 1.38 : 1.0) * (p2 <= 8 ? 1.0 + 0.52 * (p2 - 1) : (1.0 + 0.52 * 7) * wpasses / 8.0);
-    const double skinny = w.data_tiled ? 5.0 + data / 3.8e6 * wave_form : 5.0 + data / 2.8e6 * (1.0 + 0.85 * (passes - 1));
+    return {p2, wpasses, wave_form, w.data_tiled ? 5.0 + data / 3.8e6 * wave_form : 5.0 + data / 2.8e6 * (1.0 + 0.85 * (passes - 1))};
+}
+// Microseconds of int4 weights in blocks of up to 64 rows, which scale a group's sum in fp32 as the skinny GEMM does (1e30: not
+// taken).  Where the skinny GEMM is chosen and these are estimated faster, they run in its place: 321 rows of 6144 x 4096 32 us
+// against 70, of 4096 x 14336 58 against 69, of 4096 x 4096 21 against 26, 96 of 28672 x 4096 35 against 50.
+double groups_cost(const Linear& w, int M, size_t ws_bytes) {
+    return M >= 17 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
+}
+bool in_groups(const Linear& w, int M, size_t ws_bytes) { return groups_cost(w, M, ws_bytes) < skinny_cost(w, M).us; }
+GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
+    if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
+    const auto [p2, wpasses, wave_form, skinny] = skinny_cost(w, M);
+    const double data = static_cast<double>(w.data_bytes()), groups = groups_cost(w, M, ws_bytes);
     const int steps = w.K / 64;
     if (M > 128) {
         // Int4 weights: the skinny GEMM multiplies the codes and scales a group's sum in fp32, the blocks round every code times
         // its scale to bf16 first, which takes a product's error from 0.0017 of its norm to 0.0022 (K of 4096, groups of 128).
-        // So int4 weights leave the skinny GEMM only where it is estimated slower than 128-row tiles, at 512 of them to a
+        // So int4 weights leave fp32 scales only where the skinny GEMM is estimated slower than 128-row tiles, at 512 of them to a
         // round: 28672 x 4096 at once, 6144 x 4096 from 481 rows on, 4096 x 4096 from 705, 4096 x 14336 from 769.  (At 381 rows of
         // these skinny / wide blocks take 169 / 120, 45 / 42, 28 / 31 and 73 / 68 us.)
         const double high = static_cast<double>((w.N + 127) / 128) * ((M + 127) / 128);
@@ -92,7 +107,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const int fmt = fmt_code(w.kind);
         const double tiles = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
         const double blocks = tile_major(w) ? pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes) : tiles;
-        if (rows_us < blocks) return GemmPath::Skinny;
+        if (rows_us < blocks || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
         return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
     }
     const double tiles = static_cast<double>((w.N + 127) / 128);
@@ -106,6 +121,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     }
     const double columns = tile_major(w) ? pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, 0) : 1e30;
     if (columns < std::min({skinny, split, tiled})) return GemmPath::Wide;
+    if (groups < std::min({skinny, split, tiled})) return GemmPath::Skinny;
     if (split < skinny && split < tiled) return GemmPath::TiledSplitK;
     return tiled < skinny ? GemmPath::Tiled : GemmPath::Skinny;
 }
@@ -189,6 +205,12 @@ bool linear_fused(const Linear& w, const uint16_t* act, const uint16_t* norm_w, 
                               : tuned == 3 ? GemmPath::TiledSplitK
                               : tuned == 4 ? GemmPath::Wide
                                            : pick_gemm(w, M, gemm_ws_bytes);   // (forced row limit, GEMV refusal)
+        if (path == GemmPath::Skinny && in_groups(w, M, gemm_ws_bytes)) {
+            const int sg = pie_hip_gemm_groups_tiled(a, w.data_tiled, w.scale_tiled, w.group, y, M, w.N, w.K, beta, swiglu, glu,
+                                                     gemm_ws, gemm_ws_bytes, s);
+            if (sg == PIE_HIP_OK) return true;
+            if (sg != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sg);
+        }
         if (path == GemmPath::Wide) {
             const int sw = pie_hip_gemm_mfma_tiled(fmt, a, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, sbf, w.group, y, M,
                                                    w.N, w.K, beta, swiglu, glu, gemm_ws, gemm_ws_bytes, s);
@@ -710,10 +732,14 @@ void Executor::body(int N, int S, int max_kv_len) {
             if (fused_rope && !w.q_norm && w.wqkv.data_tiled &&
                 (tuned_qkv >= 0 ? tuned_qkv <= 1 : pick_gemm(w.wqkv, N, gemm_ws_bytes_) == GemmPath::Skinny)) {
                 PIE_KERNEL(pie_hip_rmsnorm(x_, w.attn_norm, xn_, N, H, m.rms_eps, s));
-                const int st = pie_hip_qkv_rope_skinny_tiled(
-                    fmt_code(w.wqkv.kind), xn_, w.wqkv.data_tiled,
-                    w.wqkv.scale_tiled ? w.wqkv.scale_tiled : w.wqkv.scale, w.wqkv.scale_bf16 ? 1 : 0,
-                    w.wqkv.group, N, H, rope_tab_, slots, q_, k_pool_[l], v_pool_[l], hq, hk, d, pairing, s);
+                const int st =
+                    in_groups(w.wqkv, N, gemm_ws_bytes_)
+                        ? pie_hip_qkv_rope_groups_tiled(xn_, w.wqkv.data_tiled, w.wqkv.scale_tiled, w.wqkv.group, N, H, rope_tab_, slots, q_,
+                                                        k_pool_[l], v_pool_[l], hq, hk, d, pairing, gemm_ws_, gemm_ws_bytes_, s)
+                        : pie_hip_qkv_rope_skinny_tiled(fmt_code(w.wqkv.kind), xn_, w.wqkv.data_tiled,
+                                                        w.wqkv.scale_tiled ? w.wqkv.scale_tiled : w.wqkv.scale, w.wqkv.scale_bf16 ? 1 : 0,
+                                                        w.wqkv.group, N, H, rope_tab_, slots, q_, k_pool_[l], v_pool_[l], hq, hk, d,
+                                                        pairing, s);
                 if (st == PIE_HIP_OK) done = true;
                 else if (st != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(st);
             }

@@ -23,6 +23,79 @@ struct GemmArgs {
     int aligned;   // wide form: y starts at a multiple of 8 bytes
 };
 
+#define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
+// s_waitcnt lgkmcnt(0) alone and vmcnt(n) alone, n < 64 (gfx9 encoding).  The no-op keeps the compiler's own wait for a
+// value loaded before from being merged into this one: merged, it counts transfers into LDS as unordered and waits for all.
+#define PIE_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
+#define PIE_WAIT_VM(n)                              \
+    do {                                            \
+        __builtin_amdgcn_sched_barrier(0);          \
+        __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14)); \
+        asm volatile("s_nop 0");                    \
+        __builtin_amdgcn_sched_barrier(0);          \
+    } while (0)
+
+#define PIE_FENCE() __builtin_amdgcn_sched_barrier(0)
+#define PIE_MEET()                         \
+    do {                                   \
+        PIE_FENCE();                       \
+        asm volatile("" ::: "memory");     \
+        __builtin_amdgcn_s_barrier();      \
+        asm volatile("" ::: "memory");     \
+        PIE_FENCE();                       \
+    } while (0)
+
+__device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
+    __builtin_amdgcn_global_load_lds(from, PIE_LDS_PTR(to), 16, 0, 0);
+}
+
+// The epilogue of row m, columns n .. n + 3 (those below N; n is a multiple of 4): SwiGLU over (gate, up) pairs rounded to
+// bf16 first, or a pointwise function and the residual.
+__device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, float* v) {
+    const int N = a.N, nout = a.swiglu ? N / 2 : N;
+    const bool whole = N % 4 == 0 && a.aligned;   // one 8- (SwiGLU: 4-) byte store
+    if (a.swiglu) {
+        uint16_t o[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            float g = v[2 * r], u = v[2 * r + 1];
+            if (a.glu.bias) {
+                g += a.glu.bias[min(n + 2 * r, N - 1)];
+                u += a.glu.bias[min(n + 2 * r + 1, N - 1)];
+            }
+            g = bf16_bits_to_f32(f32_to_bf16_bits(g));
+            u = bf16_bits_to_f32(f32_to_bf16_bits(u));
+            o[r] = f32_to_bf16_bits(glu_value(g, u, a.glu));
+        }
+        uint16_t* p = a.y + static_cast<size_t>(m) * nout + n / 2;
+        if (whole) {
+            *reinterpret_cast<uint32_t*>(p) = o[0] | static_cast<uint32_t>(o[1]) << 16;
+        } else {
+            p[0] = o[0];
+            if (n + 2 < N) p[1] = o[1];
+        }
+        return;
+    }
+    uint16_t* p = a.y + static_cast<size_t>(m) * nout + n;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = epilogue_pointwise<true>(v[r], a.pointwise);
+    if (whole) {
+        if (a.beta) {
+            const u32x2_t old = *reinterpret_cast<const u32x2_t*>(p);
+            v[0] += bf16_lo(old.x);
+            v[1] += bf16_hi(old.x);
+            v[2] += bf16_lo(old.y);
+            v[3] += bf16_hi(old.y);
+        }
+        *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else {
+        for (int r = 0; r < 4 && n + r < N; ++r) {
+            if (a.beta) v[r] += bf16_bits_to_f32(p[r]);
+            p[r] = f32_to_bf16_bits(v[r]);
+        }
+    }
+}
+
 // The problem and the rows [m0, m1) of block row `t` when problems are cut into blocks of `rows` rows one after
 // another; false behind the last.  Every lane of the wave calls it and gets the same answer.
 __device__ __forceinline__ bool grouped_place(const int32_t* __restrict__ offsets, int problems, int rows, int t, int lane,
@@ -67,6 +140,10 @@ int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, si
 // Experts' rows gathered by route, over tile-major fp8 or int8 weights.
 int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t stream);
 double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes);
+// Int4 weights with fp32 group scales, tile-major, of at least 128 values a group, in blocks of up to 64 rows; a workspace lets few blocks over a long K run
+// in shares.
+int launch_gemm_groups(const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream);
+double gemm_groups_us(int M, int N, int K, int group_size, size_t ws_bytes);
 double gemm_tiles_us(int format, int M, int N, int K);
 
 }  // namespace pie_hip

@@ -32,28 +32,6 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 constexpr int kRows = 256, kStepK = 64, kWaves = 8;
 constexpr int kActVecs = kRows * kStepK / 8;   // 16-byte vectors of an activation stage
 
-#define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
-// s_waitcnt lgkmcnt(0) alone and vmcnt(n) alone, n < 64 (gfx9 encoding).  The no-op keeps the compiler's own wait for a
-// value loaded before from being merged into this one: merged, it counts transfers into LDS as unordered and waits for all.
-#define PIE_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
-#define PIE_WAIT_VM(n)                              \
-    do {                                            \
-        __builtin_amdgcn_sched_barrier(0);          \
-        __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14)); \
-        asm volatile("s_nop 0");                    \
-        __builtin_amdgcn_sched_barrier(0);          \
-    } while (0)
-
-#define PIE_FENCE() __builtin_amdgcn_sched_barrier(0)
-#define PIE_MEET()                         \
-    do {                                   \
-        PIE_FENCE();                       \
-        asm volatile("" ::: "memory");     \
-        __builtin_amdgcn_s_barrier();      \
-        asm volatile("" ::: "memory");     \
-        PIE_FENCE();                       \
-    } while (0)
-
 // ---- what a thread stages of a step's weights: V (32 or 16) of them, loaded from the tile-major copy (blocks of 1 KiB, 16 rows
 // by 64 bytes, lane 16 q + j its bytes 16 q .. 16 q + 15 of row j), as V / 8 16-byte vectors of bf16; wave w takes the
 // tiles of 16 rows from w V / 16 on.  (Row-major, a wave's load touches 32 rows' cache lines for 32 bytes each and took
@@ -145,53 +123,6 @@ struct WBf16 {
 
 // position of granule g of tile row r (in 16-byte vectors)
 __device__ __forceinline__ int swz(int r, int g) { return r * 8 + (g ^ ((r >> 1) & 7)); }
-
-// The epilogue of row m, columns n .. n + 3 (those below N; n is a multiple of 4): SwiGLU over (gate, up) pairs rounded to
-// bf16 first, or a pointwise function and the residual.
-__device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, float* v) {
-    const int N = a.N, nout = a.swiglu ? N / 2 : N;
-    const bool whole = N % 4 == 0 && a.aligned;   // one 8- (SwiGLU: 4-) byte store
-    if (a.swiglu) {
-        uint16_t o[2];
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            float g = v[2 * r], u = v[2 * r + 1];
-            if (a.glu.bias) {
-                g += a.glu.bias[min(n + 2 * r, N - 1)];
-                u += a.glu.bias[min(n + 2 * r + 1, N - 1)];
-            }
-            g = bf16_bits_to_f32(f32_to_bf16_bits(g));
-            u = bf16_bits_to_f32(f32_to_bf16_bits(u));
-            o[r] = f32_to_bf16_bits(glu_value(g, u, a.glu));
-        }
-        uint16_t* p = a.y + static_cast<size_t>(m) * nout + n / 2;
-        if (whole) {
-            *reinterpret_cast<uint32_t*>(p) = o[0] | static_cast<uint32_t>(o[1]) << 16;
-        } else {
-            p[0] = o[0];
-            if (n + 2 < N) p[1] = o[1];
-        }
-        return;
-    }
-    uint16_t* p = a.y + static_cast<size_t>(m) * nout + n;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = epilogue_pointwise<true>(v[r], a.pointwise);
-    if (whole) {
-        if (a.beta) {
-            const u32x2_t old = *reinterpret_cast<const u32x2_t*>(p);
-            v[0] += bf16_lo(old.x);
-            v[1] += bf16_hi(old.x);
-            v[2] += bf16_lo(old.y);
-            v[3] += bf16_hi(old.y);
-        }
-        *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    } else {
-        for (int r = 0; r < 4 && n + r < N; ++r) {
-            if (a.beta) v[r] += bf16_bits_to_f32(p[r]);
-            p[r] = f32_to_bf16_bits(v[r]);
-        }
-    }
-}
 
 template <class FMT, int COLS>
 struct Wide {
@@ -436,9 +367,6 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
 // Bound by the weights: 128 fp8 experts of 1536 x 2048 at 82 routes 116 us (402 MB; the tiles through LDS 147, four routes per
 // expert 98), of 2048 x 768 74 (84 through LDS).
 constexpr int kExpertRows = 128;
-__device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
-    __builtin_amdgcn_global_load_lds(from, PIE_LDS_PTR(to), 16, 0, 0);
-}
 // The same for one matrix and up to 128 rows (64 columns per block, two groups of waves that take the steps in turn and meet at the
 // end: a block is alone on its CU, and one wave per SIMD waits out every step's chain): 77 rows of 16384 x 2048 int8 16.7 us, fp8
 // 16.4 (128 x 128 tiles 27 and 26, passes of 32 rows 26 and 24; one group 18.4 and 17.7), 40 rows 13.7 and 11.3 (18.5 and 16.6).
@@ -620,182 +548,6 @@ __global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(
     }
 }
 
-// ---- 17 to 48 rows of int4 weights: the columns form with a scale group's products summed before they are scaled -------------
-// (The passes of 16 and 32 rows side by side read the weights once each, out of the L2 the second time, and that is what they
-// wait for: 40 rows of 28672 x 4096 29.8 us, here 24.2; 32 rows 23.0 and 20.9.  What bounds it: the vector unit and the matrix
-// pipe, 145 instructions and 36 products per wave and step, which overlap little: one group of waves with a block's scaling
-// spread over the next one's products 27.8.  64 rows need more registers than a wave has: 33.8 against 31.)
-// A wave's step is a tile-major block (16 columns x 128 k-values) of each of its NG tiles.  The codes enter the products as
-// 128 + n; what 136 times the activations' sum is too much leaves with a product against ones, once for all tiles.
-constexpr int kC4Step = 128, kC4Stages = 4, kC4Groups = 2;
-// places of a row's sixteen 16-byte granules: granule c at c ^ c4_key(row).  The lanes an LDS read serves together (0 - 3 and
-// 12 - 15 of one granule's rows, 4 - 11 of the next but three) find sixteen different places.
-__device__ __forceinline__ int c4_key(int row) { return (row & 15) < 4 ? row & 15 : (row & 15) < 12 ? (row & 15) + 4 : (row & 15) - 8; }
-
-template <int RT, int NG>
-__global__ __launch_bounds__(256 * kC4Groups, 2) void gemm_columns4_kernel(const GemmArgs a) {
-    constexpr int S = kC4Stages, KP = kC4Groups, kVecs = RT * 16 * (kC4Step / 8);
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int part_id = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 256);
-    u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem) + part_id * S * kVecs;
-    const int tid = threadIdx.x & 255, lane = tid & (kWave - 1);
-    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int j = lane & 15, q = lane >> 4;
-    const int N = a.N, K = a.K, M = a.M, T = N / 16, nb = K / kC4Step;
-    const int nk = (nb - part_id + KP - 1) / KP;   // this group's steps
-    auto place = [&](int kt) { return min(part_id + KP * min(kt, max(nk, 1) - 1), nb - 1); };   // (past them, or without any: a step again)
-    const int tile0 = (static_cast<int>(blockIdx.x) * 4 + wv) * NG, groups = K >> a.g_shift, to_group = a.g_shift - 7;
-
-    uint32_t woff[NG], soff[NG];
-#pragma unroll
-    for (int i = 0; i < NG; ++i) {
-        const uint32_t tile = min(tile0 + i, T - 1);
-        woff[i] = tile * (nb * 1024u) + lane * 16u;
-        soff[i] = tile * (groups * 32u) + q * 8u;
-    }
-    u32x4_t raw[S][NG];
-    u32x2_t gs[S][NG];
-    auto load_w = [&](int kt, int slot) __attribute__((always_inline)) {
-        const int b = place(kt);
-        const unsigned char* pw = a.w + static_cast<size_t>(b) * 1024;
-        const unsigned char* ps = a.scale + static_cast<size_t>(b >> to_group) * 32;
-#pragma unroll
-        for (int i = 0; i < NG; ++i) raw[slot][i] = *reinterpret_cast<const u32x4_t*>(pw + woff[i]);
-#pragma unroll
-        for (int i = 0; i < NG; ++i) gs[slot][i] = *reinterpret_cast<const u32x2_t*>(ps + soff[i]);
-        PIE_FENCE();
-    };
-    uint32_t aoff[RT];
-#pragma unroll
-    for (int u = 0; u < RT; ++u) {
-        const int r = (u * 4 + wv) * 4 + (lane >> 4);
-        aoff[u] = static_cast<uint32_t>(min(r, M - 1)) * (2u * K) + ((lane & 15) ^ c4_key(r)) * 16;
-    }
-    auto issue_a = [&](int kt, int stage) __attribute__((always_inline)) {
-        const unsigned char* pa = reinterpret_cast<const unsigned char*>(a.act) + static_cast<size_t>(place(kt)) * (kC4Step * 2);
-#pragma unroll
-        for (int u = 0; u < RT; ++u) to_lds(pa + aoff[u], lds + stage * kVecs + (u * 4 + wv) * 64);
-        PIE_FENCE();
-    };
-    const int key = c4_key(j);
-    bf16x8_t af[2][RT], bw[2][NG];
-    auto read_a = [&](int stage, int s, int to) __attribute__((always_inline)) {
-        const u32x4_t* A = lds + stage * kVecs + j * 16 + ((4 * q + s) ^ key);
-#pragma unroll
-        for (int t = 0; t < RT; ++t) af[to][t] = __builtin_bit_cast(bf16x8_t, A[t * 256]);
-    };
-    uint32_t k128 = 0x43004300u;   // (128.0, 128.0) as a bf16 pair, opaque to the compiler
-    asm volatile("" : "+v"(k128));
-    auto decode = [&](const u32x4_t& r, int s) __attribute__((always_inline)) {
-        const uint32_t v = r[s];
-        return __builtin_bit_cast(bf16x8_t, u32x4_t{and_or(v, 0x000F000Fu, k128), and_or(v >> 4, 0x000F000Fu, k128),
-                                                    and_or(v >> 8, 0x000F000Fu, k128), and_or(v >> 12, 0x000F000Fu, k128)});
-    };
-    const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4_t{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
-    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4_t acc[RT][NG], sum[RT][NG], sx[RT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-        for (int i = 0; i < NG; ++i) acc[t][i] = zero;
-
-#pragma unroll
-    for (int i = 0; i < S; ++i) load_w(i, i);
-#pragma unroll
-    for (int i = 0; i < S; ++i) issue_a(i, i);
-    constexpr int kOps = RT + 2 * NG;
-    PIE_WAIT_VM((S - 1) * RT);
-    PIE_MEET();
-    read_a(0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < NG; ++i) bw[0][i] = decode(raw[0][i], 0);
-    auto step = [&](auto slot, int kt) __attribute__((always_inline)) {
-        constexpr int cur = decltype(slot)::value, next = (cur + 1) % S;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            PIE_FENCE();
-            if (s < 3) {
-                read_a(cur, s + 1, (s + 1) & 1);
-#pragma unroll
-                for (int i = 0; i < NG; ++i) bw[(s + 1) & 1][i] = decode(raw[cur][i], s + 1);
-            } else {
-                // step kt + 1 has come (of the first S the weights left first)
-                if (kt < S - 2) PIE_WAIT_VM((S - 2) * RT);
-                else PIE_WAIT_VM((S - 2) * kOps);
-                PIE_WAIT_LGKM0();
-                PIE_MEET();
-                read_a(next, 0, 0);
-#pragma unroll
-                for (int i = 0; i < NG; ++i) bw[0][i] = decode(raw[next][i], 0);
-            }
-#pragma unroll
-            for (int t = 0; t < RT; ++t) {
-                sx[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, af[s & 1][t], s ? sx[t] : zero, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < NG; ++i)
-                    sum[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[s & 1][i], af[s & 1][t], s ? sum[t][i] : zero, 0, 0, 0);
-            }
-#pragma unroll
-            for (int u = 0; u < RT * (NG + 1); ++u) {   // the reads ahead between the first products, the decoding between all
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                if (u < RT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-            }
-        }
-        // (lane: row j, columns 4q .. 4q + 3 of a tile)
-#pragma unroll
-        for (int i = 0; i < NG; ++i) {
-            const float sc[4] = {bf16_lo(gs[cur][i].x), bf16_hi(gs[cur][i].x), bf16_lo(gs[cur][i].y), bf16_hi(gs[cur][i].y)};
-#pragma unroll
-            for (int t = 0; t < RT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[t][i][r] = fmaf(sc[r], fmaf(-136.f, sx[t][r], sum[t][i][r]), acc[t][i][r]);
-        }
-        PIE_FENCE();
-        issue_a(kt + S, cur);
-        load_w(kt + S, cur);
-    };
-    const int rounds = (nb + KP - 1) / KP;
-    auto steps = [&](int kt, auto whole) __attribute__((always_inline)) {
-        auto one = [&](auto slot) __attribute__((always_inline)) {
-            constexpr int i = decltype(slot)::value;
-            if (decltype(whole)::value || kt + i < nk) step(slot, kt + i);
-            else if (kt + i < rounds) PIE_MEET();
-        };
-        one(std::integral_constant<int, 0>{});
-        one(std::integral_constant<int, 1>{});
-        one(std::integral_constant<int, 2>{});
-        one(std::integral_constant<int, 3>{});
-    };
-    int kt = 0;
-    for (; kt + S <= nb / KP; kt += S) steps(kt, std::true_type{});
-    if (kt < rounds) steps(kt, std::false_type{});
-    __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the sums take their place)
-    __syncthreads();
-    f32x4_t* meet = reinterpret_cast<f32x4_t*>(smem);
-    if (part_id > 0) {
-#pragma unroll
-        for (int t = 0; t < RT; ++t)
-#pragma unroll
-            for (int i = 0; i < NG; ++i) meet[(t * NG + i) * 256 + tid] = acc[t][i];
-    }
-    __syncthreads();
-    if (part_id > 0) return;
-#pragma unroll
-    for (int i = 0; i < NG; ++i) {
-        const int n = (tile0 + i) * 16 + 4 * q;
-        if (n >= N) continue;
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-            const int m = t * 16 + j;
-            if (m >= M) continue;
-            const f32x4_t o = acc[t][i] + meet[(t * NG + i) * 256 + tid];
-            float v[4] = {o[0], o[1], o[2], o[3]};
-            wide_store(a, m, n, v);
-        }
-    }
-}
-
 // Sums the K shares' partials of four columns and applies the epilogue the kernel would have applied.
 __global__ __launch_bounds__(256) void wide_reduce_kernel(const GemmArgs a, int splits) {
     const int N = a.N, quads = (N + 3) / 4;
@@ -928,28 +680,16 @@ bool fits(int format, int M, int N, int K, int group_size) {
     return 2ll * M * K <= 0xFFFFFFFFll && 2ll * (N + 15) * K <= 0xFFFFFFFFll && (M + 255ll) / 256 * ((N + 127ll) / 128) < 0x0FFFFFFF;
 }
 
-template <int RT>
-int launch_columns4(const GemmArgs& a, hipStream_t stream) {
-    constexpr int NG = 2;
-    constexpr size_t smem = kC4Groups * kC4Stages * static_cast<size_t>(RT * 16) * kC4Step * 2;
-    static_assert(static_cast<size_t>(RT) * NG * 256 * 16 <= smem, "the sums fit the activations' place");
-    constexpr auto kernel = &gemm_columns4_kernel<RT, NG>;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
-    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
-    hipLaunchKernelGGL(kernel, dim3((a.N + 64 * NG - 1) / (64 * NG)), dim3(256 * kC4Groups), smem, stream, a);
-    return launch_status();
-}
-// up to 128 rows of one-byte weights, 17 to 48 of int4 ones
+// up to 128 rows of one-byte weights, 17 to 48 of int4 ones (those in gemm_groups_mfma.hip)
 bool columns_fit(int format, int M, int N, int K, int group_size) {
     if (N % 16 != 0 || static_cast<long long>(N) * K > 0xFFFFFFFFll) return false;
     if (format == PIE_HIP_FMT_INT4B8)
-        return M > 16 && M <= 48 && K % kC4Step == 0 && group_size >= kC4Step && (group_size & (group_size - 1)) == 0 && K % group_size == 0;
+        return M > 16 && M <= 48 && gemm_groups_us(M, N, K, group_size, 0) < 1e30;
     return M <= 128 && (format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8) && K % kStepK == 0;
 }
 // A round of blocks (one to a CU, two with 64 rows' LDS) takes 4 us and 0.27 - 0.5 a step (measured at 40 - 128 rows of
 // 16384, 5120 and 3072 x 2048 and 28672 x 4096).
 double columns_us(int format, int M, int N, int K) {
-    if (format == PIE_HIP_FMT_INT4B8) return 4.0 + (N + 32767) / 32768 * (K / (2 * kC4Step)) * (M <= 32 ? 1.05 : 1.26);
     const int size = M <= 64 ? 0 : M <= 96 ? 1 : 2;
     constexpr double kStepUs[2][3] = {{0.34, 0.40, 0.51}, {0.27, 0.39, 0.50}};
     const long long blocks = (N + 63) / 64, slots = size == 0 ? 512 : 256;
@@ -974,7 +714,8 @@ int run(GemmArgs a, const Plan& p, float* ws, hipStream_t stream) {
 }  // namespace
 
 double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
-    if (columns_fit(format, M, N, K, group_size)) return columns_us(format, M, N, K);
+    if (columns_fit(format, M, N, K, group_size))
+        return format == PIE_HIP_FMT_INT4B8 ? gemm_groups_us(M, N, K, group_size, ws_bytes) : columns_us(format, M, N, K);
     return fits(format, M, N, K, group_size) ? plan_of(kRates[format], M, N, K, ws_bytes).us : 1e30;
 }
 // (the choice between its two heights is launch_gemm's)
@@ -988,10 +729,12 @@ double gemm_tiles_us(int format, int M, int N, int K) {
 }
 
 int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {
-    if (columns_fit(format, a.M, a.N, a.K, group_size) && reinterpret_cast<uintptr_t>(a.act) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0) {
+    if (format == PIE_HIP_FMT_INT4B8 && columns_fit(format, a.M, a.N, a.K, group_size)) {
+        const int st = launch_gemm_groups(a, group_size, ws, ws_bytes, stream);
+        if (st != PIE_HIP_ERR_UNSUPPORTED) return st;
+    } else if (columns_fit(format, a.M, a.N, a.K, group_size) && reinterpret_cast<uintptr_t>(a.act) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0) {
         GemmArgs b = a;
         b.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
-        if (format == PIE_HIP_FMT_INT4B8) return a.M <= 32 ? launch_columns4<2>(b, stream) : launch_columns4<3>(b, stream);
         return format == PIE_HIP_FMT_FP8 ? launch_columns<kKvFp8>(b, stream) : launch_columns<kKvInt8>(b, stream);
     }
     if (!fits(format, a.M, a.N, a.K, group_size) || reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16)

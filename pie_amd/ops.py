@@ -631,6 +631,34 @@ def gemm_mfma_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] 
     return y
 
 
+def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
+                      workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The GEMM of 17 and more rows over tile-major int4 weights whose groups are scaled in fp32; with a workspace few blocks over a
+    long K run in shares of K."""
+    _dev(act, torch.bfloat16, "act")
+    M, K = act.shape
+    if K != w.K or w.kind != "int4b8+tiled":
+        raise KernelError("act K != weight K, or not tile-major int4 weights")
+    n_out = w.N // 2 if epilogue == 1 else w.N
+    if y is None:
+        if beta:
+            raise KernelError("beta=1 needs an existing y")
+        y = torch.empty((M, n_out), dtype=torch.bfloat16, device=act.device)
+    _dev(y, torch.bfloat16, "y")
+    if tuple(y.shape) != (M, n_out):
+        raise KernelError("y shape mismatch")
+    _check(kernels().pie_hip_gemm_groups_tiled(_ptr(act), _ptr(w.data), _ptr(w.scale), w.group_size, _ptr(y), M, w.N, K, beta, epilogue, None,
+                                               _ptr(workspace), C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()),
+                                               _stream()), "pie_hip_gemm_groups_tiled")
+    return y
+
+
+def gemm_groups_us(M: int, N: int, K: int, group: int, workspace_bytes: int = 0) -> float:
+    lib = kernels()
+    lib.pie_hip_gemm_groups_us.restype = C.c_float
+    return float(lib.pie_hip_gemm_groups_us(M, N, K, group, C.c_size_t(workspace_bytes)))
+
+
 def gemm_mfma_us(kind: str, M: int, N: int, K: int, group: int, tiled: bool, workspace_bytes: int = 0) -> float:
     """Estimated microseconds of the tiled GEMMs over more than 128 rows."""
     lib = kernels()
@@ -691,10 +719,10 @@ def qkv_rope_fused(act: torch.Tensor, w: WeightView, table: torch.Tensor, kv_slo
 
 def qkv_rope_skinny_tiled(act: torch.Tensor, w: WeightView, table: torch.Tensor, kv_slots: torch.Tensor,
                           k_pages: torch.Tensor, v_pages: torch.Tensor, hq: int, hk: int, d: int,
-                          pairing: int = 1) -> torch.Tensor:
+                          pairing: int = 1, groups: bool = False, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """q|k|v projection over tile-major weights + RoPE + KV-cache write for a decode batch (act
     already normalised).  Returns q [M, hq, d]; k / v land in their slots.  pairing as for
-    `qkv_rope_fused`."""
+    `qkv_rope_fused`; `groups`: int4 weights in the form of `gemm_groups_tiled`."""
     _dev(act, torch.bfloat16, "act")
     _dev(table, torch.float32, "rope_table")
     _dev(kv_slots, torch.int64, "kv_slots")
@@ -709,6 +737,14 @@ def qkv_rope_skinny_tiled(act: torch.Tensor, w: WeightView, table: torch.Tensor,
         raise KernelError("kv slot out of range")
     q_out = torch.empty((M, hq, d), dtype=torch.bfloat16, device=act.device)
     scale_is_bf16 = int(w.scale is not None and w.scale.dtype == torch.bfloat16)
+    if groups:
+        if w.kind != "int4b8+tiled":
+            raise KernelError("tile-major int4 weights expected")
+        _check(kernels().pie_hip_qkv_rope_groups_tiled(
+            _ptr(act), _ptr(w.data), _ptr(w.scale), w.group_size, M, K, _ptr(table), _ptr(kv_slots), _ptr(q_out), _ptr(k_pages), _ptr(v_pages),
+            hq, hk, d, pairing, _ptr(workspace), C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()),
+            _stream()), "pie_hip_qkv_rope_groups_tiled")
+        return q_out
     _check(kernels().pie_hip_qkv_rope_skinny_tiled(
         FMT[w.kind[:-len("+tiled")]], _ptr(act), _ptr(w.data), _ptr(w.scale), scale_is_bf16, w.group_size,
         M, K, _ptr(table), _ptr(kv_slots), _ptr(q_out), _ptr(k_pages), _ptr(v_pages), hq, hk, d,
