@@ -287,6 +287,14 @@ int pie_hip_gemm_groups_tiled(const uint16_t* act_bf16, const void* weight, cons
                               int M, int N, int K, int beta, int epilogue, const PieHipGlu* glu, void* workspace,
                               size_t workspace_bytes, void* stream);
 float pie_hip_gemm_groups_us(int M, int N, int K, int group_size, size_t workspace_bytes);
+/* The same (any number of rows) in two or more shares of K whose fp32 sums [*shares, M, N] stay in the workspace, for
+ * pie_hip_shares_rmsnorm: x += the shares' sums in order, rounded to bf16; norm_out = x normalised as by pie_hip_rmsnorm (sums of
+ * squares in another order).  hidden % 8 == 0, up to 16384; all on 16-byte boundaries.  The estimate leaves the norm's own time out (1e30: not taken). */
+int pie_hip_gemm_groups_shares(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, int M, int N, int K,
+                               void* workspace, size_t workspace_bytes, int* shares, void* stream);
+float pie_hip_gemm_groups_shares_us(int M, int N, int K, int group_size, size_t workspace_bytes);
+int pie_hip_shares_rmsnorm(const float* partials, int shares, uint16_t* x_bf16, const uint16_t* weight_bf16, uint16_t* norm_out_bf16,
+                           int rows, int hidden, float eps, void* stream);
 /* pie_hip_qkv_rope_skinny_tiled in that form (q_out and the pools on 8-byte boundaries). */
 int pie_hip_qkv_rope_groups_tiled(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, int M, int K,
                                   const float* rope_table, const int64_t* kv_slots, uint16_t* q_out, uint16_t* k_pages,

@@ -86,6 +86,16 @@ double groups_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 17 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
 bool in_groups(const Linear& w, int M, size_t ws_bytes) { return groups_cost(w, M, ws_bytes) < skinny_cost(w, M).us; }
+// Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
+// (pie_hip_shares_rmsnorm), for 5 rows and more: 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
+// without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
+bool in_shares(const Linear& w, int M, size_t ws_bytes) {
+    if (M < 5 || w.kind != Quant::Int4b8 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return false;
+    double other = std::min(skinny_cost(w, M).us, groups_cost(w, M, ws_bytes));
+    if (M > 128) other = std::min({other, static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 0, ws_bytes)),
+                                   static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 1, ws_bytes))});
+    return pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes) < other;
+}
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
     const auto [p2, wpasses, wave_form, skinny] = skinny_cost(w, M);
@@ -693,7 +703,7 @@ void Executor::body(int N, int S, int max_kv_len) {
         const bool kvq = kv_format_ != PIE_HIP_KV_BF16;
         float* ksc = kvq && !k_scale_pool_.empty() ? k_scale_pool_[l] : nullptr;
         float* vsc = kvq && !v_scale_pool_.empty() ? v_scale_pool_[l] : nullptr;
-        // (the previous layer's MoE combine may have left this layer's normalised rows in xn_)
+        // (the previous layer's MoE combine or down projection may have left this layer's normalised rows in xn_)
         const bool prenormed = xn_holds_next_norm_;
         xn_holds_next_norm_ = false;
         if (kvq) {
@@ -731,7 +741,7 @@ void Executor::body(int N, int S, int max_kv_len) {
             const int tuned_qkv = N <= 128 ? w.wqkv.tuned[N] : -1;
             if (fused_rope && !w.q_norm && w.wqkv.data_tiled &&
                 (tuned_qkv >= 0 ? tuned_qkv <= 1 : pick_gemm(w.wqkv, N, gemm_ws_bytes_) == GemmPath::Skinny)) {
-                PIE_KERNEL(pie_hip_rmsnorm(x_, w.attn_norm, xn_, N, H, m.rms_eps, s));
+                if (!prenormed) PIE_KERNEL(pie_hip_rmsnorm(x_, w.attn_norm, xn_, N, H, m.rms_eps, s));
                 const int st =
                     in_groups(w.wqkv, N, gemm_ws_bytes_)
                         ? pie_hip_qkv_rope_groups_tiled(xn_, w.wqkv.data_tiled, w.wqkv.scale_tiled, w.wqkv.group, N, H, rope_tab_, slots, q_,
@@ -830,8 +840,22 @@ void Executor::body(int N, int S, int max_kv_len) {
         } else {
             for (const RowRun& r : runs_) attend_rows(r);
         }
-        if (!merged_into_wo)
-        linear_fused(w.wo, attn_, nullptr, m.rms_eps, x_, N, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
+        // x_ += act · W^T; true if xn_ then holds the rows under `norm`
+        auto project = [&](const Linear& lin, const uint16_t* act, const uint16_t* norm) {
+            int shares = 0;
+            if (norm && in_shares(lin, N, gemm_ws_bytes_)) {
+                const int st = pie_hip_gemm_groups_shares(act, lin.data_tiled, lin.scale_tiled, lin.group, N, lin.N, lin.K, gemm_ws_,
+                                                          gemm_ws_bytes_, &shares, s);
+                if (st == PIE_HIP_OK) {
+                    PIE_KERNEL(pie_hip_shares_rmsnorm(static_cast<const float*>(gemm_ws_), shares, x_, norm, xn_, N, H, m.rms_eps, s));
+                    return true;
+                }
+                if (st != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(st);
+            }
+            linear_fused(lin, act, nullptr, m.rms_eps, x_, N, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
+            return false;
+        };
+        const bool ffn_normed = !merged_into_wo && project(w.wo, attn_, model_.is_moe() ? nullptr : w.ffn_norm);
         if (model_.is_moe()) {
             // the next layer's rows come normalised when that layer runs the plain projection
             // (q/k norm: no fused RoPE epilogue) on more than the GEMV's four rows
@@ -839,8 +863,8 @@ void Executor::body(int N, int S, int max_kv_len) {
             moe_block(w, N, next_plain ? model_.layers[l + 1].attn_norm : nullptr, s);
             continue;
         }
-        linear_fused(w.wgu, x_, w.ffn_norm, m.rms_eps, act_, N, 0, 1, xn_, gemm_ws_, gemm_ws_bytes_, s);
-        linear_fused(w.wdown, act_, nullptr, m.rms_eps, x_, N, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
+        linear_fused(w.wgu, ffn_normed ? xn_ : x_, ffn_normed ? nullptr : w.ffn_norm, m.rms_eps, act_, N, 0, 1, xn_, gemm_ws_, gemm_ws_bytes_, s);
+        xn_holds_next_norm_ = project(w.wdown, act_, l + 1 < m.layers ? model_.layers[l + 1].attn_norm : nullptr);
     }
     // lm_head only on the sampled rows (driver/portable/src/graph_qwen3.cpp:867-896)
     const int cap = static_cast<int>(std::min<size_t>(max_tokens_, 2 * static_cast<size_t>(cfg_.batching.max_forward_requests)));

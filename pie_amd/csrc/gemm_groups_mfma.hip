@@ -1,5 +1,5 @@
 // Int4 weights times 17 and more activation rows with the group scales kept in fp32: y[M, N] = epilogue( act[M, K] · W[N, K]^T ),
-// the skinny GEMM's arithmetic (a group's code products are summed as they are and scaled once, in fp32) in blocks of 32, 48 or 64
+// the skinny GEMM's arithmetic (a group's code products are summed as they are and scaled once, in fp32) in blocks of 16 to 64
 // rows x 128 columns, two blocks of four waves to a CU.
 //
 // The skinny GEMM's passes of 32 rows read and decode the weights once each, stage their rows per wave, and their number costs in
@@ -79,7 +79,7 @@ __device__ __forceinline__ int key_of(int row) { return (row & 15) < 4 ? row & 1
 template <int RT>
 __global__ __launch_bounds__(256, 2) void gemm_groups_kernel(const GemmArgs a, const Rotation rot, int row_blocks, int per_xcd, int blocks, int per_share) {
     constexpr int S = kStages, NG = kTiles, kVecs = RT * 16 * (kStep / 8), kOps = RT + 2 * NG;
-    static_assert(RT <= 4 && NG == 2, "a quarter of a phase scales one row tile; two tiles' sums");
+    static_assert(RT >= 1 && RT <= 4 && NG == 2, "a quarter of a phase scales one row tile; two tiles' sums");
     extern __shared__ __align__(16) unsigned char smem[];
     u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem);
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -275,27 +275,32 @@ int launch(const GemmArgs& a, const Rotation& rot, int shares, hipStream_t strea
     return launch_status();
 }
 
-// Rows per block and shares of K.  A block takes 4 us and per step `alone` (a CU has one), `pair` (two); 512 run at a time,
-// and what is left over of several rounds costs a sixth of one.  The shares' sums take a second kernel, 3 us and their
-// bytes at 3.2 TB/s.  Fitted to 20 - 800 rows of 28672 x 4096, 6144 x 4096, 4096 x 4096 and 4096 x 14336: the plan taken is
-// within 6 % of the fastest of all.
+// Rows per block and shares of K.  A block alone on its CU takes 3.7 us and `alone` a step, or what its weights take at 6.3 TB/s; two to a
+// CU take 2 us more and `pair`; rounds of 512 blocks take 2 us and their steps each, what is left over a sixth of one.
+// The shares' sums meet in a second kernel: 3 us and their bytes at 3.2 TB/s, or (`norm`) 0.2 us a share on top of the norm that would run
+// anyway.  Fitted to 5 - 800 rows of 28672 x 4096, 6144 x 4096, 4096 x 4096 and 4096 x 14336: the plan taken is within 8 % of the fastest of all.
 struct Plan {
     int row_tiles = 0, shares = 1;
     double us = 1e30;
 };
-Plan plan_of(int M, int N, int K, size_t ws_bytes) {
-    constexpr double kAlone[] = {0.34, 0.50, 0.66}, kPair[] = {0.66, 0.82, 1.13};
+Plan plan_of(int M, int N, int K, size_t ws_bytes, bool norm) {
+    constexpr double kAlone[] = {0.28, 0.44, 0.60, 0.80}, kPair[] = {0.55, 0.715, 0.92, 1.19};
     const int steps = K / kStep;
     Plan best;
-    for (int rt = 2; rt <= 4; ++rt) {
+    for (int rt = 1; rt <= 4; ++rt) {
         const long long tiles = (M + rt * 16ll - 1) / (rt * 16) * ((N + kCols - 1) / kCols);
-        for (int s = 1; s <= 8; ++s) {
+        for (int s = norm ? 2 : 1; s <= 8; ++s) {
             const int per = (steps + s - 1) / s;
             const size_t bytes = static_cast<size_t>(s) * M * N * sizeof(float);
-            if (s > 1 && (per < 2 || (s - 1) * per >= steps || bytes > ws_bytes || tiles * (s - 1) >= 512)) break;
-            const long long blocks = tiles * s;
-            const double block = 4.0 + per * (blocks <= 256 ? kAlone : kPair)[rt - 2];
-            const double us = 2.5 + block * (blocks <= 512 ? 1.0 : blocks / 512.0 + 1.0 / 6.0) + (s > 1 ? 3.0 + static_cast<double>(bytes) / 3.2e6 : 0.0);
+            if (s > 1 && (per < 2 || bytes > ws_bytes || tiles * (s - 1) >= 512)) break;
+            if ((s - 1) * per >= steps) continue;   // (the last share would be empty)
+            const double n = static_cast<double>(tiles) * s, alone = kAlone[rt - 1], pair = kPair[rt - 1];
+            double us;
+            if (n <= 256) us = 3.7 + per * std::max(alone, n * 8448 / 6.3e6);
+            else if (n <= 512) us = 5.7 + per * (alone + (pair - alone) * (0.3 + 0.7 * (n - 256) / 256));
+            else us = 2.0 + (n / 512 + 1.0 / 6.0) * (2.0 + per * pair);
+            if (norm) us += 0.2 * s;
+            else if (s > 1) us += 3.0 + static_cast<double>(bytes) / 3.2e6;
             if (us < best.us) best = {rt, s, us};
         }
     }
@@ -305,17 +310,23 @@ bool fits(int M, int N, int K, int group_size) {
     return M > 0 && N % 16 == 0 && K % kStep == 0 && group_size >= kStep && (group_size & (group_size - 1)) == 0 && K % group_size == 0 &&
            static_cast<long long>(N) * K <= 0xFFFFFFFFll && 2ll * M * K <= 0xFFFFFFFFll && (M + 31ll) / 32 * ((N + kCols - 1ll) / kCols) < 0x0FFFFFFF;
 }
-int run(GemmArgs a, const Rotation& rot, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {
+// (`shares`: the sums stay in the workspace, in that many shares)
+int run(GemmArgs a, const Rotation& rot, int group_size, void* ws, size_t ws_bytes, hipStream_t stream, int* shares = nullptr) {
     if (!fits(a.M, a.N, a.K, group_size) || reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16 ||
         reinterpret_cast<uintptr_t>(a.scale) % 8)
         return PIE_HIP_ERR_UNSUPPORTED;
     if (reinterpret_cast<uintptr_t>(ws) % 16) ws = nullptr;
-    const Plan p = plan_of(a.M, a.N, a.K, ws ? ws_bytes : 0);
+    const Plan p = plan_of(a.M, a.N, a.K, ws ? ws_bytes : 0, shares != nullptr);
+    if (p.row_tiles == 0) return PIE_HIP_ERR_UNSUPPORTED;
     a.g_shift = __builtin_ctz(static_cast<unsigned>(group_size));
     a.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
     a.partial = p.shares > 1 ? static_cast<float*>(ws) : nullptr;
-    const int st = p.row_tiles == 2 ? launch<2>(a, rot, p.shares, stream) : p.row_tiles == 3 ? launch<3>(a, rot, p.shares, stream) : launch<4>(a, rot, p.shares, stream);
-    if (st != PIE_HIP_OK || p.shares == 1) return st;
+    const int st = p.row_tiles == 1   ? launch<1>(a, rot, p.shares, stream)
+                   : p.row_tiles == 2 ? launch<2>(a, rot, p.shares, stream)
+                   : p.row_tiles == 3 ? launch<3>(a, rot, p.shares, stream)
+                                      : launch<4>(a, rot, p.shares, stream);
+    if (shares) *shares = p.shares;
+    if (st != PIE_HIP_OK || p.shares == 1 || shares) return st;
     const size_t quads = static_cast<size_t>(a.M) * (a.N / 4);
     hipLaunchKernelGGL(groups_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, a, rot, p.shares);
     return launch_status();
@@ -327,13 +338,32 @@ int launch_gemm_groups(const GemmArgs& a, int group_size, void* ws, size_t ws_by
     return run(a, Rotation{}, group_size, ws, ws_bytes, stream);
 }
 double gemm_groups_us(int M, int N, int K, int group_size, size_t ws_bytes) {
-    return fits(M, N, K, group_size) ? plan_of(M, N, K, ws_bytes).us : 1e30;
+    return fits(M, N, K, group_size) ? plan_of(M, N, K, ws_bytes, false).us : 1e30;
 }
 
 }  // namespace pie_hip
 
 extern "C" float pie_hip_gemm_groups_us(int M, int N, int K, int group_size, size_t workspace_bytes) {
     return static_cast<float>(pie_hip::gemm_groups_us(M, N, K, group_size, workspace_bytes));
+}
+
+extern "C" float pie_hip_gemm_groups_shares_us(int M, int N, int K, int group_size, size_t workspace_bytes) {
+    using namespace pie_hip;
+    return static_cast<float>(fits(M, N, K, group_size) ? plan_of(M, N, K, workspace_bytes, true).us : 1e30);
+}
+
+extern "C" int pie_hip_gemm_groups_shares(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, int M, int N, int K,
+                                          void* workspace, size_t workspace_bytes, int* shares, void* stream) {
+    using namespace pie_hip;
+    if (!act_bf16 || !weight || !scale || !workspace || !shares || M <= 0 || N <= 0 || K <= 0) return PIE_HIP_ERR_INVALID;
+    GemmArgs a{};
+    a.act = act_bf16;
+    a.w = static_cast<const unsigned char*>(weight);
+    a.scale = static_cast<const unsigned char*>(scale);
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    return run(a, Rotation{}, group_size, workspace, workspace_bytes, static_cast<hipStream_t>(stream), shares);
 }
 
 extern "C" int pie_hip_gemm_groups_tiled(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, uint16_t* y_bf16,

@@ -98,6 +98,59 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* __restrict__ x,
         store_vec(v, *reinterpret_cast<const u32x4_t*>(x + base + v * 8), *reinterpret_cast<const u32x4_t*>(w + v * 8));
 }
 
+// A projection's shares of K meet the residual and the next norm: x += the shares' sums in order (bf16), y = the row normalised, as the
+// two launches.  One block per row, eight columns per thread and round.
+__global__ __launch_bounds__(1024) void shares_rmsnorm_kernel(const float* __restrict__ partial, int shares, size_t plane, uint16_t* __restrict__ x,
+                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ y, int H, float eps) {
+    __shared__ float red[16];
+    const size_t base = static_cast<size_t>(blockIdx.x) * H;
+    constexpr int kMaxVec = 2;
+    u32x4_t cache[kMaxVec], wcache[kMaxVec];
+    float local = 0.f;
+    const int nvec = H / 8;
+#pragma unroll
+    for (int c = 0; c < kMaxVec; ++c) {
+        const int v = threadIdx.x + c * blockDim.x;
+        if (v >= nvec) break;
+        wcache[c] = *reinterpret_cast<const u32x4_t*>(w + v * 8);
+        u32x4_t a = *reinterpret_cast<const u32x4_t*>(x + base + v * 8);
+        const float* p = partial + base + v * 8;
+        f32x4_t s0 = *reinterpret_cast<const f32x4_t*>(p), s1 = *reinterpret_cast<const f32x4_t*>(p + 4);
+#pragma unroll 4
+        for (int z = 1; z < shares; ++z) {
+            s0 += *reinterpret_cast<const f32x4_t*>(p + z * plane);
+            s1 += *reinterpret_cast<const f32x4_t*>(p + z * plane + 4);
+        }
+        a[0] = pack_bf16x2(s0[0] + bf16_lo(a[0]), s0[1] + bf16_hi(a[0]));
+        a[1] = pack_bf16x2(s0[2] + bf16_lo(a[1]), s0[3] + bf16_hi(a[1]));
+        a[2] = pack_bf16x2(s1[0] + bf16_lo(a[2]), s1[1] + bf16_hi(a[2]));
+        a[3] = pack_bf16x2(s1[2] + bf16_lo(a[3]), s1[3] + bf16_hi(a[3]));
+        *reinterpret_cast<u32x4_t*>(x + base + v * 8) = a;
+        cache[c] = a;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float lo = bf16_lo(a[i]), hi = bf16_hi(a[i]);
+            local += lo * lo + hi * hi;
+        }
+    }
+    local = wave_sum(local);
+    if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = local;
+    __syncthreads();
+    float total = 0.f;
+    for (int i = 0; i < static_cast<int>(blockDim.x) / kWave; ++i) total += red[i];
+    const float inv_rms = rsqrtf(total / static_cast<float>(H) + eps);
+#pragma unroll
+    for (int c = 0; c < kMaxVec; ++c) {
+        const int v = threadIdx.x + c * blockDim.x;
+        if (v >= nvec) break;
+        u32x4_t o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[i] = pack_bf16x2(bf16_lo(cache[c][i]) * inv_rms * bf16_lo(wcache[c][i]), bf16_hi(cache[c][i]) * inv_rms * bf16_hi(wcache[c][i]));
+        *reinterpret_cast<u32x4_t*>(y + base + v * 8) = o;
+    }
+}
+
 // table[n, i] = cos(pos_n * inv_freq[i]), table[n, i + d/2] = sin(...), i < d/2: the
 // per-forward cos/sin rows every layer reuses (rope_standard_table_kernel,
 // driver/cuda/src/kernels/rope.cu:35-53).  inv_freq comes from the host so that any
@@ -366,6 +419,16 @@ extern "C" int pie_hip_rmsnorm(const uint16_t* x_bf16, const uint16_t* weight_bf
     hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3(rows), dim3(256), 0,
                        static_cast<hipStream_t>(stream), const_cast<uint16_t*>(x_bf16), nullptr,
                        weight_bf16, y_bf16, hidden, eps);
+    return launch_status();
+}
+
+extern "C" int pie_hip_shares_rmsnorm(const float* partials, int shares, uint16_t* x_bf16, const uint16_t* weight_bf16, uint16_t* norm_out_bf16,
+                                      int rows, int hidden, float eps, void* stream) {
+    if (!partials || !x_bf16 || !weight_bf16 || !norm_out_bf16 || shares <= 0 || rows <= 0 || hidden <= 0) return PIE_HIP_ERR_INVALID;
+    if (hidden % 8 != 0 || hidden > 2 * 8 * 1024) return PIE_HIP_ERR_UNSUPPORTED;
+    const int nvec = hidden / 8, threads = std::min(1024, (nvec + kWave - 1) / kWave * kWave);
+    hipLaunchKernelGGL(shares_rmsnorm_kernel, dim3(rows), dim3(threads), 0, static_cast<hipStream_t>(stream), partials, shares,
+                       static_cast<size_t>(rows) * hidden, x_bf16, weight_bf16, norm_out_bf16, hidden, eps);
     return launch_status();
 }
 

@@ -653,6 +653,22 @@ def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor
     return y
 
 
+def gemm_groups_shares_norm(act: torch.Tensor, w: WeightView, x: torch.Tensor, norm_weight: torch.Tensor, eps: float, workspace: torch.Tensor):
+    """x += act . W^T in shares of K that meet in the norm's kernel; returns the normalised rows and the number of shares."""
+    for t, n in ((act, "act"), (x, "x"), (norm_weight, "norm_weight")):
+        _dev(t, torch.bfloat16, n)
+    M, K = act.shape
+    if K != w.K or w.kind != "int4b8+tiled" or tuple(x.shape) != (M, w.N) or norm_weight.numel() != w.N:
+        raise KernelError("shape mismatch, or not tile-major int4 weights")
+    shares, y = C.c_int(0), torch.empty_like(x)
+    _check(kernels().pie_hip_gemm_groups_shares(_ptr(act), _ptr(w.data), _ptr(w.scale), w.group_size, M, w.N, K, _ptr(workspace),
+                                                C.c_size_t(workspace.numel() * workspace.element_size()), C.byref(shares), _stream()),
+           "pie_hip_gemm_groups_shares")
+    _check(kernels().pie_hip_shares_rmsnorm(_ptr(workspace), shares, _ptr(x), _ptr(norm_weight), _ptr(y), M, w.N, C.c_float(eps), _stream()),
+           "pie_hip_shares_rmsnorm")
+    return y, shares.value
+
+
 def gemm_groups_us(M: int, N: int, K: int, group: int, workspace_bytes: int = 0) -> float:
     lib = kernels()
     lib.pie_hip_gemm_groups_us.restype = C.c_float

@@ -93,3 +93,24 @@ def test_qkv_rope_epilogue_equals_projection_then_rope_kernel(gpu, oracle, M, hq
         q2 = ops.qkv_rope_kvwrite(ops.gemm_groups_tiled(x, wt, workspace=ws), pools[2], pools[3], tab, sg, hq, hk, d, pairing == 1)
         assert np.array_equal(bits(q1), bits(q2))
         assert np.array_equal(bits(pools[0]), bits(pools[2])) and np.array_equal(bits(pools[1]), bits(pools[3]))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 512), (5, 4096, 640), (16, 2064, 1152), (17, 528, 896), (40, 8208, 512), (64, 16384, 384), (130, 1024, 1024)])
+def test_shares_that_meet_in_the_norm(gpu, oracle, M, N, K):
+    """Projection into the residual and the norm behind it, against the same sums added to the residual and normalised: rows of less
+    than a wave, of one and two rounds of the block's threads, shares that do not divide the steps."""
+    import torch
+    from pie_amd import ops
+
+    act, t, ref, bound = groups_case(oracle, gpu, M, N, K, 128, 870 + M)
+    g = torch.Generator(device=gpu).manual_seed(870 + M)
+    x0 = torch.randn(M, N, generator=g, device=gpu).to(torch.bfloat16)
+    w = (1 + 0.1 * torch.randn(N, generator=g, device=gpu)).to(torch.bfloat16)
+    x, ws = x0.clone(), torch.full((8 * M * N,), float("nan"), device=gpu)
+    y, shares = ops.gemm_groups_shares_norm(act, t, x, w, 1e-5, ws)
+    assert 2 <= shares <= 8
+    total = ref + x0.double()
+    assert ((x.double() - total).abs() <= 2.0 ** -8 * total.abs() + bound).all()
+    # (the norm's own rounding: two products and a reciprocal root in fp32, the sum of squares of N values in another order)
+    want = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert ((y.double() - want).abs() <= (2.0 ** -8 + N * 2.0 ** -24) * want.abs()).all()
