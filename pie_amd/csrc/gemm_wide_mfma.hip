@@ -358,15 +358,14 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
     }
 }
 
-// ---- experts: the rows of a problem gathered by route, one-byte weights, blocks of 128 rows x 64 NG columns -------------
+// ---- experts: the rows of a problem gathered by route, one-byte weights, blocks of 32 to 128 rows x 64 NG columns --------
 // A hundred rows per expert make an expert's weights as many bytes as its products are time, and each is wanted by one
-// block only.  So weights do not pass through LDS: a wave owns 16 NG columns for all 128 rows, the tile-major copy gives it
+// block only.  So weights do not pass through LDS: a wave owns 16 NG columns for all rows of the block, the tile-major copy gives it
 // the MFMAs' operand by plain loads, three or four steps ahead in registers, each decoded once.  The activations are shared in LDS,
 // as far ahead.  Two or three blocks of four waves to a CU, independent of one another: one's prologue, waits and stores run
 // beside the other's MFMAs.  A row block's column blocks stay on one chiplet and share its activations there.
-// Bound by the weights: 128 fp8 experts of 1536 x 2048 at 82 routes 116 us (402 MB; the tiles through LDS 147, four routes per
-// expert 98), of 2048 x 768 74 (84 through LDS).
-constexpr int kExpertRows = 128;
+// Bound by the weights up to 50 routes per expert (5.8 TB/s at four), above by the products too: 128 fp8 experts of 1536 x 2048 at 82 routes 118 us
+// (402 MB; the tiles through LDS 147), of 2048 x 768 75 (84 through LDS).
 // The same for one matrix and up to 128 rows (64 columns per block, two groups of waves that take the steps in turn and meet at the
 // end: a block is alone on its CU, and one wave per SIMD waits out every step's chain): 77 rows of 16384 x 2048 int8 16.7 us, fp8
 // 16.4 (128 x 128 tiles 27 and 26, passes of 32 rows 26 and 24; one group 18.4 and 17.7), 40 rows 13.7 and 11.3 (18.5 and 16.6).
@@ -646,18 +645,30 @@ size_t shares_bytes(int most_rows, int N, int K) {
     }
     return bytes;
 }
-template <int KVF, int NG, int S>
+template <int KVF, int RT>
 int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
-    constexpr size_t smem = S * static_cast<size_t>(kExpertRows) * kStepK * 2;
-    constexpr auto kernel = &gemm_columns_kernel<KVF, kExpertRows / 16, NG, S, true>;
+    constexpr int NG = 2, S = 3;   // three blocks of 128 columns to a CU: one's prologue, waits and stores run beside the others' products
+    constexpr size_t smem = S * static_cast<size_t>(RT * 16) * kStepK * 2;
+    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, NG, S, true>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
     const int cols = (a.N + 64 * NG - 1) / (64 * NG);
-    const long long rows = routes / kExpertRows + std::min(routes, a.problems);   // (no cut of the routes into problems makes more)
+    const long long rows = routes / (RT * 16) + std::min(routes, a.problems);   // (no cut of the routes into problems makes more)
     const long long blocks = (rows + 7) / 8 * 8 * cols;
     if (blocks > 0x7FFFFFFF) return PIE_HIP_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), smem, stream, a, cols);
     return launch_status();
+}
+// A block's rows by the routes an expert has on average, so that most experts are one block and few of its rows are none's.  128 fp8
+// experts of 1536 x 2048, us in blocks of 32 / 64 / 96 / 128 rows: 4 routes each 69 / 76 / 81 / 100, 20 78 / 80 / 87 / 104, 44 122 / 86 / 94 / 118, 62 - / 112 / 97 /
+// 114, 78 - / 137 / 110 / 117, 94 - / 143 / 132 / 127; of 2048 x 768 41 / 44 / 60 / 60, 46 / 49 / 62 / 64, 66 / 55 / 65 / 69, - / 73 / 70 / 75, - / 89 / 73 / 77, - / 91 / 95 / 82.
+template <int KVF>
+int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
+    const double each = static_cast<double>(routes) / a.problems;
+    return each <= 24 ? launch_experts<KVF, 2>(a, routes, stream)
+           : each <= 54 ? launch_experts<KVF, 4>(a, routes, stream)
+           : each <= 84 ? launch_experts<KVF, 6>(a, routes, stream)
+                        : launch_experts<KVF, 8>(a, routes, stream);
 }
 template <int KVF, int RT>
 int launch_columns(const GemmArgs& a, hipStream_t stream) {
@@ -756,12 +767,8 @@ int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t s
     if (a.K % kStepK != 0 || a.N % 16 != 0 || static_cast<long long>(a.N) * a.K > 0xFFFFFFFFll ||
         reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16 || a.w_stride % 16)
         return PIE_HIP_ERR_UNSUPPORTED;
-    // Three blocks of 128 columns to a CU hide one another's prologue, waits and stores better than two of 192, which read
-    // the activations less often: 128 fp8 experts of 1536 x 2048, 16 / 48 / 82 / 188 routes each 107 / 113 / 116 / 220 us against 101 / 109 /
-    // 121 / 230; of 2048 x 768, twelve steps, 59 / 64 / 74 / 152 against 63 / 75 / 82 / 167.
-    const bool wide = a.K > 1024 && routes < 64ll * a.problems;
-    if (format == PIE_HIP_FMT_FP8) return wide ? launch_experts<kKvFp8, 3, 4>(b, routes, stream) : launch_experts<kKvFp8, 2, 3>(b, routes, stream);
-    if (format == PIE_HIP_FMT_INT8) return wide ? launch_experts<kKvInt8, 3, 4>(b, routes, stream) : launch_experts<kKvInt8, 2, 3>(b, routes, stream);
+    if (format == PIE_HIP_FMT_FP8) return launch_experts<kKvFp8>(b, routes, stream);
+    if (format == PIE_HIP_FMT_INT8) return launch_experts<kKvInt8>(b, routes, stream);
     return PIE_HIP_ERR_UNSUPPORTED;
 }
 

@@ -327,6 +327,35 @@ def test_byte_experts_over_tile_major_weights(gpu, oracle, fmt, N, K):
                        ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True))
 
 
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+@pytest.mark.parametrize("height,counts", [(32, [0, 1, 31, 32, 33, 64, 0, 7]), (64, [63, 64, 65, 0, 1, 130]), (96, [95, 96, 97, 1, 193, 0]),
+                                           (128, [127, 128, 129, 1, 257])])
+def test_byte_experts_in_blocks_of_each_height(gpu, oracle, fmt, height, counts):
+    """Routes per expert choose a block's rows (32 up to 24 on average, 64 up to 54, 96 up to 84, else 128): experts at a block's edges,
+    three steps of 64 k-values and two, columns off a block.  The bound of the test above."""
+    import torch
+    from pie_amd import ops
+
+    each = sum(counts) / len(counts)
+    assert height == (32 if each <= 24 else 64 if each <= 54 else 96 if each <= 84 else 128)
+    N, K = 272, 192 if height < 96 else 128
+    rng = np.random.default_rng(580 + height)
+    E, T, routes = len(counts), 70, sum(counts)
+    offs = dev(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), gpu)
+    rows = dev(rng.integers(0, T, routes).astype(np.int32), gpu)
+    act = dev(oracle.f32_to_bf16(rng.standard_normal((T, K)).astype(np.float32)), gpu, torch.bfloat16)
+    w = dev(rng.integers(-128, 128, (E, N, K)).astype(np.int8) if fmt == "int8"
+            else rng.integers(0, 0x70, (E, N, K)).astype(np.uint8) | (rng.integers(0, 2, (E, N, K)) << 7).astype(np.uint8), gpu)
+    scale = dev(rng.uniform(0.001, 0.004, (E, N)).astype(np.float32), gpu).bfloat16()
+    t = ops.repack_mfma_tiles(ops.WeightView(fmt, w.reshape(E * N, K), scale.reshape(-1), 0, E * N, K)).data.reshape(E, N, K)
+    bound = K * 4.0 * 0.004 * (128 if fmt == "int8" else 256) * 2 * K * 2.0 ** -24
+    want = ops.moe_grouped_gemm(act, rows, offs, fmt, w, scale, N, K, 257, 0, block_rows=128).float()
+    got = ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, block_rows=0, tiled=True)
+    assert torch.all((got.float() - want).abs() <= 2.0 ** -7 * want.abs() + bound)
+    assert torch.equal(ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, True, block_rows=0, tiled=True),
+                       ops.swiglu_bf16(torch.cat([got[:, 0::2], got[:, 1::2]], dim=1).contiguous()))
+
+
 @pytest.mark.parametrize("tokens", [128, 129, 2048, 2049])
 def test_sorted_layout_of_prompts(gpu, tokens):
     """A block sorts 1025 to 16384 routes out of its registers, others out of memory: either way each expert's routes are together,
