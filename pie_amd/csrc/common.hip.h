@@ -289,12 +289,24 @@ __device__ __forceinline__ float epilogue_pointwise(float v, int code) {
     return v;
 }
 
-// The gated rule on a column pair whose biases are in; {NULL, INFINITY, 1, 0} is the plain one.
+// g / (1 + exp(-alpha g)) for outputs rounded to bf16: exp by the hardware's 2^x of the fraction of the argument (log2 e in two
+// parts, so the fraction is right to fp32), the quotient by its reciprocal: within 3 units of the last fp32 place, in 12
+// instructions where expf and the division took 40 (the epilogue of a block of 256 x 256 gate and up columns 14 -> 7 us: 2048 x 28672 x 4096
+// int4 441 -> 415 us, bf16 404 -> 370).
+__device__ __forceinline__ float silu(float g, float alpha) {
+    const float t = __builtin_amdgcn_fmed3f(-alpha * g, -150.f, 150.f);   // (exp is 0 or inf from there on)
+    const float n = __builtin_rintf(t * 1.44269502f);
+    const float f = fmaf(t, 1.92596299e-8f, fmaf(t, 1.44269502f, -n));
+    const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
+    return g * __builtin_amdgcn_rcpf(1.f + e);
+}
+// The gated rule on a column pair whose biases are in; {NULL, INFINITY, 1, 0} is the plain one.  `F32`: the output stays in fp32.
 constexpr PieHipGlu kPlainGlu = {nullptr, __builtin_inff(), 1.f, 0.f};
+template <bool F32 = false>
 __device__ __forceinline__ float glu_value(float g, float u, const PieHipGlu& r) {
     g = fminf(g, r.limit);
     u = fminf(fmaxf(u, -r.limit), r.limit);
-    return g / (1.f + expf(-r.alpha * g)) * (u + r.shift);
+    return (F32 ? g / (1.f + expf(-r.alpha * g)) : silu(g, r.alpha)) * (u + r.shift);
 }
 inline bool glu_ok(const PieHipGlu* r, int epilogue) { return !r || (epilogue == PIE_HIP_EPI_SWIGLU && r->limit >= 0.f); }
 

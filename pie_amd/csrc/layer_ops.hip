@@ -332,8 +332,7 @@ __global__ void swiglu_kernel(const uint16_t* __restrict__ gu, uint16_t* __restr
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const float g0 = bf16_lo(g[j]), g1 = bf16_hi(g[j]);
-        o[j] = pack_bf16x2(g0 / (1.f + expf(-g0)) * bf16_lo(u[j]),
-                           g1 / (1.f + expf(-g1)) * bf16_hi(u[j]));
+        o[j] = pack_bf16x2(silu(g0, 1.f) * bf16_lo(u[j]), silu(g1, 1.f) * bf16_hi(u[j]));
     }
     *reinterpret_cast<u32x4_t*>(y + n * I + i) = o;
 }

@@ -530,7 +530,7 @@ __global__ __launch_bounds__(256) void glu_f32_kernel(const float* __restrict__ 
         g += glu.bias[2 * i];
         u += glu.bias[2 * i + 1];
     }
-    y[idx] = glu_value(g, u, glu);
+    y[idx] = glu_value<true>(g, u, glu);
 }
 
 }  // namespace
