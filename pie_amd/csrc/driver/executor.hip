@@ -81,9 +81,9 @@ Skinny skinny_cost(const Linear& w, int M) {
 }
 // Microseconds of int4 weights in blocks of up to 64 rows, which scale a group's sum in fp32 as the skinny GEMM does (1e30: not
 // taken).  Where the skinny GEMM is chosen and these are estimated faster, they run in its place: 321 rows of 6144 x 4096 32 us
-// against 70, of 4096 x 14336 58 against 69, of 4096 x 4096 21 against 26, 96 of 28672 x 4096 35 against 50.
+// against 70, of 4096 x 14336 58 against 69, of 4096 x 4096 21 against 26; 5 / 16 / 32 / 96 of 28672 x 4096 14.8 / 14.3 / 17.9 / 35 against 17.5 / 18.7 / 21.9 / 50.
 double groups_cost(const Linear& w, int M, size_t ws_bytes) {
-    return M >= 17 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
+    return M >= 2 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
 bool in_groups(const Linear& w, int M, size_t ws_bytes) { return groups_cost(w, M, ws_bytes) < skinny_cost(w, M).us; }
 // Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
@@ -147,7 +147,7 @@ int model_route(const Linear& w, int M, bool has_norm, size_t ws_bytes) {
         if (M < 2 || !w.data_tiled) return 0;
         const double bytes = static_cast<double>(w.data_bytes());
         const double t_gemv = 3.4 + bytes / 5.5e6 * (M == 2 ? 1.35 : 1.0 + 0.5 * (M - 1));   // (a second row costs the GEMV less than the third and fourth)
-        const double t_skinny = 4.4 + bytes / 4.2e6 + (has_norm ? 4.8 : 0.0);
+        const double t_skinny = std::min(4.4 + bytes / 4.2e6, groups_cost(w, M, ws_bytes)) + (has_norm ? 4.8 : 0.0);
         if (t_gemv <= t_skinny) return 0;
     }
     const GemmPath p = pick_gemm(w, M, ws_bytes);
