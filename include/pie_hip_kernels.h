@@ -279,6 +279,14 @@ size_t pie_hip_gemm_mfma_tiled_workspace_bytes(int most_rows, int N, int K);
  * copy (`tiled`) or bf16 weights, pie_hip_gemm_mfma_tiled; up to 128 rows the latter alone (1e30: not taken). */
 float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes);
 
+/* The same products over tile-major int8 or fp8 weights in blocks of 32 to 128 rows x 128 columns, three to a CU: K % 64 == 0, N % 16 == 0, act
+ * and weight on 16-byte boundaries.  With a workspace few blocks over a long K run in shares of K, as many as it holds of 4 M N bytes
+ * each; the estimate in microseconds (1e30: not taken). */
+int pie_hip_gemm_rows_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale, int scale_is_bf16,
+                            uint16_t* y_bf16, int M, int N, int K, int beta, int epilogue, const PieHipGlu* glu, void* workspace,
+                            size_t workspace_bytes, void* stream);
+float pie_hip_gemm_rows_us(int format, int M, int N, int K, size_t workspace_bytes);
+
 /* pie_hip_gemm_skinny_tiled's arithmetic (int4b8 codes multiplied as they are, a group's sum scaled in fp32) in blocks of up to 64 rows x 128
  * columns, over the tile-major copy: K % 128 == 0, N % 16 == 0, groups a power of two from 128 on, act and weight on 16-byte and scales
  * on 8-byte boundaries.  With a workspace few blocks over a long K run in shares of K, as many as it holds of 4 M N bytes each.

@@ -86,6 +86,14 @@ double groups_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 2 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
 bool in_groups(const Linear& w, int M, size_t ws_bytes) { return groups_cost(w, M, ws_bytes) < skinny_cost(w, M).us; }
+// Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
+// where they are estimated faster.
+double rows_cost(const Linear& w, int M, size_t ws_bytes) {
+    return M > 128 && tile_major(w) ? pie_hip_gemm_rows_us(fmt_code(w.kind), M, w.N, w.K, ws_bytes) : 1e30;
+}
+bool in_rows(const Linear& w, int M, size_t ws_bytes) {
+    return rows_cost(w, M, ws_bytes) < pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes);
+}
 // Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
 // (pie_hip_shares_rmsnorm), for 5 rows and more: 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
 // without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
@@ -116,7 +124,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const double rows_us = w.data_tiled ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * prompt_form : skinny;
         const int fmt = fmt_code(w.kind);
         const double tiles = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
-        const double blocks = tile_major(w) ? pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes) : tiles;
+        const double blocks = std::min(rows_cost(w, M, ws_bytes), tile_major(w) ? static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes)) : tiles);
         if (rows_us < blocks || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
         return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
     }
@@ -220,6 +228,11 @@ bool linear_fused(const Linear& w, const uint16_t* act, const uint16_t* norm_w, 
                                                      gemm_ws, gemm_ws_bytes, s);
             if (sg == PIE_HIP_OK) return true;
             if (sg != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sg);
+        }
+        if (path == GemmPath::Wide && in_rows(w, M, gemm_ws_bytes)) {
+            const int sr = pie_hip_gemm_rows_tiled(fmt, a, w.data_tiled, w.scale, sbf, y, M, w.N, w.K, beta, swiglu, glu, gemm_ws, gemm_ws_bytes, s);
+            if (sr == PIE_HIP_OK) return true;
+            if (sr != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sr);
         }
         if (path == GemmPath::Wide) {
             const int sw = pie_hip_gemm_mfma_tiled(fmt, a, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, sbf, w.group, y, M,

@@ -370,8 +370,12 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
 // end: a block is alone on its CU, and one wave per SIMD waits out every step's chain): 77 rows of 16384 x 2048 int8 16.7 us, fp8
 // 16.4 (128 x 128 tiles 27 and 26, passes of 32 rows 26 and 24; one group 18.4 and 17.7), 40 rows 13.7 and 11.3 (18.5 and 16.6).
 // RT row tiles of 16, NG column tiles per wave, S steps of 64 k-values in flight (LDS stages and weight registers).
-template <int KVF, int RT, int NG, int S, bool EXPERTS, int KP = 1>
-__global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(GemmArgs a, int col_blocks) {
+// Whole: one block has all rows; Experts: rows gathered by route; Rows: blocks of a matrix of many rows, in shares of K (blockIdx.z) where
+// they are few.
+enum class Form { Whole, Experts, Rows };
+template <int KVF, int RT, int NG, int S, Form FORM, int KP = 1>
+__global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(GemmArgs a, int col_blocks, int row_blocks, int per_share) {
+    constexpr bool EXPERTS = FORM == Form::Experts;
     constexpr int kRowsB = RT * 16, kVecs = kRowsB * kStepK / 8, HT = RT / 2, AC = RT / 2;   // a half's row tiles; chunks of eight rows per wave
     extern __shared__ __align__(16) unsigned char smem[];
     const int part = KP == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 256);
@@ -379,21 +383,27 @@ __global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(
     const int tid = threadIdx.x & 255, lane = tid & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int j = lane & 15, q = lane >> 4;
-    const int at = EXPERTS ? static_cast<int>(blockIdx.x >> 3) : static_cast<int>(blockIdx.x);
-    int problem = 0, m0 = 0, M = a.M;
+    // (Rows: each XCD's blocks are neighbours, the row blocks of a column block side by side)
+    const int at = EXPERTS            ? static_cast<int>(blockIdx.x >> 3)
+                   : FORM == Form::Rows ? static_cast<int>((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3))
+                                        : static_cast<int>(blockIdx.x);
+    if (FORM == Form::Rows && at >= row_blocks * col_blocks) return;
+    int problem = 0, m0 = FORM == Form::Rows ? at % row_blocks * kRowsB : 0, M = a.M;
     if constexpr (EXPERTS)
         if (!grouped_place(a.offsets, a.problems, kRowsB, at / col_blocks * 8 + static_cast<int>(blockIdx.x & 7), lane, problem, m0, M)) return;
-    const int N = a.N, K = a.K, nk_all = K / kStepK, T = (N + 15) / 16;
+    const int N = a.N, K = a.K, nk_matrix = K / kStepK, T = (N + 15) / 16;
+    const int first = FORM == Form::Rows ? static_cast<int>(blockIdx.z) * per_share : 0;
+    const int nk_all = FORM == Form::Rows ? min(per_share, nk_matrix - first) : nk_matrix;
     const int nk = (nk_all - part + KP - 1) / KP;   // this group's steps: part, part + KP, ..
-    auto place = [&](int kt) { return min(part + KP * min(kt, max(nk, 1) - 1), nk_all - 1); };   // (past them, or without any: a step again)
-    const int tile0 = (at % col_blocks * 4 + wv) * NG;
+    auto place = [&](int kt) { return first + min(part + KP * min(kt, max(nk, 1) - 1), nk_all - 1); };   // (past them, or without any: a step again)
+    const int tile0 = ((FORM == Form::Rows ? at / row_blocks : at % col_blocks) * 4 + wv) * NG;
     const unsigned char* w = a.w + static_cast<size_t>(problem) * a.w_stride;
     const unsigned char* scale = a.scale + static_cast<size_t>(problem) * a.scale_stride;
 
     // the weights first: they depend on the problem alone, the activations on the routes' rows too
     uint32_t woff[NG];
 #pragma unroll
-    for (int i = 0; i < NG; ++i) woff[i] = static_cast<uint32_t>(min(tile0 + i, T - 1)) * (nk_all * 1024u) + lane * 16u;
+    for (int i = 0; i < NG; ++i) woff[i] = static_cast<uint32_t>(min(tile0 + i, T - 1)) * (nk_matrix * 1024u) + lane * 16u;
     u32x4_t raw[S][NG];
     auto load_w = [&](int kt, int slot) __attribute__((always_inline)) {
         const unsigned char* pw = w + static_cast<size_t>(place(kt)) * 1024;
@@ -542,7 +552,8 @@ __global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = acc[t][i][r] * rs[r];
-            wide_store(a, m, n, v);
+            if (FORM == Form::Rows && a.partial) *reinterpret_cast<f32x4_t*>(a.partial + (static_cast<size_t>(blockIdx.z) * M + m) * N + n) = f32x4_t{v[0], v[1], v[2], v[3]};
+            else wide_store(a, m, n, v);
         }
     }
 }
@@ -649,14 +660,14 @@ template <int KVF, int RT>
 int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
     constexpr int NG = 2, S = 3;   // three blocks of 128 columns to a CU: one's prologue, waits and stores run beside the others' products
     constexpr size_t smem = S * static_cast<size_t>(RT * 16) * kStepK * 2;
-    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, NG, S, true>;
+    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, NG, S, Form::Experts>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
     const int cols = (a.N + 64 * NG - 1) / (64 * NG);
     const long long rows = routes / (RT * 16) + std::min(routes, a.problems);   // (no cut of the routes into problems makes more)
     const long long blocks = (rows + 7) / 8 * 8 * cols;
     if (blocks > 0x7FFFFFFF) return PIE_HIP_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), smem, stream, a, cols);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), smem, stream, a, cols, 0, 0);
     return launch_status();
 }
 // A block's rows by the routes an expert has on average, so that most experts are one block and few of its rows are none's.  128 fp8
@@ -671,14 +682,25 @@ int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
                         : launch_experts<KVF, 8>(a, routes, stream);
 }
 template <int KVF, int RT>
+int launch_rows(const GemmArgs& a, int shares, hipStream_t stream) {
+    constexpr int NG = 2, S = 3;
+    constexpr size_t smem = S * static_cast<size_t>(RT * 16) * kStepK * 2;
+    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, NG, S, Form::Rows>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+    const int rows = (a.M + RT * 16 - 1) / (RT * 16), cols = (a.N + 64 * NG - 1) / (64 * NG), steps = a.K / kStepK;
+    hipLaunchKernelGGL(kernel, dim3((rows * cols + 7) / 8 * 8, 1, shares), dim3(256), smem, stream, a, cols, rows, (steps + shares - 1) / shares);
+    return launch_status();
+}
+template <int KVF, int RT>
 int launch_columns(const GemmArgs& a, hipStream_t stream) {
     constexpr int S = 4, KP = 2;
     constexpr size_t smem = KP * S * static_cast<size_t>(RT * 16) * kStepK * 2;
-    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, 1, S, false, KP>;
+    constexpr auto kernel = &gemm_columns_kernel<KVF, RT, 1, S, Form::Whole, KP>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
     const int cols = (a.N + 63) / 64;
-    hipLaunchKernelGGL(kernel, dim3(cols), dim3(256 * KP), smem, stream, a, cols);
+    hipLaunchKernelGGL(kernel, dim3(cols), dim3(256 * KP), smem, stream, a, cols, 1, 0);
     return launch_status();
 }
 template <int KVF>
@@ -707,6 +729,57 @@ double columns_us(int format, int M, int N, int K) {
     const long long blocks = (N + 63) / 64, slots = size == 0 ? 512 : 256;
     const double crowd = size == 0 && blocks > 256 ? 1.6 : 1.0;
     return 4.0 + static_cast<double>((blocks + slots - 1) / slots) * (K / kStepK) * kStepUs[format == PIE_HIP_FMT_FP8][size] * crowd;
+}
+
+// ---- one-byte weights and many rows in blocks of 32 to 128 rows x 128 columns ---------------------------------------------------
+// (The blocks of 256 rows pass the decoded weights through LDS, in rounds of one block to a CU, and pad their rows.  Three small blocks to a CU
+// fill the machine from some hundred rows on and hide one another's prologue and stores; us there / here, fp8: 400 / 1250 / 1900 rows of
+// 5120 x 2048 29.2 / 36.4 / 64.2 and 15.8 / 34.0 / 46.6, of 2048 x 4096 25.5 / 36.3 / 45.1 and 17.6 / 31.1 / 36.1; 320 / 550 rows of 28672 x 4096 107 / 171 and
+// 84 / 129; 1900 of 4096 x 14336 190 / 199.)
+// A round of up to 768 blocks takes `fixed` and `step` by how many a CU has (one, two, three), the steps past 128 half as much again (long
+// rows); more rounds in proportion and a seventh of one.  Shares' sums as in gemm_groups_mfma.hip.  Fitted to 65 - 1900 rows of ten matrices.
+struct RowsPlan {
+    int row_tiles = 0, shares = 1;
+    double us = 1e30;
+};
+RowsPlan rows_plan(int format, int M, int N, int K, size_t ws_bytes) {
+    struct Round {
+        double fixed, step;
+    };
+    constexpr Round kRounds[4][3] = {{{6.2, 0.185}, {7.0, 0.22}, {4.0, 0.40}},
+                                     {{7.7, 0.28}, {8.0, 0.40}, {6.0, 0.65}},
+                                     {{9.5, 0.30}, {10.5, 0.53}, {9.0, 0.86}},
+                                     {{11.0, 0.375}, {13.0, 0.68}, {13.0, 1.10}}};
+    const int steps = K / kStepK;
+    RowsPlan best;
+    for (int half = 1; half <= 4; ++half) {
+        const long long tiles = (M + half * 32ll - 1) / (half * 32) * ((N + 127) / 128);
+        for (int s = 1; s <= 6; ++s) {
+            const int per = (steps + s - 1) / s;
+            const size_t bytes = static_cast<size_t>(s) * M * N * sizeof(float);
+            if (s > 1 && (per < 4 || bytes > ws_bytes || tiles * (s - 1) >= 768)) break;
+            if ((s - 1) * per >= steps) continue;   // (the last share would be empty)
+            const long long n = tiles * s;
+            const Round& r = kRounds[half - 1][n <= 256 ? 0 : n <= 512 ? 1 : 2];
+            const double round = r.fixed + r.step * (per + 0.5 * std::max(0, per - 128));
+            double us = n <= 768 ? round : round * (static_cast<double>(n) / 768.0 + 1.0 / 7.0);
+            if (format == PIE_HIP_FMT_INT8) us *= 1.05;
+            if (s > 1) us += 3.0 + static_cast<double>(bytes) / 3.2e6;
+            if (us < best.us) best = {half * 2, s, us};
+        }
+    }
+    return best;
+}
+bool rows_fit(int format, int M, int N, int K) {
+    return (format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8) && M > 0 && N > 0 && N % 16 == 0 && K > 0 && K % kStepK == 0 &&
+           static_cast<long long>(N) * K <= 0xFFFFFFFFll && (M + 31ll) / 32 * ((N + 127ll) / 128) < 0x0FFFFFFF;
+}
+template <int KVF>
+int launch_rows(const GemmArgs& a, const RowsPlan& p, hipStream_t stream) {
+    return p.row_tiles == 2   ? launch_rows<KVF, 2>(a, p.shares, stream)
+           : p.row_tiles == 4 ? launch_rows<KVF, 4>(a, p.shares, stream)
+           : p.row_tiles == 6 ? launch_rows<KVF, 6>(a, p.shares, stream)
+                              : launch_rows<KVF, 8>(a, p.shares, stream);
 }
 
 template <class F>
@@ -773,6 +846,44 @@ int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t s
 }
 
 }  // namespace pie_hip
+
+extern "C" float pie_hip_gemm_rows_us(int format, int M, int N, int K, size_t workspace_bytes) {
+    return pie_hip::rows_fit(format, M, N, K) ? static_cast<float>(pie_hip::rows_plan(format, M, N, K, workspace_bytes).us) : 1e30f;
+}
+
+extern "C" int pie_hip_gemm_rows_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale, int scale_is_bf16,
+                                       uint16_t* y_bf16, int M, int N, int K, int beta, int epilogue, const PieHipGlu* glu,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace pie_hip;
+    if (!glu_ok(glu, epilogue)) return PIE_HIP_ERR_INVALID;
+    if (!act_bf16 || !weight || !scale || !y_bf16 || M <= 0 || N <= 0 || K <= 0) return PIE_HIP_ERR_INVALID;
+    const int pointwise = pointwise_code(epilogue), swiglu = epilogue == PIE_HIP_EPI_SWIGLU ? 1 : 0;
+    if ((swiglu && N % 2 != 0) || ((swiglu || pointwise) && beta)) return PIE_HIP_ERR_INVALID;
+    if (!rows_fit(format, M, N, K) || reinterpret_cast<uintptr_t>(act_bf16) % 16 || reinterpret_cast<uintptr_t>(weight) % 16) return PIE_HIP_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(workspace) % 16) workspace = nullptr;
+    const RowsPlan p = rows_plan(format, M, N, K, workspace ? workspace_bytes : 0);
+    GemmArgs a{};
+    a.act = act_bf16;
+    a.w = static_cast<const unsigned char*>(weight);
+    a.scale = static_cast<const unsigned char*>(scale);
+    a.y = y_bf16;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.beta = beta;
+    a.swiglu = swiglu;
+    a.pointwise = pointwise;
+    if (glu) a.glu = *glu;
+    a.scale_is_bf16 = scale_is_bf16;
+    a.aligned = reinterpret_cast<uintptr_t>(y_bf16) % 8 == 0;
+    a.partial = p.shares > 1 ? static_cast<float*>(workspace) : nullptr;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int st = format == PIE_HIP_FMT_FP8 ? launch_rows<kKvFp8>(a, p, s) : launch_rows<kKvInt8>(a, p, s);
+    if (st != PIE_HIP_OK || p.shares == 1) return st;
+    const size_t quads = static_cast<size_t>(M) * (N / 4);
+    hipLaunchKernelGGL(wide_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s, a, p.shares);
+    return launch_status();
+}
 
 extern "C" float pie_hip_gemm_mfma_us(int format, int M, int N, int K, int group_size, int tiled, size_t workspace_bytes) {
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return 1e30f;

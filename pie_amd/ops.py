@@ -631,6 +631,29 @@ def gemm_mfma_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] 
     return y
 
 
+def gemm_rows_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
+                    workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The GEMM over tile-major int8 or fp8 weights in blocks of 32 to 128 rows; with a workspace few blocks over a long K run in
+    shares of K."""
+    _dev(act, torch.bfloat16, "act")
+    M, K = act.shape
+    if K != w.K or w.kind not in ("int8+tiled", "fp8+tiled"):
+        raise KernelError("act K != weight K, or not tile-major one-byte weights")
+    n_out = w.N // 2 if epilogue == 1 else w.N
+    if y is None:
+        if beta:
+            raise KernelError("beta=1 needs an existing y")
+        y = torch.empty((M, n_out), dtype=torch.bfloat16, device=act.device)
+    _dev(y, torch.bfloat16, "y")
+    if tuple(y.shape) != (M, n_out):
+        raise KernelError("y shape mismatch")
+    _check(kernels().pie_hip_gemm_rows_tiled(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale),
+                                             int(w.scale.dtype == torch.bfloat16), _ptr(y), M, w.N, K, beta, epilogue, None, _ptr(workspace),
+                                             C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream()),
+           "pie_hip_gemm_rows_tiled")
+    return y
+
+
 def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
                       workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The GEMM of 17 and more rows over tile-major int4 weights whose groups are scaled in fp32; with a workspace few blocks over a

@@ -332,3 +332,27 @@ def test_columns_of_few_rows_int4(gpu, oracle, M, N, K, G):
     pairs = ops.gemm_mfma_tiled(act, t)
     assert torch.equal(ops.gemm_mfma_tiled(act, t, epilogue=1),
                        ops.swiglu_bf16(torch.cat([pairs[:, 0::2], pairs[:, 1::2]], dim=1).contiguous()))
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (33, 144, 128), (65, 256, 192), (97, 1040, 320), (129, 512, 1088), (200, 5136, 256), (700, 4096, 192), (1300, 8208, 128)])
+def test_rows_in_blocks_of_each_height(gpu, oracle, kind, M, N, K):
+    """Many rows of one-byte weights against the exact sums: row counts off a block, columns off a block of 128, one step of 64 k-values
+    to remainders of those in flight, one to several rounds of blocks; with shares of K too."""
+    import torch
+    from pie_amd import ops
+
+    act, w, t = wide_case(oracle, gpu, kind, M, N, K, 780 + M)
+    codes = w.data.double() if kind == "int8" else w.data.view(torch.float8_e4m3fn).double()
+    wd = codes.reshape(N, K) * w.scale.double().reshape(N, 1)
+    x = act.double()
+    bound = K * 2.0 ** -23 * (x.abs() @ wd.abs().T)
+    ref = x @ wd.T
+    for ws in (None, torch.full((4 << 20,), float("nan"), device=gpu)):
+        got = ops.gemm_rows_tiled(act, t, workspace=ws)
+        assert torch.isfinite(got).all() and ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + bound).all()
+        y0 = torch.randn(M, N, device=gpu).to(torch.bfloat16)
+        res = ops.gemm_rows_tiled(act, t, y=y0.clone(), beta=1, workspace=ws).double()
+        assert ((res - ref - y0.double()).abs() <= 2.0 ** -8 * (ref + y0.double()).abs() + 2 * bound).all()
+        assert torch.equal(ops.gemm_rows_tiled(act, t, epilogue=1, workspace=ws),
+                           ops.swiglu_bf16(torch.cat([got[:, 0::2], got[:, 1::2]], dim=1).contiguous()))
