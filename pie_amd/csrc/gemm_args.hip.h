@@ -21,6 +21,7 @@ struct GemmArgs {
     size_t w_stride, scale_stride;
     int problems, tiled;
     int aligned;   // wide form: y starts at a multiple of 8 bytes
+    int lines;     // whole tile pairs, y on 16 bytes: see store_pair
 };
 
 #define PIE_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
@@ -94,6 +95,58 @@ __device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, floa
             p[r] = f32_to_bf16_bits(v[r]);
         }
     }
+}
+
+inline int stores_lines(const uint16_t* y, int N) { return N % 32 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0; }
+// The same for columns n .. n + 3 and n + 16 .. n + 19, n = 32 k + 4 q with q the lane's sixteenth of the wave (a.lines): neighbouring
+// sixteenths swap half of their values, the even ones end with eight columns of the first tile and the odd ones of the second, so that
+// a store is 16 bytes and a row's four lanes fill 64 (SwiGLU: 8 and 32).
+__device__ __forceinline__ void store_pair(const GemmArgs& a, int m, int n, int q, float* v0, float* v1) {
+    const int nout = a.swiglu ? a.N / 2 : a.N, at = q & 1 ? n + 12 : n;
+    if (a.swiglu) {
+        uint32_t o[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float* v = i ? v1 : v0;
+            float w[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                float g = v[2 * r], u = v[2 * r + 1];
+                if (a.glu.bias) {
+                    g += a.glu.bias[n + 16 * i + 2 * r];
+                    u += a.glu.bias[n + 16 * i + 2 * r + 1];
+                }
+                g = bf16_bits_to_f32(f32_to_bf16_bits(g));
+                u = bf16_bits_to_f32(f32_to_bf16_bits(u));
+                w[r] = glu_value(g, u, a.glu);
+            }
+            o[i] = pack_bf16x2(w[0], w[1]);
+        }
+        const auto s = __builtin_amdgcn_permlane16_swap(o[0], o[1], false, false);
+        *reinterpret_cast<u32x2_t*>(a.y + static_cast<size_t>(m) * nout + at / 2) = u32x2_t{s[0], s[1]};
+        return;
+    }
+    u32x4_t* p = reinterpret_cast<u32x4_t*>(a.y + static_cast<size_t>(m) * nout + at);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        v0[r] = epilogue_pointwise<true>(v0[r], a.pointwise);
+        v1[r] = epilogue_pointwise<true>(v1[r], a.pointwise);
+    }
+    if (a.beta) {
+        const u32x4_t old = *p;
+        const auto x = __builtin_amdgcn_permlane16_swap(old[0], old[2], false, false), y = __builtin_amdgcn_permlane16_swap(old[1], old[3], false, false);
+        v0[0] += bf16_lo(x[0]);
+        v0[1] += bf16_hi(x[0]);
+        v0[2] += bf16_lo(y[0]);
+        v0[3] += bf16_hi(y[0]);
+        v1[0] += bf16_lo(x[1]);
+        v1[1] += bf16_hi(x[1]);
+        v1[2] += bf16_lo(y[1]);
+        v1[3] += bf16_hi(y[1]);
+    }
+    const auto x = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v0[0], v0[1]), pack_bf16x2(v1[0], v1[1]), false, false);
+    const auto y = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v0[2], v0[3]), pack_bf16x2(v1[2], v1[3]), false, false);
+    *p = u32x4_t{x[0], y[0], x[1], y[1]};
 }
 
 // The problem and the rows [m0, m1) of block row `t` when problems are cut into blocks of `rows` rows one after

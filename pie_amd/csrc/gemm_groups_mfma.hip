@@ -234,6 +234,22 @@ __global__ __launch_bounds__(256, 2) void gemm_groups_kernel(const GemmArgs a, c
 #pragma unroll
     for (int t = 0; t < RT; ++t) scale(1, t);
     __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the block ends)
+    if (a.lines && !a.partial && !rot.table) {
+        const int n = tile0 * 16 + 4 * q;
+        if (n >= N) return;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int m = m0 + t * 16 + j;
+            if (m >= M) continue;
+            float v[2][4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[i][r] = acc[t][i][r];
+            store_pair(a, m, n, q, v[0], v[1]);
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
         const int n = (tile0 + i) * 16 + 4 * q;
@@ -320,6 +336,7 @@ int run(GemmArgs a, const Rotation& rot, int group_size, void* ws, size_t ws_byt
     if (p.row_tiles == 0) return PIE_HIP_ERR_UNSUPPORTED;
     a.g_shift = __builtin_ctz(static_cast<unsigned>(group_size));
     a.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+    a.lines = stores_lines(a.y, a.N);
     a.partial = p.shares > 1 ? static_cast<float*>(ws) : nullptr;
     const int st = p.row_tiles == 1   ? launch<1>(a, rot, p.shares, stream)
                    : p.row_tiles == 2 ? launch<2>(a, rot, p.shares, stream)

@@ -326,6 +326,34 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
     __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the block ends)
 
     // ---- epilogue: a lane holds four neighbouring columns of one row per tile ----
+    if (a.lines && !a.partial) {
+#pragma unroll
+        for (int nt = 0; nt < 4; nt += 2) {
+            const int n = n0 + wn * 64 + nt * 16 + 4 * q;
+            if (n >= N) continue;
+            float rs[2][4];
+            if constexpr (F::kRowScale) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        rs[i][r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[n + 16 * i + r])
+                                                   : reinterpret_cast<const float*>(a.scale)[n + 16 * i + r];
+            }
+#pragma unroll
+            for (int t = 0; t < 4 * AH; ++t) {
+                const int m = m0 + wm * 64 * AH + t * 16 + j;
+                if (m >= M) continue;
+                float v[2][4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[i][r] = F::kRowScale ? acc[t][nt + i][r] * rs[i][r] : acc[t][nt + i][r];
+                store_pair(a, m, n, q, v[0], v[1]);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
         const int n = n0 + wn * 64 + nt * 16 + 4 * q;
@@ -535,6 +563,30 @@ __global__ __launch_bounds__(256 * KP, S == 3 ? 3 : 2) void gemm_columns_kernel(
         for (int t = 0; t < RT; ++t) acc[t][0] += meet[t * 256 + tid];
     }
 
+    if constexpr (NG == 2)
+        if (a.lines && !(FORM == Form::Rows && a.partial)) {
+            const int n = tile0 * 16 + 4 * q;
+            if (n >= N) return;
+            float rs[2][4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    rs[i][r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(scale)[n + 16 * i + r])
+                                               : reinterpret_cast<const float*>(scale)[n + 16 * i + r];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                const int m = m0 + t * 16 + j;
+                if (m >= M) continue;
+                float v[2][4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[i][r] = acc[t][i][r] * rs[i][r];
+                store_pair(a, m, n, q, v[0], v[1]);
+            }
+            return;
+        }
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
         const int n = (tile0 + i) * 16 + 4 * q;
@@ -786,6 +838,7 @@ template <class F>
 int run(GemmArgs a, const Plan& p, float* ws, hipStream_t stream) {
     int st = PIE_HIP_OK;
     a.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+    a.lines = stores_lines(a.y, a.N);
     if (p.splits > 1) a.partial = ws;
     if (p.first) st = launch<F, 256>(a, 0, p.first, 1, stream);
     const int rest = (std::max(0, a.N - p.first * 256) + 127) / 128;
@@ -837,6 +890,7 @@ int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, si
 int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t stream) {
     GemmArgs b = a;
     b.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
+    b.lines = stores_lines(a.y, a.N);
     if (a.K % kStepK != 0 || a.N % 16 != 0 || static_cast<long long>(a.N) * a.K > 0xFFFFFFFFll ||
         reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16 || a.w_stride % 16)
         return PIE_HIP_ERR_UNSUPPORTED;
@@ -876,6 +930,7 @@ extern "C" int pie_hip_gemm_rows_tiled(int format, const uint16_t* act_bf16, con
     if (glu) a.glu = *glu;
     a.scale_is_bf16 = scale_is_bf16;
     a.aligned = reinterpret_cast<uintptr_t>(y_bf16) % 8 == 0;
+    a.lines = stores_lines(y_bf16, N);
     a.partial = p.shares > 1 ? static_cast<float*>(workspace) : nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int st = format == PIE_HIP_FMT_FP8 ? launch_rows<kKvFp8>(a, p, s) : launch_rows<kKvInt8>(a, p, s);
