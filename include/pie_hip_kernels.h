@@ -640,7 +640,8 @@ int pie_hip_attn_decode_paged(const uint16_t* q, const uint16_t* k_pages, const 
  * num_requests = num_rows.
  */
 /* How a decode attention launch over (num_rows, num_kv_heads, max_kv_len) splits its rows:
- * units_per_split 16-token units per split, num_splits splits per row (1: no workspace, no merge). */
+ * at most num_splits splits per row (1: no workspace, no merge), equally long but the last and of at least units_per_split 16-token
+ * units each (a row of fewer has one). */
 int pie_hip_attn_decode_plan(int num_rows, int num_kv_heads, int max_kv_len, int* units_per_split,
                              int* num_splits);
 /* Whether a decode attention launch without custom masks over pools of kv_format takes the chunked

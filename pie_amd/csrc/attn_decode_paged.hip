@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kAttnBlock) void attn_decode_split_kernel(
     const uint32_t* __restrict__ row_begin, const int32_t* __restrict__ row_len,
     float* __restrict__ part_o, float* __restrict__ part_ml, uint16_t* __restrict__ o_direct,
     float* __restrict__ lse, const uint16_t* __restrict__ mask_bits, int mask_stride, int hq,
-    int hk, int ps, int units_per_split, int nsplit, float scale_log2e) {
+    int hk, int ps, int least_units, int nsplit, float scale_log2e) {
     using U = UnitRegs<D, GQA, KVF>;
     using KV = typename KvVec<KVF>::type;
     constexpr int LPR = U::LPR, TPI = U::TPI, IPU = U::IPU;
@@ -92,9 +92,9 @@ __global__ __launch_bounds__(kAttnBlock) void attn_decode_split_kernel(
     const uint32_t pg_lo = ext.pg_lo;
     const int kv_len = ext.kv_len;
     const int nunits = (kv_len + kUnitTokens - 1) / kUnitTokens;
-    const int u_begin = split * units_per_split;
+    const int units = split_units(nunits, least_units, nsplit), u_begin = split * units;
     if (u_begin >= nunits) return;
-    const int u_end = min(u_begin + units_per_split, nunits);
+    const int u_end = min(u_begin + units, nunits);
 
     // q for the GQA heads of this kv head: 8 dims per lane per head, as bf16 pairs.
     u32x4_t qv[GQA];
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void attn_decode_mfma_kernel(
     const uint32_t* __restrict__ row_begin, const int32_t* __restrict__ row_len,
     float* __restrict__ part_o, float* __restrict__ part_ml, uint16_t* __restrict__ o_direct,
     float* __restrict__ lse, const uint16_t* __restrict__ mask_bits, int mask_stride, int hq, int hk,
-    int ps, int ps_shift, int units_per_split, int nsplit, float scale_log2e, int num_rows,
+    int ps, int ps_shift, int least_units, int nsplit, float scale_log2e, int num_rows,
     int* __restrict__ row_pieces) {
     static_assert(!(CHUNKS && MASKED), "the chunked launch takes no custom masks");
     static_assert(CHUNKS || NW == kAttnWaves || NW == 2 * kAttnWaves, "the gridded launch has four or eight waves per block");
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void attn_decode_mfma_kernel(
         pg_lo = ext.pg_lo;
         const int kv_len = ext.kv_len;
         nunits = (kv_len + kUnitTokens - 1) / kUnitTokens;
-        const int u_begin = split * units_per_split;
+        const int units = split_units(nunits, least_units, nsplit), u_begin = split * units;
         if (u_begin >= nunits) {
             // (one split per row: a row without keys gets its zeros and its -inf here, no launch
             // of its own for that)
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void attn_decode_mfma_kernel(
             return;
         }
         k_begin = u_begin * kUnitTokens;
-        k_end = min(min(u_begin + units_per_split, nunits) * kUnitTokens, kv_len);
+        k_end = min(min(u_begin + units, nunits) * kUnitTokens, kv_len);
     }
 
     // Q^T fragment: column l16 = query head l16 of this kv head's group (zero beyond GQA)
@@ -871,7 +871,7 @@ __global__ __launch_bounds__(D) void attn_decode_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
     const uint32_t* __restrict__ page_indptr, const uint32_t* __restrict__ last_lens,
     const uint32_t* __restrict__ row_begin, const int32_t* __restrict__ row_len,
-    uint16_t* __restrict__ o, float* __restrict__ lse, int hq, int ps, int units_per_split,
+    uint16_t* __restrict__ o, float* __restrict__ lse, int hq, int ps, int least_units,
     int nsplit) {
     __shared__ float s_w[kMaxSplits];
     __shared__ float s_red[2 * (D / kWave)];
@@ -893,7 +893,7 @@ __global__ __launch_bounds__(D) void attn_decode_merge_kernel(
     if (dd < nsplit) mine_ml = *reinterpret_cast<const float2*>(ml + 2 * dd);
     const int kv_len = row_extent(page_indptr, last_lens, row_begin, row_len, r, ps).kv_len;
     const int nunits = (kv_len + kUnitTokens - 1) / kUnitTokens;
-    const int ns = min(nsplit, (nunits + units_per_split - 1) / units_per_split);
+    const int units = split_units(nunits, least_units, nsplit), ns = min(nsplit, (nunits + units - 1) / units);
 
     float mloc = dd < ns ? mine_ml.x : -INFINITY;
     for (int s = dd + D; s < ns; s += D) mloc = fmaxf(mloc, ml[2 * s]);
@@ -1025,7 +1025,7 @@ __global__ __launch_bounds__(D) void attn_decode_merge_chunks_kernel(
 }
 
 struct SplitPlan {
-    int units_per_split;
+    int least_units;   // of a split (split_units)
     int nsplit;
     int waves = kAttnWaves;   // per block of the gridded launch (eight: whole rows by blocks of twice the width)
 };
@@ -1101,7 +1101,8 @@ SplitPlan plan_splits(int R, int hk, int max_kv_len, bool uniform = false) {
             long long u = (max_units + ns - 1) / ns;
             if (u < 2 * kAttnWaves) u = 2 * kAttnWaves;   // >= 2 units per wave amortises the merge
             if (u > max_units) u = max_units;
-            return {static_cast<int>(u), static_cast<int>((max_units + u - 1) / u)};
+            // (shorter rows fill their slots too, from two units per wave on)
+            return {static_cast<int>(std::min<long long>(u, 2 * kAttnWaves)), static_cast<int>((max_units + u - 1) / u)};
         }
     }
     long long ups = (max_units + want_split - 1) / want_split;
@@ -1188,7 +1189,7 @@ int launch_decode(const uint16_t* q, const void* k_pages, const void* v_pages,
                     hipLaunchKernelGGL((attn_decode_mfma_kernel<D, GQA, KVF, false, false, 2 * kAttnWaves>), dim3(hk, 1, R),
                                        dim3(2 * kAttnBlock), 0, stream, q, k_pages, v_pages, k_scales, v_scales,
                                        page_indices, page_indptr, last_lens, row_begin, row_len, nullptr, nullptr, o, lse,
-                                       nullptr, 0, hq, hk, ps, ps_shift, plan.units_per_split, 1, scale_log2e, R, nullptr);
+                                       nullptr, 0, hq, hk, ps, ps_shift, plan.least_units, 1, scale_log2e, R, nullptr);
                     return launch_status();
                 }
             }
@@ -1197,7 +1198,7 @@ int launch_decode(const uint16_t* q, const void* k_pages, const void* v_pages,
                                    stream, q, k_pages, v_pages, k_scales, v_scales, page_indices, page_indptr,
                                    last_lens, row_begin, row_len,
                                    nullptr, nullptr, o, lse, mask_bits, mask_stride, hq, hk, ps, ps_shift,
-                                   plan.units_per_split, 1, scale_log2e, R, nullptr);
+                                   plan.least_units, 1, scale_log2e, R, nullptr);
                 return launch_status();
             }
             const size_t n_part = static_cast<size_t>(R) * hq * plan.nsplit;
@@ -1209,11 +1210,11 @@ int launch_decode(const uint16_t* q, const void* k_pages, const void* v_pages,
                                stream, q, k_pages, v_pages, k_scales, v_scales, page_indices, page_indptr,
                                last_lens, row_begin, row_len,
                                part_o, part_ml, nullptr, nullptr, mask_bits, mask_stride, hq, hk, ps, ps_shift,
-                               plan.units_per_split, plan.nsplit, scale_log2e, R, nullptr);
+                               plan.least_units, plan.nsplit, scale_log2e, R, nullptr);
             if (!t_defer_merge)
                 hipLaunchKernelGGL((attn_decode_merge_kernel<D>), dim3(R * hq), dim3(D), 0, stream, part_o,
                                    part_ml, page_indptr, last_lens, row_begin, row_len, o, lse, hq, ps,
-                                   plan.units_per_split, plan.nsplit);
+                                   plan.least_units, plan.nsplit);
             return launch_status();
         }
     }
@@ -1223,7 +1224,7 @@ int launch_decode(const uint16_t* q, const void* k_pages, const void* v_pages,
         hipLaunchKernelGGL((attn_decode_split_kernel<D, GQA, MASKED, KVF>), dim3(hk, 1, R),
                            dim3(kAttnBlock), 0, stream, q, k_pages, v_pages, k_scales, v_scales, page_indices,
                            page_indptr, last_lens, row_begin, row_len, nullptr, nullptr, o, lse,
-                           mask_bits, mask_stride, hq, hk, ps, plan.units_per_split, 1, scale_log2e);
+                           mask_bits, mask_stride, hq, hk, ps, plan.least_units, 1, scale_log2e);
         return launch_status();
     }
     const size_t n_part = static_cast<size_t>(R) * hq * plan.nsplit;
@@ -1234,11 +1235,11 @@ int launch_decode(const uint16_t* q, const void* k_pages, const void* v_pages,
     hipLaunchKernelGGL((attn_decode_split_kernel<D, GQA, MASKED, KVF>), dim3(hk, plan.nsplit, R),
                        dim3(kAttnBlock), 0, stream, q, k_pages, v_pages, k_scales, v_scales, page_indices, page_indptr,
                        last_lens, row_begin, row_len, part_o, part_ml, nullptr, nullptr, mask_bits,
-                       mask_stride, hq, hk, ps, plan.units_per_split, plan.nsplit, scale_log2e);
+                       mask_stride, hq, hk, ps, plan.least_units, plan.nsplit, scale_log2e);
     if (!t_defer_merge)
         hipLaunchKernelGGL((attn_decode_merge_kernel<D>), dim3(R * hq), dim3(D), 0, stream, part_o,
                            part_ml, page_indptr, last_lens, row_begin, row_len, o, lse, hq, ps,
-                           plan.units_per_split,
+                           plan.least_units,
                            plan.nsplit);
     return launch_status();
 }
@@ -1399,7 +1400,7 @@ extern "C" int pie_hip_attn_decode_plan(int num_rows, int num_kv_heads, int max_
     if (num_rows <= 0 || num_kv_heads <= 0 || max_kv_len < 0 || !units_per_split || !num_splits)
         return PIE_HIP_ERR_INVALID;
     const pie_hip::SplitPlan plan = pie_hip::plan_splits(num_rows, num_kv_heads, max_kv_len);
-    *units_per_split = plan.units_per_split;
+    *units_per_split = plan.least_units;
     *num_splits = plan.nsplit;
     return PIE_HIP_OK;
 }

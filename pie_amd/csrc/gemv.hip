@@ -279,7 +279,7 @@ struct GemvArgs {
     const float* mg_part_o;      // [M, hq, nsplit, d] f32
     const float* mg_part_ml;     // [M, hq, nsplit, 2] f32 (max, sum)
     const int32_t* mg_row_len;   // visible keys per row
-    int mg_nsplit, mg_units_per_split, mg_hq, mg_d;
+    int mg_nsplit, mg_least_units, mg_hq, mg_d;
     int pointwise;   // PIE_HIP_EPI_RELU2 and above: applied to the sum (0: nothing)
     PieHipGlu glu = kPlainGlu;   // swiglu
 };
@@ -484,7 +484,8 @@ __global__ __launch_bounds__(kBlock) void gemv_kernel(const GemvArgs a) {
                 }
                 const int kv_len = a.mg_row_len[m];
                 const int nunits = (kv_len + kAttnUnitTokens - 1) / kAttnUnitTokens;
-                mg_ns[m] = min(a.mg_nsplit, (nunits + a.mg_units_per_split - 1) / a.mg_units_per_split);
+                const int units = split_units(nunits, a.mg_least_units, a.mg_nsplit);
+                mg_ns[m] = min(a.mg_nsplit, (nunits + units - 1) / units);
             }
         } else {
 #pragma unroll
@@ -1207,7 +1208,7 @@ extern "C" int pie_hip_linear_attn_merge(int format, const void* attn_workspace,
     a.mg_part_ml = a.mg_part_o + n_part * head_dim;
     a.mg_row_len = row_kv_len;
     a.mg_nsplit = num_splits;
-    a.mg_units_per_split = units_per_split;
+    a.mg_least_units = units_per_split;
     a.mg_hq = num_q_heads;
     a.mg_d = head_dim;
     hipStream_t st = static_cast<hipStream_t>(stream);
