@@ -6,7 +6,8 @@
 // int4 weights takes as many of those as half the MFMAs' time, and every step ended in a wait for all transfers.  Here:
 //   - eight waves, two to a SIMD, the second four one barrier behind the first: one wave's operand reads and transfers run
 //     beside the other's MFMAs; a wave's tile of 128 x 64 needs 24 reads of 16 bytes per 64 MFMAs;
-//   - the weights are the MFMAs' first operand, so that a lane ends with four neighbouring columns and stores 8 bytes;
+//   - the weights are the MFMAs' first operand, so that a lane ends with four neighbouring columns, and
+//     stores 16 bytes with its neighbour's (store_pair: 1.8 % of an 8b prompt of 2048 tokens; the figures below are from before it);
 //   - weights are decoded between the MFMAs, one vector per phase, from the tile-major copy;
 //   - transfers into LDS run one to two steps ahead and no wait drains them;
 //   - a chiplet's blocks are neighbours (the row blocks of a column block share its weights in one L2).
