@@ -286,6 +286,8 @@ int pie_hip_gemm_rows_tiled(int format, const uint16_t* act_bf16, const void* we
                             uint16_t* y_bf16, int M, int N, int K, int beta, int epilogue, const PieHipGlu* glu, void* workspace,
                             size_t workspace_bytes, void* stream);
 float pie_hip_gemm_rows_us(int format, int M, int N, int K, size_t workspace_bytes);
+/* The rows of a block and the shares of K that such a call runs in. */
+int pie_hip_gemm_rows_plan(int format, int M, int N, int K, size_t workspace_bytes, int* block_rows, int* shares);
 
 /* pie_hip_gemm_skinny_tiled's arithmetic (int4b8 codes multiplied as they are, a group's sum scaled in fp32) in blocks of up to 64 rows x 128
  * columns, over the tile-major copy: K % 128 == 0, N % 16 == 0, groups a power of two from 128 on, act and weight on 16-byte and scales

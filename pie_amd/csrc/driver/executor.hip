@@ -124,8 +124,11 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const double rows_us = w.data_tiled ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * prompt_form : skinny;
         const int fmt = fmt_code(w.kind);
         const double tiles = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
-        const double blocks = std::min(rows_cost(w, M, ws_bytes), tile_major(w) ? static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes)) : tiles);
-        if (rows_us < blocks || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
+        const double rows = rows_cost(w, M, ws_bytes), wide = tile_major(w) ? static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes)) : tiles;
+        const double blocks = std::min(rows, wide);
+        // (on narrow outputs blocks of few rows and the passes are close, and the passes' estimate is the one that is too high: 160 rows of 3072 x 4096 and
+        // 320 of 2048 x 2048 fp8 13.9 and 13.7 us in passes, 17.0 and 14.7 in blocks)
+        if (rows_us < std::min(1.12 * rows, wide) || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
         return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
     }
     const double tiles = static_cast<double>((w.N + 127) / 128);

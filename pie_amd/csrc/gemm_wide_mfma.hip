@@ -787,11 +787,13 @@ double columns_us(int format, int M, int N, int K) {
 
 // ---- one-byte weights and many rows in blocks of 32 to 128 rows x 128 columns ---------------------------------------------------
 // (The blocks of 256 rows pass the decoded weights through LDS, in rounds of one block to a CU, and pad their rows.  Three small blocks to a CU
-// fill the machine from some hundred rows on and hide one another's prologue and stores; us there / here, fp8: 400 / 1250 / 1900 rows of
-// 5120 x 2048 29.2 / 36.4 / 64.2 and 15.8 / 34.0 / 46.6, of 2048 x 4096 25.5 / 36.3 / 45.1 and 17.6 / 31.1 / 36.1; 320 / 550 rows of 28672 x 4096 107 / 171 and
-// 84 / 129; 1900 of 4096 x 14336 190 / 199.)
-// A round of up to 768 blocks takes `fixed` and `step` by how many a CU has (one, two, three), the steps past 128 half as much again (long
-// rows); more rounds in proportion and a seventh of one.  Shares' sums as in gemm_groups_mfma.hip.  Fitted to 65 - 1900 rows of ten matrices.
+// fill the machine from some hundred rows on and hide one another's prologue and stores.  Weights from HBM, us there / here, fp8: 400 / 1300 / 2048
+// rows of 5120 x 2048 30.9 / 17.0, 37.3 / 33.8 and 60.2 / 46.9; 320 / 512 rows of 28672 x 4096 109 / 84 and 114 / 112; int8: 400 of 2048 x 4096 26.1 / 20.5.)
+// Blocks that share a CU with c - 1 others take `fixed` and `step` of the c-th column (four: more in proportion), where only some CUs have the c-th up to an
+// eighth less.  A block alone waits for its weights from HBM at every step, three of which are in flight: 0.33 - 0.54 us a step whatever the
+// rows, which is why a long K of few blocks pays for shares.  Shares' sums meet in a second kernel, 3 us and their bytes at 3.6 TB/s.  Measured over 50
+// matrices of 1024 - 28672 x 1024 - 14336 and 129 - 2048 rows, each call's weights out of HBM: 3 % rms, the faster of both kernels missed by 1 % on
+// average and by at most 7.
 struct RowsPlan {
     int row_tiles = 0, shares = 1;
     double us = 1e30;
@@ -800,10 +802,14 @@ RowsPlan rows_plan(int format, int M, int N, int K, size_t ws_bytes) {
     struct Round {
         double fixed, step;
     };
-    constexpr Round kRounds[4][3] = {{{6.2, 0.185}, {7.0, 0.22}, {4.0, 0.40}},
-                                     {{7.7, 0.28}, {8.0, 0.40}, {6.0, 0.65}},
-                                     {{9.5, 0.30}, {10.5, 0.53}, {9.0, 0.86}},
-                                     {{11.0, 0.375}, {13.0, 0.68}, {13.0, 1.10}}};
+    constexpr Round kRounds[2][4][4] = {{{{3.8, 0.325}, {4.6, 0.364}, {5.1, 0.547}, {5.6, 0.705}},
+                                         {{4.4, 0.463}, {5.9, 0.529}, {7.9, 0.735}, {8.6, 0.959}},
+                                         {{5.6, 0.481}, {8.4, 0.647}, {10.0, 0.952}, {12.2, 1.275}},
+                                         {{7.1, 0.538}, {9.8, 0.830}, {11.4, 1.220}, {14.5, 1.611}}},
+                                        {{{3.5, 0.430}, {4.4, 0.466}, {5.9, 0.585}, {6.3, 0.751}},
+                                         {{4.6, 0.468}, {6.3, 0.571}, {7.8, 0.813}, {8.7, 1.050}},
+                                         {{5.7, 0.512}, {8.0, 0.716}, {10.0, 1.026}, {11.7, 1.398}},
+                                         {{7.1, 0.586}, {9.8, 0.889}, {11.6, 1.295}, {14.1, 1.731}}}};
     const int steps = K / kStepK;
     RowsPlan best;
     for (int half = 1; half <= 4; ++half) {
@@ -814,11 +820,12 @@ RowsPlan rows_plan(int format, int M, int N, int K, size_t ws_bytes) {
             if (s > 1 && (per < 4 || bytes > ws_bytes || tiles * (s - 1) >= 768)) break;
             if ((s - 1) * per >= steps) continue;   // (the last share would be empty)
             const long long n = tiles * s;
-            const Round& r = kRounds[half - 1][n <= 256 ? 0 : n <= 512 ? 1 : 2];
-            const double round = r.fixed + r.step * (per + 0.5 * std::max(0, per - 128));
-            double us = n <= 768 ? round : round * (static_cast<double>(n) / 768.0 + 1.0 / 7.0);
-            if (format == PIE_HIP_FMT_INT8) us *= 1.05;
-            if (s > 1) us += 3.0 + static_cast<double>(bytes) / 3.2e6;
+            const int c = static_cast<int>(std::min(4ll, (n + 255) / 256));
+            const Round& r = kRounds[format == PIE_HIP_FMT_INT8][half - 1][c - 1];
+            double us = r.fixed + r.step * per;
+            if (n > 1024) us *= static_cast<double>(n) / 1024.0;
+            else us *= 1.0 - (c == 1 ? 0.04 : 0.13) * (c - n / 256.0);
+            if (s > 1) us += 3.0 + static_cast<double>(bytes) / 3.6e6;
             if (us < best.us) best = {half * 2, s, us};
         }
     }
@@ -905,6 +912,15 @@ int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t s
 
 extern "C" float pie_hip_gemm_rows_us(int format, int M, int N, int K, size_t workspace_bytes) {
     return pie_hip::rows_fit(format, M, N, K) ? static_cast<float>(pie_hip::rows_plan(format, M, N, K, workspace_bytes).us) : 1e30f;
+}
+
+extern "C" int pie_hip_gemm_rows_plan(int format, int M, int N, int K, size_t workspace_bytes, int* block_rows, int* shares) {
+    if (!block_rows || !shares) return PIE_HIP_ERR_INVALID;
+    if (!pie_hip::rows_fit(format, M, N, K)) return PIE_HIP_ERR_UNSUPPORTED;
+    const pie_hip::RowsPlan p = pie_hip::rows_plan(format, M, N, K, workspace_bytes);
+    *block_rows = p.row_tiles * 16;
+    *shares = p.shares;
+    return PIE_HIP_OK;
 }
 
 extern "C" int pie_hip_gemm_rows_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale, int scale_is_bf16,

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -690,6 +690,19 @@ def gemm_groups_shares_norm(act: torch.Tensor, w: WeightView, x: torch.Tensor, n
     _check(kernels().pie_hip_shares_rmsnorm(_ptr(workspace), shares, _ptr(x), _ptr(norm_weight), _ptr(y), M, w.N, C.c_float(eps), _stream()),
            "pie_hip_shares_rmsnorm")
     return y, shares.value
+
+
+def gemm_rows_us(kind: str, M: int, N: int, K: int, workspace_bytes: int = 0) -> float:
+    lib = kernels()
+    lib.pie_hip_gemm_rows_us.restype = C.c_float
+    return float(lib.pie_hip_gemm_rows_us(FMT[kind], M, N, K, C.c_size_t(workspace_bytes)))
+
+
+def gemm_rows_plan(kind: str, M: int, N: int, K: int, workspace_bytes: int = 0) -> Tuple[int, int]:
+    """Rows of a block and shares of K of `gemm_rows_tiled`."""
+    rows, shares = C.c_int(0), C.c_int(0)
+    _check(kernels().pie_hip_gemm_rows_plan(FMT[kind], M, N, K, C.c_size_t(workspace_bytes), C.byref(rows), C.byref(shares)), "pie_hip_gemm_rows_plan")
+    return rows.value, shares.value
 
 
 def gemm_groups_us(M: int, N: int, K: int, group: int, workspace_bytes: int = 0) -> float:

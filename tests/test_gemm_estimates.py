@@ -1,0 +1,40 @@
+"""The estimates that choose a GEMM's kernel, its blocks and its shares of K, against times measured on an MI355X with each call's weights
+out of HBM (host-only entry points, no GPU call)."""
+import pytest
+
+WORKSPACE = 32 << 20
+
+# (format, rows, N, K): microseconds in blocks of 256 rows, and in blocks of (rows, shares of K) for every way within an eighth of the fastest.
+# On the long K of these, a few blocks without shares wait for HBM at each of 128 and 224 steps and take up to 1.45 times as long.
+ONE_BYTE = {
+    ("int8", 256, 4096, 14336): (45.2, {(64, 4): 45.1, (96, 5): 46.1, (128, 4): 46.9, (64, 6): 48.1, (128, 6): 50.1, (96, 4): 50.3}),
+    ("int8", 800, 2048, 8192): (45.3, {(96, 3): 41.5, (128, 4): 42.8, (64, 2): 44.6, (96, 4): 44.7, (64, 3): 45.2, (96, 5): 45.6, (64, 4): 46.0}),
+    ("int8", 192, 8192, 8192): (48.6, {(96, 4): 40.3, (96, 3): 43.3, (64, 4): 44.5, (128, 4): 45.3}),
+    ("int8", 256, 8192, 8192): (48.3, {(128, 4): 49.2, (64, 2): 49.2, (128, 2): 50.8, (64, 3): 51.5, (128, 3): 52.8, (96, 2): 53.5, (96, 4): 54.3}),
+    ("int8", 400, 5120, 8192): (54.4, {(128, 3): 52.8, (96, 2): 53.7, (64, 2): 54.8, (96, 3): 56.5, (64, 3): 57.1, (128, 4): 59.4}),
+    ("fp8", 1024, 2048, 8192): (47.0, {(128, 4): 45.2, (64, 2): 45.2, (64, 3): 46.3, (128, 2): 47.1, (128, 3): 48.9, (96, 4): 49.8, (96, 2): 50.1, (96, 3): 50.1}),
+    ("fp8", 256, 4096, 14336): (44.6, {(96, 5): 44.0, (128, 4): 44.6, (64, 4): 45.0, (64, 6): 47.6, (96, 4): 47.8, (128, 6): 48.8}),
+    ("fp8", 512, 3072, 8192): (41.6, {(96, 3): 39.5, (64, 4): 40.3, (128, 5): 40.6, (128, 4): 41.9, (64, 5): 44.0, (64, 3): 44.2, (64, 2): 44.4}),
+    ("fp8", 400, 5120, 8192): (54.0, {(128, 3): 50.4, (64, 2): 50.5, (96, 2): 50.6, (32, 1): 54.0, (96, 3): 54.3, (64, 3): 54.5, (128, 4): 56.6}),
+    ("fp8", 700, 2048, 14336): (55.5, {(96, 4): 51.1, (128, 5): 54.2, (96, 3): 55.5, (64, 4): 55.7}),
+    ("fp8", 1300, 2048, 4096): (43.8, {(32, 1): 33.3, (64, 1): 35.9, (96, 2): 37.0, (96, 1): 37.0}),
+    ("fp8", 1300, 5120, 2048): (37.3, {(128, 1): 33.8, (64, 1): 34.5, (96, 1): 35.2}),
+    ("fp8", 400, 5120, 2048): (30.9, {(32, 1): 17.0}),
+    ("fp8", 320, 28672, 4096): (109.2, {(128, 1): 83.7, (64, 1): 86.0, (96, 1): 87.6}),
+    ("int8", 1300, 6144, 4096): (103.5, {(96, 1): 70.0, (64, 1): 72.7}),
+}
+
+
+@pytest.mark.parametrize("shape", ONE_BYTE, ids=str)
+def test_one_byte_prompts_take_a_way_within_an_eighth_of_the_fastest(shape):
+    from pie_amd import ops
+
+    kind, M, N, K = shape
+    tall, ways = ONE_BYTE[shape]
+    fastest = min(tall, *ways.values())
+    us = ops.gemm_rows_us(kind, M, N, K, WORKSPACE)
+    if us < ops.gemm_mfma_us(kind, M, N, K, 0, True, WORKSPACE):
+        plan = ops.gemm_rows_plan(kind, M, N, K, WORKSPACE)
+        assert plan in ways and abs(us / ways[plan] - 1) < 0.2
+    else:
+        assert tall <= 1.125 * fastest
