@@ -619,6 +619,15 @@ bool Executor::alloc_pools() {
     return true;
 }
 
+bool Executor::few_in_blocks(Quant kind, long long routes, int experts, int hidden, int inner) {
+    if ((kind != Quant::Int8 && kind != Quant::Fp8) || grouped_in_blocks(kind, routes, experts)) return false;
+    auto both = [&](int blocks) {
+        return pie_hip_moe_few_routes_us(fmt_code(kind), static_cast<int>(routes), experts, 2 * inner, hidden, 1, blocks) +
+               pie_hip_moe_few_routes_us(fmt_code(kind), static_cast<int>(routes), experts, hidden, inner, 0, blocks);
+    };
+    return 1.03f * both(1) < both(0);
+}
+
 // x += sum_k w_k * down_e(swiglu(gate_up_e(norm(x)))) over each token's top-k experts
 // (driver/portable/src/graph_common.cpp:237-345; kernel-by-kernel form
 // driver/cuda/src/model/kimi_forward.cpp:662-714): norm, router GEMM, one routing kernel, two
@@ -654,13 +663,11 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     auto wptr = [&](const Linear& l) { return tiled ? l.data_tiled : l.data; };
     auto sptr = [&](const Linear& l) { return tiled && l.scale_tiled ? l.scale_tiled : l.scale; };
     // many routes per expert (a prompt's tokens): blocks of an expert's routes on the tiled GEMM (widths that the passes
-    // refuse stay refused).  One-byte tile-major weights take blocks of 32 to 128 rows for any number of routes: 128 fp8 experts of 1536 x 2048 and
-    // 2048 x 768, passes / blocks of 2, 16, 64, 128 and 256 tokens of eight routes: 26 / 23, 91 / 83, 118 / 111, 129 / 115 and 173 / 119 us.
+    // refuse stay refused); one-byte tile-major weights take smaller blocks for few routes too, by an estimate
     const int unit = w.wgu.kind == Quant::Bf16 ? 64 : 256;
     const bool fits = H % unit == 0 && Ie % unit == 0;
     bool done = false;
-    const bool one_byte = w.wgu.kind == Quant::Int8 || w.wgu.kind == Quant::Fp8;
-    if (grouped_in_blocks(w.wgu.kind, N * K, E) || (one_byte && tiled)) {
+    if (grouped_in_blocks(w.wgu.kind, N * K, E) || (tiled && few_in_blocks(w.wgu.kind, N * K, E, H, Ie))) {
         auto blocks = [&](const Linear& l, const uint16_t* act, const int32_t* rows, uint16_t* y, int rows_out, int cols, int epilogue) {
             return pie_hip_moe_grouped_gemm_mfma_fmt(fmt, act, rows, moe_offsets_, E, N * K, wptr(l), l.data_bytes() / E, l.scale,
                                                      l.scale_bytes() / E, sbf, l.group, y, rows_out, cols, epilogue, tiled ? 1 : 0,
@@ -1335,12 +1342,15 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
 }
 
 // The same for a mixture's experts: whether `routes` over `experts` of a storage format run in blocks of an expert's routes (1)
-// or in passes of 16 (0).
-extern "C" int pie_hip_driver_experts_in_blocks(int format, long long routes, int experts) {
+// or in passes of 16 (0); with sizes (`hidden` > 0) those of tile-major experts.
+extern "C" int pie_hip_driver_experts_in_blocks(int format, long long routes, int experts, int hidden, int inner) {
     using namespace pie_hip_driver;
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || routes <= 0 || experts <= 0) return -1;
     constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
-    return Executor::grouped_in_blocks(kinds[format], routes, experts) ? 1 : 0;
+    return Executor::grouped_in_blocks(kinds[format], routes, experts) ||
+                   (hidden > 0 && inner > 0 && Executor::few_in_blocks(kinds[format], routes, experts, hidden, inner))
+               ? 1
+               : 0;
 }
 
 // And for a batch's attention: the rows of request r are qo_indptr[r] .. qo_indptr[r + 1] (of R requests), row i sees

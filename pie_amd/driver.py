@@ -163,7 +163,7 @@ def lib() -> C.CDLL:
         l.pie_hip_driver_linear_route.restype = C.c_int
         l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
         l.pie_hip_driver_experts_in_blocks.restype = C.c_int
-        l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int]
+        l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int, C.c_int, C.c_int]
         l.pie_hip_driver_attention_cut.restype = C.c_longlong
         l.pie_hip_driver_attention_cut.argtypes = [C.c_void_p, C.c_int, C.c_void_p] + [C.c_int] * 4 + [C.c_void_p, C.c_size_t]
         l.pie_driver_hip_run_inproc.restype = C.c_int
@@ -476,9 +476,10 @@ def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: 
     return LINEAR_ROUTES[route]
 
 
-def experts_in_blocks(kind: str, routes: int, experts: int) -> bool:
-    """Host-only: whether a mixture's routes run in blocks of an expert's routes (else in passes of 16)."""
-    return lib().pie_hip_driver_experts_in_blocks(_FORMATS.index(kind), routes, experts) == 1
+def experts_in_blocks(kind: str, routes: int, experts: int, hidden: int = 0, inner: int = 0) -> bool:
+    """Host-only: whether a mixture's routes run in blocks of an expert's routes (else in passes of 16); tile-major experts of
+    hidden x inner with the sizes, row-major ones without."""
+    return lib().pie_hip_driver_experts_in_blocks(_FORMATS.index(kind), routes, experts, hidden, inner) == 1
 
 
 def attention_cut(requests: Sequence[tuple], q_heads: int, kv_heads: int, head_dim: int, one_byte: bool = False) -> dict:

@@ -38,3 +38,32 @@ def test_one_byte_prompts_take_a_way_within_an_eighth_of_the_fastest(shape):
         assert plan in ways and abs(us / ways[plan] - 1) < 0.2
     else:
         assert tall <= 1.125 * fastest
+
+
+# (format, experts, hidden, inner): microseconds of gate|up and down by routes, in passes of 16 and in blocks of 32
+FEW_ROUTES = {
+    ("fp8", 8, 4096, 14336): {2: (76, 151), 4: (143, 192), 8: (162, 219), 32: (243, 248), 64: (245, 250)},
+    ("int8", 8, 4096, 14336): {2: (81, 179), 4: (147, 222), 8: (165, 248), 32: (244, 278), 64: (246, 281)},
+    ("fp8", 128, 2048, 768): {8: (21, 18), 16: (24, 21), 32: (39, 31), 128: (83, 75), 256: (110, 102)},
+    ("int8", 128, 2048, 768): {8: (25, 22), 16: (27, 25), 32: (43, 33), 128: (84, 79), 256: (109, 106)},
+    ("fp8", 16, 4096, 2048): {2: (28, 31), 4: (30, 32), 8: (39, 36), 32: (66, 64), 64: (70, 66)},
+    ("int8", 16, 4096, 2048): {2: (32, 38), 4: (33, 39), 8: (45, 41), 32: (67, 67), 64: (70, 67)},
+    ("fp8", 32, 1024, 256): {4: (11, 13), 8: (11, 13), 16: (12, 13), 64: (13, 14), 128: (14, 15)},
+    ("int8", 32, 1024, 256): {4: (12, 14), 8: (12, 15), 16: (12, 15), 64: (14, 15), 128: (14, 16)},
+    ("fp8", 64, 2048, 1024): {8: (21, 19), 16: (27, 25), 32: (44, 35), 128: (71, 66), 256: (80, 74)},
+    ("int8", 64, 2048, 1024): {8: (26, 23), 16: (29, 27), 32: (47, 37), 128: (72, 67), 256: (79, 77)},
+    ("fp8", 8, 2048, 4096): {2: (21, 35), 4: (28, 36), 8: (30, 40), 32: (42, 46), 64: (43, 45)},
+    ("int8", 8, 2048, 4096): {2: (22, 41), 4: (30, 42), 8: (32, 46), 32: (43, 52), 64: (44, 51)},
+    ("fp8", 16, 4096, 6400): {2: (41, 79), 4: (66, 86), 8: (104, 114), 32: (199, 192), 64: (209, 198)},
+    ("int8", 16, 4096, 6400): {2: (52, 88), 4: (68, 94), 8: (101, 124), 32: (194, 202), 64: (201, 205)},
+}
+
+
+@pytest.mark.parametrize("mixture", FEW_ROUTES, ids=str)
+def test_few_routes_per_expert_leave_the_passes_only_where_blocks_are_no_slower(mixture):
+    from pie_amd import driver as drv
+
+    kind, experts, hidden, inner = mixture
+    for routes, (passes, blocks) in FEW_ROUTES[mixture].items():
+        taken = blocks if drv.experts_in_blocks(kind, routes, experts, hidden, inner) else passes
+        assert taken <= 1.06 * passes and taken <= 1.3 * blocks, (routes, passes, blocks)
