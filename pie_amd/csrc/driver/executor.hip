@@ -80,26 +80,43 @@ Skinny skinny_cost(const Linear& w, int M) {
     return {p2, wpasses, wave_form, w.data_tiled ? 5.0 + data / 3.8e6 * wave_form : 5.0 + data / 2.8e6 * (1.0 + 0.85 * (passes - 1))};
 }
 // Microseconds of int4 weights in blocks of up to 64 rows, which scale a group's sum in fp32 as the skinny GEMM does (1e30: not
-// taken).  Where the skinny GEMM is chosen and these are estimated faster, they run in its place: 321 rows of 6144 x 4096 32 us
-// against 70, of 4096 x 14336 58 against 69, of 4096 x 4096 21 against 26; 5 / 16 / 32 / 96 of 28672 x 4096 14.8 / 14.3 / 17.9 / 35 against 17.5 / 18.7 / 21.9 / 50.
+// taken).  Where the skinny GEMM is chosen and these are estimated faster, they run in its place: 320 rows of 4096 x 14336 50 us
+// against 68, of 4096 x 4096 21 against 28; 2 / 16 / 32 / 96 of 28672 x 4096 14.5 / 13.8 / 17.4 / 34.5 against 18.4 / 19.8 / 21.9 / 47.4; 321 of q|k|v with the
+// rotation, 6144 x 4096, 33 against 73.
 double groups_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 2 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
-bool in_groups(const Linear& w, int M, size_t ws_bytes) { return groups_cost(w, M, ws_bytes) < skinny_cost(w, M).us; }
+// The skinny GEMM of tile-major int4 weights as those blocks are compared with: up to 128 rows fitted to 50 matrices of 1024 - 28672 x 1024 - 14336 with
+// weights out of HBM, 7 - 11 % rms.  (The estimate above prices all matrices by their bytes alone: it is 40 % above what few rows of large ones take, and
+// blocks chosen by it ran 1.2 to 1.5 times as long as the passes: 2 rows of 8192 x 8192 12.0 us against 9.9, 8 of 8192 x 1024 5.7 against 4.5.)
+double passes_cost(const Linear& w, int M) {
+    struct Fit {
+        int rows;
+        double fixed, rate, per_n, per_k;
+    };
+    constexpr Fit kFits[] = {{4, 3.21, 6.95e6, 0.061e-3, 0.288e-3},  {16, 3.65, 6.49e6, 0.056e-3, 0.390e-3}, {32, 4.22, 4.20e6, 0.089e-3, 0.337e-3},
+                             {64, 4.53, 3.47e6, 0.195e-3, 0.633e-3}, {96, 4.65, 1.93e6, 0.350e-3, 0.524e-3}, {128, 4.83, 1.72e6, 0.331e-3, 0.555e-3}};
+    for (const Fit& f : kFits)
+        if (M <= f.rows) return f.fixed + static_cast<double>(w.data_bytes()) / f.rate + w.N * f.per_n + w.K * f.per_k;
+    return skinny_cost(w, M).us;
+}
+// (up to 32 rows both are short, and ties stay where they are)
+bool in_groups(const Linear& w, int M, size_t ws_bytes) { return (M <= 32 ? 1.05 : 1.0) * groups_cost(w, M, ws_bytes) < passes_cost(w, M); }
 // Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
 // where they are estimated faster.
 double rows_cost(const Linear& w, int M, size_t ws_bytes) {
     return M > 128 && tile_major(w) ? pie_hip_gemm_rows_us(fmt_code(w.kind), M, w.N, w.K, ws_bytes) : 1e30;
 }
 bool in_rows(const Linear& w, int M, size_t ws_bytes) {
-    return rows_cost(w, M, ws_bytes) < pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes);
+    const double rows = rows_cost(w, M, ws_bytes);
+    return rows < 1e29 && rows < pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes);
 }
 // Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
 // (pie_hip_shares_rmsnorm), for 5 rows and more: 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
 // without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
 bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     if (M < 5 || w.kind != Quant::Int4b8 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return false;
-    double other = std::min(skinny_cost(w, M).us, groups_cost(w, M, ws_bytes));
+    double other = in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M);
     if (M > 128) other = std::min({other, static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 0, ws_bytes)),
                                    static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 1, ws_bytes))});
     return pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes) < other;
@@ -158,7 +175,7 @@ int model_route(const Linear& w, int M, bool has_norm, size_t ws_bytes) {
         if (M < 2 || !w.data_tiled) return 0;
         const double bytes = static_cast<double>(w.data_bytes());
         const double t_gemv = 3.4 + bytes / 5.5e6 * (M == 2 ? 1.35 : 1.0 + 0.5 * (M - 1));   // (a second row costs the GEMV less than the third and fourth)
-        const double t_skinny = std::min(4.4 + bytes / 4.2e6, groups_cost(w, M, ws_bytes)) + (has_norm ? 4.8 : 0.0);
+        const double t_skinny = std::min(4.4 + bytes / 4.2e6, in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : 1e30) + (has_norm ? 4.8 : 0.0);
         if (t_gemv <= t_skinny) return 0;
     }
     const GemmPath p = pick_gemm(w, M, ws_bytes);
@@ -1339,6 +1356,22 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
     int there = 0;   // (only whether a copy is there counts)
     if (tile_major) w.data_tiled = w.scale_tiled = &there;
     return model_route(w, M, false, workspace_bytes);
+}
+
+// And in which form that kernel runs before any measurement: bit 0 int4 rows in blocks that scale groups in fp32 (in the skinny GEMM's place), bit 1 an int4
+// projection into the residual in shares of K that meet in the norm's kernel, bit 2 one-byte rows in blocks of 32 to 128 (in the wide GEMM's place).
+extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, int K, size_t workspace_bytes) {
+    using namespace pie_hip_driver;
+    if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return -1;
+    constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
+    Linear w;
+    w.kind = kinds[format];
+    w.N = N;
+    w.K = K;
+    w.group = group;
+    int there = 0;
+    w.data_tiled = w.scale_tiled = &there;
+    return (in_groups(w, M, workspace_bytes) ? 1 : 0) | (in_shares(w, M, workspace_bytes) ? 2 : 0) | (in_rows(w, M, workspace_bytes) ? 4 : 0);
 }
 
 // The same for a mixture's experts: whether `routes` over `experts` of a storage format run in blocks of an expert's routes (1)

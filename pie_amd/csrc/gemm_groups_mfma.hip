@@ -293,8 +293,8 @@ int launch(const GemmArgs& a, const Rotation& rot, int shares, hipStream_t strea
 
 // Rows per block and shares of K.  A block alone on its CU takes 3.7 us and `alone` a step, or what its weights take at 6.3 TB/s; two to a
 // CU take 2 us more and `pair`; rounds of 512 blocks take 2 us and their steps each, what is left over a sixth of one.
-// The shares' sums meet in a second kernel: 3 us and their bytes at 3.2 TB/s, or (`norm`) 0.2 us a share on top of the norm that would run
-// anyway.  Fitted to 5 - 800 rows of 28672 x 4096, 6144 x 4096, 4096 x 4096 and 4096 x 14336: the plan taken is within 8 % of the fastest of all.
+// The shares' sums meet in a second kernel: 3 us and their bytes at 3.2 TB/s, or (`norm`) 0.1 us a share and their bytes at 4 TB/s on top of the norm
+// that would run anyway.  Fitted to 5 - 800 rows of 28672 x 4096, 6144 x 4096, 4096 x 4096 and 4096 x 14336: the plan taken is within 8 % of the fastest of all.
 struct Plan {
     int row_tiles = 0, shares = 1;
     double us = 1e30;
@@ -315,7 +315,7 @@ Plan plan_of(int M, int N, int K, size_t ws_bytes, bool norm) {
             if (n <= 256) us = 3.7 + per * std::max(alone, n * 8448 / 6.3e6);
             else if (n <= 512) us = 5.7 + per * (alone + (pair - alone) * (0.3 + 0.7 * (n - 256) / 256));
             else us = 2.0 + (n / 512 + 1.0 / 6.0) * (2.0 + per * pair);
-            if (norm) us += 0.2 * s;
+            if (norm) us += 0.1 * s + static_cast<double>(bytes) / 4e6;
             else if (s > 1) us += 3.0 + static_cast<double>(bytes) / 3.2e6;
             if (us < best.us) best = {rt, s, us};
         }

@@ -162,6 +162,8 @@ def lib() -> C.CDLL:
                                           C.c_void_p, C.c_size_t, C.c_char_p, C.c_size_t]
         l.pie_hip_driver_linear_route.restype = C.c_int
         l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
+        l.pie_hip_driver_linear_forms.restype = C.c_int
+        l.pie_hip_driver_linear_forms.argtypes = [C.c_int] * 5 + [C.c_size_t]
         l.pie_hip_driver_experts_in_blocks.restype = C.c_int
         l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int, C.c_int, C.c_int]
         l.pie_hip_driver_attention_cut.restype = C.c_longlong
@@ -474,6 +476,15 @@ def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: 
     if route < 0:
         raise ValueError("linear_route")
     return LINEAR_ROUTES[route]
+
+
+def linear_forms(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 32 << 20) -> dict:
+    """Host-only: the forms the driver's estimates give tile-major weights: `groups` (int4 rows in blocks in the skinny GEMM's place), `shares` (a
+    projection into the residual whose sums meet in the norm), `rows` (one-byte rows in blocks in the wide GEMM's place)."""
+    bits = lib().pie_hip_driver_linear_forms(_FORMATS.index(kind), group, M, N, K, workspace_bytes)
+    if bits < 0:
+        raise ValueError("linear_forms")
+    return {name: bool(bits >> i & 1) for i, name in enumerate(("groups", "shares", "rows"))}
 
 
 def experts_in_blocks(kind: str, routes: int, experts: int, hidden: int = 0, inner: int = 0) -> bool:

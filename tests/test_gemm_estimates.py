@@ -67,3 +67,40 @@ def test_few_routes_per_expert_leave_the_passes_only_where_blocks_are_no_slower(
     for routes, (passes, blocks) in FEW_ROUTES[mixture].items():
         taken = blocks if drv.experts_in_blocks(kind, routes, experts, hidden, inner) else passes
         assert taken <= 1.06 * passes and taken <= 1.3 * blocks, (routes, passes, blocks)
+
+
+# (rows, N, K): microseconds of int4 weights in the skinny GEMM's passes and in blocks that scale groups in fp32
+INT4 = {
+    (2, 8192, 8192): (9.9, 11.4), (2, 8192, 1024): (4.1, 6.2), (3, 5120, 8192): (8.2, 10.4), (4, 6144, 14336): (11.9, 14.3),
+    (4, 28672, 4096): (18.3, 13.7), (8, 8192, 1024): (4.5, 5.7), (16, 28672, 4096): (19.8, 13.8), (16, 2048, 2048): (5.7, 7.5),
+    (17, 3072, 2048): (5.4, 7.4), (24, 4096, 8192): (10.2, 11.7), (32, 28672, 4096): (21.9, 17.4), (40, 2048, 2048): (6.9, 7.8),
+    (64, 6144, 4096): (12.3, 12.7), (96, 28672, 4096): (47.4, 34.5),
+}
+# (rows, N, K): the faster of both and the norm behind it, and in shares of K that meet in the norm's kernel
+INT4_SHARES = {
+    (16, 4096, 14336): (21.5, 13.0), (64, 4096, 14336): (21.8, 19.5), (64, 4096, 4096): (13.3, 11.8), (96, 8192, 8192): (28.2, 25.1),
+    (128, 4096, 8192): (21.9, 19.9), (200, 4096, 4096): (19.8, 20.3), (256, 4096, 4096): (20.1, 21.0), (400, 2048, 2048): (13.6, 15.9),
+    (400, 1024, 8192): (20.9, 19.3),
+}
+
+
+@pytest.mark.parametrize("shape", INT4, ids=str)
+def test_int4_rows_leave_the_passes_only_for_faster_blocks(shape):
+    from pie_amd import driver as drv
+
+    M, N, K = shape
+    passes, blocks = INT4[shape]
+    forms = drv.linear_forms("int4b8", M, N, K, 128)
+    assert not forms["rows"]
+    taken = blocks if forms["groups"] else passes
+    assert taken <= 1.06 * passes and taken <= 1.15 * blocks
+
+
+@pytest.mark.parametrize("shape", INT4_SHARES, ids=str)
+def test_int4_projections_meet_in_the_norm_where_that_is_no_slower(shape):
+    from pie_amd import driver as drv
+
+    M, N, K = shape
+    apart, met = INT4_SHARES[shape]
+    taken = met if drv.linear_forms("int4b8", M, N, K, 128)["shares"] else apart
+    assert taken <= 1.06 * apart and taken <= 1.15 * met
