@@ -157,9 +157,11 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const int per = (steps + shares - 1) / shares;
         split = 15.0 + (per + 3) * (M <= 64 ? 1.06 : 1.36) * std::ceil(tiles * shares / 512.0);
     }
-    const double columns = tile_major(w) ? pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, 0) : 1e30;
-    if (columns < std::min({skinny, split, tiled})) return GemmPath::Wide;
-    if (groups < std::min({skinny, split, tiled})) return GemmPath::Skinny;
+    if (w.kind == Quant::Int4b8) {   // (blocks with fp32 group scales run in the skinny GEMM's place; up to 48 rows of wide outputs that is the wide GEMM's own form)
+        if (groups < std::min(split, tiled)) return M <= 48 && w.N >= 16384 && in_groups(w, M, ws_bytes) ? GemmPath::Wide : GemmPath::Skinny;
+    } else if (tile_major(w) && pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes) < std::min({skinny, split, tiled})) {
+        return GemmPath::Wide;
+    }
     if (split < skinny && split < tiled) return GemmPath::TiledSplitK;
     return tiled < skinny ? GemmPath::Tiled : GemmPath::Skinny;
 }
@@ -525,7 +527,8 @@ void Executor::tune_linears() {
                     continue;
                 if (cand >= 2 && l0.K % 64 != 0) continue;
                 double t = time_us(r, M, cand);
-                if (cand >= 2) t += r.tiled_handicap_us;
+                // (up to 48 rows of int4 weights the wide GEMM's form has the rotation in its epilogue too)
+                if (cand >= 2 && !(cand == 4 && l0.kind == Quant::Int4b8 && M <= 48)) t += r.tiled_handicap_us;
                 if (cand == by_model) model_t = t;
                 if (t < best_t) {
                     best_t = t;
@@ -781,11 +784,12 @@ void Executor::body(int N, int S, int max_kv_len) {
             // in its epilogue too (one launch less per layer)
             bool done = false;
             const int tuned_qkv = N <= 128 ? w.wqkv.tuned[N] : -1;
-            if (fused_rope && !w.q_norm && w.wqkv.data_tiled &&
-                (tuned_qkv >= 0 ? tuned_qkv <= 1 : pick_gemm(w.wqkv, N, gemm_ws_bytes_) == GemmPath::Skinny)) {
+            const GemmPath path = tuned_qkv < 0 ? pick_gemm(w.wqkv, N, gemm_ws_bytes_) : tuned_qkv <= 1 ? GemmPath::Skinny : tuned_qkv == 4 ? GemmPath::Wide : GemmPath::Tiled;
+            const bool groups = in_groups(w.wqkv, N, gemm_ws_bytes_);
+            if (fused_rope && !w.q_norm && w.wqkv.data_tiled && (path == GemmPath::Skinny || (path == GemmPath::Wide && groups && N <= 48))) {
                 if (!prenormed) PIE_KERNEL(pie_hip_rmsnorm(x_, w.attn_norm, xn_, N, H, m.rms_eps, s));
                 const int st =
-                    in_groups(w.wqkv, N, gemm_ws_bytes_)
+                    groups
                         ? pie_hip_qkv_rope_groups_tiled(xn_, w.wqkv.data_tiled, w.wqkv.scale_tiled, w.wqkv.group, N, H, rope_tab_, slots, q_,
                                                         k_pool_[l], v_pool_[l], hq, hk, d, pairing, gemm_ws_, gemm_ws_bytes_, s)
                         : pie_hip_qkv_rope_skinny_tiled(fmt_code(w.wqkv.kind), xn_, w.wqkv.data_tiled,

@@ -777,8 +777,8 @@ bool columns_fit(int format, int M, int N, int K, int group_size) {
 }
 // A round of blocks (one to a CU, two with 64 rows' LDS) takes 4 us and 0.27 - 0.5 a step (measured at 40 - 128 rows of
 // 16384, 5120 and 3072 x 2048 and 28672 x 4096).
-double columns_us(int format, int M, int N, int K) {
-    if (format == PIE_HIP_FMT_INT4B8) return 4.0 + (N + 32767) / 32768 * (K / 256) * (M <= 32 ? 1.05 : 1.26);   // (one block to a CU, no shares)
+double columns_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
+    if (format == PIE_HIP_FMT_INT4B8) return gemm_groups_us(M, N, K, group_size, ws_bytes);
     const int size = M <= 64 ? 0 : M <= 96 ? 1 : 2;
     constexpr double kStepUs[2][3] = {{0.34, 0.40, 0.51}, {0.27, 0.39, 0.50}};
     const long long blocks = (N + 63) / 64, slots = size == 0 ? 512 : 256;
@@ -880,7 +880,7 @@ int run(GemmArgs a, const Plan& p, float* ws, hipStream_t stream) {
 }  // namespace
 
 double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
-    if (columns_fit(format, M, N, K, group_size)) return columns_us(format, M, N, K);
+    if (columns_fit(format, M, N, K, group_size)) return columns_us(format, M, N, K, group_size, ws_bytes);
     return fits(format, M, N, K, group_size) ? plan_of(kRates[format], M, N, K, ws_bytes).us : 1e30;
 }
 // (the choice between its two heights is launch_gemm's)

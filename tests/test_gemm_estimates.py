@@ -104,3 +104,15 @@ def test_int4_projections_meet_in_the_norm_where_that_is_no_slower(shape):
     apart, met = INT4_SHARES[shape]
     taken = met if drv.linear_forms("int4b8", M, N, K, 128)["shares"] else apart
     assert taken <= 1.06 * apart and taken <= 1.15 * met
+
+
+@pytest.mark.parametrize("M", [17, 32, 40, 48])
+def test_few_int4_rows_have_one_estimate(M):
+    """The wide GEMM runs 17 to 48 rows of int4 weights in the blocks that scale groups in fp32: either way to them costs the same."""
+    from pie_amd import driver as drv, ops
+
+    for N, K in ((28672, 4096), (6144, 4096), (4096, 14336), (2048, 2048)):
+        for ws in (0, WORKSPACE):
+            assert ops.gemm_mfma_us("int4b8", M, N, K, 128, True, ws) == ops.gemm_groups_us(M, N, K, 128, ws)
+        if drv.linear_route("int4b8", M, N, K, 128) == "wide":
+            assert drv.linear_forms("int4b8", M, N, K, 128)["groups"]
