@@ -526,12 +526,24 @@ extern "C" size_t pie_hip_driver_export_tensor(PieHipDriver* d, const char* name
     if (nm == "info.tuned") {
         // the kernel each decoder linear runs per row count, as the start-up measurement left it:
         // int8 [4 linears (wqkv, wo, wgu, wdown)][129 row counts] of layer 0 (every layer holds the
-        // same), -1 = the cost model decides, 0 GEMV, 1 skinny GEMM, 2 tiled GEMM, 3 tiled GEMM in K shares
+        // same), -1 = the cost model decides, 0 GEMV, 1 skinny GEMM, 2 tiled GEMM, 3 tiled GEMM in K shares,
+        // 4 tiled GEMM over the tile-major copy
         const auto& lw = d->model.layers.at(0);
         const Linear* lins[4] = {&lw.wqkv, &lw.wo, &lw.wgu, &lw.wdown};
         int8_t tab[4][129];
         for (int i = 0; i < 4; ++i)
             for (int m = 0; m <= 128; ++m) tab[i][m] = lins[i]->tuned[static_cast<size_t>(m)];
+        if (dst && cap >= sizeof(tab)) std::memcpy(dst, tab, sizeof(tab));
+        return sizeof(tab);
+    }
+    if (nm == "info.tuned_forms") {
+        // what it left of the int4 forms: int8 [2][4 linears][129 row counts], blocks that scale groups in fp32 in the skinny GEMM's place and shares of K that
+        // meet in the norm; 0 or 1, -1 = by estimate
+        const auto& lw = d->model.layers.at(0);
+        const Linear* lins[4] = {&lw.wqkv, &lw.wo, &lw.wgu, &lw.wdown};
+        int8_t tab[2][4][129];
+        for (int i = 0; i < 4; ++i)
+            for (size_t m = 0; m <= 128; ++m) tab[0][i][m] = lins[i]->groups[m], tab[1][i][m] = lins[i]->shares[m];
         if (dst && cap >= sizeof(tab)) std::memcpy(dst, tab, sizeof(tab));
         return sizeof(tab);
     }

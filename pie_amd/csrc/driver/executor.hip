@@ -101,7 +101,12 @@ double passes_cost(const Linear& w, int M) {
     return skinny_cost(w, M).us;
 }
 // (up to 32 rows both are short, and ties stay where they are)
-bool in_groups(const Linear& w, int M, size_t ws_bytes) { return (M <= 32 ? 1.05 : 1.0) * groups_cost(w, M, ws_bytes) < passes_cost(w, M); }
+bool in_groups(const Linear& w, int M, size_t ws_bytes) {
+    const double us = groups_cost(w, M, ws_bytes);
+    if (us > 1e29) return false;
+    if (M <= 128 && w.groups[M] >= 0) return w.groups[M] == 1;   // (measured at start-up)
+    return (M <= 32 ? 1.05 : 1.0) * us < passes_cost(w, M);
+}
 // Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
 // where they are estimated faster.
 double rows_cost(const Linear& w, int M, size_t ws_bytes) {
@@ -116,10 +121,13 @@ bool in_rows(const Linear& w, int M, size_t ws_bytes) {
 // without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
 bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     if (M < 5 || w.kind != Quant::Int4b8 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return false;
+    const double us = pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes);
+    if (us > 1e29) return false;
+    if (M <= 128 && w.shares[M] >= 0) return w.shares[M] == 1;   // (measured at start-up)
     double other = in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M);
     if (M > 128) other = std::min({other, static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 0, ws_bytes)),
                                    static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 1, ws_bytes))});
-    return pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes) < other;
+    return us < other;
 }
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
@@ -481,17 +489,13 @@ void Executor::tune_linears() {
     int rot = 0;
     // (the smaller of two timed rounds: a round disturbed by something else on the machine would
     // otherwise decide the dispatch for the life of the process)
-    auto time_us = [&](const Role& r, int M, int force) -> double {
+    auto time_us = [&](auto&& launch) -> double {   // launch(layer): false where it does not take the shape
         constexpr int kWarm = 1, kReps = 4, kRounds = 2;
         double best = 1e30;
         for (int round = 0; round < kRounds; ++round) {
             for (int i = 0; i < kWarm + kReps; ++i) {
                 if (i == kWarm) PIE_HIP_CHECK(hipEventRecord(e0, s));
-                LayerWeights& lw = model_.layers[static_cast<size_t>(rot++ % L)];
-                const uint16_t* nw = r.norm ? lw.*(r.norm) : nullptr;
-                if (!linear_fused(lw.*(r.lin), r.act, nw, m.rms_eps, r.y, M, r.beta, r.swiglu, xn_, gemm_ws_,
-                                  gemm_ws_bytes_, s, force))
-                    return 1e30;
+                if (!launch(model_.layers[static_cast<size_t>(rot++ % L)])) return 1e30;
             }
             PIE_HIP_CHECK(hipEventRecord(e1, s));
             PIE_HIP_CHECK(hipEventSynchronize(e1));
@@ -501,6 +505,16 @@ void Executor::tune_linears() {
         }
         return best;
     };
+    auto time_route = [&](const Role& r, int M, int force) {
+        return time_us([&](LayerWeights& lw) {
+            const uint16_t* nw = r.norm ? lw.*(r.norm) : nullptr;
+            return linear_fused(lw.*(r.lin), r.act, nw, m.rms_eps, r.y, M, r.beta, r.swiglu, xn_, gemm_ws_, gemm_ws_bytes_, s, force);
+        });
+    };
+    // A measurement overrides the cost model only where it is clearly faster (a tenth and
+    // half a microsecond): candidates that tie keep the model's kernel, so that timing noise
+    // does not change which kernel — and with it which rounding — a restart gets.
+    auto clearly = [](double us, double than) { return us < 0.9 * than && us + 0.5 < than; };
     const int ladder[] = {2, 3, 4, 17, 24, 32, 33, 40, 48, 56, 64, 65, 72, 80, 88, 96, 97, 104, 112, 120, 128};
     for (const Role& r : roles) {
         const Linear& l0 = model_.layers[0].*(r.lin);
@@ -517,6 +531,23 @@ void Executor::tune_linears() {
                 prev = M;
                 continue;
             }
+            // rows 5..16 stay with the skinny GEMM; a rung decides for the row counts above the
+            // previous rung up to itself
+            const int lo = M <= 4 ? M : std::max(prev + 1, 17);
+            auto set = [&](std::array<int8_t, 129> Linear::*table, int value, int from) {
+                for (auto& lw : model_.layers)
+                    for (int mm = from; mm <= M; ++mm) (lw.*(r.lin).*table)[static_cast<size_t>(mm)] = static_cast<int8_t>(value);
+            };
+            // int4 weights where the skinny GEMM is chosen: its passes, or the blocks that scale groups in fp32
+            if (groups_cost(l0, M, gemm_ws_bytes_) < 1e29) {
+                const int guess = in_groups(l0, M, gemm_ws_bytes_) ? 1 : 0;
+                double us[2];
+                for (int form = 0; form < 2; ++form) {
+                    set(&Linear::groups, form, M);
+                    us[form] = time_route(r, M, 1);
+                }
+                set(&Linear::groups, clearly(us[1 - guess], us[guess]) ? 1 - guess : guess, lo);
+            }
             int best = -1;
             double best_t = 1e30, model_t = 1e30;
             const int by_model = model_route(l0, M, r.norm != nullptr, gemm_ws_bytes_);
@@ -526,7 +557,7 @@ void Executor::tune_linears() {
                                   pie_hip_gemm_mfma_workspace_bytes(M, l0.N, l0.K) > gemm_ws_bytes_))
                     continue;
                 if (cand >= 2 && l0.K % 64 != 0) continue;
-                double t = time_us(r, M, cand);
+                double t = time_route(r, M, cand);
                 // (up to 48 rows of int4 weights the wide GEMM's form has the rotation in its epilogue too)
                 if (cand >= 2 && !(cand == 4 && l0.kind == Quant::Int4b8 && M <= 48)) t += r.tiled_handicap_us;
                 if (cand == by_model) model_t = t;
@@ -535,16 +566,21 @@ void Executor::tune_linears() {
                     best = cand;
                 }
             }
-            // A measurement overrides the cost model only where it is clearly faster (a tenth and
-            // half a microsecond): candidates that tie keep the model's kernel, so that timing noise
-            // does not change which kernel — and with it which rounding — a restart gets.
-            if (model_t < 1e29 && !(best_t < 0.9 * model_t && best_t + 0.5 < model_t)) best = by_model;
-            // rows 5..16 stay with the skinny GEMM; a rung decides for the row counts above the
-            // previous rung up to itself
-            const int lo = M <= 4 ? M : std::max(prev + 1, 17);
-            if (best >= 0)
-                for (auto& lw : model_.layers)
-                    for (int mm = lo; mm <= M; ++mm) (lw.*(r.lin)).tuned[static_cast<size_t>(mm)] = static_cast<int8_t>(best);
+            if (model_t < 1e29 && !clearly(best_t, model_t)) best = by_model;
+            if (best >= 0) set(&Linear::tuned, best, lo);
+            // the projections into the residual: this route and the norm behind it, or shares of K that meet in the norm
+            const bool residual = r.beta && !model_.is_moe();
+            if (best >= 0 && M > 4 && residual && l0.kind == Quant::Int4b8 && pie_hip_gemm_groups_shares_us(M, l0.N, l0.K, l0.group, gemm_ws_bytes_) < 1e29f) {
+                const int guess = in_shares(l0, M, gemm_ws_bytes_) ? 1 : 0;
+                double us[2];
+                us[0] = time_us([&](LayerWeights& lw) {
+                    const bool done = linear_fused(lw.*(r.lin), r.act, nullptr, m.rms_eps, r.y, M, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
+                    PIE_KERNEL(pie_hip_rmsnorm(x_, lw.ffn_norm, xn_, M, H, m.rms_eps, s));
+                    return done;
+                });
+                us[1] = time_us([&](LayerWeights& lw) { return project_in_shares(lw.*(r.lin), r.act, lw.ffn_norm, M); });
+                set(&Linear::shares, us[1] < 1e29 && clearly(us[1 - guess], us[guess]) ? 1 - guess : us[1] < 1e29 ? guess : 0, lo);
+            }
             prev = M;
         }
     }
@@ -721,6 +757,17 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     }
 }
 
+// x_ += act · W^T in shares of K that meet in the kernel of the norm, whose rows go to xn_; false where the shape is not taken.
+bool Executor::project_in_shares(const Linear& w, const uint16_t* act, const uint16_t* norm, int N) {
+    const ModelConfig& m = model_.cfg();
+    int shares = 0;
+    const int st = pie_hip_gemm_groups_shares(act, w.data_tiled, w.scale_tiled, w.group, N, w.N, w.K, gemm_ws_, gemm_ws_bytes_, &shares, stream_);
+    if (st == PIE_HIP_ERR_UNSUPPORTED) return false;
+    PIE_KERNEL(st);
+    PIE_KERNEL(pie_hip_shares_rmsnorm(static_cast<const float*>(gemm_ws_), shares, x_, norm, xn_, N, m.hidden, m.rms_eps, stream_));
+    return true;
+}
+
 void Executor::body(int N, int S, int max_kv_len) {
     if (model_.cfg().is_stack()) return stack_body(N, S, max_kv_len);
     xn_holds_next_norm_ = false;
@@ -888,16 +935,7 @@ void Executor::body(int N, int S, int max_kv_len) {
         }
         // x_ += act · W^T; true if xn_ then holds the rows under `norm`
         auto project = [&](const Linear& lin, const uint16_t* act, const uint16_t* norm) {
-            int shares = 0;
-            if (norm && in_shares(lin, N, gemm_ws_bytes_)) {
-                const int st = pie_hip_gemm_groups_shares(act, lin.data_tiled, lin.scale_tiled, lin.group, N, lin.N, lin.K, gemm_ws_,
-                                                          gemm_ws_bytes_, &shares, s);
-                if (st == PIE_HIP_OK) {
-                    PIE_KERNEL(pie_hip_shares_rmsnorm(static_cast<const float*>(gemm_ws_), shares, x_, norm, xn_, N, H, m.rms_eps, s));
-                    return true;
-                }
-                if (st != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(st);
-            }
+            if (norm && in_shares(lin, N, gemm_ws_bytes_) && project_in_shares(lin, act, norm, N)) return true;
             linear_fused(lin, act, nullptr, m.rms_eps, x_, N, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
             return false;
         };
@@ -1362,9 +1400,10 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
     return model_route(w, M, false, workspace_bytes);
 }
 
-// And in which form that kernel runs before any measurement: bit 0 int4 rows in blocks that scale groups in fp32 (in the skinny GEMM's place), bit 1 an int4
+// And in which form that kernel runs, by what a measurement said (0 or 1; -1: by estimate): bit 0 int4 rows in blocks that scale groups in fp32 (in the skinny GEMM's place), bit 1 an int4
 // projection into the residual in shares of K that meet in the norm's kernel, bit 2 one-byte rows in blocks of 32 to 128 (in the wide GEMM's place).
-extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, int K, size_t workspace_bytes) {
+extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, int K, int measured_groups, int measured_shares,
+                                           size_t workspace_bytes) {
     using namespace pie_hip_driver;
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return -1;
     constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
@@ -1375,6 +1414,8 @@ extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, 
     w.group = group;
     int there = 0;
     w.data_tiled = w.scale_tiled = &there;
+    w.groups.fill(static_cast<int8_t>(measured_groups));
+    w.shares.fill(static_cast<int8_t>(measured_shares));
     return (in_groups(w, M, workspace_bytes) ? 1 : 0) | (in_shares(w, M, workspace_bytes) ? 2 : 0) | (in_rows(w, M, workspace_bytes) ? 4 : 0);
 }
 

@@ -882,6 +882,21 @@ def test_start_up_warm_up_changes_no_result(gpu):
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
 
 
+def test_start_up_measurement_leaves_the_int4_forms(gpu):
+    """Which int4 rows run in blocks that scale groups in fp32 and which projections meet in the norm: measured per rung from 17 rows on
+    (two to four too, but for q|k|v), 5 to 16 rows and everything without the measurement by estimate."""
+    from pie_amd import driver as drvmod
+
+    for tune in (True, False):
+        with drvmod.Driver(toml_config(tune_linears=tune)) as d:
+            forms = d.export_tensor("info.tuned_forms", np.int8).reshape(2, 4, 129)
+            assert np.all((forms >= -1) & (forms <= 1)) and np.all(forms[:, :, 5:17] == -1)
+            if not tune:
+                assert np.all(forms == -1)
+            else:
+                assert np.all(forms[0, :, 17:] >= 0) and np.all(forms[1, 1::2, 17:] >= 0) and np.all(forms[1, 0::2] == -1)
+
+
 def test_start_up_kernel_measurement_keeps_results_within_rounding(gpu, oracle):
     """[runtime] tune_linears times each decoder linear's candidate kernels at start-up and may route
     a row count to another kernel than the cost model: the kernels sum in different orders, so the

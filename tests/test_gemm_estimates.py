@@ -116,3 +116,17 @@ def test_few_int4_rows_have_one_estimate(M):
             assert ops.gemm_mfma_us("int4b8", M, N, K, 128, True, ws) == ops.gemm_groups_us(M, N, K, 128, ws)
         if drv.linear_route("int4b8", M, N, K, 128) == "wide":
             assert drv.linear_forms("int4b8", M, N, K, 128)["groups"]
+
+
+def test_a_measurement_decides_the_forms_of_up_to_128_int4_rows():
+    """What the start-up measurement found goes before the estimates, where the form takes the shape at all."""
+    from pie_amd import driver as drv
+
+    for M, N, K in ((17, 2048, 2048), (40, 4096, 14336), (128, 4096, 4096)):
+        for form in ("groups", "shares"):
+            got = [drv.linear_forms("int4b8", M, N, K, 128, **{f"measured_{form}": v})[form] for v in (0, 1)]
+            assert got == [False, True], (M, N, K, form)
+            assert not drv.linear_forms("int4b8", M, N, K, 64, **{f"measured_{form}": 1})[form]   # (groups of half a step)
+    assert not drv.linear_forms("int4b8", 40, 4096, 14336, 128, workspace_bytes=0, measured_shares=1)["shares"]
+    for v in (0, 1):   # (more rows are not measured)
+        assert drv.linear_forms("int4b8", 129, 4096, 14336, 128, measured_groups=v, measured_shares=v) == drv.linear_forms("int4b8", 129, 4096, 14336, 128)
