@@ -345,11 +345,13 @@ int pie_hip_moe_grouped_gemm_mfma(const uint16_t* act_bf16, const int32_t* route
                                   int num_experts, int num_routes, const void* weights_bf16, size_t weight_stride_bytes,
                                   uint16_t* y_bf16, int N, int K, int epilogue, int tiled, const PieHipGlu* glu,
                                   int block_rows, void* stream);
+/* The routes of a block in such a call over tile-major int8 or fp8 experts (0: refused). */
+int pie_hip_moe_block_rows(int num_routes, int num_experts, int block_rows);
 /* Estimated microseconds of such a product over tile-major int8 or fp8 experts that have fewer than 16 routes each: in blocks of 32 routes
  * (`in_blocks`), or in the passes of pie_hip_moe_grouped_gemm_tiled. */
 float pie_hip_moe_few_routes_us(int format, int num_routes, int num_experts, int N, int K, int swiglu, int in_blocks);
-/* The same over experts in any storage format, row-major (bf16, fp8 and int8 also tile-major; the latter two in blocks of
- * 128 routes); `scales` as in pie_hip_moe_grouped_gemm.  Int4 groups are powers of two from 32 on; each int4 code times its
+/* The same over experts in any storage format, row-major (bf16, fp8 and int8 also tile-major; the latter two with block_rows 128, or 0: blocks of 32 to
+ * 128 routes by pie_hip_moe_block_rows); `scales` as in pie_hip_moe_grouped_gemm.  Int4 groups are powers of two from 32 on; each int4 code times its
  * scale is rounded to bf16 (pie_hip_moe_grouped_gemm scales a group's sum in fp32). */
 int pie_hip_moe_grouped_gemm_mfma_fmt(int format, const uint16_t* act_bf16, const int32_t* route_act_rows,
                                       const int32_t* expert_offsets, int num_experts, int num_routes,

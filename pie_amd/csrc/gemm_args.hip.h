@@ -190,8 +190,8 @@ __device__ __forceinline__ bool grouped_place(const int32_t* __restrict__ offset
 // tile-major for int4); a workspace lets few blocks over a long K run in shares.  What it and the tiles of
 // gemm_mfma.hip take, in microseconds (1e30: it does not take the shape).
 int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream);
-// Experts' rows gathered by route, over tile-major fp8 or int8 weights.
-int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t stream);
+// Experts' rows gathered by route, over tile-major fp8 or int8 weights (block_rows: 32, 64, 96, 128; 0: by the routes an expert has).
+int launch_gemm_experts(int format, const GemmArgs& a, int routes, int block_rows, hipStream_t stream);
 double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_bytes);
 // Int4 weights with fp32 group scales, tile-major, of at least 128 values a group, in blocks of up to 64 rows; a workspace lets few blocks over a long K run
 // in shares.

@@ -626,7 +626,7 @@ extern "C" int pie_hip_moe_grouped_gemm_mfma_fmt(int format, const uint16_t* act
     a.N = N;
     a.K = K;
     if (glu) a.glu = *glu;
-    if (tiled && bytes) return launch_gemm_experts(format, a, num_routes, static_cast<hipStream_t>(stream));
+    if (tiled && bytes) return launch_gemm_experts(format, a, num_routes, block_rows, static_cast<hipStream_t>(stream));
     // (64 bf16 experts of 3072 x 4096, routes per expert 16 / 64 / 256: 295 / 367 / 985 us in blocks of 64, 310 / 324 / 746
     // of 128, 377 / 412 / 679 of 256; passes of 16 rows: 390 / 1161 / 4300)
     // (128 fp8 experts of 1536 x 2048, routes per expert 24 / 64 / 88 / 128 / 192 / 512: 100 / 153 / 195 / 279 / - / - us in blocks

@@ -728,13 +728,18 @@ int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
 // A block's rows by the routes an expert has on average, so that most experts are one block and few of its rows are none's.  128 fp8
 // experts of 1536 x 2048, us in blocks of 32 / 64 / 96 / 128 rows: 4 routes each 69 / 76 / 81 / 100, 20 78 / 80 / 87 / 104, 44 122 / 86 / 94 / 118, 62 - / 112 / 97 /
 // 114, 78 - / 137 / 110 / 117, 94 - / 143 / 132 / 127; of 2048 x 768 41 / 44 / 60 / 60, 46 / 49 / 62 / 64, 66 / 55 / 65 / 69, - / 73 / 70 / 75, - / 89 / 73 / 77, - / 91 / 95 / 82.
+int expert_rows(int routes, int experts) {
+    const double each = static_cast<double>(routes) / experts;
+    return each <= 24 ? 32 : each <= 54 ? 64 : each <= 84 ? 96 : 128;
+}
 template <int KVF>
-int launch_experts(const GemmArgs& a, int routes, hipStream_t stream) {
-    const double each = static_cast<double>(routes) / a.problems;
-    return each <= 24 ? launch_experts<KVF, 2>(a, routes, stream)
-           : each <= 54 ? launch_experts<KVF, 4>(a, routes, stream)
-           : each <= 84 ? launch_experts<KVF, 6>(a, routes, stream)
-                        : launch_experts<KVF, 8>(a, routes, stream);
+int launch_experts(const GemmArgs& a, int routes, int block_rows, hipStream_t stream) {
+    switch (block_rows ? block_rows : expert_rows(routes, a.problems)) {
+        case 32: return launch_experts<KVF, 2>(a, routes, stream);
+        case 64: return launch_experts<KVF, 4>(a, routes, stream);
+        case 96: return launch_experts<KVF, 6>(a, routes, stream);
+        default: return launch_experts<KVF, 8>(a, routes, stream);
+    }
 }
 template <int KVF, int RT>
 int launch_rows(const GemmArgs& a, int shares, hipStream_t stream) {
@@ -915,19 +920,24 @@ int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, si
     }
 }
 
-int launch_gemm_experts(int format, const GemmArgs& a, int routes, hipStream_t stream) {
+int launch_gemm_experts(int format, const GemmArgs& a, int routes, int block_rows, hipStream_t stream) {
     GemmArgs b = a;
     b.aligned = reinterpret_cast<uintptr_t>(a.y) % 8 == 0;
     b.lines = stores_lines(a.y, a.N);
     if (a.K % kStepK != 0 || a.N % 16 != 0 || static_cast<long long>(a.N) * a.K > 0xFFFFFFFFll ||
         reinterpret_cast<uintptr_t>(a.act) % 16 || reinterpret_cast<uintptr_t>(a.w) % 16 || a.w_stride % 16)
         return PIE_HIP_ERR_UNSUPPORTED;
-    if (format == PIE_HIP_FMT_FP8) return launch_experts<kKvFp8>(b, routes, stream);
-    if (format == PIE_HIP_FMT_INT8) return launch_experts<kKvInt8>(b, routes, stream);
+    if (format == PIE_HIP_FMT_FP8) return launch_experts<kKvFp8>(b, routes, block_rows, stream);
+    if (format == PIE_HIP_FMT_INT8) return launch_experts<kKvInt8>(b, routes, block_rows, stream);
     return PIE_HIP_ERR_UNSUPPORTED;
 }
 
 }  // namespace pie_hip
+
+extern "C" int pie_hip_moe_block_rows(int num_routes, int num_experts, int block_rows) {
+    if (num_routes <= 0 || num_experts <= 0 || (block_rows != 0 && block_rows != 128)) return 0;
+    return block_rows ? block_rows : pie_hip::expert_rows(num_routes, num_experts);
+}
 
 extern "C" float pie_hip_moe_few_routes_us(int format, int num_routes, int num_experts, int N, int K, int swiglu, int in_blocks) {
     if ((format != PIE_HIP_FMT_FP8 && format != PIE_HIP_FMT_INT8) || num_routes <= 0 || num_experts <= 0 || N <= 0 || K <= 0) return 1e30f;

@@ -692,6 +692,11 @@ def gemm_groups_shares_norm(act: torch.Tensor, w: WeightView, x: torch.Tensor, n
     return y, shares.value
 
 
+def moe_block_rows(routes: int, experts: int, block_rows: int = 0) -> int:
+    """Routes of a block of tile-major one-byte experts (0: not a height they take)."""
+    return int(kernels().pie_hip_moe_block_rows(routes, experts, block_rows))
+
+
 def gemm_rows_us(kind: str, M: int, N: int, K: int, workspace_bytes: int = 0) -> float:
     lib = kernels()
     lib.pie_hip_gemm_rows_us.restype = C.c_float

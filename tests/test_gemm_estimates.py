@@ -130,3 +130,11 @@ def test_a_measurement_decides_the_forms_of_up_to_128_int4_rows():
     assert not drv.linear_forms("int4b8", 40, 4096, 14336, 128, workspace_bytes=0, measured_shares=1)["shares"]
     for v in (0, 1):   # (more rows are not measured)
         assert drv.linear_forms("int4b8", 129, 4096, 14336, 128, measured_groups=v, measured_shares=v) == drv.linear_forms("int4b8", 129, 4096, 14336, 128)
+
+
+def test_blocks_of_tile_major_experts_have_the_rows_that_were_asked_for():
+    from pie_amd import ops
+
+    assert [ops.moe_block_rows(each * 8, 8) for each in (1, 24, 25, 54, 55, 84, 85, 4000)] == [32, 32, 64, 64, 96, 96, 128, 128]
+    assert all(ops.moe_block_rows(each * 8, 8, 128) == 128 for each in (1, 50, 500))
+    assert [ops.moe_block_rows(80, 8, rows) for rows in (16, 64, 96, 256)] == [0] * 4

@@ -356,6 +356,28 @@ def test_byte_experts_in_blocks_of_each_height(gpu, oracle, fmt, height, counts)
                        ops.swiglu_bf16(torch.cat([got[:, 0::2], got[:, 1::2]], dim=1).contiguous()))
 
 
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+def test_byte_experts_in_blocks_of_128_where_asked(gpu, oracle, fmt):
+    """block_rows = 128 with few routes: the same sums as in the smaller blocks the rule takes; other heights are refused."""
+    import torch
+    from pie_amd import ops
+
+    counts, T, N, K = [0, 1, 31, 33, 7], 40, 160, 192
+    rng = np.random.default_rng(599)
+    E, routes = len(counts), sum(counts)
+    assert ops.moe_block_rows(routes, E) == 32 and ops.moe_block_rows(routes, E, 128) == 128
+    offs = dev(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), gpu)
+    rows = dev(rng.integers(0, T, routes).astype(np.int32), gpu)
+    act = dev(oracle.f32_to_bf16(rng.standard_normal((T, K)).astype(np.float32)), gpu, torch.bfloat16)
+    w = dev(rng.integers(-128, 128, (E, N, K)).astype(np.int8) if fmt == "int8" else rng.integers(0, 0x70, (E, N, K)).astype(np.uint8), gpu)
+    scale = dev(rng.uniform(0.001, 0.004, (E, N)).astype(np.float32), gpu).bfloat16()
+    t = ops.repack_mfma_tiles(ops.WeightView(fmt, w.reshape(E * N, K), scale.reshape(-1), 0, E * N, K)).data.reshape(E, N, K)
+    call = lambda block_rows: ops.moe_grouped_gemm(act, rows, offs, fmt, t, scale, N, K, 257, 0, block_rows=block_rows, tiled=True)  # noqa: E731
+    assert torch.equal(call(128), call(0))
+    with pytest.raises(ops.KernelError):
+        call(64)
+
+
 @pytest.mark.parametrize("tokens", [128, 129, 2048, 2049])
 def test_sorted_layout_of_prompts(gpu, tokens):
     """A block sorts 1025 to 16384 routes out of its registers, others out of memory: either way each expert's routes are together,
