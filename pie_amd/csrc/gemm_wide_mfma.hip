@@ -566,7 +566,8 @@ __global__ __launch_bounds__(256 * KP, S == 3 ? (RT == 2 ? 6 : 3) : 2) void gemm
         for (int t = 0; t < RT; ++t) acc[t][0] += meet[t * 256 + tid];
     }
 
-    if constexpr (NG == 2 && !(EXPERTS && RT == 2))   // (a decode batch's few rows: nothing to gain, registers to lose)
+    // (a decode batch's few rows: nothing to gain, registers to lose; 128 routes of int8 experts: one register more than three blocks to a CU leave)
+    if constexpr (NG == 2 && !(EXPERTS && (RT == 2 || (RT == 8 && KVF == kKvInt8))))
         if (a.lines && !(FORM == Form::Rows && a.partial)) {
             const int n = tile0 * 16 + 4 * q;
             if (n >= N) return;
