@@ -647,8 +647,10 @@ int pie_hip_attn_decode_paged(const uint16_t* q, const uint16_t* k_pages, const 
  * num_requests = num_rows.
  */
 /* How a decode attention launch over (num_rows, num_kv_heads, max_kv_len) splits its rows:
- * at most num_splits splits per row (1: no workspace, no merge), equally long but the last and of at least units_per_split 16-token
- * units each (a row of fewer has one). */
+ * at most num_splits splits per row (1: no workspace, no merge), one for every units_per_split 16-token units of the row that are begun, equally long but
+ * the last.  pie_hip_attn_row_split: the units of each split of a row of kv_len keys under such a plan: units_per_split at most and more than half as many,
+ * until a row is so long that num_splits splits have to hold it. */
+int pie_hip_attn_row_split(int kv_len, int units_per_split, int num_splits);
 int pie_hip_attn_decode_plan(int num_rows, int num_kv_heads, int max_kv_len, int* units_per_split,
                              int* num_splits);
 /* Whether a decode attention launch without custom masks over pools of kv_format takes the chunked
@@ -856,6 +858,8 @@ int pie_hip_qkv_rope_kvwrite(const uint16_t* packed_qkv, uint16_t* q_out, uint16
  * swiglu.hpp:82). */
 int pie_hip_swiglu(const uint16_t* gate_up_bf16, uint16_t* y_bf16, int num_tokens,
                    int intermediate, void* stream);
+/* y[i] = g / (1 + exp(-alpha g)), g = gate[i], as the epilogues of bf16 outputs compute it before the product with u. */
+int pie_hip_silu(const float* gate, float alpha, float* y, int n, void* stream);
 
 /* out_idx[r] = argmax_i logits[r, i]; ties -> lowest index; NaN never wins.  vocab % 8 == 0.
  * Reference: argmax_bf16_kernel, driver/cuda/src/kernels/argmax.cu:36-80. */

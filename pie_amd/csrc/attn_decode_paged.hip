@@ -1025,7 +1025,7 @@ __global__ __launch_bounds__(D) void attn_decode_merge_chunks_kernel(
 }
 
 struct SplitPlan {
-    int least_units;   // of a split (split_units)
+    int least_units;   // one split for each that is begun (split_units)
     int nsplit;
     int waves = kAttnWaves;   // per block of the gridded launch (eight: whole rows by blocks of twice the width)
 };
@@ -1101,7 +1101,7 @@ SplitPlan plan_splits(int R, int hk, int max_kv_len, bool uniform = false) {
             long long u = (max_units + ns - 1) / ns;
             if (u < 2 * kAttnWaves) u = 2 * kAttnWaves;   // >= 2 units per wave amortises the merge
             if (u > max_units) u = max_units;
-            // (shorter rows fill their slots too, from two units per wave on)
+            // (shorter rows fill their slots too: a split for every two units per wave begun)
             return {static_cast<int>(std::min<long long>(u, 2 * kAttnWaves)), static_cast<int>((max_units + u - 1) / u)};
         }
     }
@@ -1393,6 +1393,11 @@ extern "C" int pie_hip_attn_decode_is_chunked(int kv_format, int num_rows, int n
     if (num_rows <= 0 || num_kv_heads <= 0 || max_kv_len < 0) return 0;
     const pie_hip::SplitPlan plan = pie_hip::plan_splits(num_rows, num_kv_heads, max_kv_len);
     return pie_hip::plan_chunks(num_rows, num_kv_heads, max_kv_len, plan, kv_format != PIE_HIP_KV_BF16).use ? 1 : 0;
+}
+
+extern "C" int pie_hip_attn_row_split(int kv_len, int units_per_split, int num_splits) {
+    if (kv_len < 0 || units_per_split <= 0 || num_splits <= 0) return 0;
+    return pie_hip::split_units((kv_len + pie_hip::kAttnUnitTokens - 1) / pie_hip::kAttnUnitTokens, units_per_split, num_splits);
 }
 
 extern "C" int pie_hip_attn_decode_plan(int num_rows, int num_kv_heads, int max_kv_len, int* units_per_split,

@@ -129,14 +129,16 @@ __device__ __forceinline__ float wave_max(float v) {
 // splits are merged by attn_decode_merge_kernel or by the output projection's prologue).
 constexpr int kAttnUnitTokens = 16;
 
-// Units of each split of a row of `nunits` units: the row in as many splits as have `least` units, at most `nsplit`, all but the last of
-// them equally long (a whole number of 32-key steps).  The plan is made for the longest row, in a captured graph for the longest of its
+// Units of each split of a row of `nunits` units: the row in one split per `least` units begun, at most `nsplit`, all but the last of
+// them equally long (a whole number of 32-key steps).  Up to `nsplit` of them hold `least` units at most and more than half as many (9 units by 8 are 6 and 3, not 8 and
+// 1).  The plan is made for the longest row, in a captured graph for the longest of its
 // bucket: with its split length for every row 16 rows of 1024 - 2048 keys left a third of the resident blocks idle (24.5 us a layer of 8 kv
 // heads, so 22.9; 23 rows of 720 - 1200 keys 22.7, so 21.3).
-__device__ __forceinline__ int split_units(int nunits, int least, int nsplit) {
-    if (nsplit <= 1) return max(nunits, 1);
-    const int n = max(1, min(nsplit, (nunits + least - 1) / least));
-    return max(1, ((nunits + n - 1) / n + 1) & ~1);
+__host__ __device__ __forceinline__ int split_units(int nunits, int least, int nsplit) {
+    if (nsplit <= 1) return nunits > 1 ? nunits : 1;
+    const int begun = (nunits + least - 1) / least, n = begun < 1 ? 1 : begun < nsplit ? begun : nsplit;
+    const int units = ((nunits + n - 1) / n + 1) & ~1;
+    return units > 1 ? units : 1;
 }
 
 // A query row's KV extent comes either from the wire arrays of a decode batch
@@ -299,10 +301,11 @@ __device__ __forceinline__ float epilogue_pointwise(float v, int code) {
     return v;
 }
 
-// g / (1 + exp(-alpha g)), bit for bit what expf and the division give for every bf16 g (checked over all of them at alpha 1, 1.702 and 0.5), in 19
+// g / (1 + exp(-alpha g)), bit for bit what expf and the division give for every bf16 g (at alpha 1, 1.702 and 0.5: pie_hip_silu's test), in 19
 // instructions where those took 28: the exponent's product with log2 e in two parts and the hardware's 2^x of its fraction, no tests of the range
-// (exp is 0 or inf from 150 on); the quotient by the reciprocal and one correction, both sides a quarter so that no reciprocal
-// is subnormal.  The epilogue of a block of 256 x 256 gate and up columns is made of this.
+// (exp is 0 or inf from 150 on); the quotient by the reciprocal and one correction, both sides a quarter so that up to expf's overflow no reciprocal
+// is subnormal.  (Past it, where a quarter of the divisor is still finite, the reciprocal's is: v_rcp_f32 gives zero, and the quotient is the -0 of a division by
+// inf.)  The epilogue of a block of 256 x 256 gate and up columns is made of this.
 __device__ __forceinline__ float silu(float g, float alpha) {
     const float t = __builtin_amdgcn_fmed3f(-alpha * g, -150.f, 150.f);
     const float hi = t * 1.44269502f, lo = fmaf(t, 1.92596299e-8f, fmaf(t, 1.44269502f, -hi));

@@ -316,6 +316,11 @@ __global__ __launch_bounds__(512) void qkv_rope_kvwrite_vec_kernel(
     }
 }
 
+__global__ __launch_bounds__(256) void silu_kernel(const float* __restrict__ g, float alpha, float* __restrict__ y, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) y[i] = silu(g[i], alpha);
+}
+
 // y[n, i] = bf16( silu(g) * u ), g = gu[n, i], u = gu[n, I + i] over a fused gate/up row
 // [N, 2I] (swiglu_bf16_kernel, driver/cuda/src/kernels/swiglu.cu:9-22; fused-row form
 // chunked_swiglu, swiglu.hpp:82).  8 elements per thread.
@@ -492,6 +497,12 @@ extern "C" int pie_hip_qkv_rope_kvwrite(const uint16_t* packed_qkv, uint16_t* q_
                        dim3(64), 0, static_cast<hipStream_t>(stream), packed_qkv, q_out, k_pages,
                        v_pages, q_norm_weight, k_norm_weight, rope_table, kv_slots, num_q_heads,
                        num_kv_heads, head_dim, interleaved, eps);
+    return launch_status();
+}
+
+extern "C" int pie_hip_silu(const float* gate, float alpha, float* y, int n, void* stream) {
+    if (!gate || !y || n <= 0) return PIE_HIP_ERR_INVALID;
+    hipLaunchKernelGGL(silu_kernel, dim3((n + 255u) / 256u), dim3(256), 0, static_cast<hipStream_t>(stream), gate, alpha, y, n);
     return launch_status();
 }
 

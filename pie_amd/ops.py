@@ -308,6 +308,28 @@ def swiglu_bf16(gate_up: torch.Tensor) -> torch.Tensor:
     return y
 
 
+def silu(gate: torch.Tensor, alpha: float = 1.0) -> torch.Tensor:
+    """gate / (1 + exp(-alpha gate)) in fp32, as the epilogues of bf16 outputs compute it."""
+    _dev(gate, torch.float32, "gate")
+    y = torch.empty_like(gate)
+    _check(kernels().pie_hip_silu(_ptr(gate), C.c_float(alpha), _ptr(y), gate.numel(), _stream()), "pie_hip_silu")
+    return y
+
+
+def glu_f32(x: torch.Tensor, rule: Glu) -> torch.Tensor:
+    """The gated rule on fp32 columns (gate_0, up_0, gate_1, ..) by expf and the division."""
+    _dev(x, torch.float32, "x")
+    M, N = x.shape
+    y = torch.empty((M, N // 2), dtype=torch.float32, device=x.device)
+    _check(kernels().pie_hip_glu_f32(_ptr(x), C.byref(rule), _ptr(y), M, N // 2, _stream()), "pie_hip_glu_f32")
+    return y
+
+
+def attn_row_split(kv_len: int, units_per_split: int, num_splits: int) -> int:
+    """16-token units of each split of a decode row under such a plan."""
+    return int(kernels().pie_hip_attn_row_split(kv_len, units_per_split, num_splits))
+
+
 def argmax_bf16(logits: torch.Tensor) -> torch.Tensor:
     _dev(logits, torch.bfloat16, "logits")
     rows, V = logits.shape
@@ -1451,10 +1473,7 @@ def linear_glu(form: str, act: torch.Tensor, w: torch.Tensor, rule: Glu) -> torc
     N, lib = w.shape[0], kernels()
     _dev(w, torch.bfloat16, "w")
     if form == "f32":
-        x = linear_f32(act, w)
-        y = torch.empty((M, N // 2), dtype=torch.float32, device=act.device)
-        _check(lib.pie_hip_glu_f32(_ptr(x), C.byref(rule), _ptr(y), M, N // 2, _stream()), "pie_hip_glu_f32")
-        return y
+        return glu_f32(linear_f32(act, w), rule)
     y = torch.empty((M, N // 2), dtype=torch.bfloat16, device=act.device)
     head = (3, _ptr(act))
     if form == "gemv":

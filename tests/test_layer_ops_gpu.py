@@ -139,6 +139,22 @@ def test_swiglu(gpu, oracle):
     assert d.max() <= 1 and (d == 0).mean() > 0.98
 
 
+@pytest.mark.parametrize("alpha", [1.0, 1.702, 0.5])
+def test_silu_of_every_bf16_gate_is_that_of_expf_and_the_division(gpu, alpha):
+    """The bf16 epilogues' gate against the fp32 rule's, which calls expf and divides: every bf16 value, the ends of expf's range and the
+    infinities among them, bit for bit (the fp32 rule clamps NaN to its limit)."""
+    import torch
+    from pie_amd import ops
+
+    gates = torch.arange(1 << 16, device=gpu, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).float()
+    gates = gates[~torch.isnan(gates)]
+    want = ops.glu_f32(torch.stack([gates, torch.ones_like(gates)], dim=1).contiguous(), ops.glu(alpha=alpha)).flatten()
+    got = ops.silu(gates, alpha)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    there = ~torch.isnan(want)
+    assert there.sum() > 65000 and torch.equal(got[there].view(torch.int32), want[there].view(torch.int32))
+
+
 def test_argmax_ties_nan_and_vocab(gpu, oracle):
     import torch
     from pie_amd import ops
