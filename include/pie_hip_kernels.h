@@ -303,6 +303,8 @@ float pie_hip_gemm_groups_us(int M, int N, int K, int group_size, size_t workspa
 int pie_hip_gemm_groups_shares(const uint16_t* act_bf16, const void* weight, const void* scale, int group_size, int M, int N, int K,
                                void* workspace, size_t workspace_bytes, int* shares, void* stream);
 float pie_hip_gemm_groups_shares_us(int M, int N, int K, int group_size, size_t workspace_bytes);
+/* The rows of a block and the shares of K that a call of either runs in (`norm`: pie_hip_gemm_groups_shares). */
+int pie_hip_gemm_groups_plan(int M, int N, int K, int group_size, size_t workspace_bytes, int norm, int* block_rows, int* shares);
 int pie_hip_shares_rmsnorm(const float* partials, int shares, uint16_t* x_bf16, const uint16_t* weight_bf16, uint16_t* norm_out_bf16,
                            int rows, int hidden, float eps, void* stream);
 /* pie_hip_qkv_rope_skinny_tiled in that form (q_out and the pools on 8-byte boundaries). */

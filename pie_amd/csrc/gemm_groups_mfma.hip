@@ -1,4 +1,4 @@
-// Int4 weights times 17 and more activation rows with the group scales kept in fp32: y[M, N] = epilogue( act[M, K] · W[N, K]^T ),
+// Int4 weights times two and more activation rows with the group scales kept in fp32: y[M, N] = epilogue( act[M, K] · W[N, K]^T ),
 // the skinny GEMM's arithmetic (a group's code products are summed as they are and scaled once, in fp32) in blocks of 16 to 64
 // rows x 128 columns, two blocks of four waves to a CU.
 //
@@ -362,6 +362,16 @@ double gemm_groups_us(int M, int N, int K, int group_size, size_t ws_bytes) {
 
 extern "C" float pie_hip_gemm_groups_us(int M, int N, int K, int group_size, size_t workspace_bytes) {
     return static_cast<float>(pie_hip::gemm_groups_us(M, N, K, group_size, workspace_bytes));
+}
+
+extern "C" int pie_hip_gemm_groups_plan(int M, int N, int K, int group_size, size_t workspace_bytes, int norm, int* block_rows, int* shares) {
+    using namespace pie_hip;
+    if (!block_rows || !shares) return PIE_HIP_ERR_INVALID;
+    const Plan p = fits(M, N, K, group_size) ? plan_of(M, N, K, workspace_bytes, norm != 0) : Plan{};
+    if (p.row_tiles == 0) return PIE_HIP_ERR_UNSUPPORTED;
+    *block_rows = p.row_tiles * 16;
+    *shares = p.shares;
+    return PIE_HIP_OK;
 }
 
 extern "C" float pie_hip_gemm_groups_shares_us(int M, int N, int K, int group_size, size_t workspace_bytes) {

@@ -394,8 +394,8 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
 // the MFMAs' operand by plain loads, three or four steps ahead in registers, each decoded once.  The activations are shared in LDS,
 // as far ahead.  Two or three blocks of four waves to a CU, independent of one another: one's prologue, waits and stores run
 // beside the other's MFMAs.  A row block's column blocks stay on one chiplet and share its activations there.
-// Bound by the weights up to 50 routes per expert (5.8 TB/s at four), above by the products too: 128 fp8 experts of 1536 x 2048 at 82 routes 118 us
-// (402 MB; the tiles through LDS 147), of 2048 x 768 75 (84 through LDS).
+// Bound by the weights up to 50 routes per expert (5.8 TB/s at four), above by the products too: 128 fp8 experts of 1536 x 2048 at 82 routes 111 us
+// (402 MB; the tiles through LDS 147), of 2048 x 768 74 (84 through LDS).
 // The same for one matrix and up to 128 rows (64 columns per block, two groups of waves that take the steps in turn and meet at the
 // end: a block is alone on its CU, and one wave per SIMD waits out every step's chain): 77 rows of 16384 x 2048 int8 16.7 us, fp8
 // 16.4 (128 x 128 tiles 27 and 26, passes of 32 rows 26 and 24; one group 18.4 and 17.7), 40 rows 13.7 and 11.3 (18.5 and 16.6).
@@ -650,7 +650,9 @@ int launch(const GemmArgs& a, int first_col, int col_blocks, int splits, hipStre
 
 // What a launch takes, in microseconds: a round of up to one block per CU is `fixed` and, per step of 64 k-values, `step` for
 // a few blocks; `fixed_full` and `step_full` more when all 256 CUs have one (shared caches, stores, power), most of it only
-// when nearly all have.  Fitted to 160 - 4096 rows of 4096 x 14336, 28672 x 4096, 16384 x 2048 and 4096 x 4096 (within 7 %).
+// when nearly all have.  Fitted to 160 - 4096 rows of 4096 x 14336, 28672 x 4096, 16384 x 2048 and 4096 x 4096 (within 7 %), before the blocks stored 16
+// bytes a lane.  Over 50 matrices of 129 - 2048 rows with these stores and each call's weights out of HBM: int8 and fp8 within 6 % at the median from K of 2048 on and up
+// to a fifth low at 1024, int4 at most 11 % high.  (Int4 stays so: lower figures would take rows from the blocks that scale groups in fp32.)
 struct Rate {
     double fixed, step, fixed_full, step_full;
 };

@@ -654,7 +654,7 @@ def gemm_mfma_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] 
 
 
 def gemm_rows_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
-                    workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    workspace: Optional[torch.Tensor] = None, rule: Optional[Glu] = None) -> torch.Tensor:
     """The GEMM over tile-major int8 or fp8 weights in blocks of 32 to 128 rows; with a workspace few blocks over a long K run in
     shares of K."""
     _dev(act, torch.bfloat16, "act")
@@ -670,15 +670,16 @@ def gemm_rows_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] 
     if tuple(y.shape) != (M, n_out):
         raise KernelError("y shape mismatch")
     _check(kernels().pie_hip_gemm_rows_tiled(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale),
-                                             int(w.scale.dtype == torch.bfloat16), _ptr(y), M, w.N, K, beta, epilogue, None, _ptr(workspace),
+                                             int(w.scale.dtype == torch.bfloat16), _ptr(y), M, w.N, K, beta, epilogue,
+                                             None if rule is None else C.byref(rule), _ptr(workspace),
                                              C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream()),
            "pie_hip_gemm_rows_tiled")
     return y
 
 
 def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
-                      workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """The GEMM of 17 and more rows over tile-major int4 weights whose groups are scaled in fp32; with a workspace few blocks over a
+                      workspace: Optional[torch.Tensor] = None, rule: Optional[Glu] = None) -> torch.Tensor:
+    """The GEMM over tile-major int4 weights whose groups are scaled in fp32, in blocks of up to 64 rows; with a workspace few blocks over a
     long K run in shares of K."""
     _dev(act, torch.bfloat16, "act")
     M, K = act.shape
@@ -692,7 +693,8 @@ def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor
     _dev(y, torch.bfloat16, "y")
     if tuple(y.shape) != (M, n_out):
         raise KernelError("y shape mismatch")
-    _check(kernels().pie_hip_gemm_groups_tiled(_ptr(act), _ptr(w.data), _ptr(w.scale), w.group_size, _ptr(y), M, w.N, K, beta, epilogue, None,
+    _check(kernels().pie_hip_gemm_groups_tiled(_ptr(act), _ptr(w.data), _ptr(w.scale), w.group_size, _ptr(y), M, w.N, K, beta, epilogue,
+                                               None if rule is None else C.byref(rule),
                                                _ptr(workspace), C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()),
                                                _stream()), "pie_hip_gemm_groups_tiled")
     return y
@@ -736,6 +738,14 @@ def gemm_groups_us(M: int, N: int, K: int, group: int, workspace_bytes: int = 0)
     lib = kernels()
     lib.pie_hip_gemm_groups_us.restype = C.c_float
     return float(lib.pie_hip_gemm_groups_us(M, N, K, group, C.c_size_t(workspace_bytes)))
+
+
+def gemm_groups_plan(M: int, N: int, K: int, group: int, workspace_bytes: int = 0, norm: bool = False) -> Tuple[int, int]:
+    """Rows of a block and shares of K of `gemm_groups_tiled`, or (norm) of `gemm_groups_shares_norm`."""
+    rows, shares = C.c_int(0), C.c_int(0)
+    _check(kernels().pie_hip_gemm_groups_plan(M, N, K, group, C.c_size_t(workspace_bytes), int(norm), C.byref(rows), C.byref(shares)),
+           "pie_hip_gemm_groups_plan")
+    return rows.value, shares.value
 
 
 def gemm_mfma_us(kind: str, M: int, N: int, K: int, group: int, tiled: bool, workspace_bytes: int = 0) -> float:

@@ -30,7 +30,8 @@ def groups_case(oracle, gpu, M, N, K, G, seed):
                                      (49, 112, 768, 256), (64, 256, 1152, 128), (65, 1040, 896, 128), (130, 2064, 1408, 128), (321, 16528, 512, 128)])
 def test_blocks_of_group_scaled_rows(gpu, oracle, M, N, K, G):
     """Row counts around each block height, columns off a block of 128, one to eleven steps of 128 k-values (four in flight, their
-    remainders), groups of several steps, more blocks than run at once; with shares of K too."""
+    remainders), groups of several steps, more blocks than run at once, without and with a workspace: mostly in blocks of 16 rows and without shares.  (Each height and
+    shares by the plan: test_gemm_stores_gpu.py.)"""
     import torch
     from pie_amd import ops
 
@@ -113,4 +114,47 @@ def test_shares_that_meet_in_the_norm(gpu, oracle, M, N, K):
     assert ((x.double() - total).abs() <= 2.0 ** -8 * total.abs() + bound).all()
     # (the norm's own rounding: two products and a reciprocal root in fp32, the sum of squares of N values in another order)
     want = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert ((y.double() - want).abs() <= (2.0 ** -8 + N * 2.0 ** -24) * want.abs()).all()
+
+
+@pytest.mark.parametrize("M,hq,hk,d,K,rows,shares", [(18, 4, 2, 64, 2048, 16, 8), (16, 32, 8, 128, 4096, 16, 4), (30, 32, 8, 128, 2944, 32, 5),
+                                                     (37, 16, 4, 128, 4096, 48, 8), (180, 16, 4, 128, 4096, 64, 3)])
+def test_qkv_rope_epilogue_of_shares(gpu, oracle, M, hq, hk, d, K, rows, shares):
+    """The rotation and the cache's rows behind sums that meet in shares of K, every height of a block."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(890 + M)
+    N = (hq + 2 * hk) * d
+    ws = torch.full((6 << 20,), float("nan"), device=gpu)
+    assert ops.gemm_groups_plan(M, N, K, 128, ws.numel() * 4) == (rows, shares)
+    _, mk = make_weight(oracle, rng, "int4b8", N, K)
+    wt = ops.repack_mfma_tiles(mk(gpu))
+    x = dev(oracle.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32)), gpu, torch.bfloat16)
+    tab = ops.rope_table(dev(rng.integers(0, 500, M).astype(np.int32), gpu), dev(oracle.rope_inv_freq(d, 10000.0), gpu), d)
+    slots = rng.permutation(256)[:M].astype(np.int64)
+    slots[1] = -1
+    sg = dev(slots, gpu)
+    for pairing, w in ((1, wt), (2, ops.repack_mfma_tiles(ops.pair_qk_rows(mk(gpu), hq, hk, d)))):
+        pools = [torch.full((256, hk, d), 0.5, device=gpu, dtype=torch.bfloat16) for _ in range(4)]
+        q1 = ops.qkv_rope_skinny_tiled(x, w, tab, sg, pools[0], pools[1], hq, hk, d, pairing=pairing, groups=True, workspace=ws)
+        q2 = ops.qkv_rope_kvwrite(ops.gemm_groups_tiled(x, wt, workspace=ws), pools[2], pools[3], tab, sg, hq, hk, d, pairing == 1)
+        assert np.array_equal(bits(q1), bits(q2))
+        assert np.array_equal(bits(pools[0]), bits(pools[2])) and np.array_equal(bits(pools[1]), bits(pools[3]))
+
+
+@pytest.mark.parametrize("M,N,K,rows,shares", [(1, 16, 384, 16, 2), (17, 8208, 384, 32, 2), (33, 8208, 384, 48, 2), (49, 8208, 384, 64, 2)])
+def test_shares_that_meet_in_the_norm_by_height(gpu, oracle, M, N, K, rows, shares):
+    import torch
+    from pie_amd import ops
+
+    ws = torch.full((8 * M * N,), float("nan"), device=gpu)
+    assert ops.gemm_groups_plan(M, N, K, 128, ws.numel() * 4, True) == (rows, shares)
+    act, t, ref, bound = groups_case(oracle, gpu, M, N, K, 128, 895 + M)
+    x0 = torch.randn(M, N, generator=torch.Generator(device=gpu).manual_seed(895), device=gpu).to(torch.bfloat16)
+    x = x0.clone()
+    y, got = ops.gemm_groups_shares_norm(act, t, x, torch.ones(N, device=gpu, dtype=torch.bfloat16), 1e-5, ws)
+    total = ref + x0.double()
+    assert got == shares and ((x.double() - total).abs() <= 2.0 ** -8 * total.abs() + bound).all()
+    want = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5)
     assert ((y.double() - want).abs() <= (2.0 ** -8 + N * 2.0 ** -24) * want.abs()).all()

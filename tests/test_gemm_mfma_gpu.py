@@ -338,7 +338,7 @@ def test_columns_of_few_rows_int4(gpu, oracle, M, N, K, G):
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (33, 144, 128), (65, 256, 192), (97, 1040, 320), (129, 512, 1088), (200, 5136, 256), (700, 4096, 192), (1300, 8208, 128)])
 def test_rows_in_blocks_of_each_height(gpu, oracle, kind, M, N, K):
     """Many rows of one-byte weights against the exact sums: row counts off a block, columns off a block of 128, one step of 64 k-values
-    to remainders of those in flight, one to several rounds of blocks; with shares of K too."""
+    to remainders of those in flight, one to several rounds of blocks, without and with a workspace.  (Each height and shares by the plan: test_gemm_stores_gpu.py.)"""
     import torch
     from pie_amd import ops
 

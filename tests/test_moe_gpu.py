@@ -297,8 +297,8 @@ def test_quantised_experts_in_blocks_of_routes(gpu, oracle, fmt, K, G, block_row
 @pytest.mark.parametrize("fmt", ["fp8", "int8"])
 @pytest.mark.parametrize("N,K", [(144, 64), (192, 192), (400, 320), (16, 768), (208, 1088)])
 def test_byte_experts_over_tile_major_weights(gpu, oracle, fmt, N, K):
-    """Blocks of 128 routes over the tile-major copy against those over row-major weights: an expert without routes, with one,
-    at the edges of a block, columns off a block, one step of 64 k-values and remainders of those in flight (K above 1024 and few routes: the other block).
+    """Blocks by the routes an expert has (here 64 and 96) over the tile-major copy against blocks of 128 over row-major weights: an expert without routes, with one,
+    at the edges of a block, columns off a block, one step of 64 k-values and remainders of those in flight.
     The same exact products in fp32, in another order: the bound of the test above."""
     import torch
     from pie_amd import ops
