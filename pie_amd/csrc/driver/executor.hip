@@ -116,6 +116,13 @@ bool in_rows(const Linear& w, int M, size_t ws_bytes) {
     const double rows = rows_cost(w, M, ws_bytes);
     return rows < 1e29 && rows < pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes);
 }
+// Microseconds of an int4 projection whose sums do not wait for the norm.
+double apart_cost(const Linear& w, int M, size_t ws_bytes) {
+    double us = in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M);
+    if (M > 128) us = std::min({us, static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 0, ws_bytes)),
+                                static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 1, ws_bytes))});
+    return us;
+}
 // Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
 // (pie_hip_shares_rmsnorm), for 5 rows and more: 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
 // without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
@@ -124,11 +131,10 @@ bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     const double us = pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes);
     if (us > 1e29) return false;
     if (M <= 128 && w.shares[M] >= 0) return w.shares[M] == 1;   // (measured at start-up)
-    double other = in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M);
-    if (M > 128) other = std::min({other, static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 0, ws_bytes)),
-                                   static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 1, ws_bytes))});
-    return us < other;
+    return us < apart_cost(w, M, ws_bytes);
 }
+// The tiled GEMM, up to 128 rows.
+double tiled_cost(const Linear& w, int M) { return 2.0 + w.K / 64 * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, (w.N + 127) / 128 / 512.0); }
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
     const auto [p2, wpasses, wave_form, skinny] = skinny_cost(w, M);
@@ -156,8 +162,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         if (rows_us < std::min(1.12 * rows, wide) || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
         return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
     }
-    const double tiles = static_cast<double>((w.N + 127) / 128);
-    const double tiled = 2.0 + steps * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, tiles / 512.0);
+    const double tiles = static_cast<double>((w.N + 127) / 128), tiled = tiled_cost(w, M);
     double split = 1e30;
     const size_t need = pie_hip_gemm_mfma_workspace_bytes(M, w.N, w.K);
     if (need && need <= ws_bytes) {
@@ -515,6 +520,8 @@ void Executor::tune_linears() {
     // half a microsecond): candidates that tie keep the model's kernel, so that timing noise
     // does not change which kernel — and with it which rounding — a restart gets.
     auto clearly = [](double us, double than) { return us < 0.9 * than && us + 0.5 < than; };
+    // (int4 forms that the estimates put a fifth apart are not measured: all of them take 55 ms of an 8B driver's start-up, so 20)
+    auto close = [](double a, double b) { return std::max(a, b) < 1.2 * std::min(a, b); };
     const int ladder[] = {2, 3, 4, 17, 24, 32, 33, 40, 48, 56, 64, 65, 72, 80, 88, 96, 97, 104, 112, 120, 128};
     for (const Role& r : roles) {
         const Linear& l0 = model_.layers[0].*(r.lin);
@@ -539,25 +546,31 @@ void Executor::tune_linears() {
                     for (int mm = from; mm <= M; ++mm) (lw.*(r.lin).*table)[static_cast<size_t>(mm)] = static_cast<int8_t>(value);
             };
             // int4 weights where the skinny GEMM is chosen: its passes, or the blocks that scale groups in fp32
+            double skinny_t = 1e30;
             if (groups_cost(l0, M, gemm_ws_bytes_) < 1e29) {
-                const int guess = in_groups(l0, M, gemm_ws_bytes_) ? 1 : 0;
-                double us[2];
-                for (int form = 0; form < 2; ++form) {
-                    set(&Linear::groups, form, M);
-                    us[form] = time_route(r, M, 1);
+                int form = in_groups(l0, M, gemm_ws_bytes_) ? 1 : 0;
+                if (close(groups_cost(l0, M, gemm_ws_bytes_), passes_cost(l0, M))) {
+                    double us[2];
+                    for (int f = 0; f < 2; ++f) {
+                        set(&Linear::groups, f, M);
+                        us[f] = time_route(r, M, 1);
+                    }
+                    if (clearly(us[1 - form], us[form])) form = 1 - form;
+                    skinny_t = us[form];
                 }
-                set(&Linear::groups, clearly(us[1 - guess], us[guess]) ? 1 - guess : guess, lo);
+                set(&Linear::groups, form, lo);
             }
             int best = -1;
             double best_t = 1e30, model_t = 1e30;
             const int by_model = model_route(l0, M, r.norm != nullptr, gemm_ws_bytes_);
             for (int cand = M <= 4 ? 0 : 1; cand <= (M <= 4 ? 1 : 4); ++cand) {
                 if (cand == 4 && by_model != 4) continue;   // (far slower where the model does not expect it)
+                if (cand == 2 && by_model != 2 && l0.kind == Quant::Int4b8 && l0.data_tiled && tiled_cost(l0, M) > 2.0 * passes_cost(l0, M)) continue;   // (likewise)
                 if (cand == 3 && (M > 128 || pie_hip_gemm_mfma_workspace_bytes(M, l0.N, l0.K) == 0 ||
                                   pie_hip_gemm_mfma_workspace_bytes(M, l0.N, l0.K) > gemm_ws_bytes_))
                     continue;
                 if (cand >= 2 && l0.K % 64 != 0) continue;
-                double t = time_route(r, M, cand);
+                double t = cand == 1 && skinny_t < 1e29 ? skinny_t : time_route(r, M, cand);
                 // (up to 48 rows of int4 weights the wide GEMM's form has the rotation in its epilogue too)
                 if (cand >= 2 && !(cand == 4 && l0.kind == Quant::Int4b8 && M <= 48)) t += r.tiled_handicap_us;
                 if (cand == by_model) model_t = t;
@@ -571,15 +584,14 @@ void Executor::tune_linears() {
             // the projections into the residual: this route and the norm behind it, or shares of K that meet in the norm
             const bool residual = r.beta && !model_.is_moe();
             if (best >= 0 && M > 4 && residual && l0.kind == Quant::Int4b8 && pie_hip_gemm_groups_shares_us(M, l0.N, l0.K, l0.group, gemm_ws_bytes_) < 1e29f) {
-                const int guess = in_shares(l0, M, gemm_ws_bytes_) ? 1 : 0;
-                double us[2];
-                us[0] = time_us([&](LayerWeights& lw) {
-                    const bool done = linear_fused(lw.*(r.lin), r.act, nullptr, m.rms_eps, r.y, M, 1, 0, xn_, gemm_ws_, gemm_ws_bytes_, s);
-                    PIE_KERNEL(pie_hip_rmsnorm(x_, lw.ffn_norm, xn_, M, H, m.rms_eps, s));
-                    return done;
-                });
-                us[1] = time_us([&](LayerWeights& lw) { return project_in_shares(lw.*(r.lin), r.act, lw.ffn_norm, M); });
-                set(&Linear::shares, us[1] < 1e29 && clearly(us[1 - guess], us[guess]) ? 1 - guess : us[1] < 1e29 ? guess : 0, lo);
+                int form = in_shares(l0, M, gemm_ws_bytes_) ? 1 : 0;
+                if (close(pie_hip_gemm_groups_shares_us(M, l0.N, l0.K, l0.group, gemm_ws_bytes_), apart_cost(l0, M, gemm_ws_bytes_)) || best != by_model) {
+                    double us[2];
+                    us[0] = (best == by_model ? model_t : best_t) + time_us([&](LayerWeights& lw) { return pie_hip_rmsnorm(x_, lw.ffn_norm, xn_, M, H, m.rms_eps, s) == PIE_HIP_OK; });
+                    us[1] = time_us([&](LayerWeights& lw) { return project_in_shares(lw.*(r.lin), r.act, lw.ffn_norm, M); });
+                    if (clearly(us[1 - form], us[form])) form = 1 - form;
+                }
+                set(&Linear::shares, form, lo);
             }
             prev = M;
         }
