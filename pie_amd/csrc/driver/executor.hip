@@ -126,9 +126,12 @@ double apart_cost(const Linear& w, int M, size_t ws_bytes) {
 // Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
 // (pie_hip_shares_rmsnorm), for 5 rows and more: 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
 // without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
+double shares_cost(const Linear& w, int M, size_t ws_bytes) {   // (1e30: not taken, by the product's kernel or the norm's)
+    if (M < 5 || w.kind != Quant::Int4b8 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return 1e30;
+    return pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes);
+}
 bool in_shares(const Linear& w, int M, size_t ws_bytes) {
-    if (M < 5 || w.kind != Quant::Int4b8 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return false;
-    const double us = pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes);
+    const double us = shares_cost(w, M, ws_bytes);
     if (us > 1e29) return false;
     if (M <= 128 && w.shares[M] >= 0) return w.shares[M] == 1;   // (measured at start-up)
     return us < apart_cost(w, M, ws_bytes);
@@ -583,9 +586,10 @@ void Executor::tune_linears() {
             if (best >= 0) set(&Linear::tuned, best, lo);
             // the projections into the residual: this route and the norm behind it, or shares of K that meet in the norm
             const bool residual = r.beta && !model_.is_moe();
-            if (best >= 0 && M > 4 && residual && l0.kind == Quant::Int4b8 && pie_hip_gemm_groups_shares_us(M, l0.N, l0.K, l0.group, gemm_ws_bytes_) < 1e29f) {
+            const double shares = residual ? shares_cost(l0, M, gemm_ws_bytes_) : 1e30;
+            if (best >= 0 && shares < 1e29) {
                 int form = in_shares(l0, M, gemm_ws_bytes_) ? 1 : 0;
-                if (close(pie_hip_gemm_groups_shares_us(M, l0.N, l0.K, l0.group, gemm_ws_bytes_), apart_cost(l0, M, gemm_ws_bytes_)) || best != by_model) {
+                if (close(shares, apart_cost(l0, M, gemm_ws_bytes_)) || best != by_model) {
                     double us[2];
                     us[0] = (best == by_model ? model_t : best_t) + time_us([&](LayerWeights& lw) { return pie_hip_rmsnorm(x_, lw.ffn_norm, xn_, M, H, m.rms_eps, s) == PIE_HIP_OK; });
                     us[1] = time_us([&](LayerWeights& lw) { return project_in_shares(lw.*(r.lin), r.act, lw.ffn_norm, M); });

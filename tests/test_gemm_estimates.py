@@ -128,6 +128,7 @@ def test_a_measurement_decides_the_forms_of_up_to_128_int4_rows():
             assert got == [False, True], (M, N, K, form)
             assert not drv.linear_forms("int4b8", M, N, K, 64, **{f"measured_{form}": 1})[form]   # (groups of half a step)
     assert not drv.linear_forms("int4b8", 40, 4096, 14336, 128, workspace_bytes=0, measured_shares=1)["shares"]
+    assert not drv.linear_forms("int4b8", 40, 16400, 16384, 128, measured_shares=1)["shares"]   # (a row the norm's kernel does not hold)
     for v in (0, 1):   # (more rows are not measured)
         assert drv.linear_forms("int4b8", 129, 4096, 14336, 128, measured_groups=v, measured_shares=v) == drv.linear_forms("int4b8", 129, 4096, 14336, 128)
 
