@@ -129,15 +129,24 @@ __device__ __forceinline__ float wave_max(float v) {
 // splits are merged by attn_decode_merge_kernel or by the output projection's prologue).
 constexpr int kAttnUnitTokens = 16;
 
+// a / b for a >= 0, b > 0.  (a + 1/2) / b is at least 1 / (2 b) away from a whole number, and the reciprocal and the product are off by less than 2^-22 of it: the
+// whole part is right for a below 2^20 (16 million keys), larger ones divide.
+__host__ __device__ __forceinline__ int div_small(int a, int b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if (a < (1 << 20)) return static_cast<int>((static_cast<float>(a) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(b)));
+#endif
+    return a / b;
+}
 // Units of each split of a row of `nunits` units: the row in one split per `least` units begun, at most `nsplit`, all but the last of
 // them equally long (a whole number of 32-key steps).  Up to `nsplit` of them hold `least` units at most and more than half as many (9 units by 8 are 6 and 3, not 8 and
 // 1).  The plan is made for the longest row, in a captured graph for the longest of its
 // bucket: with its split length for every row 16 rows of 1024 - 2048 keys left a third of the resident blocks idle (24.5 us a layer of 8 kv
 // heads, so 22.9; 23 rows of 720 - 1200 keys 22.7, so 21.3).
+// (every block of both launches starts with this, so the divisions count: a decode launch of 40 rows of 20 keys and its merge 16.0 us with the compiler's, so 15.7)
 __host__ __device__ __forceinline__ int split_units(int nunits, int least, int nsplit) {
     if (nsplit <= 1) return nunits > 1 ? nunits : 1;
-    const int begun = (nunits + least - 1) / least, n = begun < 1 ? 1 : begun < nsplit ? begun : nsplit;
-    const int units = ((nunits + n - 1) / n + 1) & ~1;
+    const int begun = div_small(nunits + least - 1, least), n = begun < 1 ? 1 : begun < nsplit ? begun : nsplit;
+    const int units = (div_small(nunits + n - 1, n) + 1) & ~1;
     return units > 1 ? units : 1;
 }
 
