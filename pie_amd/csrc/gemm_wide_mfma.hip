@@ -801,8 +801,8 @@ double columns_us(int format, int M, int N, int K, int group_size, size_t ws_byt
 // Blocks that share a CU with c - 1 others take `fixed` and `step` of the c-th column (four: more in proportion), where only some CUs have the c-th up to an
 // eighth less.  A block alone waits for its weights from HBM at every step, three of which are in flight: 0.33 - 0.54 us a step whatever the
 // rows, which is why a long K of few blocks pays for shares.  Shares' sums meet in a second kernel, 3 us and their bytes at 3.6 TB/s.  Measured over 50
-// matrices of 1024 - 28672 x 1024 - 14336 and 129 - 2048 rows, each call's weights out of HBM: 3 % rms, the faster of both kernels missed by 1 % on
-// average and by at most 7.
+// matrices of 1024 - 28672 x 1024 - 14336 and 129 - 2048 rows, each call's weights out of HBM: 6 % rms, the faster of both kernels missed by 1 % on
+// average.
 struct RowsPlan {
     int row_tiles = 0, shares = 1;
     double us = 1e30;
@@ -810,7 +810,7 @@ struct RowsPlan {
 struct Round {
     double fixed, step;
 };
-constexpr Round kRowRounds[2][4][4] = {{{{3.8, 0.325}, {4.6, 0.364}, {5.1, 0.547}, {5.6, 0.705}},
+constexpr Round kRowRounds[2][4][4] = {{{{3.8, 0.325}, {4.6, 0.364}, {5.0, 0.490}, {5.3, 0.660}},
                                      {{4.4, 0.463}, {5.9, 0.529}, {7.9, 0.735}, {8.6, 0.959}},
                                      {{5.6, 0.481}, {8.4, 0.647}, {10.0, 0.952}, {12.2, 1.275}},
                                      {{7.1, 0.538}, {9.8, 0.830}, {11.4, 1.220}, {14.5, 1.611}}},
@@ -818,12 +818,16 @@ constexpr Round kRowRounds[2][4][4] = {{{{3.8, 0.325}, {4.6, 0.364}, {5.1, 0.547
                                      {{4.6, 0.468}, {6.3, 0.571}, {7.8, 0.813}, {8.7, 1.050}},
                                      {{5.7, 0.512}, {8.0, 0.716}, {10.0, 1.026}, {11.7, 1.398}},
                                      {{7.1, 0.586}, {9.8, 0.889}, {11.6, 1.295}, {14.1, 1.731}}}};
-// Microseconds of `n` blocks of 16 `row_tiles` rows, `per` steps each.
-double row_blocks_us(int format, int row_tiles, long long n, int per) {
+// Microseconds of `n` blocks of 16 `row_tiles` rows, `per` steps each, over a matrix of `mb` million weights.
+double row_blocks_us(int format, int row_tiles, long long n, int per, double mb) {
     const int c = static_cast<int>(std::min(4ll, (n + 255) / 256));
     const Round& r = kRowRounds[format == PIE_HIP_FMT_INT8][row_tiles / 2 - 1][c - 1];
     const double us = r.fixed + r.step * per;
-    return n > 1024 ? us * static_cast<double>(n) / 1024.0 : us * (1.0 - (c == 1 ? 0.04 : 0.13) * (c - n / 256.0));
+    // (32 rows of fp8 from three to a CU on: as fast as their steps, up to a fifth less where only some CUs have the third, and the matrix besides,
+    // which each chiplet reads for few rows: 1237 x 2048 x 4096 34.5 us, priced at 33.2 and at 37.2 without, where 96 rows took 38.1.)
+    const bool thin = row_tiles == 2 && c >= 3 && format == PIE_HIP_FMT_FP8;
+    const double less = c == 1 ? 0.04 : thin && c == 3 ? 0.19 : 0.13;
+    return (n > 1024 ? us * static_cast<double>(n) / 1024.0 : us * (1.0 - less * (c - n / 256.0))) + (thin ? 0.09 * mb : 0.0);
 }
 RowsPlan rows_plan(int format, int M, int N, int K, size_t ws_bytes) {
     const int steps = K / kStepK;
@@ -835,7 +839,7 @@ RowsPlan rows_plan(int format, int M, int N, int K, size_t ws_bytes) {
             const size_t bytes = static_cast<size_t>(s) * M * N * sizeof(float);
             if (s > 1 && (per < 4 || bytes > ws_bytes || tiles * (s - 1) >= 768)) break;
             if ((s - 1) * per >= steps) continue;   // (the last share would be empty)
-            double us = row_blocks_us(format, half * 2, tiles * s, per);
+            double us = row_blocks_us(format, half * 2, tiles * s, per, 1e-6 * N * K);
             if (s > 1) us += 3.0 + static_cast<double>(bytes) / 3.6e6;
             if (us < best.us) best = {half * 2, s, us};
         }
@@ -855,7 +859,7 @@ double few_routes_us(int format, int routes, int experts, int N, int K, bool swi
     const double each = static_cast<double>(routes) / experts, touched = experts * (1.0 - std::exp(-each)), mb = 1e-6 * N * K;
     if (blocks) {
         const long long per_chiplet = static_cast<long long>(std::ceil(touched / 8.0 - 1e-9));
-        return std::max({row_blocks_us(format, 2, per_chiplet * 8 * ((N + 127) / 128), K / kStepK), 4.0 + touched * mb / 6.05, 4.0 + per_chiplet * mb / 0.9});
+        return std::max({row_blocks_us(format, 2, per_chiplet * 8 * ((N + 127) / 128), K / kStepK, 0.0), 4.0 + touched * mb / 6.05, 4.0 + per_chiplet * mb / 0.9});
     }
     // (gathered rows and the gate's epilogue: 2.5 us from a second chunk of K on)
     const double gate = swiglu ? std::min(1.0, std::max(0.0, K / 1000.0 - 1.0)) : 0.0;

@@ -109,8 +109,8 @@ def test_blocks_that_scale_groups_in_fp32(gpu, M, N, K, rows, shares):
 ROWS = {"int8": [(33, 16, 320, 32, 1), (33, 1056, 320, 32, 1), (300, 8208, 320, 64, 1), (300, 8224, 320, 64, 1), (1300, 2064, 320, 96, 1), (1300, 2080, 320, 96, 1),
                  (1100, 6160, 1088, 128, 1), (1100, 6176, 1088, 128, 1), (33, 16, 1088, 32, 5), (1100, 528, 3136, 64, 5), (1300, 272, 4160, 96, 6),
                  (200, 6160, 6208, 128, 5)],
-        "fp8": [(33, 16, 320, 32, 1), (33, 1056, 320, 32, 1), (1100, 3088, 320, 64, 1), (1100, 3104, 320, 64, 1), (900, 3088, 1088, 96, 1), (900, 3104, 1088, 96, 1),
-                (1100, 6160, 1088, 128, 1), (1100, 6176, 1088, 128, 1), (33, 16, 1088, 32, 5), (1300, 528, 4160, 64, 4), (1300, 1040, 6208, 96, 4),
+        "fp8": [(33, 16, 320, 32, 1), (33, 1056, 320, 32, 1), (900, 4112, 448, 64, 1), (900, 4128, 448, 64, 1), (1300, 4112, 1088, 96, 1), (1300, 4128, 1088, 96, 1),
+                (1100, 6160, 1088, 128, 1), (1100, 6176, 1088, 128, 1), (33, 16, 1088, 32, 5), (900, 1040, 4160, 64, 3), (1300, 1040, 6208, 96, 4),
                 (200, 6160, 8256, 128, 5)]}
 
 
