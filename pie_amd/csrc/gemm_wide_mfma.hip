@@ -824,7 +824,7 @@ double row_blocks_us(int format, int row_tiles, long long n, int per, double mb)
     const Round& r = kRowRounds[format == PIE_HIP_FMT_INT8][row_tiles / 2 - 1][c - 1];
     const double us = r.fixed + r.step * per;
     // (32 rows of fp8 from three to a CU on: as fast as their steps, up to a fifth less where only some CUs have the third, and the matrix besides,
-    // which each chiplet reads for few rows: 1237 x 2048 x 4096 34.5 us, priced at 33.2 and at 37.2 without, where 96 rows took 38.1.)
+    // which each chiplet reads for few rows: 1237 x 2048 x 4096 34.5 us, priced at 33.2 and at 37.2 without, where 64 rows took 38.1.)
     const bool thin = row_tiles == 2 && c >= 3 && format == PIE_HIP_FMT_FP8;
     const double less = c == 1 ? 0.04 : thin && c == 3 ? 0.19 : 0.13;
     return (n > 1024 ? us * static_cast<double>(n) / 1024.0 : us * (1.0 - less * (c - n / 256.0))) + (thin ? 0.09 * mb : 0.0);
