@@ -810,7 +810,7 @@ struct RowsPlan {
 struct Round {
     double fixed, step;
 };
-constexpr Round kRowRounds[2][4][4] = {{{{3.8, 0.325}, {4.6, 0.364}, {5.0, 0.490}, {5.3, 0.660}},
+constexpr Round kRowRounds[2][4][4] = {{{{3.8, 0.325}, {4.6, 0.364}, {5.0, 0.490}, {5.6, 0.705}},
                                      {{4.4, 0.463}, {5.9, 0.529}, {7.9, 0.735}, {8.6, 0.959}},
                                      {{5.6, 0.481}, {8.4, 0.647}, {10.0, 0.952}, {12.2, 1.275}},
                                      {{7.1, 0.538}, {9.8, 0.830}, {11.4, 1.220}, {14.5, 1.611}}},
@@ -823,10 +823,10 @@ double row_blocks_us(int format, int row_tiles, long long n, int per, double mb)
     const int c = static_cast<int>(std::min(4ll, (n + 255) / 256));
     const Round& r = kRowRounds[format == PIE_HIP_FMT_INT8][row_tiles / 2 - 1][c - 1];
     const double us = r.fixed + r.step * per;
-    // (32 rows of fp8 from three to a CU on: as fast as their steps, up to a fifth less where only some CUs have the third, and the matrix besides,
-    // which each chiplet reads for few rows: 1237 x 2048 x 4096 34.5 us, priced at 33.2 and at 37.2 without, where 64 rows took 38.1.)
-    const bool thin = row_tiles == 2 && c >= 3 && format == PIE_HIP_FMT_FP8;
-    const double less = c == 1 ? 0.04 : thin && c == 3 ? 0.19 : 0.13;
+    // (32 rows of fp8, three to a CU: a fifth less where only some CUs have the third, and a part that goes with the matrix, which each chiplet reads
+    // for few rows.  1237 x 2048 x 4096 takes 34.5 us: priced at 33.2, at 37.2 by the others' rule, where 64 rows take 38.1.)
+    const bool thin = row_tiles == 2 && c == 3 && format == PIE_HIP_FMT_FP8;
+    const double less = c == 1 ? 0.04 : thin ? 0.19 : 0.13;
     return (n > 1024 ? us * static_cast<double>(n) / 1024.0 : us * (1.0 - less * (c - n / 256.0))) + (thin ? 0.09 * mb : 0.0);
 }
 RowsPlan rows_plan(int format, int M, int N, int K, size_t ws_bytes) {

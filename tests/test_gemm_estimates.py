@@ -40,6 +40,20 @@ def test_one_byte_prompts_take_a_way_within_an_eighth_of_the_fastest(shape):
         assert tall <= 1.125 * fastest
 
 
+# fp8 rows, N, K: microseconds in blocks of 32 rows and of the faster of 64 and 96, none in shares of K
+THIN = {(1250, 2048, 4096): (33.6, 36.3), (900, 3072, 2048): (18.6, 21.0), (900, 3072, 4096): (32.8, 37.5), (600, 4096, 4096): (31.5, 35.1),
+        (448, 5120, 2048): (17.5, 19.4), (448, 6144, 1024): (12.3, 13.5), (1400, 3072, 1024): (17.4, 16.2), (700, 6144, 1024): (18.3, 16.7)}
+
+
+@pytest.mark.parametrize("shape", THIN, ids=str)
+def test_fp8_prompts_take_blocks_of_32_rows_where_they_are_faster(shape):
+    from pie_amd import ops
+
+    thin, others = THIN[shape]
+    rows, shares = ops.gemm_rows_plan("fp8", *shape, WORKSPACE)
+    assert shares == 1 and (rows == 32) == (thin < others)
+
+
 # (format, experts, hidden, inner): microseconds of gate|up and down by routes, in passes of 16 and in blocks of 32
 FEW_ROUTES = {
     ("fp8", 8, 4096, 14336): {2: (76, 151), 4: (143, 192), 8: (162, 219), 32: (243, 248), 64: (245, 250)},
