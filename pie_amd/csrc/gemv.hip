@@ -13,7 +13,7 @@
 //   * the grid is sized to the machine, not to the problem: `waves_per_simd`
 //     resident waves on each of the 1024 SIMDs, every wave owning one contiguous,
 //     balanced slice of the output rows, so all CUs start and finish together;
-//   * a wave walks its slice R rows at a time; every lane streams 16-byte pieces of
+//   * a wave walks its slice R rows at a time (pick_rows); every lane streams 16-byte pieces of
 //     each row, so one wave instruction covers 1 KiB of a row, fully coalesced.
 //     Loads are branch-free and run a ring of two work units (R rows x one 1 KiB chunk)
 //     ahead of the arithmetic, so 2R independent 16 B loads per lane are in flight
@@ -953,6 +953,35 @@ int launch_m(int M, const GemvArgs& a, int wps, hipStream_t stream) {
     }
 }
 
+// A wave's rows at a time where the slice is shorter than four, else four.
+int slice_rows(int N, int waves_per_simd) {
+    const long long per_wave = N / (static_cast<long long>(kNumCU) * 4 * waves_per_simd);
+    return per_wave >= 4 ? 4 : (per_wave >= 3 ? 3 : (per_wave >= 2 ? 2 : 1));
+}
+
+// Rows of a step and waves of a SIMD, for `rows` activation rows in one pass.  Below 8192 weight rows a wave of two per SIMD has one
+// step to make and takes its slice at once.  From there two rows a step are better than four: what waits in front of the first step
+// and behind the last is half as long, and eight or more half as long steps are spread more evenly.  With int4, where the waves wait
+// for their own decoding, and with several activation rows, four waves a SIMD then hide it better than two.  Over 65536 rows (int4)
+// or 32768 the ends count for nothing, and four rows at a time share their reads of the activations.  Weights out of memory, us,
+// (4 rows, 2 waves) / (2, 2) / (2, 4):
+//   int4, 1 row: 8192 x 4096 6.9 / 6.1 / 6.7, 12288 x 4096 9.1 / 7.7 / 8.9, 16384 x 4096 10.1 / 10.0 / 9.8, 20480 x 4096 12.6 / 11.6 / 11.0,
+//     28672 x 4096 15.2 / 14.6 / 13.5, 28672 x 8192 27.2 / 26.5 / 23.9, 65536 x 2048 16.2 / 17.8 / 15.0, 128256 x 4096 47.4 / 55.4 / 49.3;
+//     2 rows 28672 x 4096 20.5 / 19.9 / 17.6, 4 rows 30.3 / 27.9 / 26.8
+//   int8, 1 row: 8192 x 4096 9.5 / 8.6 / 9.2, 16384 x 2048 8.7 / 8.5 / 8.3, 28672 x 4096 23.2 / 21.8 / 21.8, 16384 x 8192 25.9 / 24.2 / 27.3;
+//     2 rows 28672 x 4096 26.4 / 27.1 / 23.1, 4 rows 16384 x 2048 13.5 / 13.4 / 12.9, 2 rows 128256 x 2048 46.7 / 54.4 / 48.8 (fp8: the same)
+//   bf16, 1 row: 8192 x 6144 19.1 / 18.4 / 19.1, 16384 x 2048 14.2 / 13.0 / 14.1, 28672 x 4096 39.9 / 38.3 / 39.1, 32768 x 1024 13.0 / 14.5 / 12.5,
+//     16384 x 8192 47.3 / 49.5 / 59.5
+template <class F>
+void pick_rows(const GemvArgs& a, int rows, int* rows_per_wave, int* waves_per_simd) {
+    constexpr bool kInt4 = std::is_same<F, FmtInt4>::value, kBf16 = std::is_same<F, FmtBf16>::value;
+    *waves_per_simd = 2;
+    *rows_per_wave = slice_rows(a.N, 2);
+    if (a.N < 8192 || a.N > (kInt4 ? 65536 : 32768) || (kBf16 && a.N >= 16384 && (a.K > 4096 || a.N >= 32768))) return;
+    *rows_per_wave = 2;
+    if (!kBf16 && a.N >= 16384 && (kInt4 || rows >= 2)) *waves_per_simd = 4;
+}
+
 // rows_per_wave (R) in {1,2,3,4}; waves_per_simd in 1..8.  0 = pick.
 template <class F>
 int dispatch(GemvArgs a, int M, int rows_per_wave, int waves_per_simd, hipStream_t stream) {
@@ -960,18 +989,8 @@ int dispatch(GemvArgs a, int M, int rows_per_wave, int waves_per_simd, hipStream
     if (a.K % F::WPP != 0) return PIE_HIP_ERR_UNSUPPORTED;
     if (a.norm_w && a.K % 8 != 0) return PIE_HIP_ERR_UNSUPPORTED;
     if (a.swiglu && (a.N % 2 != 0 || a.beta)) return PIE_HIP_ERR_INVALID;
-    // Measured on MI355X: two resident waves per SIMD, each walking its slice four rows
-    // at a time (fewer when the slice is shorter), is within a few percent of the best
-    // (rows, waves) pair for every decode shape of an 8B-class model.
-    a.g_shift = (a.G > 0 && (a.G & (a.G - 1)) == 0) ? __builtin_ctz(static_cast<unsigned>(a.G)) : -1;
-    if (waves_per_simd <= 0) waves_per_simd = 2;
     if (waves_per_simd > 8) return PIE_HIP_ERR_INVALID;
-    if (rows_per_wave <= 0) {
-        const long long per_wave =
-            a.N / (static_cast<long long>(kNumCU) * 4 * waves_per_simd);
-        rows_per_wave = per_wave >= 4 ? 4 : (per_wave >= 3 ? 3 : (per_wave >= 2 ? 2 : 1));
-    }
-    if ((a.swiglu || a.rope_table) && rows_per_wave % 2 != 0) rows_per_wave = rows_per_wave == 3 ? 4 : 2;
+    a.g_shift = (a.G > 0 && (a.G & (a.G - 1)) == 0) ? __builtin_ctz(static_cast<unsigned>(a.G)) : -1;
     // Up to four activation rows share one pass over the weights (fewer when their staged
     // copies would not fit in 64 KiB of LDS); larger M re-reads the weights per group.
     constexpr int kChunkK = kWave * F::WPP;
@@ -979,6 +998,10 @@ int dispatch(GemvArgs a, int M, int rows_per_wave, int waves_per_simd, hipStream
     if (per_m > 64 * 1024) return PIE_HIP_ERR_UNSUPPORTED;
     int mcap = static_cast<int>(64 * 1024 / per_m);
     if (mcap > 4) mcap = 4;
+    if (rows_per_wave <= 0 && waves_per_simd <= 0) pick_rows<F>(a, M < mcap ? M : mcap, &rows_per_wave, &waves_per_simd);
+    if (waves_per_simd <= 0) waves_per_simd = 2;
+    if (rows_per_wave <= 0) rows_per_wave = slice_rows(a.N, waves_per_simd);
+    if ((a.swiglu || a.rope_table) && rows_per_wave % 2 != 0) rows_per_wave = rows_per_wave == 3 ? 4 : 2;
     if (a.mg_part_o && M > mcap) return PIE_HIP_ERR_UNSUPPORTED;   // (the merge prologue indexes rows from 0)
     const uint16_t* act = a.act;
     uint16_t* y = a.y;

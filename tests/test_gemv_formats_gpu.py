@@ -102,6 +102,54 @@ def test_bf16(gpu, oracle, M, N, K):
     check(oracle, bits(y), truth.astype(np.float64), ab, 2e-6)
 
 
+@pytest.mark.parametrize("kind", ["int4b8", "int8", "fp8", "bf16"])
+@pytest.mark.parametrize("M", [1, 2, 4])
+@pytest.mark.parametrize("N", [8190, 8194, 16382, 16390, 32770, 65538])
+def test_rows_and_waves_by_size(gpu, kind, M, N):
+    """Both sides of the sizes at which the rows of a step and the waves of a SIMD change, slices that do not
+    divide, plain and as gate|up pairs behind a norm, against float64 sums of the decoded weights.  An output
+    is off by its bf16 rounding (2^-8) and by float32 sums of K offset codes (up to 136, 128 against 8 codes or
+    127): 2^-24 K 17 of the products' magnitudes, well under 2e-4."""
+    import torch
+    from pie_amd import ops
+
+    K = 512
+    g = torch.Generator(device=gpu).manual_seed(N + M)
+    act = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+    if kind == "int4b8":
+        q = torch.randint(-2**31, 2**31 - 1, (N, K // 8), generator=g, device=gpu, dtype=torch.int64).to(torch.int32)
+        s = (torch.rand(N, K // 128, generator=g, device=gpu) * 0.01 + 0.002).bfloat16()
+        w = ops.int4b8_view(q, s, 128)
+        codes = torch.stack([(q >> (4 * i)) & 15 for i in range(8)], -1).reshape(N, K).double() - 8
+        full = (codes.view(N, -1, 128) * s.double()[:, :, None]).view(N, K)
+    elif kind == "bf16":
+        data = (torch.randn(N, K, generator=g, device=gpu) * 0.05).bfloat16()
+        w, full = ops.WeightView(kind, data, None, 0, N, K), data.double()
+    else:
+        s = torch.rand(N, generator=g, device=gpu) * 0.01 + 0.002
+        if kind == "int8":
+            data = torch.randint(-127, 128, (N, K), generator=g, device=gpu, dtype=torch.int64).to(torch.int8)
+            codes = data.double()
+        else:
+            e4m3 = torch.randn(N, K, generator=g, device=gpu).to(torch.float8_e4m3fn)
+            data, codes = e4m3.view(torch.uint8), e4m3.double()
+        w, full = ops.WeightView(kind, data, s, 0, N, K), codes * s.double()[:, None]
+    truth, mass = act.double() @ full.T, act.double().abs() @ full.abs().T
+    y = ops.linear_fused(act, w).double()
+    assert ((y - truth).abs() <= 2.0 ** -8 * truth.abs() + 2e-4 * mass + 1e-30).all()
+    # pairs: the same sums of normed rows, through the gate
+    nw = (torch.rand(K, generator=g, device=gpu) + 0.5).bfloat16()
+    h = (act.double() * torch.rsqrt(act.double().pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()).bfloat16().double()
+    truth, mass = h @ full.T, h.abs() @ full.abs().T
+    gate, up = truth[:, 0::2], truth[:, 1::2]
+    # (the normed row may round the other way: 2^-8 of each product; gate and up are rounded to bf16 on the way)
+    err = (2.0 ** -8 + 2e-4) * mass + 2.0 ** -8 * truth.abs()
+    got = ops.linear_fused(act, w, norm_weight=nw, swiglu=True).double()
+    want = torch.nn.functional.silu(gate) * up
+    bound = 1.1 * err[:, 0::2] * (up.abs() + err[:, 1::2]) + (gate.abs() + err[:, 0::2]) * err[:, 1::2] + 2.0 ** -7 * want.abs() + 1e-6
+    assert ((got - want).abs() <= bound).all()
+
+
 def test_bf16_lm_head_shape_and_greedy_token(gpu, oracle):
     """lm_head [128256, 2048] at batch 1: the argmax of the GPU logits is the oracle's token
     (ties/near-ties resolved against the fp64 logits)."""
