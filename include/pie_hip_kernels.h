@@ -421,6 +421,14 @@ int pie_hip_moe_route(const uint16_t* router_logits_bf16, int32_t* topk_idx, flo
 int pie_hip_moe_route_opt(const uint16_t* router_logits_bf16, int32_t* topk_idx, float* topk_weight,
                       int32_t* expert_offsets, int32_t* route_token, int32_t* route_pos,
                       int num_tokens, int num_experts, int top_k, int renormalize, void* stream);
+/* The same from the tokens' normalised rows: the router logits bf16(sum_k act[t, k] * router[e, k]) over the bf16 router matrix
+ * [E, hidden] (fp32 sums in this entry's own order), made in shares of K whose sums lie in `workspace` (16-byte aligned; as many shares
+ * as it holds, at least num_tokens * E * 4 bytes for E a multiple of four), then the choice on them.  router_logits may be NULL (not stored).
+ * hidden: a multiple of 256.  PIE_HIP_ERR_UNSUPPORTED: other shapes, alignments or too small a workspace; nothing has been launched. */
+int pie_hip_moe_router_route(const uint16_t* act_bf16, const uint16_t* router_bf16, uint16_t* router_logits_bf16,
+                             int32_t* topk_idx, float* topk_weight, int32_t* expert_offsets, int32_t* route_token,
+                             int32_t* route_pos, int num_tokens, int hidden, int num_experts, int top_k, int renormalize,
+                             void* workspace, size_t workspace_bytes, void* stream);
 /* The same from fp32 logits (rows of ld_logits), with the experts in num_groups equal groups of neighbours:
  * a token chooses among the experts of the keep_groups groups whose best expert has the largest probability
  * (ties to the lowest group); weight = p / (sum of the chosen p + 1e-20) * weight_scale.  top_k <= 64 and at most

@@ -709,22 +709,33 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     const int H = m.hidden, E = m.num_experts, K = m.top_k, Ie = m.expert_intermediate;
     const int fmt = fmt_code(w.wgu.kind);
     const int sbf = w.wgu.scale_bf16 ? 1 : 0;
-    // a decode batch: norm, router logits and top-k per token in one launch (every token's block
-    // reads the router matrix through the L2, which stops paying at a few hundred rows)
+    // a decode batch: norm, router logits and top-k per token in one launch, where the router is small: every token's block reads all of it through
+    // its CU's L2 port.  From kFusedRouteValues on, and for more tokens than kFusedRouteRows, the norm, the logits in shares of K and the choice run one
+    // by one.  us for 1 / 64 / 256 tokens, in one launch / one by one: 8 experts of 4096 9.3 / 9.8 / 10.6, 12.0 / 12.3 / 13.1; 64 of 4096 13.0 / 14.0 / 16.8,
+    // 13.8 / 13.9 / 15.7; 128 of 2048 14.5 / 15.5 / 18.4, 12.9 / 14.0 / 15.8; 256 of 2048 23.3 / 24.7 / 28.0, 15.5 / 16.3 / 18.9
     // (PIE_MOE_FUSED=0: the separate launches, for measurement)
     static const bool fused_on = [] { const char* e = getenv("PIE_MOE_FUSED"); return !e || atoi(e) != 0; }();
     if (!fused_on) next_norm = nullptr;
+    const bool by_token = fused_on && N <= kFusedRouteRows && w.router.kind == Quant::Bf16;
+    auto in_one = [&] {
+        return pie_hip_moe_norm_route(x_, w.ffn_norm, m.rms_eps, static_cast<const uint16_t*>(w.router.data), xn_, moe_logits_, moe_idx_, moe_w_,
+                                      moe_offsets_, moe_route_token_, moe_route_pos_, N, H, E, K, m.norm_topk ? 1 : 0, s);
+    };
     int routed = PIE_HIP_ERR_UNSUPPORTED;
-    if (fused_on && N <= kFusedRouteRows && w.router.kind == Quant::Bf16)
-        routed = pie_hip_moe_norm_route(x_, w.ffn_norm, m.rms_eps, static_cast<const uint16_t*>(w.router.data), xn_,
-                                        moe_logits_, moe_idx_, moe_w_, moe_offsets_, moe_route_token_,
-                                        moe_route_pos_, N, H, E, K, m.norm_topk ? 1 : 0, s);
-    if (routed == PIE_HIP_ERR_UNSUPPORTED) {
-    PIE_KERNEL(pie_hip_rmsnorm(x_, w.ffn_norm, xn_, N, H, m.rms_eps, s));
-    linear_fused(w.router, xn_, nullptr, m.rms_eps, moe_logits_, N, 0, 0, nullptr, gemm_ws_, gemm_ws_bytes_, s);
-    PIE_KERNEL(pie_hip_moe_route_opt(moe_logits_, moe_idx_, moe_w_, moe_offsets_, moe_route_token_,
-                                     moe_route_pos_, N, E, K, m.norm_topk ? 1 : 0, s));
+    if (by_token && (E * H < kFusedRouteValues || H % 256 != 0)) routed = in_one();
+    if (routed != PIE_HIP_ERR_UNSUPPORTED) {
+        PIE_KERNEL(routed);
     } else {
+        PIE_KERNEL(pie_hip_rmsnorm(x_, w.ffn_norm, xn_, N, H, m.rms_eps, s));
+        // (the shares' sums in the products' workspace; where it is too small a decode batch goes as above after all)
+        if (fused_on && w.router.kind == Quant::Bf16)
+            routed = pie_hip_moe_router_route(xn_, static_cast<const uint16_t*>(w.router.data), moe_logits_, moe_idx_, moe_w_, moe_offsets_,
+                                              moe_route_token_, moe_route_pos_, N, H, E, K, m.norm_topk ? 1 : 0, gemm_ws_, gemm_ws_bytes_, s);
+        if (routed == PIE_HIP_ERR_UNSUPPORTED && by_token) routed = in_one();
+        if (routed == PIE_HIP_ERR_UNSUPPORTED) {
+            linear_fused(w.router, xn_, nullptr, m.rms_eps, moe_logits_, N, 0, 0, nullptr, gemm_ws_, gemm_ws_bytes_, s);
+            routed = pie_hip_moe_route_opt(moe_logits_, moe_idx_, moe_w_, moe_offsets_, moe_route_token_, moe_route_pos_, N, E, K, m.norm_topk ? 1 : 0, s);
+        }
         PIE_KERNEL(routed);
     }
     const int hint = std::max(1, std::min(N, 2 * ((N * K + E - 1) / E)));

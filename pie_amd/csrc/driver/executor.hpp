@@ -160,7 +160,8 @@ class Executor {
     void collect_samplers(const BatchPlan& plan, SampleOutputs& out);
     void moe_block(const LayerWeights& w, int N, const uint16_t* next_norm, hipStream_t s);
     bool project_in_shares(const Linear& w, const uint16_t* act, const uint16_t* norm, int N);
-    static constexpr int kFusedRouteRows = 256;   // batches up to this size take pie_hip_moe_norm_route
+    // batches of up to so many rows and routers of fewer values take pie_hip_moe_norm_route
+    static constexpr int kFusedRouteRows = 256, kFusedRouteValues = 128 * 2048;
     static constexpr size_t kMergeProjMaxBytes = 64 * 1024;   // partial results a merging output projection reads per block
     bool xn_holds_next_norm_ = false;             // (while a forward is being enqueued) xn_ = the coming layer's normalised rows
     void alloc_kv();

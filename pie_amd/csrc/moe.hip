@@ -17,8 +17,9 @@
 //   pie_hip_moe_combine: out[t] (+)= sum_k w[t, k] * y_route[pos[t, k]] in top-k order, fp32,
 //   one rounding (token_batched_weighted_sum[_add]_bf16_kernel,
 //   driver/cuda/src/kernels/moe_dispatch.cu:152-196).
-#include "common.hip.h"
+#include "gemm_args.hip.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace pie_hip {
@@ -365,6 +366,110 @@ __global__ __launch_bounds__(kNormRouteThreads) void moe_norm_route_kernel(
         topk_idx[static_cast<size_t>(t) * K + tid] = sel_e[tid];
         topk_w[static_cast<size_t>(t) * K + tid] = renorm ? sel_w[tid] * inv_w : sel_w[tid];
     }
+}
+
+// ---- the router of a prompt: logits in shares of K, summed where the experts are chosen -----------------------------------------
+// Blocks of 32 tokens x up to 128 experts x 256 k-values, whose 80 KiB are all requested at once and multiplied when they are there (two blocks to a CU:
+// one waits while the other multiplies); a wave takes 32 experts.  The fp32 sums of up to eight shares go to memory, and the wave that chooses a token's
+// experts adds them in the order of K.
+// What bounds it: the time to the first byte; a launch's share of the bytes is small.  1237 tokens x 128 experts x 2048, us: the skinny GEMM, whose 624 blocks of
+// 16 x 16 walk all of K (128 KiB each), and the choice and the sort 31; here 20, 12 of them the choice and the sort.  64 tokens behind a norm of 2.6: 11.6, 4 tokens
+// 10.7 (one launch for norm, logits and choice and the sort 15.5 and 14.6: there every CU that has a token reads the whole router, here a quarter to a
+// sixteenth).  (Blocks of one wave and 32 experts, for few tokens: the same to 3 us more.)
+constexpr int kRouterRows = 32, kRouterStep = 256, kRouterExperts = 128, kRouterShares = 8;
+constexpr int kRouterBlocks = 512;   // two to a CU: no more shares than fill them once
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+struct RouterPlan {
+    int shares, per_share;   // per_share: steps of 256 k-values
+    size_t bytes;            // of the shares' sums
+};
+RouterPlan plan_router(int N, int H, int E, size_t ws_bytes) {
+    const int steps = H / kRouterStep, ld = (E + 3) / 4 * 4;
+    const long long tiles = (N + kRouterRows - 1ll) / kRouterRows * ((E + kRouterExperts - 1) / kRouterExperts);
+    const size_t plane = static_cast<size_t>(N) * ld * sizeof(float);
+    const long long most = std::min<long long>({kRouterShares, steps, std::max(1ll, kRouterBlocks / tiles), static_cast<long long>(ws_bytes / plane)});
+    if (most < 1) return {0, 0, 0};
+    const int per = static_cast<int>((steps + most - 1) / most), shares = (steps + per - 1) / per;
+    return {shares, per, shares * plane};
+}
+__global__ __launch_bounds__(256) void moe_router_shares_kernel(const uint16_t* __restrict__ act, const uint16_t* __restrict__ router,
+                                                                float* __restrict__ part, int N, int H, int E, int per_share) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    u32x4_t* lds = reinterpret_cast<u32x4_t*>(smem);   // 32 tokens' rows of 32 pieces, then the experts'
+    constexpr int kPieces = kRouterStep / 8;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int j = lane & 15, q = lane >> 4;
+    const int t0 = blockIdx.x * kRouterRows, e0 = blockIdx.y * kRouterExperts, share = blockIdx.z;
+    const int steps = H / kRouterStep, first = share * per_share, last = min(first + per_share, steps);
+    const int experts = min(E - e0, kRouterExperts), expert_rows = (experts + 31) / 32 * 32;
+    f32x4_t acc[2][2];   // [token tile][expert tile]
+#pragma unroll
+    for (int t = 0; t < 2; ++t) acc[t][0] = acc[t][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int r2 = lane >> 5;   // a wave's transfer moves two rows
+    for (int step = first; step < last; ++step) {
+        if (step > first) __syncthreads();   // (everybody has read the step before)
+        // piece p of row r lies at p ^ (r % 16): the sixteen rows an LDS read serves find different banks
+        for (int r = wv * 2; r < kRouterRows + expert_rows; r += 8) {
+            const int row = r + r2;
+            const uint16_t* from = row < kRouterRows ? act + static_cast<size_t>(min(t0 + row, N - 1)) * H
+                                                     : router + static_cast<size_t>(min(e0 + row - kRouterRows, E - 1)) * H;
+            to_lds(reinterpret_cast<const unsigned char*>(from + step * kRouterStep + ((lane & 31) ^ (row & 15)) * 8), lds + r * kPieces);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0070);
+        __syncthreads();
+        if (wv * 32 < experts) {
+#pragma unroll
+            for (int k = 0; k < kRouterStep / 32; ++k) {
+                const int at = (4 * k + q) ^ j;
+                bf16x8_t a[2], w[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[i] = __builtin_bit_cast(bf16x8_t, lds[(i * 16 + j) * kPieces + at]);
+                    w[i] = __builtin_bit_cast(bf16x8_t, lds[(kRouterRows + wv * 32 + i * 16 + j) * kPieces + at]);
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], a[t], acc[t][i], 0, 0, 0);
+            }
+        }
+    }
+    // (a lane has experts 4 q .. 4 q + 3 of token j of a tile; rows of whole groups of four)
+    const int ld = (E + 3) / 4 * 4;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int token = t0 + t * 16 + j;
+        if (token >= N) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int e = e0 + wv * 32 + i * 16 + 4 * q;
+            if (e < E) *reinterpret_cast<f32x4_t*>(part + (static_cast<size_t>(share) * N + token) * ld + e) = acc[t][i];
+        }
+    }
+}
+// moe_topk_kernel on the shares' sums; the logits are stored as a GEMM would have (`logits_out` may be null).
+__global__ __launch_bounds__(256) void moe_topk_shares_kernel(const float* __restrict__ part, int shares, uint16_t* __restrict__ logits_out,
+                                                              int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, int N, int E, int K,
+                                                              int renorm) {
+    const int t = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    if (t >= N) return;
+    const int ld = (E + 3) / 4 * 4;
+    const size_t plane = static_cast<size_t>(N) * ld;
+    const float* row = part + static_cast<size_t>(t) * ld;
+    auto logit = [&](int e) {
+        float p[kRouterShares];
+#pragma unroll
+        for (int z = 0; z < kRouterShares; ++z) p[z] = row[min(z, shares - 1) * plane + e];
+        float sum = p[0];
+#pragma unroll
+        for (int z = 1; z < kRouterShares; ++z) sum = z < shares ? sum + p[z] : sum;
+        const uint16_t b = f32_to_bf16_bits(sum);
+        if (logits_out) logits_out[static_cast<size_t>(t) * E + e] = b;
+        return bf16_bits_to_f32(b);
+    };
+    if (E <= 2 * kWave) topk_of_token<decltype(logit), NoGroups, 2>(logit, lane, t, topk_idx, topk_w, E, K, renorm);
+    else topk_of_token(logit, lane, t, topk_idx, topk_w, E, K, renorm);
 }
 
 // One block: rank of every route inside its expert, expert offsets, sorted positions.  The first `shared` routes of
@@ -729,6 +834,35 @@ extern "C" int pie_hip_moe_route_opt(const uint16_t* router_logits_bf16, int32_t
                        renormalize ? 1 : 0);
     hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kRouteThreads), 0, st, topk_idx, expert_offsets,
                        route_token, route_pos, num_tokens, num_experts, top_k, 0);
+    return launch_status();
+}
+
+extern "C" int pie_hip_moe_router_route(const uint16_t* act_bf16, const uint16_t* router_bf16, uint16_t* router_logits_bf16,
+                                        int32_t* topk_idx, float* topk_weight, int32_t* expert_offsets, int32_t* route_token,
+                                        int32_t* route_pos, int num_tokens, int hidden, int num_experts, int top_k, int renormalize,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace pie_hip;
+    if (!act_bf16 || !router_bf16 || !topk_idx || !topk_weight || !expert_offsets || !route_token || !route_pos || num_tokens <= 0 || hidden <= 0)
+        return PIE_HIP_ERR_INVALID;
+    if (num_experts <= 0 || num_experts > kMaxExperts || top_k <= 0 || top_k > kMaxTopK || top_k > num_experts || hidden % kRouterStep != 0 ||
+        (reinterpret_cast<uintptr_t>(act_bf16) | reinterpret_cast<uintptr_t>(router_bf16) | reinterpret_cast<uintptr_t>(workspace)) % 16)
+        return PIE_HIP_ERR_UNSUPPORTED;
+    const RouterPlan p = plan_router(num_tokens, hidden, num_experts, workspace ? workspace_bytes : 0);
+    if (p.shares == 0) return PIE_HIP_ERR_UNSUPPORTED;
+    constexpr int kMostBytes = (kRouterRows + kRouterExperts) * kRouterStep * 2;
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_router_shares_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kMostBytes);
+    if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int expert_rows = (std::min(num_experts, kRouterExperts) + 31) / 32 * 32;
+    const size_t smem = static_cast<size_t>(kRouterRows + expert_rows) * kRouterStep * 2;
+    hipLaunchKernelGGL(moe_router_shares_kernel,
+                       dim3((num_tokens + kRouterRows - 1) / kRouterRows, (num_experts + kRouterExperts - 1) / kRouterExperts, p.shares), dim3(256), smem, st,
+                       act_bf16, router_bf16, static_cast<float*>(workspace), num_tokens, hidden, num_experts, p.per_share);
+    hipLaunchKernelGGL(moe_topk_shares_kernel, dim3((num_tokens + 3) / 4), dim3(256), 0, st, static_cast<const float*>(workspace), p.shares,
+                       router_logits_bf16, topk_idx, topk_weight, num_tokens, num_experts, top_k, renormalize ? 1 : 0);
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kRouteThreads), 0, st, topk_idx, expert_offsets, route_token, route_pos, num_tokens,
+                       num_experts, top_k, 0);
     return launch_status();
 }
 

@@ -525,6 +525,28 @@ def moe_route(router_logits: torch.Tensor, top_k: int, renormalize: bool = True)
     return idx, w, offs, rtok, rpos
 
 
+def moe_router_route(act: torch.Tensor, router: torch.Tensor, top_k: int, renormalize: bool = True, workspace: Optional[torch.Tensor] = None):
+    """`moe_route` from the tokens' normalised rows [T, H] and the router matrix [E, H].  Returns (logits, then as `moe_route`)."""
+    _dev(act, torch.bfloat16, "act")
+    _dev(router, torch.bfloat16, "router")
+    T, H = act.shape
+    E = router.shape[0]
+    d = act.device
+    if router.shape[1] != H:
+        raise KernelError("router K != act K")
+    ws = workspace if workspace is not None else torch.empty(8 * T * ((E + 3) // 4 * 4), dtype=torch.float32, device=d)
+    logits = torch.empty((T, E), dtype=torch.bfloat16, device=d)
+    idx = torch.empty((T, top_k), dtype=torch.int32, device=d)
+    w = torch.empty((T, top_k), dtype=torch.float32, device=d)
+    offs = torch.empty(E + 1, dtype=torch.int32, device=d)
+    rtok = torch.empty(T * top_k, dtype=torch.int32, device=d)
+    rpos = torch.empty(T * top_k, dtype=torch.int32, device=d)
+    _check(kernels().pie_hip_moe_router_route(_ptr(act), _ptr(router), _ptr(logits), _ptr(idx), _ptr(w), _ptr(offs), _ptr(rtok), _ptr(rpos), T, H, E,
+                                              top_k, int(renormalize), _ptr(ws), C.c_size_t(ws.numel() * ws.element_size()), _stream()),
+           "pie_hip_moe_router_route")
+    return logits, idx, w, offs, rtok, rpos
+
+
 def moe_combine(y_routes: torch.Tensor, route_pos: torch.Tensor, topk_w: torch.Tensor,
                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[t] (+)= sum_k w[t,k] * y_routes[route_pos[t,k]]; `out` given = accumulate onto it."""

@@ -91,6 +91,37 @@ def test_norm_route_in_one_launch(gpu, oracle, T, H, E, K):
         assert np.array_equal(ref[0].cpu().numpy(), idx) and np.array_equal(ref[1].cpu().numpy(), w)
 
 
+@pytest.mark.parametrize("T,H,E,K,planes", [(1, 256, 1, 1, 8), (31, 512, 6, 2, 8), (33, 2048, 128, 8, 8), (64, 2304, 130, 8, 8), (257, 2048, 128, 8, 3),
+                                            (40, 7168, 384, 8, 8), (2080, 256, 512, 16, 1), (5, 1280, 64, 4, 1)])
+def test_router_in_shares_of_k(gpu, oracle, T, H, E, K, planes):
+    """pie_hip_moe_router_route over tiles of 32 tokens and 128 experts that are full, one over and one short, one to eight shares of K that
+    divide its steps or not, and a workspace of `planes` shares: the logits are the oracle's bf16 products up to the order of the fp32 sum (one
+    bf16 step where it rounds the other way), and the choice on the logits it stored is pie_hip_moe_route_opt's exactly."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(560 + T + E)
+    act = oracle.f32_to_bf16(rng.standard_normal((T, H)).astype(np.float32))
+    router = oracle.f32_to_bf16(rng.standard_normal((E, H)).astype(np.float32) * (1.0 / np.sqrt(H)))
+    ws = torch.full((planes * T * ((E + 3) // 4 * 4),), float("nan"), device=gpu)
+    want = oracle.gemm_bf16(act, router, mode=0)[1]
+    for renorm in (True, False):
+        lg, idx, w, offs, rtok, rpos = ops.moe_router_route(dev(act, gpu, torch.bfloat16), dev(router, gpu, torch.bfloat16), K, renorm, ws)
+        # (sums of a cancelling row differ by more of its own small steps: 2^-20 of the products' magnitude, as float32 sums of K <= 7168 do)
+        truth, _, ab = oracle.gemm_bf16(act, router, mode=2, want_abs=True)
+        off = np.abs(oracle.bf16_to_f32(bits(lg)).astype(np.float64) - truth)
+        assert (off <= 2.0 ** -8 * np.abs(truth) + 2.0 ** -20 * ab + 1e-30).all() and (bits(lg) == want).mean() > 0.97
+        ref = ops.moe_route(lg, K, renormalize=renorm)
+        assert torch.equal(ref[0], idx) and torch.equal(ref[1], w) and torch.equal(ref[2], offs)
+        idx, offs, rtok, rpos = (t.cpu().numpy() for t in (idx, offs, rtok, rpos))
+        flat = idx.reshape(-1)
+        assert np.array_equal(np.sort(rpos), np.arange(T * K)) and np.array_equal(rtok[rpos], np.arange(T * K) // K)
+        assert np.all(rpos >= offs[flat]) and np.all(rpos < offs[flat + 1])
+    for bad in ((act[:, :H - 8], router[:, :H - 8], ws), (act, router, ws[:T * E // 2])):
+        with pytest.raises(ops.KernelError):
+            ops.moe_router_route(dev(np.ascontiguousarray(bad[0]), gpu, torch.bfloat16), dev(np.ascontiguousarray(bad[1]), gpu, torch.bfloat16), K, True, bad[2])
+
+
 @pytest.mark.parametrize("T,K,H", [(64, 8, 2048), (3, 2, 512), (130, 6, 8192)])
 def test_combine_with_the_next_norm_equals_the_two_launches(gpu, oracle, T, K, H):
     import torch
