@@ -66,6 +66,47 @@ def test_tiles_match_oracle_and_row_kernel(gpu, oracle, hq, hk, d, ps, half):
     assert (ulp <= 1).mean() > 0.97
 
 
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("hq,hk,d,ps", [(8, 2, 128, 16), (4, 4, 64, 48), (8, 1, 64, 16), (32, 8, 128, 64)])
+def test_scores_that_outgrow_their_reference(gpu, oracle, hq, hk, d, ps, half):
+    """Keys that grow along the context, shrink along it, or jump at its end: what the exponents are relative to has to move at many
+    steps, at the first only, or at the last, past contexts of one to several pages and steps that end inside a page.  Against the oracle: a
+    bf16 rounding, and weights off by the float32 sums of d products behind them (2^-24 d of the products' magnitude, twice: a weight
+    and its sum)."""
+    import torch
+
+    from pie_amd import ops
+
+    rng = np.random.default_rng(90 + hq + d + ps)
+    ctx = [300, 97, 33, 161]
+    b = make_paged_batch(rng, ctx, hk, d, ps, f32_to_bf16=oracle.f32_to_bf16)
+    k = oracle.bf16_to_f32(b["k_pages"]).copy()
+    grow = [lambda x: 0.2 + 6.0 * x, lambda x: 6.2 - 6.0 * x, lambda x: np.where(x > 0.9, 8.0, 0.1), lambda x: 0.2 + 6.0 * x * x]
+    for r, n in enumerate(ctx):
+        for j in range(n):
+            page = b["page_indices"][int(b["page_indptr"][r]) + j // ps]
+            k[page, j % ps] *= grow[r](j / n)
+    kb = oracle.f32_to_bf16(k.astype(np.float32)).reshape(b["k_pages"].shape)
+    tr = ops.attn_prefill_tile_rows(hq, hk) // (2 if half else 1)
+    chunks = [(220, 80), (0, 97), (0, 33), (155, 6)]
+    row_begin, row_len, tile_start, tile_n = build_rows(b, ctx, chunks, tr)
+    rows = len(row_begin)
+    q = oracle.f32_to_bf16(3.0 * rng.standard_normal((rows, hq, d)).astype(np.float32))
+    dev = lambda a, dt=None: (lambda t: t.view(dt) if dt is not None else t)(
+        torch.from_numpy(np.ascontiguousarray(a)).to(gpu))
+    o = ops.attention_prefill_tiles(dev(q, torch.bfloat16), dev(kb, torch.bfloat16), dev(b["v_pages"], torch.bfloat16),
+                                    dev(b["page_indices"].view(np.int32)), dev(row_begin), dev(row_len), dev(tile_start), dev(tile_n),
+                                    rows_per_tile=tr)
+    got = oracle.bf16_to_f32(o.view(torch.uint16).cpu().numpy()).astype(np.float64)
+    truth, _, _ = oracle.attn_rows_masked(q, kb, b["v_pages"], b["page_indices"], row_begin, row_len, hq, hk, d, ps, [None] * rows)
+    qf, vf = np.abs(oracle.bf16_to_f32(q)), np.abs(oracle.bf16_to_f32(b["v_pages"]))
+    mass = (qf.reshape(rows, -1, d) * np.abs(k).max(axis=(0, 1)).max(axis=0)).sum(-1).max() / np.sqrt(d)
+    tol = 2.0 ** -8 * np.maximum(np.abs(truth), np.abs(got)) + 2 * d * 2.0 ** -24 * mass * vf.max()
+    err = np.abs(got - truth)
+    assert np.all(err <= tol), f"worst {np.max(err / tol):.2f}x"
+    assert np.sqrt((err ** 2).mean()) <= 2.0 ** -9 * np.sqrt((truth ** 2).mean())
+
+
 @pytest.mark.parametrize("fmt", ["fp8_e4m3", "int8_per_token_head", "fp8_per_token_head", "fp8_e5m2"])
 @pytest.mark.parametrize("hq,hk,d,ps", [(8, 2, 128, 16), (4, 4, 64, 16), (32, 8, 128, 32)])
 @pytest.mark.parametrize("half", [False, True])
