@@ -7,6 +7,7 @@
 #include "common.hip.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace pie_hip {
 namespace {
@@ -99,7 +100,11 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* __restrict__ x,
 }
 
 // A projection's shares of K meet the residual and the next norm: x += the shares' sums in order (bf16), y = the row normalised, as the
-// two launches.  One block per row, eight columns per thread and round.
+// two launches.  One block per row, eight columns per thread and round.  What bounds it: the way to the shares, which other chiplets have
+// just written.  All SHARES are asked for at once (0: any number, four at a time
+// and the rest one by one).  us behind their product, four at a time / at once: 16 rows of 4096 in seven shares 4.3 / 4.0, 5 in seven 4.9 / 3.9, 40 in eight 5.7 / 5.3,
+// 64 in four 4.8 / 4.5 (a launch that reads nothing 1.9).
+template <int SHARES>
 __global__ __launch_bounds__(1024) void shares_rmsnorm_kernel(const float* __restrict__ partial, int shares, size_t plane, uint16_t* __restrict__ x,
                                                               const uint16_t* __restrict__ w, uint16_t* __restrict__ y, int H, float eps) {
     __shared__ float red[16];
@@ -115,11 +120,30 @@ __global__ __launch_bounds__(1024) void shares_rmsnorm_kernel(const float* __res
         wcache[c] = *reinterpret_cast<const u32x4_t*>(w + v * 8);
         u32x4_t a = *reinterpret_cast<const u32x4_t*>(x + base + v * 8);
         const float* p = partial + base + v * 8;
-        f32x4_t s0 = *reinterpret_cast<const f32x4_t*>(p), s1 = *reinterpret_cast<const f32x4_t*>(p + 4);
+        f32x4_t s0, s1;
+        if constexpr (SHARES > 0) {
+            f32x4_t all[SHARES][2];
+#pragma unroll
+            for (int z = 0; z < SHARES; ++z) {
+                all[z][0] = *reinterpret_cast<const f32x4_t*>(p + z * plane);
+                all[z][1] = *reinterpret_cast<const f32x4_t*>(p + z * plane + 4);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // (all of them before the first sum)
+            s0 = all[0][0];
+            s1 = all[0][1];
+#pragma unroll
+            for (int z = 1; z < SHARES; ++z) {
+                s0 += all[z][0];
+                s1 += all[z][1];
+            }
+        } else {
+            s0 = *reinterpret_cast<const f32x4_t*>(p);
+            s1 = *reinterpret_cast<const f32x4_t*>(p + 4);
 #pragma unroll 4
-        for (int z = 1; z < shares; ++z) {
-            s0 += *reinterpret_cast<const f32x4_t*>(p + z * plane);
-            s1 += *reinterpret_cast<const f32x4_t*>(p + z * plane + 4);
+            for (int z = 1; z < shares; ++z) {
+                s0 += *reinterpret_cast<const f32x4_t*>(p + z * plane);
+                s1 += *reinterpret_cast<const f32x4_t*>(p + z * plane + 4);
+            }
         }
         a[0] = pack_bf16x2(s0[0] + bf16_lo(a[0]), s0[1] + bf16_hi(a[0]));
         a[1] = pack_bf16x2(s0[2] + bf16_lo(a[1]), s0[3] + bf16_hi(a[1]));
@@ -431,9 +455,21 @@ extern "C" int pie_hip_shares_rmsnorm(const float* partials, int shares, uint16_
     if (!partials || !x_bf16 || !weight_bf16 || !norm_out_bf16 || shares <= 0 || rows <= 0 || hidden <= 0) return PIE_HIP_ERR_INVALID;
     if (hidden % 8 != 0 || hidden > 2 * 8 * 1024) return PIE_HIP_ERR_UNSUPPORTED;
     const int nvec = hidden / 8, threads = std::min(1024, (nvec + kWave - 1) / kWave * kWave);
-    hipLaunchKernelGGL(shares_rmsnorm_kernel, dim3(rows), dim3(threads), 0, static_cast<hipStream_t>(stream), partials, shares,
-                       static_cast<size_t>(rows) * hidden, x_bf16, weight_bf16, norm_out_bf16, hidden, eps);
-    return launch_status();
+    auto launch = [&](auto count) {
+        hipLaunchKernelGGL(shares_rmsnorm_kernel<decltype(count)::value>, dim3(rows), dim3(threads), 0, static_cast<hipStream_t>(stream), partials, shares,
+                           static_cast<size_t>(rows) * hidden, x_bf16, weight_bf16, norm_out_bf16, hidden, eps);
+        return launch_status();
+    };
+    switch (shares) {
+        case 2: return launch(std::integral_constant<int, 2>{});
+        case 3: return launch(std::integral_constant<int, 3>{});
+        case 4: return launch(std::integral_constant<int, 4>{});
+        case 5: return launch(std::integral_constant<int, 5>{});
+        case 6: return launch(std::integral_constant<int, 6>{});
+        case 7: return launch(std::integral_constant<int, 7>{});
+        case 8: return launch(std::integral_constant<int, 8>{});
+        default: return launch(std::integral_constant<int, 0>{});
+    }
 }
 
 extern "C" int pie_hip_residual_rmsnorm(uint16_t* hidden_bf16, const uint16_t* residual_bf16,
