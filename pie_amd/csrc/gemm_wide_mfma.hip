@@ -652,7 +652,9 @@ int launch(const GemmArgs& a, int first_col, int col_blocks, int splits, hipStre
 // a few blocks; `fixed_full` and `step_full` more when all 256 CUs have one (shared caches, stores, power), most of it only
 // when nearly all have.  Fitted to 160 - 4096 rows of 4096 x 14336, 28672 x 4096, 16384 x 2048 and 4096 x 4096 (within 7 %), before the blocks stored 16
 // bytes a lane.  Over 50 matrices of 129 - 2048 rows with these stores and each call's weights out of HBM: int8 and fp8 within 6 % at the median from K of 2048 on and up
-// to a fifth low at 1024, int4 at most 11 % high.  (Int4 stays so: lower figures would take rows from the blocks that scale groups in fp32.)
+// to a fifth low at 1024, int4 at most 11 % high.  Bf16 with these stores and short K, us by 256 rows of 8 waves / blocks of 128 columns / of 256: 2011 x 8192 x 512 37.0 /
+// 29.9 / 25.7, x 256 29.8 / 22.2 / 20.0, x 1024 50.4 / 44.4 / 36.0, 500 x 16384 x 256 17.4 / 13.3 / 18.2, 2011 x 4096 x 1024 26.8 / 22.6 / 30.4, 1000 x 2048 x 1024 14.4 / 18.3 /
+// 26.9 (blocks of 128 rows): within 7 % where two of them are close.  (Int4 stays so: lower figures would take rows from the blocks that scale groups in fp32.)
 struct Rate {
     double fixed, step, fixed_full, step_full;
 };
@@ -665,7 +667,7 @@ constexpr Rates kRates[] = {
     /* int4 */ {{14.0, 1.36, 8.0, 0.26}, {6.0, 0.76, 1.0, 0.15}, 0.57, 0.20, 0.64, 1.14},
     /* int8 */ {{14.0, 1.31, 10.0, 0.22}, {7.0, 0.72, 2.0, 0.12}, 0.54, 0.20, 0.62, 1.10},
     /* fp8 */ {{14.0, 1.31, 10.0, 0.20}, {7.0, 0.71, 2.0, 0.12}, 0.47, 0.17, 0.58, 1.08},
-    /* bf16 */ {{14.0, 0.90, 10.0, 0.43}, {6.0, 0.62, 1.0, 0.19}, 0.36, 0.21, 0.57, 0.98},
+    /* bf16 */ {{9.0, 0.90, 2.8, 0.43}, {6.0, 0.62, 1.0, 0.19}, 0.36, 0.21, 0.57, 0.93},
 };
 double launch_us(const Rate& r, long long blocks, int steps) {
     const long long rounds = blocks / 256;
@@ -901,8 +903,14 @@ double gemm_tiles_us(int format, int M, int N, int K) {
     const long long cols = (N + 127) / 128, low = cols * ((M + 127) / 128), high = cols * ((M + 255) / 256);
     const long long low_rounds = (low + 255) / 256, high_rounds = (high + 255) / 256;
     const double steps = K / kStepK;
-    if (1.85 * static_cast<double>(high_rounds) < static_cast<double>(low_rounds)) return high_rounds * (5.0 + steps * r.tall);
-    return (format == PIE_HIP_FMT_BF16 ? 9.0 : 7.0) + steps * (low <= 256 ? r.few + r.many * static_cast<double>(low) / 256.0 : r.round * static_cast<double>(low_rounds));
+    // (bf16: a round of either height starts and stores for a while, which at a short K is most of it)
+    const bool tall = 1.85 * static_cast<double>(high_rounds) < static_cast<double>(low_rounds);
+    if (format == PIE_HIP_FMT_BF16) {
+        if (tall) return 3.0 + high_rounds * (9.8 + steps * r.tall);
+        return 3.5 + 5.5 * static_cast<double>(low_rounds) + steps * (low <= 256 ? r.few + r.many * static_cast<double>(low) / 256.0 : r.round * static_cast<double>(low_rounds));
+    }
+    if (tall) return high_rounds * (5.0 + steps * r.tall);
+    return 7.0 + steps * (low <= 256 ? r.few + r.many * static_cast<double>(low) / 256.0 : r.round * static_cast<double>(low_rounds));
 }
 
 int launch_gemm_wide(int format, const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream) {

@@ -40,6 +40,20 @@ def test_one_byte_prompts_take_a_way_within_an_eighth_of_the_fastest(shape):
         assert tall <= 1.125 * fastest
 
 
+# bf16 rows, N, K: microseconds in blocks of 128 columns and two heights (the faster is the entry's choice), and of 256 rows of 8 waves by 128 or 256 columns
+SHORT_K = {(500, 2048, 256): (8.9, 10.0), (300, 14336, 256): (15.8, 11.9), (2011, 8192, 256): (30.8, 20.4), (2011, 14336, 256): (55.0, 34.7), (3000, 4096, 256): (26.1, 19.2),
+           (2011, 8192, 512): (38.7, 25.6), (2011, 14336, 512): (70.4, 46.1), (1000, 4096, 512): (12.0, 14.2), (700, 8192, 768): (21.5, 18.1),
+           (1000, 2048, 1024): (14.4, 18.3), (2011, 4096, 1024): (26.8, 22.6), (3000, 16384, 1024): (147.8, 101.2), (2011, 2176, 1536): (29.7, 25.6),
+           (4000, 6144, 2048): (112.5, 95.1), (2011, 8192, 4096): (127.4, 100.2), (200, 4096, 4096): (37.4, 51.7), (2011, 2176, 4096): (58.1, 50.9)}
+
+
+@pytest.mark.parametrize("shape", SHORT_K, ids=str)
+def test_bf16_prompts_of_short_k_are_priced_at_the_faster_form(shape):
+    from pie_amd import ops
+
+    assert abs(ops.gemm_mfma_us("bf16", *shape, 0, False) / min(SHORT_K[shape]) - 1) < 0.2
+
+
 # fp8 rows, N, K: microseconds in blocks of 32 rows and of the faster of 64 and 96, none in shares of K
 THIN = {(1250, 2048, 4096): (33.6, 36.3), (900, 3072, 2048): (18.6, 21.0), (900, 3072, 4096): (32.8, 37.5), (600, 4096, 4096): (31.5, 35.1),
         (448, 5120, 2048): (17.5, 19.4), (448, 6144, 1024): (12.3, 13.5), (1400, 3072, 1024): (17.4, 16.2), (700, 6144, 1024): (18.3, 16.7)}
