@@ -711,8 +711,8 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
     const int sbf = w.wgu.scale_bf16 ? 1 : 0;
     // a decode batch: norm, router logits and top-k per token in one launch, where the router is small: every token's block reads all of it through
     // its CU's L2 port.  From kFusedRouteValues on, and for more tokens than kFusedRouteRows, the norm, the logits in shares of K and the choice run one
-    // by one.  us for 1 / 64 / 256 tokens, in one launch / one by one: 8 experts of 4096 9.3 / 9.8 / 10.6, 12.0 / 12.3 / 13.1; 64 of 4096 13.0 / 14.0 / 16.8,
-    // 13.8 / 13.9 / 15.7; 128 of 2048 14.5 / 15.5 / 18.4, 12.9 / 14.0 / 15.8; 256 of 2048 23.3 / 24.7 / 28.0, 15.5 / 16.3 / 18.9
+    // by one.  us for 1 / 64 / 256 tokens, in one launch / one by one: 8 experts of 4096 9.3 / 9.8 / 10.6, 10.4 / 12.5 / 13.0; 64 of 4096 13.0 / 14.0 / 16.8,
+    // 11.7 / 13.9 / 15.5; 128 of 2048 14.5 / 15.5 / 18.4, 11.3 / 14.0 / 15.8; 256 of 2048 23.3 / 24.7 / 28.0, 13.5 / 16.3 / 18.5
     // (PIE_MOE_FUSED=0: the separate launches, for measurement)
     static const bool fused_on = [] { const char* e = getenv("PIE_MOE_FUSED"); return !e || atoi(e) != 0; }();
     if (!fused_on) next_norm = nullptr;

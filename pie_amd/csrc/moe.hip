@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kNormRouteThreads) void moe_norm_route_kernel(
 // experts adds them in the order of K.
 // What bounds it: the time to the first byte; a launch's share of the bytes is small.  1237 tokens x 128 experts x 2048, us: the skinny GEMM, whose 624 blocks of
 // 16 x 16 walk all of K (128 KiB each), and the choice and the sort 31; here 20, 12 of them the choice and the sort.  64 tokens behind a norm of 2.6: 11.6, 4 tokens
-// 10.7 (one launch for norm, logits and choice and the sort 15.5 and 14.6: there every CU that has a token reads the whole router, here a quarter to a
+// 9.3 (one launch for norm, logits and choice and the sort 15.5 and 14.6: there every CU that has a token reads the whole router, here a quarter to a
 // sixteenth).  (Blocks of one wave and 32 experts, for few tokens: the same to 3 us more.)
 constexpr int kRouterRows = 32, kRouterStep = 256, kRouterExperts = 128, kRouterShares = 8;
 constexpr int kRouterBlocks = 512;   // two to a CU: no more shares than fill them once
@@ -448,12 +448,10 @@ __global__ __launch_bounds__(256) void moe_router_shares_kernel(const uint16_t* 
         }
     }
 }
-// moe_topk_kernel on the shares' sums; the logits are stored as a GEMM would have (`logits_out` may be null).
-__global__ __launch_bounds__(256) void moe_topk_shares_kernel(const float* __restrict__ part, int shares, uint16_t* __restrict__ logits_out,
-                                                              int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, int N, int E, int K,
-                                                              int renorm) {
-    const int t = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    if (t >= N) return;
+// The choice of token t by one wave, on the shares' sums; the logits are stored as a GEMM would have (`logits_out` may be null).
+__device__ __forceinline__ void choose_from_shares(const float* __restrict__ part, int shares, uint16_t* __restrict__ logits_out,
+                                                   int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, int N, int E, int K, int renorm,
+                                                   int t, int lane) {
     const int ld = (E + 3) / 4 * 4;
     const size_t plane = static_cast<size_t>(N) * ld;
     const float* row = part + static_cast<size_t>(t) * ld;
@@ -470,6 +468,12 @@ __global__ __launch_bounds__(256) void moe_topk_shares_kernel(const float* __res
     };
     if (E <= 2 * kWave) topk_of_token<decltype(logit), NoGroups, 2>(logit, lane, t, topk_idx, topk_w, E, K, renorm);
     else topk_of_token(logit, lane, t, topk_idx, topk_w, E, K, renorm);
+}
+__global__ __launch_bounds__(256) void moe_topk_shares_kernel(const float* __restrict__ part, int shares, uint16_t* __restrict__ logits_out,
+                                                              int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, int N, int E, int K,
+                                                              int renorm) {
+    const int t = blockIdx.x * 4 + threadIdx.x / kWave;
+    if (t < N) choose_from_shares(part, shares, logits_out, topk_idx, topk_w, N, E, K, renorm, t, threadIdx.x & (kWave - 1));
 }
 
 // One block: rank of every route inside its expert, expert offsets, sorted positions.  The first `shared` routes of
@@ -551,6 +555,18 @@ __global__ __launch_bounds__(kRouteThreads) void moe_sort_kernel(
     const int32_t* __restrict__ topk_idx, int32_t* __restrict__ expert_offsets,
     int32_t* __restrict__ route_token, int32_t* __restrict__ route_pos, int N, int E, int K, int shared) {
     sort_routes(topk_idx, expert_offsets, route_token, route_pos, N, E, K, shared);
+}
+// The choice and the sort in one launch, a wave per token.  us with the logits of 2048 values, in one launch / in two: 1 token of 128 experts 8.9 / 10.3, 16 10.9 / 11.5; 4
+// of 256 11.7 / 13.2, but 16 14.5 / 13.6: the sixteen waves share four SIMDs, and a choice is the longer the more experts there are.
+constexpr int kRouteInOneTokens = kRouteThreads / kWave, kRouteInOneLogits = 2048;
+__global__ __launch_bounds__(kRouteThreads) void moe_route_shares_kernel(const float* __restrict__ part, int shares, uint16_t* __restrict__ logits_out,
+                                                                         int32_t* topk_idx, float* __restrict__ topk_w, int32_t* __restrict__ expert_offsets,
+                                                                         int32_t* __restrict__ route_token, int32_t* __restrict__ route_pos, int N, int E,
+                                                                         int K, int renorm) {
+    const int t = threadIdx.x / kWave;
+    if (t < N) choose_from_shares(part, shares, logits_out, topk_idx, topk_w, N, E, K, renorm, t, threadIdx.x & (kWave - 1));
+    __syncthreads();   // (a block's stores are seen by its own threads after the barrier)
+    sort_routes(topk_idx, expert_offsets, route_token, route_pos, N, E, K);
 }
 
 // fp32 logits and groups of experts: one wave per token, four to a block.
@@ -859,6 +875,11 @@ extern "C" int pie_hip_moe_router_route(const uint16_t* act_bf16, const uint16_t
     hipLaunchKernelGGL(moe_router_shares_kernel,
                        dim3((num_tokens + kRouterRows - 1) / kRouterRows, (num_experts + kRouterExperts - 1) / kRouterExperts, p.shares), dim3(256), smem, st,
                        act_bf16, router_bf16, static_cast<float*>(workspace), num_tokens, hidden, num_experts, p.per_share);
+    if (num_tokens <= kRouteInOneTokens && num_tokens * num_experts <= kRouteInOneLogits) {
+        hipLaunchKernelGGL(moe_route_shares_kernel, dim3(1), dim3(kRouteThreads), 0, st, static_cast<const float*>(workspace), p.shares, router_logits_bf16,
+                           topk_idx, topk_weight, expert_offsets, route_token, route_pos, num_tokens, num_experts, top_k, renormalize ? 1 : 0);
+        return launch_status();
+    }
     hipLaunchKernelGGL(moe_topk_shares_kernel, dim3((num_tokens + 3) / 4), dim3(256), 0, st, static_cast<const float*>(workspace), p.shares,
                        router_logits_bf16, topk_idx, topk_weight, num_tokens, num_experts, top_k, renormalize ? 1 : 0);
     hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kRouteThreads), 0, st, topk_idx, expert_offsets, route_token, route_pos, num_tokens,

@@ -92,10 +92,11 @@ def test_norm_route_in_one_launch(gpu, oracle, T, H, E, K):
 
 
 @pytest.mark.parametrize("T,H,E,K,planes", [(1, 256, 1, 1, 8), (31, 512, 6, 2, 8), (33, 2048, 128, 8, 8), (64, 2304, 130, 8, 8), (257, 2048, 128, 8, 3),
-                                            (40, 7168, 384, 8, 8), (2080, 256, 512, 16, 1), (5, 1280, 64, 4, 1)])
+                                            (40, 7168, 384, 8, 8), (2080, 256, 512, 16, 1), (5, 1280, 64, 4, 1),
+                                            (16, 2048, 128, 8, 8), (17, 512, 64, 4, 2), (8, 512, 257, 8, 2), (7, 512, 257, 8, 2)])
 def test_router_in_shares_of_k(gpu, oracle, T, H, E, K, planes):
     """pie_hip_moe_router_route over tiles of 32 tokens and 128 experts that are full, one over and one short, one to eight shares of K that
-    divide its steps or not, and a workspace of `planes` shares: the logits are the oracle's bf16 products up to the order of the fp32 sum (one
+    divide its steps or not, a workspace of `planes` shares, and the choice and the sort in one launch and in two: the logits are the oracle's bf16 products up to the order of the fp32 sum (one
     bf16 step where it rounds the other way), and the choice on the logits it stored is pie_hip_moe_route_opt's exactly."""
     import torch
     from pie_amd import ops
