@@ -15,7 +15,7 @@
 //     balanced slice of the output rows, so all CUs start and finish together;
 //   * a wave walks its slice R rows at a time (pick_rows); every lane streams 16-byte pieces of
 //     each row, so one wave instruction covers 1 KiB of a row, fully coalesced.
-//     Loads are branch-free and run a ring of two work units (R rows x one 1 KiB chunk)
+//     Loads are branch-free and run a ring of two or four work units (R rows x one 1 KiB chunk)
 //     ahead of the arithmetic, so 2R independent 16 B loads per lane are in flight
 //     while the previous unit is being reduced;
 //   * the first units are requested before the activation row is staged, so the
@@ -47,7 +47,6 @@ namespace {
 constexpr int kBlock = 512;  // 8 waves: two per SIMD of a CU, so one block's prologue serves the whole CU
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kNumCU = 256;
-constexpr int kUnits = 2;   // work units in flight per wave
 
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
@@ -342,7 +341,8 @@ __device__ __forceinline__ u32x4_t merge_splits(const f32x4_t (&po)[NSP][2], con
 // it fetches and every instruction ahead of the first weight request delays it, so short rows
 // get a prologue with no idle trips.
 // MG: 0, or the most splits (4 or 8) of the attention-merge prologue (PJ = 1, no norm, no RoPE).
-template <class F, int R, int M, bool ROPE, bool GS1, int PJ, int MG = 0>
+// kUnits: work units in flight per wave.
+template <class F, int R, int M, bool ROPE, bool GS1, int PJ, int MG = 0, int kUnits = 2>
 __global__ __launch_bounds__(kBlock) void gemv_kernel(const GemvArgs a) {
     constexpr int WPP = F::WPP, XV = F::XV;
     constexpr int kChunkK = kWave * WPP;  // weights covered by one wave-wide 16 B load
@@ -431,8 +431,7 @@ __global__ __launch_bounds__(kBlock) void gemv_kernel(const GemvArgs a) {
     };
 
     // kUnits work units are requested before the activations are staged and stay in flight
-    // from then on.  (Measured: deeper rings than two lose on every decode shape of an 8B
-    // model, 1.84 / 1.94 / 2.03 ms per decode step for 2 / 3 / 4 units.)
+    // from then on.
     float best_v = -INFINITY;   // lm_head form: largest output of this lane so far, and its row
     int best_i = 0x7FFFFFFF;
     Unit<R> un[kUnits];
@@ -869,6 +868,13 @@ int gemv_grid(int N, bool pairs, int waves_per_simd) {
     return grid > max_grid ? max_grid : grid;
 }
 
+// From so many chunks of a row on a wave that takes one row at a time has four units in flight.  With two, a unit being 1 KiB, the chip has 4 MB in flight, where 6 TB/s
+// from HBM need ten.  Where a wave has few units the deeper ring costs more than it gives, as it does with two rows at a time (4096 x 4096 int4 4.8 us with two
+// units, 5.9 with four).  us with two / four, 1 row: int8 2048 x 8192 6.8 / 6.1, x 14336 9.8 / 8.5, 2560 x 6912 (7 chunks) 8.7 / 8.3, 2048 x 5120 (5) 5.2 / 5.5; fp8 2048 x
+// 8192 6.7 / 5.9; bf16 2048 x 8192 9.4 / 8.1, 3584 x 18944 33.2 / 26.1, 1536 x 4608 (9) 6.1 / 6.0; int4 2048 x 16384 (8) 8.2 / 7.9, x 14336 (7) 7.5 / 7.2 but 2 rows 8.2 / 8.3.
+template <class F>
+constexpr int kDeepChunks = F::kGroupScale ? 8 : 7;
+
 template <class F, int R, int M>
 int launch(const GemvArgs& a_in, int waves_per_simd, hipStream_t stream) {
     constexpr int kChunkK = kWave * F::WPP;
@@ -900,6 +906,12 @@ int launch(const GemvArgs& a_in, int waves_per_simd, hipStream_t stream) {
                     hipLaunchKernelGGL((gemv_kernel<F, R, M, false, kOne, 1, 4>), dim3(grid), dim3(kBlock), smem, stream, a);
                 else if constexpr (M == 1)
                     hipLaunchKernelGGL((gemv_kernel<F, R, M, false, kOne, 1, 8>), dim3(grid), dim3(kBlock), smem, stream, a);
+                return;
+            }
+        }
+        if constexpr (R == 1 && kPj != 1) {
+            if (nchunks >= kDeepChunks<F> && !t_start_event) {
+                hipLaunchKernelGGL((gemv_kernel<F, R, M, kRope, kOne, kPj, 0, 4>), dim3(grid), dim3(kBlock), smem, stream, a);
                 return;
             }
         }

@@ -102,6 +102,44 @@ def test_bf16(gpu, oracle, M, N, K):
     check(oracle, bits(y), truth.astype(np.float64), ab, 2e-6)
 
 
+@pytest.mark.parametrize("kind,K", [("int8", 6144), ("int8", 6144 + 16), ("int8", 8192), ("fp8", 14336), ("bf16", 4608), ("bf16", 4096 + 8), ("bf16", 18944),
+                                    ("int4b8", 14336), ("int4b8", 14336 + 128), ("int4b8", 18944)])
+@pytest.mark.parametrize("M", [1, 3])
+@pytest.mark.parametrize("N", [3, 515, 2048, 4095])
+def test_long_rows_one_at_a_time(gpu, oracle, kind, K, M, N):
+    """Rows of as many chunks as take the deeper ring and one fewer, chunks that end inside a wave, fewer rows than waves and two rows to some waves, with and
+    without a residual: against the oracle, to the bars of the tests of each format."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(80 + N + K)
+    act = oracle.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    yin = oracle.f32_to_bf16(rng.standard_normal((M, N)).astype(np.float32))
+    a = dev(act, gpu, torch.bfloat16)
+    s = rng.uniform(1e-4, 1e-3, N).astype(np.float32)
+    if kind == "int4b8":
+        q = torch.randint(-2**31, 2**31 - 1, (N, K // 8), dtype=torch.int64).to(torch.int32)
+        gs = (torch.rand(N, K // 128) * 0.01 + 0.002).bfloat16()
+        w = ops.int4b8_view(q.to(gpu), gs.to(gpu), 128)
+        codes = torch.stack([(q >> (4 * i)) & 15 for i in range(8)], -1).reshape(N, K).double() - 8
+        full, acc = (codes.view(N, -1, 128) * gs.double()[:, :, None]).view(N, K).numpy(), 1e-4
+    elif kind == "bf16":
+        wb = oracle.f32_to_bf16(rng.standard_normal((N, K)).astype(np.float32) * 0.02)
+        w, full, acc = ops.WeightView(kind, dev(wb, gpu, torch.bfloat16), None, 0, N, K), oracle.bf16_to_f32(wb).astype(np.float64), 2e-6
+    elif kind == "int8":
+        q = rng.integers(-127, 128, size=(N, K), dtype=np.int8)
+        w, full, acc = ops.WeightView(kind, dev(q, gpu), dev(s, gpu), 0, N, K), q.astype(np.float64) * s[:, None], 2e-5
+    else:
+        e = (torch.randn(N, K) * 0.5).to(torch.float8_e4m3fn)
+        w, full, acc = ops.WeightView(kind, e.view(torch.uint8).to(gpu), dev(s, gpu), 0, N, K), e.double().numpy() * s[:, None], 2e-6
+    x = oracle.bf16_to_f32(act).astype(np.float64)
+    truth, mass = x @ full.T, np.abs(x) @ np.abs(full).T
+    check(oracle, bits(ops.linear_fused(a, w)), truth, mass, acc)
+    y = dev(yin, gpu, torch.bfloat16)
+    before = oracle.bf16_to_f32(yin).astype(np.float64)
+    check(oracle, bits(ops.linear_fused(a, w, y=y, beta=1)), truth + before, mass + np.abs(before), acc)
+
+
 @pytest.mark.parametrize("kind", ["int4b8", "int8", "fp8", "bf16"])
 @pytest.mark.parametrize("M", [1, 2, 4])
 @pytest.mark.parametrize("N", [8190, 8194, 16382, 16390, 32770, 65538])
