@@ -56,10 +56,11 @@ struct TileLds {
 // bf16 pools: a step's rows as they are stored, moved without registers.  A transfer of a wave fills 1 KiB in the order of its lanes (4 rows of 128 values, 8 of 64),
 // so rows have no padding; a row's 16-byte pieces change places instead, K's by the row (the sixteen rows an operand read takes find
 // different banks), V's in pairs by the row (the eight rows of 32 bytes that half a wave's transposing read takes).
-template <int D, int S>
+constexpr int kRawStages = 2;
+template <int D>
 struct RawLds {
-    alignas(256) uint16_t k[S][kStepKeys * D];
-    alignas(256) uint16_t v[S][kStepKeys * D];
+    alignas(256) uint16_t k[kRawStages][kStepKeys * D];
+    alignas(256) uint16_t v[kRawStages][kStepKeys * D];
 };
 template <int D>
 __device__ __forceinline__ int raw_k(int key, int piece) { return piece ^ (key / (128 / D) & (D / 8 - 1)); }
@@ -86,11 +87,11 @@ __device__ __forceinline__ void read_transposed(uint32_t a0, uint32_t a1, uint32
 #pragma unroll
     for (int i = 0; i < 4; ++i) out[i] = __builtin_bit_cast(bf16x8_t, u32x4_t{r[2 * i].x, r[2 * i].y, r[2 * i + 1].x, r[2 * i + 1].y});
 }
-template <int D, bool Q8, int S>
-constexpr size_t kTileBytes = Q8 ? sizeof(TileLds<D, Q8>) : sizeof(RawLds<D, S>);
+template <int D, bool Q8>
+constexpr size_t kTileBytes = Q8 ? sizeof(TileLds<D, Q8>) : sizeof(RawLds<D>);
 // ... or a group's accumulators, maxima and sums at the end
-template <int D, bool Q8, int S>
-constexpr size_t kGroupBytes = kTileBytes<D, Q8, S> > (D / 16 + 1) * kTileThreads * 16 ? kTileBytes<D, Q8, S> : (D / 16 + 1) * kTileThreads * 16;
+template <int D, bool Q8>
+constexpr size_t kGroupBytes = kTileBytes<D, Q8> > (D / 16 + 1) * kTileThreads * 16 ? kTileBytes<D, Q8> : (D / 16 + 1) * kTileThreads * 16;
 
 // slot of key kappa (0..31) inside a V^T row
 __device__ __forceinline__ int vt_slot(int kappa) {
@@ -102,7 +103,6 @@ __device__ __forceinline__ int vt_slot(int kappa) {
 // KVF: one-byte pools (the codes become bf16 — exactly — on the way into the LDS tiles, one
 // 16-code piece per thread and matrix; the step's per-(token, kv head) scales sit in LDS and
 // multiply the scores (K) and the probabilities (V): float(code) * scale as in the row kernels).
-// S: steps of bf16 rows in LDS.
 // KP: groups of four waves that take a tile's steps in turn and meet at the end (in LDS, in fp32).  A block alone on its
 // CU is one wave per SIMD, which waits out every step's chain of products, exponentials and barrier: 1.25 us for 32 keys.
 // Up to 512 blocks of one 16-row tile per wave run in two groups: 358 rows behind 300 keys (32 heads over 8 of 128, 184
@@ -114,7 +114,7 @@ __device__ __forceinline__ int vt_slot(int kappa) {
 // 128: 489 rows 16.0 / 12.9, 1024 34.5 / 24.4, 2048 86 / 67, 4096 278 / 207 (in 128-row tiles 270 / 199), 8192 978 / 737, 128 behind 2000 46 / 34; three
 // prompts of 412 with 32 heads over 4 20.5 / 17.3; 2048 rows of 32 heads over 8 of 64 57 / 43.  (Page ids kept in the lanes, three stages, tiles dealt long and
 // short in turn: the same.)
-template <int D, int GQA, int QT, int KVF = kKvBf16, int KP = 1, int S = 2>
+template <int D, int GQA, int QT, int KVF = kKvBf16, int KP = 1>
 __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ k_pages_raw,
     const void* __restrict__ v_pages_raw, const float* __restrict__ k_scales,
@@ -151,9 +151,8 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
     const int l16 = lane & 15, g = lane >> 4;
     const int s0 = tile_start[tile], n_rows = tile_rows[tile];
     const uint32_t pg_lo = row_begin[s0];
-    L& lds = *reinterpret_cast<L*>(smem + part * kGroupBytes<D, Q8, S>);
-    using Raw = RawLds<D, S>;
-    Raw& raw = *reinterpret_cast<Raw*>(smem + part * kGroupBytes<D, Q8, S>);
+    L& lds = *reinterpret_cast<L*>(smem + part * kGroupBytes<D, Q8>);
+    RawLds<D>& raw = *reinterpret_cast<RawLds<D>*>(smem + part * kGroupBytes<D, Q8>);
 
     // (every wave finds the longest extent for itself: no barrier between the loads that lead to the first keys)
     int longest = row_len[s0 + min(lane, max(n_rows, 1) - 1)];
@@ -344,7 +343,7 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
         // bf16 pools: V^T out of the stored rows, four tiles at a time, the first beside the products above
         [[maybe_unused]] bf16x8_t vraw[4];
         auto v_read = [&](auto first_tag) {
-            constexpr int d0 = decltype(first_tag)::value, at = offsetof(Raw, v) + slot * sizeof(raw.v[0]);
+            constexpr int d0 = decltype(first_tag)::value, at = offsetof(RawLds<D>, v) + slot * sizeof(raw.v[0]);
             read_transposed<at, at + 16 * D * 2>(v_at[d0], v_at[d0 + 1], v_at[d0 + 2], v_at[d0 + 3], vraw);
         };
         if constexpr (!Q8) v_read(std::integral_constant<int, 0>{});
@@ -449,28 +448,18 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
             }
         }
     } else {
-        // one barrier a step: behind it everybody's transfers of the step have landed (those of later steps stay in flight) and the stage of the
-        // step before is free
-        static_assert(S == 2 || S == 4, "the waits below");
-#pragma unroll
-        for (int i = 0; i < S - 1; ++i)
-            if (first + i * advance < kmax) issue(i, first + i * advance);
-        auto turn = [&](auto slot_tag, int j0) __attribute__((always_inline)) {
+        // one barrier a step: behind it everybody's transfers of the step have landed and the stage of the step before is free
+        if (first < kmax) issue(0, first);
+        auto turn = [&](auto slot_tag, int j0) {
             constexpr int slot = decltype(slot_tag)::value;
-            if (S == 4 && first + j0 + 2 * advance < kmax) PIE_WAIT_VM(4 * MOVES);
-            else if (S == 4 && first + j0 + advance < kmax) PIE_WAIT_VM(2 * MOVES);
-            else PIE_WAIT_VM(0);
+            PIE_WAIT_VM(0);
             PIE_MEET();
-            if (first + j0 + (S - 1) * advance < kmax) issue((slot + S - 1) % S, first + j0 + (S - 1) * advance);
+            if (first + j0 + advance < kmax) issue(slot ^ 1, first + j0 + advance);
             if (KP == 1 || first + j0 < kmax) step(slot_tag, first + j0);
         };
-        for (int j0 = 0; j0 < kmax; j0 += S * advance) {
+        for (int j0 = 0; j0 < kmax; j0 += 2 * advance) {
             turn(std::integral_constant<int, 0>{}, j0);
             if (j0 + advance < kmax) turn(std::integral_constant<int, 1>{}, j0 + advance);
-            if constexpr (S == 4) {
-                if (j0 + 2 * advance < kmax) turn(std::integral_constant<int, 2>{}, j0 + 2 * advance);
-                if (j0 + 3 * advance < kmax) turn(std::integral_constant<int, 3>{}, j0 + 3 * advance);
-            }
         }
         __syncthreads();
     }
@@ -488,7 +477,7 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
         const float c = Q8 ? 1.f : scale_log2e;
 #pragma unroll
         for (int other = 1; other < KP && shared; ++other) {
-            const f32x4_t* its = reinterpret_cast<const f32x4_t*>(smem + other * kGroupBytes<D, Q8, S>);
+            const f32x4_t* its = reinterpret_cast<const f32x4_t*>(smem + other * kGroupBytes<D, Q8>);
             const f32x4_t st = its[DT * kTileThreads + tid];
             const float m_new = fmaxf(mx[0], st[0]), safe = m_new == -INFINITY ? 0.f : m_new;
             const float wa = __builtin_amdgcn_exp2f((mx[0] - safe) * c), wb = __builtin_amdgcn_exp2f((st[0] - safe) * c);
@@ -525,25 +514,22 @@ int launch_tiles(int kv_format, const uint16_t* q, const void* k_pages, const vo
                  const int32_t* tile_start, const int32_t* tile_rows, int num_tiles, int hq, int hk,
                  int ps, float scale, hipStream_t stream) {
     const float sl = scale * 1.4426950408889634f;
-    auto run = [&](auto format, auto groups, auto stages) {
-        constexpr int KVF = decltype(format)::value, KP = decltype(groups)::value, S = KVF == kKvBf16 ? decltype(stages)::value : 2;
-        constexpr size_t smem = KP * kGroupBytes<D, KVF != kKvBf16, S>;
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_tile_kernel<D, GQA, QT, KVF, KP, S>),
+    auto run = [&](auto format, auto groups) {
+        constexpr int KVF = decltype(format)::value, KP = decltype(groups)::value;
+        constexpr size_t smem = KP * kGroupBytes<D, KVF != kKvBf16>;
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_tile_kernel<D, GQA, QT, KVF, KP>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
         if (attr != hipSuccess) return PIE_HIP_ERR_LAUNCH;
-        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, KVF, KP, S>), dim3(num_tiles, hk), dim3(kTileThreads * KP), smem, stream, q,
+        hipLaunchKernelGGL((attn_prefill_tile_kernel<D, GQA, QT, KVF, KP>), dim3(num_tiles, hk), dim3(kTileThreads * KP), smem, stream, q,
                            k_pages, v_pages, k_scales, v_scales, o, page_indices, row_begin, row_len, tile_start, tile_rows, hq, hk, ps, sl);
         return launch_status();
     };
     auto grouped = [&](auto format) {
         if constexpr (QT == 1) {
             const long long blocks = static_cast<long long>(num_tiles) * hk;
-            // (a block alone on its CU has room for four steps: all of a short prompt's keys, just written by other chiplets, are asked for at once.  A
-            // prompt of 77 of a 1B model 1194 us with two steps, 1184 before they went straight into LDS, with four 1178; from caches 489 rows 13.0 and 13.4)
-            if (blocks <= 256) return run(format, std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
-            if (blocks <= 512) return run(format, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+            if (blocks <= 512) return run(format, std::integral_constant<int, 2>{});
         }
-        return run(format, std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
+        return run(format, std::integral_constant<int, 1>{});
     };
     if (kv_format == PIE_HIP_KV_BF16) return grouped(std::integral_constant<int, kKvBf16>{});
     if (kv_format == PIE_HIP_KV_INT8_PER_TOKEN_HEAD) return grouped(std::integral_constant<int, kKvInt8>{});
