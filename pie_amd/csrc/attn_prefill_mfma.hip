@@ -204,6 +204,7 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
     uint32_t k_off = (raw_key & 15) * row_bytes + raw_k<D>(raw_key, lane % LPR) * 16, v_off = (raw_key & 15) * row_bytes + raw_v<D>(raw_key, lane % LPR) * 16;
     const int ps_shift = (ps & (ps - 1)) == 0 ? __builtin_ctz(static_cast<unsigned>(ps)) : -1;
     const uint32_t page_bytes = static_cast<uint32_t>(ps) * row_bytes;
+    const bool aligned = (reinterpret_cast<uintptr_t>(k_bytes) | reinterpret_cast<uintptr_t>(v_bytes)) % 16 == 0;
     const unsigned char *k_head = k_bytes + kvh * (D * 2), *v_head = v_bytes + kvh * (D * 2);
     // a 32-key step touches at most two pages (page_size % 16 == 0): their ids come through
     // scalar loads, so the vector-memory queue holds K/V loads only, in step order
@@ -238,26 +239,35 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
         } else {
             u32x4_t* kl = reinterpret_cast<u32x4_t*>(raw.k[slot]) + wave * kWave;
             u32x4_t* vl = reinterpret_cast<u32x4_t*>(raw.v[slot]) + wave * kWave;
-            if (j0 + kStepKeys <= kmax) {
-                // a whole step: sixteen keys are in one page, and scalars find where; a lane adds its own offset
-                asm volatile("" : "+v"(k_off), "+v"(v_off));   // (32-bit offsets from scalar bases, not 64-bit sums)
+            auto move_all = [&](auto direct) __attribute__((always_inline)) {
+                auto move = [&](const unsigned char* from, u32x4_t* to) __attribute__((always_inline)) {
+                    if constexpr (decltype(direct)::value) to_lds(from, to);
+                    else to[lane] = *reinterpret_cast<const u32x4_t*>(from);
+                };
+                if (j0 + kStepKeys <= kmax) {
+                    // a whole step: sixteen keys are in one page, and scalars find where; a lane adds its own offset
+                    asm volatile("" : "+v"(k_off), "+v"(v_off));   // (32-bit offsets from scalar bases, not 64-bit sums)
 #pragma unroll
-                for (int u = 0; u < MOVES; ++u) {
-                    const int key = D == 128 ? 16 * u : wave * MKEYS / 16 * 16;   // 0 or 16
-                    const bool in_b = key && pa_end - j0 == 16;
-                    const size_t at = static_cast<uint64_t>(in_b ? pid_b : pid_a) * page_bytes + (in_b ? 0u : static_cast<uint32_t>(j0 + key - pa_end + ps) * row_bytes);
-                    to_lds(k_head + at + k_off, kl + u * kTileThreads);
-                    to_lds(v_head + at + v_off, vl + u * kTileThreads);
-                }
-            } else {
+                    for (int u = 0; u < MOVES; ++u) {
+                        const int key = D == 128 ? 16 * u : wave * MKEYS / 16 * 16;   // 0 or 16
+                        const bool in_b = key && pa_end - j0 == 16;
+                        const size_t at = static_cast<uint64_t>(in_b ? pid_b : pid_a) * page_bytes + (in_b ? 0u : static_cast<uint32_t>(j0 + key - pa_end + ps) * row_bytes);
+                        move(k_head + at + k_off, kl + u * kTileThreads);
+                        move(v_head + at + v_off, vl + u * kTileThreads);
+                    }
+                } else {
 #pragma unroll
-                for (int u = 0; u < MOVES; ++u) {
-                    const int key = u * (kTileWaves * MKEYS) + raw_key;
-                    const size_t at = token_head(key) * (D * 2);
-                    to_lds(k_bytes + at + raw_k<D>(key, lane % LPR) * 16, kl + u * kTileThreads);
-                    to_lds(v_bytes + at + raw_v<D>(key, lane % LPR) * 16, vl + u * kTileThreads);
+                    for (int u = 0; u < MOVES; ++u) {
+                        const int key = u * (kTileWaves * MKEYS) + raw_key;
+                        const size_t at = token_head(key) * (D * 2);
+                        move(k_bytes + at + raw_k<D>(key, lane % LPR) * 16, kl + u * kTileThreads);
+                        move(v_bytes + at + raw_v<D>(key, lane % LPR) * 16, vl + u * kTileThreads);
+                    }
                 }
-            }
+            };
+            // (pools off a 16-byte boundary pass through registers)
+            if (aligned) move_all(std::true_type{});
+            else move_all(std::false_type{});
         }
     };
     auto stage = [&](int slot) {   // one-byte pools: register slot = LDS buffer
@@ -452,7 +462,7 @@ __global__ __launch_bounds__(kTileThreads* KP, 2) void attn_prefill_tile_kernel(
         if (first < kmax) issue(0, first);
         auto turn = [&](auto slot_tag, int j0) {
             constexpr int slot = decltype(slot_tag)::value;
-            PIE_WAIT_VM(0);
+            __builtin_amdgcn_s_waitcnt(0x0070);   // (LDS writes too: pools off a 16-byte boundary)
             PIE_MEET();
             if (first + j0 + advance < kmax) issue(slot ^ 1, first + j0 + advance);
             if (KP == 1 || first + j0 < kmax) step(slot_tag, first + j0);

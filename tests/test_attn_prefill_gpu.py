@@ -107,6 +107,36 @@ def test_scores_that_outgrow_their_reference(gpu, oracle, hq, hk, d, ps, half):
     assert np.sqrt((err ** 2).mean()) <= 2.0 ** -9 * np.sqrt((truth ** 2).mean())
 
 
+@pytest.mark.parametrize("off_k,off_v", [(4, 0), (0, 4), (4, 4)])
+@pytest.mark.parametrize("hq,hk,d,ps", [(8, 2, 128, 16), (4, 4, 64, 48)])
+def test_pools_off_a_16_byte_boundary(gpu, oracle, hq, hk, d, ps, off_k, off_v):
+    """Pools that begin 8 bytes behind one (which transfers into LDS do not take) give the same bytes."""
+    import torch
+
+    from pie_amd import ops
+
+    rng = np.random.default_rng(95 + d)
+    ctx = [200, 75, 33, 1]
+    b = make_paged_batch(rng, ctx, hk, d, ps, f32_to_bf16=oracle.f32_to_bf16)
+    tr = ops.attn_prefill_tile_rows(hq, hk) // 2
+    row_begin, row_len, tile_start, tile_n = build_rows(b, ctx, [(120, 80), (0, 75), (0, 33), (0, 1)], tr)
+    q = oracle.f32_to_bf16(rng.standard_normal((len(row_begin), hq, d)).astype(np.float32))
+    dev = lambda a, dt=None: (lambda t: t.view(dt) if dt is not None else t)(
+        torch.from_numpy(np.ascontiguousarray(a)).to(gpu))
+
+    def shifted(t, off):
+        flat = torch.zeros(t.numel() + 8, dtype=t.dtype, device=t.device)
+        assert flat.data_ptr() % 16 == 0
+        flat[off:off + t.numel()] = t.reshape(-1)
+        return flat[off:off + t.numel()].view(t.shape)
+
+    qd, k, v = dev(q, torch.bfloat16), dev(b["k_pages"], torch.bfloat16), dev(b["v_pages"], torch.bfloat16)
+    rest = (dev(b["page_indices"].view(np.int32)), dev(row_begin), dev(row_len), dev(tile_start), dev(tile_n))
+    want = ops.attention_prefill_tiles(qd, k, v, *rest, rows_per_tile=tr)
+    got = ops.attention_prefill_tiles(qd, shifted(k, off_k), shifted(v, off_v), *rest, rows_per_tile=tr)
+    assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
 @pytest.mark.parametrize("fmt", ["fp8_e4m3", "int8_per_token_head", "fp8_per_token_head", "fp8_e5m2"])
 @pytest.mark.parametrize("hq,hk,d,ps", [(8, 2, 128, 16), (4, 4, 64, 16), (32, 8, 128, 32)])
 @pytest.mark.parametrize("half", [False, True])
