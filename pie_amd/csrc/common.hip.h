@@ -44,11 +44,10 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float acc) {
 
 // (a & mask) | bits in one VALU op.  On gfx9-family encodings a three-source VALU op may
 // read one scalar operand and no literal, so the mask rides in an SGPR and `bits` in a VGPR;
-// written as asm because the compiler otherwise splits it into v_and + v_or.
+// `a & b | c` is split into v_and + v_or by the compiler, and in asm it would not see the waits between
+// the result and a matrix product around it (a write of that product's addend while it is still being read among them).
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask_sgpr, uint32_t bits_vgpr) {
-    uint32_t d;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask_sgpr), "v"(bits_vgpr));
-    return d;
+    return __builtin_amdgcn_bitop3_b32(a, mask_sgpr, bits_vgpr, 0xEA);   // (the truth table of a & b | c)
 }
 
 template <int CTRL, int ROW_MASK = 0xF, int BANK_MASK = 0xF>
