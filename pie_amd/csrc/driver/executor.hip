@@ -86,18 +86,25 @@ Skinny skinny_cost(const Linear& w, int M) {
 double groups_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 2 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
-// The skinny GEMM of tile-major int4 weights as those blocks are compared with: up to 128 rows fitted to 50 matrices of 1024 - 28672 x 1024 - 14336 with
-// weights out of HBM, 7 - 11 % rms.  (The estimate above prices all matrices by their bytes alone: it is 40 % above what few rows of large ones take, and
-// blocks chosen by it ran 1.2 to 1.5 times as long as the passes: 2 rows of 8192 x 8192 12.0 us against 9.9, 8 of 8192 x 1024 5.7 against 4.5.)
+// The skinny GEMM of tile-major weights as the other forms are compared with it: up to 128 rows fitted to 50 matrices (one-byte weights, and int4 to 320 rows: 15) of 1024 - 28672 x 1024 - 14336 with
+// weights out of HBM, 5 - 11 % rms.  (The estimate above prices all matrices by their bytes alone: it is 40 % above what few rows of large ones take, and
+// blocks chosen by it ran 1.2 to 1.5 times as long as the passes: 2 rows of 8192 x 8192 int4 12.0 us against 9.9, 8 of 8192 x 1024 5.7 against 4.5.)
 double passes_cost(const Linear& w, int M) {
     struct Fit {
         int rows;
         double fixed, rate, per_n, per_k;
     };
-    constexpr Fit kFits[] = {{4, 3.21, 6.95e6, 0.061e-3, 0.288e-3},  {16, 3.65, 6.49e6, 0.056e-3, 0.390e-3}, {32, 4.22, 4.20e6, 0.089e-3, 0.337e-3},
-                             {64, 4.53, 3.47e6, 0.195e-3, 0.633e-3}, {96, 4.65, 1.93e6, 0.350e-3, 0.524e-3}, {128, 4.83, 1.72e6, 0.331e-3, 0.555e-3}};
-    for (const Fit& f : kFits)
-        if (M <= f.rows) return f.fixed + static_cast<double>(w.data_bytes()) / f.rate + w.N * f.per_n + w.K * f.per_k;
+    constexpr Fit kFits[3][10] = {{{4, 3.21, 6.95e6, 0.061e-3, 0.288e-3},  {16, 3.65, 6.49e6, 0.056e-3, 0.390e-3}, {32, 4.22, 4.20e6, 0.089e-3, 0.337e-3},
+                                  {64, 4.53, 3.47e6, 0.195e-3, 0.633e-3}, {96, 4.65, 1.93e6, 0.350e-3, 0.524e-3}, {128, 4.83, 1.72e6, 0.331e-3, 0.555e-3},
+                                   {160, 3.00, 1.17e6, 0.730e-3, 0.975e-3}, {192, 3.47, 1.05e6, 0.786e-3, 0.968e-3},
+                                   {256, 3.47, 1.01e6, 1.001e-3, 1.087e-3}, {320, 3.85, 0.57e6, 1.097e-3, 1.135e-3}},
+                                 /* int8 */ {{8, 3.64, 5.22e6, 0.051e-3, 0.153e-3}, {16, 3.72, 5.74e6, 0.096e-3, 0.443e-3}, {32, 4.11, 4.64e6, 0.140e-3, 0.340e-3},
+                                             {64, 3.87, 4.94e6, 0.447e-3, 0.727e-3}, {96, 4.22, 2.32e6, 0.471e-3, 0.563e-3}, {128, 4.31, 2.38e6, 0.582e-3, 0.686e-3}},
+                                 /* fp8 */ {{8, 3.26, 5.38e6, 0.050e-3, 0.160e-3}, {16, 3.40, 5.52e6, 0.068e-3, 0.399e-3}, {32, 3.67, 4.62e6, 0.111e-3, 0.314e-3},
+                                            {64, 3.26, 4.78e6, 0.357e-3, 0.683e-3}, {96, 3.57, 2.36e6, 0.359e-3, 0.529e-3}, {128, 3.42, 2.47e6, 0.497e-3, 0.712e-3}}};
+    if (w.kind != Quant::Bf16 && tile_major(w))
+        for (const Fit& f : kFits[w.kind == Quant::Int4b8 ? 0 : w.kind == Quant::Int8 ? 1 : 2])
+            if (M <= f.rows) return f.fixed + static_cast<double>(w.data_bytes()) / f.rate + w.N * f.per_n + w.K * f.per_k;
     return skinny_cost(w, M).us;
 }
 // (up to 32 rows both are short, and ties stay where they are)
@@ -107,28 +114,48 @@ bool in_groups(const Linear& w, int M, size_t ws_bytes) {
     if (M <= 128 && w.groups[M] >= 0) return w.groups[M] == 1;   // (measured at start-up)
     return (M <= 32 ? 1.05 : 1.0) * us < passes_cost(w, M);
 }
+// Microseconds of quantised weights in blocks whose waves take the steps of K in turn (1e30: not taken); they run in the skinny GEMM's place where they
+// are estimated faster than its passes and than blocks that scale groups: over 16 - 320 rows of 15 matrices the choice takes 0.81 of what the others' fastest
+// does for int8, 0.87 for fp8 and 0.90 for int4, 0.4 - 0.6 % more than the fastest of all each time.
+double waves_cost(const Linear& w, int M, size_t ws_bytes) {
+    return M >= 5 && w.kind != Quant::Bf16 && tile_major(w) ? pie_hip_gemm_waves_us(fmt_code(w.kind), M, w.N, w.K, w.group, ws_bytes, 0) : 1e30;
+}
+double skinny_or_groups(const Linear& w, int M, size_t ws_bytes) { return in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M); }
+bool in_waves(const Linear& w, int M, size_t ws_bytes) {
+    const double us = waves_cost(w, M, ws_bytes);
+    if (us > 1e29) return false;
+    if (M <= 128 && w.waves[M] >= 0) return w.waves[M] == 1;   // (measured at start-up)
+    return (M <= 8 ? 1.1 : 1.0) * us < skinny_or_groups(w, M, ws_bytes);   // (of few rows both are short)
+}
 // Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
 // where they are estimated faster.
+// (from 65 rows on: of 28672 x 4096 96 int8 rows take 42 us so and 54 in blocks of 64 columns, 128 44 and 62; below 129 the estimate is 6 % low)
 double rows_cost(const Linear& w, int M, size_t ws_bytes) {
-    return M > 128 && tile_major(w) ? pie_hip_gemm_rows_us(fmt_code(w.kind), M, w.N, w.K, ws_bytes) : 1e30;
+    return M > 64 && tile_major(w) ? (M > 128 ? 1.0 : 1.06) * pie_hip_gemm_rows_us(fmt_code(w.kind), M, w.N, w.K, ws_bytes) : 1e30;
 }
 bool in_rows(const Linear& w, int M, size_t ws_bytes) {
     const double rows = rows_cost(w, M, ws_bytes);
     return rows < 1e29 && rows < pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes);
 }
-// Microseconds of an int4 projection whose sums do not wait for the norm.
+// Microseconds of a quantised projection whose sums do not wait for the norm.
 double apart_cost(const Linear& w, int M, size_t ws_bytes) {
-    double us = in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M);
-    if (M > 128) us = std::min({us, static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 0, ws_bytes)),
-                                static_cast<double>(pie_hip_gemm_mfma_us(PIE_HIP_FMT_INT4B8, M, w.N, w.K, w.group, 1, ws_bytes))});
+    const int fmt = fmt_code(w.kind);
+    double us = in_waves(w, M, ws_bytes) ? waves_cost(w, M, ws_bytes) : skinny_or_groups(w, M, ws_bytes);
+    if (w.kind != Quant::Int4b8) us = std::min({us, rows_cost(w, M, ws_bytes), static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes))});
+    else if (M > 128) us = std::min({us, static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes)),
+                                     static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes))});
     return us;
 }
-// Whether an int4 projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
-// (pie_hip_shares_rmsnorm), for 5 rows and more: 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
-// without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.
-double shares_cost(const Linear& w, int M, size_t ws_bytes) {   // (1e30: not taken, by the product's kernel or the norm's)
-    if (M < 5 || w.kind != Quant::Int4b8 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return 1e30;
-    return pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes);
+// Whether a quantised projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
+// (pie_hip_shares_rmsnorm), for 5 rows and more: int4 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
+// without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.  (1e30: not taken, by the products' kernels or the norm's)
+double groups_shares_cost(const Linear& w, int M, size_t ws_bytes) {
+    return w.kind == Quant::Int4b8 ? pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
+}
+double waves_shares_cost(const Linear& w, int M, size_t ws_bytes) { return pie_hip_gemm_waves_us(fmt_code(w.kind), M, w.N, w.K, w.group, ws_bytes, 1); }
+double shares_cost(const Linear& w, int M, size_t ws_bytes) {
+    if (M < 5 || w.kind == Quant::Bf16 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return 1e30;
+    return std::min(groups_shares_cost(w, M, ws_bytes), waves_shares_cost(w, M, ws_bytes));
 }
 bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     const double us = shares_cost(w, M, ws_bytes);
@@ -140,7 +167,9 @@ bool in_shares(const Linear& w, int M, size_t ws_bytes) {
 double tiled_cost(const Linear& w, int M) { return 2.0 + w.K / 64 * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, (w.N + 127) / 128 / 512.0); }
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
-    const auto [p2, wpasses, wave_form, skinny] = skinny_cost(w, M);
+    const auto [p2, wpasses, wave_form, passes] = skinny_cost(w, M);
+    const double waves = in_waves(w, M, ws_bytes) ? waves_cost(w, M, ws_bytes) : 1e30;   // (in the skinny GEMM's place)
+    const double skinny = std::min(w.kind == Quant::Int8 || w.kind == Quant::Fp8 ? passes_cost(w, M) : passes, waves);
     const double data = static_cast<double>(w.data_bytes()), groups = groups_cost(w, M, ws_bytes);
     const int steps = w.K / 64;
     if (M > 128) {
@@ -162,6 +191,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const double blocks = std::min(rows, wide);
         // (on narrow outputs blocks of few rows and the passes are close, and the passes' estimate is the one that is too high: 160 rows of 3072 x 4096 and
         // 320 of 2048 x 2048 fp8 13.9 and 13.7 us in passes, 17.0 and 14.7 in blocks)
+        if (waves < std::min({rows, wide, tiles})) return GemmPath::Skinny;
         if (rows_us < std::min(1.12 * rows, wide) || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
         return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
     }
@@ -174,8 +204,10 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         split = 15.0 + (per + 3) * (M <= 64 ? 1.06 : 1.36) * std::ceil(tiles * shares / 512.0);
     }
     if (w.kind == Quant::Int4b8) {   // (blocks with fp32 group scales run in the skinny GEMM's place; up to 48 rows of wide outputs that is the wide GEMM's own form)
-        if (groups < std::min(split, tiled)) return M <= 48 && w.N >= 16384 && in_groups(w, M, ws_bytes) ? GemmPath::Wide : GemmPath::Skinny;
-    } else if (tile_major(w) && pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes) < std::min({skinny, split, tiled})) {
+        if (std::min(waves, groups) < std::min(split, tiled))
+            return M <= 48 && w.N >= 16384 && waves > 1e29 && in_groups(w, M, ws_bytes) ? GemmPath::Wide : GemmPath::Skinny;
+    } else if (tile_major(w) && std::min(rows_cost(w, M, ws_bytes), static_cast<double>(pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes))) <
+                                    std::min({skinny, split, tiled})) {
         return GemmPath::Wide;
     }
     if (split < skinny && split < tiled) return GemmPath::TiledSplitK;
@@ -261,6 +293,12 @@ bool linear_fused(const Linear& w, const uint16_t* act, const uint16_t* norm_w, 
                               : tuned == 3 ? GemmPath::TiledSplitK
                               : tuned == 4 ? GemmPath::Wide
                                            : pick_gemm(w, M, gemm_ws_bytes);   // (forced row limit, GEMV refusal)
+        if (path == GemmPath::Skinny && in_waves(w, M, gemm_ws_bytes)) {
+            const int sv = pie_hip_gemm_waves_tiled(fmt, a, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, sbf, w.group, y, M, w.N, w.K, beta, swiglu, glu,
+                                                    gemm_ws, gemm_ws_bytes, s);
+            if (sv == PIE_HIP_OK) return true;
+            if (sv != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sv);
+        }
         if (path == GemmPath::Skinny && in_groups(w, M, gemm_ws_bytes)) {
             const int sg = pie_hip_gemm_groups_tiled(a, w.data_tiled, w.scale_tiled, w.group, y, M, w.N, w.K, beta, swiglu, glu,
                                                      gemm_ws, gemm_ws_bytes, s);
@@ -563,6 +601,22 @@ void Executor::tune_linears() {
                 }
                 set(&Linear::groups, form, lo);
             }
+            // likewise that or the blocks whose waves take the steps in turn
+            if (waves_cost(l0, M, gemm_ws_bytes_) < 1e29) {
+                int form = in_waves(l0, M, gemm_ws_bytes_) ? 1 : 0;
+                if (close(waves_cost(l0, M, gemm_ws_bytes_), skinny_or_groups(l0, M, gemm_ws_bytes_))) {
+                    double us[2];
+                    for (int f = 0; f < 2; ++f) {
+                        set(&Linear::waves, f, M);
+                        us[f] = time_route(r, M, 1);
+                    }
+                    if (clearly(us[1 - form], us[form])) form = 1 - form;
+                    skinny_t = us[form];
+                } else if (form == 1) {
+                    skinny_t = 1e30;   // (what was measured above does not run)
+                }
+                set(&Linear::waves, form, lo);
+            }
             int best = -1;
             double best_t = 1e30, model_t = 1e30;
             const int by_model = model_route(l0, M, r.norm != nullptr, gemm_ws_bytes_);
@@ -803,7 +857,10 @@ void Executor::moe_block(const LayerWeights& w, int N, const uint16_t* next_norm
 bool Executor::project_in_shares(const Linear& w, const uint16_t* act, const uint16_t* norm, int N) {
     const ModelConfig& m = model_.cfg();
     int shares = 0;
-    const int st = pie_hip_gemm_groups_shares(act, w.data_tiled, w.scale_tiled, w.group, N, w.N, w.K, gemm_ws_, gemm_ws_bytes_, &shares, stream_);
+    const bool waves = waves_shares_cost(w, N, gemm_ws_bytes_) < groups_shares_cost(w, N, gemm_ws_bytes_);
+    const int st = waves ? pie_hip_gemm_waves_shares(fmt_code(w.kind), act, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, w.scale_bf16 ? 1 : 0, w.group, N,
+                                                     w.N, w.K, gemm_ws_, gemm_ws_bytes_, &shares, stream_)
+                         : pie_hip_gemm_groups_shares(act, w.data_tiled, w.scale_tiled, w.group, N, w.N, w.K, gemm_ws_, gemm_ws_bytes_, &shares, stream_);
     if (st == PIE_HIP_ERR_UNSUPPORTED) return false;
     PIE_KERNEL(st);
     PIE_KERNEL(pie_hip_shares_rmsnorm(static_cast<const float*>(gemm_ws_), shares, x_, norm, xn_, N, m.hidden, m.rms_eps, stream_));
@@ -874,11 +931,14 @@ void Executor::body(int N, int S, int max_kv_len) {
             bool done = false;
             const int tuned_qkv = N <= 128 ? w.wqkv.tuned[N] : -1;
             const GemmPath path = tuned_qkv < 0 ? pick_gemm(w.wqkv, N, gemm_ws_bytes_) : tuned_qkv <= 1 ? GemmPath::Skinny : tuned_qkv == 4 ? GemmPath::Wide : GemmPath::Tiled;
-            const bool groups = in_groups(w.wqkv, N, gemm_ws_bytes_);
+            const bool waves = path == GemmPath::Skinny && in_waves(w.wqkv, N, gemm_ws_bytes_), groups = !waves && in_groups(w.wqkv, N, gemm_ws_bytes_);
             if (fused_rope && !w.q_norm && w.wqkv.data_tiled && (path == GemmPath::Skinny || (path == GemmPath::Wide && groups && N <= 48))) {
                 if (!prenormed) PIE_KERNEL(pie_hip_rmsnorm(x_, w.attn_norm, xn_, N, H, m.rms_eps, s));
                 const int st =
-                    groups
+                    waves ? pie_hip_qkv_rope_waves_tiled(fmt_code(w.wqkv.kind), xn_, w.wqkv.data_tiled, w.wqkv.scale_tiled ? w.wqkv.scale_tiled : w.wqkv.scale,
+                                                         w.wqkv.scale_bf16 ? 1 : 0, w.wqkv.group, N, H, rope_tab_, slots, q_, k_pool_[l], v_pool_[l], hq, hk, d,
+                                                         pairing, gemm_ws_, gemm_ws_bytes_, s)
+                    : groups
                         ? pie_hip_qkv_rope_groups_tiled(xn_, w.wqkv.data_tiled, w.wqkv.scale_tiled, w.wqkv.group, N, H, rope_tab_, slots, q_,
                                                         k_pool_[l], v_pool_[l], hq, hk, d, pairing, gemm_ws_, gemm_ws_bytes_, s)
                         : pie_hip_qkv_rope_skinny_tiled(fmt_code(w.wqkv.kind), xn_, w.wqkv.data_tiled,
@@ -1443,7 +1503,8 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
 }
 
 // And in which form that kernel runs, by what a measurement said (0 or 1; -1: by estimate): bit 0 int4 rows in blocks that scale groups in fp32 (in the skinny GEMM's place), bit 1 an int4
-// projection into the residual in shares of K that meet in the norm's kernel, bit 2 one-byte rows in blocks of 32 to 128 (in the wide GEMM's place).
+// projection into the residual in shares of K that meet in the norm's kernel, bit 2 one-byte rows in blocks of 32 to 128 (in the wide GEMM's place), bit 3 rows in
+// blocks whose waves take the steps of K in turn (in the skinny GEMM's place).
 extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, int K, int measured_groups, int measured_shares,
                                            size_t workspace_bytes) {
     using namespace pie_hip_driver;
@@ -1458,7 +1519,8 @@ extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, 
     w.data_tiled = w.scale_tiled = &there;
     w.groups.fill(static_cast<int8_t>(measured_groups));
     w.shares.fill(static_cast<int8_t>(measured_shares));
-    return (in_groups(w, M, workspace_bytes) ? 1 : 0) | (in_shares(w, M, workspace_bytes) ? 2 : 0) | (in_rows(w, M, workspace_bytes) ? 4 : 0);
+    return (in_groups(w, M, workspace_bytes) ? 1 : 0) | (in_shares(w, M, workspace_bytes) ? 2 : 0) | (in_rows(w, M, workspace_bytes) ? 4 : 0) |
+           (in_waves(w, M, workspace_bytes) ? 8 : 0);
 }
 
 // The same for a mixture's experts: whether `routes` over `experts` of a storage format run in blocks of an expert's routes (1)

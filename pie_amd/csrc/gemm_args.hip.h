@@ -149,6 +149,53 @@ __device__ __forceinline__ void store_pair(const GemmArgs& a, int m, int n, int 
     *p = u32x4_t{x[0], y[0], x[1], y[1]};
 }
 
+// q|k|v rows: adjacent columns of q and k heads are rotated, q goes to y [rows, hq * d], k and v to slot slots[row] of the pools
+struct Rotation {
+    const float* table = nullptr;   // [rows, d]: cos (d / 2), then sin (d / 2); null: plain outputs
+    const int64_t* slots = nullptr; // negative: the row writes no K/V
+    uint16_t *k_pages = nullptr, *v_pages = nullptr;
+    int hq = 0, hk = 0, d = 0, half_out = 0;   // half_out: pair (2i, 2i + 1) goes to places (i, i + d / 2)
+};
+
+// Row m, columns n .. n + 3: the projection's bf16 values, then the rotation of qkv_rope_kvwrite_kernel, same operations and rounding.
+__device__ __forceinline__ void store_rotated(const GemmArgs& a, const Rotation& r, int m, int n, const float* v) {
+    const int shift = __builtin_ctz(static_cast<unsigned>(r.d)), head = n >> shift, dd = n & (r.d - 1);
+    float b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
+    const int64_t slot = r.slots[m];
+    if (head >= r.hq + r.hk) {
+        if (slot >= 0)
+            *reinterpret_cast<u32x2_t*>(r.v_pages + (static_cast<size_t>(slot) * r.hk + (head - r.hq - r.hk)) * r.d + dd) =
+                u32x2_t{pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
+        return;
+    }
+    if (head >= r.hq && slot < 0) return;
+    const float* tab = r.table + static_cast<size_t>(m) * r.d + (dd >> 1);
+    uint16_t* dst = head < r.hq ? a.y + (static_cast<size_t>(m) * r.hq + head) * r.d
+                                : r.k_pages + (static_cast<size_t>(slot) * r.hk + (head - r.hq)) * r.d;
+    uint32_t o[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float c = tab[i], s = tab[(r.d >> 1) + i], x = b[2 * i], y = b[2 * i + 1];
+        o[i] = pack_bf16x2(x * c - y * s, y * c + x * s);
+    }
+    if (r.half_out) {
+        *reinterpret_cast<uint32_t*>(dst + (dd >> 1)) = __builtin_amdgcn_perm(o[1], o[0], 0x05040100u);
+        *reinterpret_cast<uint32_t*>(dst + (dd >> 1) + (r.d >> 1)) = __builtin_amdgcn_perm(o[1], o[0], 0x07060302u);
+    } else {
+        *reinterpret_cast<u32x2_t*>(dst + dd) = u32x2_t{o[0], o[1]};
+    }
+}
+__device__ __forceinline__ void store4(const GemmArgs& a, const Rotation& r, int m, int n, float* v) {
+    if (r.table) store_rotated(a, r, m, n, v);
+    else wide_store(a, m, n, v);
+}
+
+// places of a row's sixteen 16-byte granules: granule c at c ^ key(row).  The lanes an LDS read serves together (0 - 3 and
+// 12 - 15 of one granule's rows, 4 - 11 of the next but three) find sixteen different places.
+__device__ __forceinline__ int key_of(int row) { return (row & 15) < 4 ? row & 15 : (row & 15) < 12 ? (row & 15) + 4 : (row & 15) - 8; }
+
 // The problem and the rows [m0, m1) of block row `t` when problems are cut into blocks of `rows` rows one after
 // another; false behind the last.  Every lane of the wave calls it and gets the same answer.
 __device__ __forceinline__ bool grouped_place(const int32_t* __restrict__ offsets, int problems, int rows, int t, int lane,
@@ -197,6 +244,8 @@ double gemm_wide_us(int format, int M, int N, int K, int group_size, size_t ws_b
 // in shares.
 int launch_gemm_groups(const GemmArgs& a, int group_size, void* ws, size_t ws_bytes, hipStream_t stream);
 double gemm_groups_us(int M, int N, int K, int group_size, size_t ws_bytes);
+// The shares' fp32 sums in a.partial [shares, M, N], added in order, and the epilogue (N % 4 == 0, 16-byte boundaries).
+int launch_shares_reduce(const GemmArgs& a, const Rotation& rot, int shares, hipStream_t stream);
 double gemm_tiles_us(int format, int M, int N, int K);
 
 }  // namespace pie_hip

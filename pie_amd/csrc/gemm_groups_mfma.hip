@@ -29,53 +29,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int kStep = 128, kStages = 4, kTiles = 2;   // k-values of a step; steps in flight; column tiles of a wave
 constexpr int kCols = 4 * kTiles * 16;                // columns of a block
 
-// q|k|v rows: adjacent columns of q and k heads are rotated, q goes to y [rows, hq * d], k and v to slot slots[row] of the pools
-struct Rotation {
-    const float* table = nullptr;   // [rows, d]: cos (d / 2), then sin (d / 2); null: plain outputs
-    const int64_t* slots = nullptr; // negative: the row writes no K/V
-    uint16_t *k_pages = nullptr, *v_pages = nullptr;
-    int hq = 0, hk = 0, d = 0, half_out = 0;   // half_out: pair (2i, 2i + 1) goes to places (i, i + d / 2)
-};
-
-// Row m, columns n .. n + 3: the projection's bf16 values, then the rotation of qkv_rope_kvwrite_kernel, same operations and rounding.
-__device__ __forceinline__ void store_rotated(const GemmArgs& a, const Rotation& r, int m, int n, const float* v) {
-    const int shift = __builtin_ctz(static_cast<unsigned>(r.d)), head = n >> shift, dd = n & (r.d - 1);
-    float b[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) b[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
-    const int64_t slot = r.slots[m];
-    if (head >= r.hq + r.hk) {
-        if (slot >= 0)
-            *reinterpret_cast<u32x2_t*>(r.v_pages + (static_cast<size_t>(slot) * r.hk + (head - r.hq - r.hk)) * r.d + dd) =
-                u32x2_t{pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
-        return;
-    }
-    if (head >= r.hq && slot < 0) return;
-    const float* tab = r.table + static_cast<size_t>(m) * r.d + (dd >> 1);
-    uint16_t* dst = head < r.hq ? a.y + (static_cast<size_t>(m) * r.hq + head) * r.d
-                                : r.k_pages + (static_cast<size_t>(slot) * r.hk + (head - r.hq)) * r.d;
-    uint32_t o[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const float c = tab[i], s = tab[(r.d >> 1) + i], x = b[2 * i], y = b[2 * i + 1];
-        o[i] = pack_bf16x2(x * c - y * s, y * c + x * s);
-    }
-    if (r.half_out) {
-        *reinterpret_cast<uint32_t*>(dst + (dd >> 1)) = __builtin_amdgcn_perm(o[1], o[0], 0x05040100u);
-        *reinterpret_cast<uint32_t*>(dst + (dd >> 1) + (r.d >> 1)) = __builtin_amdgcn_perm(o[1], o[0], 0x07060302u);
-    } else {
-        *reinterpret_cast<u32x2_t*>(dst + dd) = u32x2_t{o[0], o[1]};
-    }
-}
-__device__ __forceinline__ void store4(const GemmArgs& a, const Rotation& r, int m, int n, float* v) {
-    if (r.table) store_rotated(a, r, m, n, v);
-    else wide_store(a, m, n, v);
-}
-
-// places of a row's sixteen 16-byte granules: granule c at c ^ key(row).  The lanes an LDS read serves together (0 - 3 and
-// 12 - 15 of one granule's rows, 4 - 11 of the next but three) find sixteen different places.
-__device__ __forceinline__ int key_of(int row) { return (row & 15) < 4 ? row & 15 : (row & 15) < 12 ? (row & 15) + 4 : (row & 15) - 8; }
-
 template <int RT>
 __global__ __launch_bounds__(256, 2) void gemm_groups_kernel(const GemmArgs a, const Rotation rot, int row_blocks, int per_xcd, int blocks, int per_share) {
     constexpr int S = kStages, NG = kTiles, kVecs = RT * 16 * (kStep / 8), kOps = RT + 2 * NG;
@@ -266,7 +219,7 @@ __global__ __launch_bounds__(256, 2) void gemm_groups_kernel(const GemmArgs a, c
 }
 
 // The shares' sums in the order of K, and the epilogue.
-__global__ __launch_bounds__(256) void groups_reduce_kernel(const GemmArgs a, const Rotation rot, int shares) {
+__global__ __launch_bounds__(256) void shares_reduce_kernel(const GemmArgs a, const Rotation rot, int shares) {
     const int quads = a.N / 4;
     const size_t idx = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= static_cast<size_t>(a.M) * quads) return;
@@ -278,6 +231,14 @@ __global__ __launch_bounds__(256) void groups_reduce_kernel(const GemmArgs a, co
     float v[4] = {sum[0], sum[1], sum[2], sum[3]};
     store4(a, rot, m, n, v);
 }
+
+}  // namespace
+int launch_shares_reduce(const GemmArgs& a, const Rotation& rot, int shares, hipStream_t stream) {
+    const size_t quads = static_cast<size_t>(a.M) * (a.N / 4);
+    hipLaunchKernelGGL(shares_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, a, rot, shares);
+    return launch_status();
+}
+namespace {
 
 template <int RT>
 int launch(const GemmArgs& a, const Rotation& rot, int shares, hipStream_t stream) {
@@ -344,9 +305,7 @@ int run(GemmArgs a, const Rotation& rot, int group_size, void* ws, size_t ws_byt
                                       : launch<4>(a, rot, p.shares, stream);
     if (shares) *shares = p.shares;
     if (st != PIE_HIP_OK || p.shares == 1 || shares) return st;
-    const size_t quads = static_cast<size_t>(a.M) * (a.N / 4);
-    hipLaunchKernelGGL(groups_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, a, rot, p.shares);
-    return launch_status();
+    return launch_shares_reduce(a, rot, p.shares, stream);
 }
 
 }  // namespace

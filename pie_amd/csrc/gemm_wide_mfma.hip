@@ -785,15 +785,15 @@ bool columns_fit(int format, int M, int N, int K, int group_size) {
         return M > 16 && M <= 48 && gemm_groups_us(M, N, K, group_size, 0) < 1e30;
     return M <= 128 && (format == PIE_HIP_FMT_FP8 || format == PIE_HIP_FMT_INT8) && K % kStepK == 0;
 }
-// A round of blocks (one to a CU, two with 64 rows' LDS) takes 4 us and 0.27 - 0.5 a step (measured at 40 - 128 rows of
-// 16384, 5120 and 3072 x 2048 and 28672 x 4096).
+// A round of blocks (one to a CU, two with 64 rows' LDS) takes 4 to 5.5 us and, a step, 0.19 - 0.35 for a few blocks and 0.08 - 0.13 more when all CUs have
+// one, or what the weights take at 6 TB/s (measured at 17 - 128 rows of 15 matrices of 1024 - 28672 x 1024 - 14336, weights out of HBM: 9 % rms).
 double columns_us(int format, int M, int N, int K, int group_size, size_t ws_bytes) {
     if (format == PIE_HIP_FMT_INT4B8) return gemm_groups_us(M, N, K, group_size, ws_bytes);
-    const int size = M <= 64 ? 0 : M <= 96 ? 1 : 2;
-    constexpr double kStepUs[2][3] = {{0.34, 0.40, 0.51}, {0.27, 0.39, 0.50}};
+    const int size = M <= 64 ? 0 : M <= 96 ? 1 : 2, fp8 = format == PIE_HIP_FMT_FP8;
+    constexpr double kFixed[3] = {3.8, 4.6, 5.5}, kStepUs[2][3] = {{0.23, 0.30, 0.35}, {0.19, 0.28, 0.34}}, kFull[2][3] = {{0.10, 0.12, 0.12}, {0.08, 0.13, 0.13}};
     const long long blocks = (N + 63) / 64, slots = size == 0 ? 512 : 256;
-    const double crowd = size == 0 && blocks > 256 ? 1.6 : 1.0;
-    return 4.0 + static_cast<double>((blocks + slots - 1) / slots) * (K / kStepK) * kStepUs[format == PIE_HIP_FMT_FP8][size] * crowd;
+    const double crowd = size == 0 && blocks > 256 ? (fp8 ? 1.8 : 1.42) : 1.0, step = (kStepUs[fp8][size] + kFull[fp8][size] * std::min(1.0, blocks / 256.0)) * crowd;
+    return std::max(kFixed[size] + static_cast<double>((blocks + slots - 1) / slots) * (K / kStepK) * step, 2.6 + 1e-6 * N * K / 6.0);
 }
 
 // ---- one-byte weights and many rows in blocks of 32 to 128 rows x 128 columns ---------------------------------------------------

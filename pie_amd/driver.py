@@ -483,11 +483,12 @@ def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: 
 def linear_forms(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 32 << 20, measured_groups: int = -1,
                  measured_shares: int = -1) -> dict:
     """Host-only: the forms the driver's estimates (or measurements: 0, 1) give tile-major weights: `groups` (int4 rows in blocks in the skinny GEMM's place), `shares` (a
-    projection into the residual whose sums meet in the norm), `rows` (one-byte rows in blocks in the wide GEMM's place)."""
+    projection into the residual whose sums meet in the norm), `rows` (one-byte rows in blocks in the wide GEMM's place), `waves` (rows in blocks whose waves take the
+    steps of K in turn, in the skinny GEMM's place)."""
     bits = lib().pie_hip_driver_linear_forms(_FORMATS.index(kind), group, M, N, K, measured_groups, measured_shares, workspace_bytes)
     if bits < 0:
         raise ValueError("linear_forms")
-    return {name: bool(bits >> i & 1) for i, name in enumerate(("groups", "shares", "rows"))}
+    return {name: bool(bits >> i & 1) for i, name in enumerate(("groups", "shares", "rows", "waves"))}
 
 
 def experts_in_blocks(kind: str, routes: int, experts: int, hidden: int = 0, inner: int = 0) -> bool:

@@ -722,6 +722,60 @@ def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor
     return y
 
 
+def gemm_waves_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
+                     workspace: Optional[torch.Tensor] = None, rule: Optional[Glu] = None) -> torch.Tensor:
+    """The GEMM over tile-major int4, int8 or fp8 weights in blocks whose waves take the steps of K in turn (up to 512 rows); with a
+    workspace few blocks over a long K run in shares of K."""
+    _dev(act, torch.bfloat16, "act")
+    M, K = act.shape
+    if K != w.K or not w.kind.endswith("+tiled"):
+        raise KernelError("act K != weight K, or not tile-major weights")
+    n_out = w.N // 2 if epilogue == 1 else w.N
+    if y is None:
+        if beta:
+            raise KernelError("beta=1 needs an existing y")
+        y = torch.empty((M, n_out), dtype=torch.bfloat16, device=act.device)
+    _dev(y, torch.bfloat16, "y")
+    if tuple(y.shape) != (M, n_out):
+        raise KernelError("y shape mismatch")
+    _check(kernels().pie_hip_gemm_waves_tiled(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale),
+                                              int(w.scale.dtype == torch.bfloat16), w.group_size, _ptr(y), M, w.N, K, beta, epilogue,
+                                              None if rule is None else C.byref(rule), _ptr(workspace),
+                                              C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream()),
+           "pie_hip_gemm_waves_tiled")
+    return y
+
+
+def gemm_waves_shares_norm(act: torch.Tensor, w: WeightView, x: torch.Tensor, norm_weight: torch.Tensor, eps: float, workspace: torch.Tensor):
+    """x += act . W^T in that form, in shares of K that meet in the norm's kernel; returns the normalised rows and the number of shares."""
+    for t, n in ((act, "act"), (x, "x"), (norm_weight, "norm_weight")):
+        _dev(t, torch.bfloat16, n)
+    M, K = act.shape
+    if K != w.K or not w.kind.endswith("+tiled") or tuple(x.shape) != (M, w.N) or norm_weight.numel() != w.N:
+        raise KernelError("shape mismatch, or not tile-major weights")
+    shares, y = C.c_int(0), torch.empty_like(x)
+    _check(kernels().pie_hip_gemm_waves_shares(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale), int(w.scale.dtype == torch.bfloat16),
+                                               w.group_size, M, w.N, K, _ptr(workspace), C.c_size_t(workspace.numel() * workspace.element_size()),
+                                               C.byref(shares), _stream()), "pie_hip_gemm_waves_shares")
+    _check(kernels().pie_hip_shares_rmsnorm(_ptr(workspace), shares, _ptr(x), _ptr(norm_weight), _ptr(y), M, w.N, C.c_float(eps), _stream()),
+           "pie_hip_shares_rmsnorm")
+    return y, shares.value
+
+
+def gemm_waves_us(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 0, norm: bool = False) -> float:
+    lib = kernels()
+    lib.pie_hip_gemm_waves_us.restype = C.c_float
+    return float(lib.pie_hip_gemm_waves_us(FMT[kind], M, N, K, group, C.c_size_t(workspace_bytes), int(norm)))
+
+
+def gemm_waves_plan(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 0, norm: bool = False) -> Tuple[int, int, int]:
+    """Rows and columns of a block and shares of K of `gemm_waves_tiled` (norm: of `gemm_waves_shares_norm`)."""
+    rows, cols, shares = C.c_int(0), C.c_int(0), C.c_int(0)
+    _check(kernels().pie_hip_gemm_waves_plan(FMT[kind], M, N, K, group, C.c_size_t(workspace_bytes), int(norm), C.byref(rows), C.byref(cols), C.byref(shares)),
+           "pie_hip_gemm_waves_plan")
+    return rows.value, cols.value, shares.value
+
+
 def gemm_groups_shares_norm(act: torch.Tensor, w: WeightView, x: torch.Tensor, norm_weight: torch.Tensor, eps: float, workspace: torch.Tensor):
     """x += act . W^T in shares of K that meet in the norm's kernel; returns the normalised rows and the number of shares."""
     for t, n in ((act, "act"), (x, "x"), (norm_weight, "norm_weight")):
@@ -842,10 +896,10 @@ def qkv_rope_fused(act: torch.Tensor, w: WeightView, table: torch.Tensor, kv_slo
 
 def qkv_rope_skinny_tiled(act: torch.Tensor, w: WeightView, table: torch.Tensor, kv_slots: torch.Tensor,
                           k_pages: torch.Tensor, v_pages: torch.Tensor, hq: int, hk: int, d: int,
-                          pairing: int = 1, groups: bool = False, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+                          pairing: int = 1, groups: bool = False, workspace: Optional[torch.Tensor] = None, waves: bool = False) -> torch.Tensor:
     """q|k|v projection over tile-major weights + RoPE + KV-cache write for a decode batch (act
     already normalised).  Returns q [M, hq, d]; k / v land in their slots.  pairing as for
-    `qkv_rope_fused`; `groups`: int4 weights in the form of `gemm_groups_tiled`."""
+    `qkv_rope_fused`; `groups`: int4 weights in the form of `gemm_groups_tiled`; `waves`: in the form of `gemm_waves_tiled`."""
     _dev(act, torch.bfloat16, "act")
     _dev(table, torch.float32, "rope_table")
     _dev(kv_slots, torch.int64, "kv_slots")
@@ -860,6 +914,12 @@ def qkv_rope_skinny_tiled(act: torch.Tensor, w: WeightView, table: torch.Tensor,
         raise KernelError("kv slot out of range")
     q_out = torch.empty((M, hq, d), dtype=torch.bfloat16, device=act.device)
     scale_is_bf16 = int(w.scale is not None and w.scale.dtype == torch.bfloat16)
+    if waves:
+        _check(kernels().pie_hip_qkv_rope_waves_tiled(
+            FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale), scale_is_bf16, w.group_size, M, K, _ptr(table), _ptr(kv_slots), _ptr(q_out),
+            _ptr(k_pages), _ptr(v_pages), hq, hk, d, pairing, _ptr(workspace),
+            C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream()), "pie_hip_qkv_rope_waves_tiled")
+        return q_out
     if groups:
         if w.kind != "int4b8+tiled":
             raise KernelError("tile-major int4 weights expected")
