@@ -87,24 +87,31 @@ double groups_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 2 && w.kind == Quant::Int4b8 && tile_major(w) ? pie_hip_gemm_groups_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
 // The skinny GEMM of tile-major weights as the other forms are compared with it: up to 128 rows fitted to 50 matrices (one-byte weights, and int4 to 320 rows: 15) of 1024 - 28672 x 1024 - 14336 with
-// weights out of HBM, 5 - 11 % rms.  (The estimate above prices all matrices by their bytes alone: it is 40 % above what few rows of large ones take, and
+// weights out of HBM, 5 - 11 % rms; bf16 over 17 matrices to 320 rows, with a copy or row-major, 8 - 13 %, past 128 rows 13 - 22.  (The estimate above prices all matrices by their bytes alone: it is 40 % above what few rows of large ones take, and
 // blocks chosen by it ran 1.2 to 1.5 times as long as the passes: 2 rows of 8192 x 8192 int4 12.0 us against 9.9, 8 of 8192 x 1024 5.7 against 4.5.)
 double passes_cost(const Linear& w, int M) {
     struct Fit {
         int rows;
         double fixed, rate, per_n, per_k;
     };
-    constexpr Fit kFits[3][10] = {{{4, 3.21, 6.95e6, 0.061e-3, 0.288e-3},  {16, 3.65, 6.49e6, 0.056e-3, 0.390e-3}, {32, 4.22, 4.20e6, 0.089e-3, 0.337e-3},
+    constexpr Fit kFits[5][10] = {{{4, 3.21, 6.95e6, 0.061e-3, 0.288e-3},  {16, 3.65, 6.49e6, 0.056e-3, 0.390e-3}, {32, 4.22, 4.20e6, 0.089e-3, 0.337e-3},
                                   {64, 4.53, 3.47e6, 0.195e-3, 0.633e-3}, {96, 4.65, 1.93e6, 0.350e-3, 0.524e-3}, {128, 4.83, 1.72e6, 0.331e-3, 0.555e-3},
                                    {160, 3.00, 1.17e6, 0.730e-3, 0.975e-3}, {192, 3.47, 1.05e6, 0.786e-3, 0.968e-3},
                                    {256, 3.47, 1.01e6, 1.001e-3, 1.087e-3}, {320, 3.85, 0.57e6, 1.097e-3, 1.135e-3}},
                                  /* int8 */ {{8, 3.64, 5.22e6, 0.051e-3, 0.153e-3}, {16, 3.72, 5.74e6, 0.096e-3, 0.443e-3}, {32, 4.11, 4.64e6, 0.140e-3, 0.340e-3},
                                              {64, 3.87, 4.94e6, 0.447e-3, 0.727e-3}, {96, 4.22, 2.32e6, 0.471e-3, 0.563e-3}, {128, 4.31, 2.38e6, 0.582e-3, 0.686e-3}},
                                  /* fp8 */ {{8, 3.26, 5.38e6, 0.050e-3, 0.160e-3}, {16, 3.40, 5.52e6, 0.068e-3, 0.399e-3}, {32, 3.67, 4.62e6, 0.111e-3, 0.314e-3},
-                                            {64, 3.26, 4.78e6, 0.357e-3, 0.683e-3}, {96, 3.57, 2.36e6, 0.359e-3, 0.529e-3}, {128, 3.42, 2.47e6, 0.497e-3, 0.712e-3}}};
-    if (w.kind != Quant::Bf16 && tile_major(w))
-        for (const Fit& f : kFits[w.kind == Quant::Int4b8 ? 0 : w.kind == Quant::Int8 ? 1 : 2])
-            if (M <= f.rows) return f.fixed + static_cast<double>(w.data_bytes()) / f.rate + w.N * f.per_n + w.K * f.per_k;
+                                            {64, 3.26, 4.78e6, 0.357e-3, 0.683e-3}, {96, 3.57, 2.36e6, 0.359e-3, 0.529e-3}, {128, 3.42, 2.47e6, 0.497e-3, 0.712e-3}},
+                                 /* bf16 */ {{8, 3.43, 5.89e6, 0.000e-3, 0.025e-3}, {16, 3.81, 5.77e6, 0.000e-3, 0.179e-3}, {32, 3.99, 4.65e6, 0.000e-3, 0.000e-3},
+                                             {64, 4.21, 4.45e6, 0.116e-3, 0.246e-3}, {96, 4.38, 2.62e6, 0.014e-3, 0.117e-3}, {128, 4.70, 2.47e6, 0.082e-3, 0.074e-3},
+                                             {192, 4.39, 1.53e6, 0.076e-3, 0.000e-3}, {320, 5.01, 1.21e6, 0.283e-3, 0.000e-3}},
+                                 /* row-major */ {{8, 4.80, 6.01e6, 0.191e-3, 0.474e-3}, {16, 5.16, 6.06e6, 0.208e-3, 0.693e-3}, {32, 6.06, 2.93e6, 0.000e-3, 0.160e-3},
+                                                  {64, 6.35, 1.97e6, 0.024e-3, 0.449e-3}, {96, 8.00, 1.43e6, 0.000e-3, 0.726e-3}, {128, 8.00, 1.04e6, 0.000e-3, 0.102e-3},
+                                                  {192, 8.00, 0.77e6, 0.191e-3, 0.859e-3}, {320, 6.28, 0.46e6, 0.123e-3, 0.209e-3}}};
+    if (w.kind == Quant::Bf16 || tile_major(w))
+        for (const Fit& f : kFits[w.kind == Quant::Int4b8 ? 0 : w.kind == Quant::Int8 ? 1 : w.kind == Quant::Fp8 ? 2 : tile_major(w) ? 3 : 4])
+            if (M <= f.rows)   // (a list's unused places have no rows)
+                return f.fixed + static_cast<double>(w.data_bytes()) / f.rate + w.N * f.per_n + w.K * f.per_k;
     return skinny_cost(w, M).us;
 }
 // (up to 32 rows both are short, and ties stay where they are)
@@ -114,18 +121,19 @@ bool in_groups(const Linear& w, int M, size_t ws_bytes) {
     if (M <= 128 && w.groups[M] >= 0) return w.groups[M] == 1;   // (measured at start-up)
     return (M <= 32 ? 1.05 : 1.0) * us < passes_cost(w, M);
 }
-// Microseconds of quantised weights in blocks whose waves take the steps of K in turn (1e30: not taken); they run in the skinny GEMM's place where they
+// Microseconds of weights in blocks whose waves take the steps of K in turn (1e30: not taken); they run in the skinny GEMM's place where they
 // are estimated faster than its passes and than blocks that scale groups: over 16 - 320 rows of 15 matrices the choice takes 0.81 of what the others' fastest
-// does for int8, 0.87 for fp8 and 0.90 for int4, 0.4 - 0.6 % more than the fastest of all each time.
+// does for int8, 0.87 for fp8 and 0.90 for int4, 0.4 - 0.6 % more than the fastest of all each time.  Bf16, 5 - 512 rows of 17 matrices: the kernel
+// chosen took 1.26 of what the fastest of all does on average, row-major 1.53, and with these takes 1.01.
 double waves_cost(const Linear& w, int M, size_t ws_bytes) {
-    return M >= 5 && w.kind != Quant::Bf16 && tile_major(w) ? pie_hip_gemm_waves_us(fmt_code(w.kind), M, w.N, w.K, w.group, ws_bytes, 0) : 1e30;
+    return M >= 5 && (w.kind == Quant::Bf16 || tile_major(w)) ? pie_hip_gemm_waves_us(fmt_code(w.kind), tile_major(w) ? 1 : 0, M, w.N, w.K, w.group, ws_bytes, 0) : 1e30;
 }
 double skinny_or_groups(const Linear& w, int M, size_t ws_bytes) { return in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M); }
 bool in_waves(const Linear& w, int M, size_t ws_bytes) {
     const double us = waves_cost(w, M, ws_bytes);
     if (us > 1e29) return false;
     if (M <= 128 && w.waves[M] >= 0) return w.waves[M] == 1;   // (measured at start-up)
-    return (M <= 8 ? 1.1 : 1.0) * us < skinny_or_groups(w, M, ws_bytes);   // (of few rows both are short)
+    return (M <= 8 && w.kind != Quant::Bf16 ? 1.1 : 1.0) * us < skinny_or_groups(w, M, ws_bytes);   // (of few rows both are short)
 }
 // Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
 // where they are estimated faster.
@@ -137,7 +145,7 @@ bool in_rows(const Linear& w, int M, size_t ws_bytes) {
     const double rows = rows_cost(w, M, ws_bytes);
     return rows < 1e29 && rows < pie_hip_gemm_mfma_us(fmt_code(w.kind), M, w.N, w.K, w.group, 1, ws_bytes);
 }
-// Microseconds of a quantised projection whose sums do not wait for the norm.
+// Microseconds of a projection whose sums do not wait for the norm.
 double apart_cost(const Linear& w, int M, size_t ws_bytes) {
     const int fmt = fmt_code(w.kind);
     double us = in_waves(w, M, ws_bytes) ? waves_cost(w, M, ws_bytes) : skinny_or_groups(w, M, ws_bytes);
@@ -146,15 +154,15 @@ double apart_cost(const Linear& w, int M, size_t ws_bytes) {
                                      static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes))});
     return us;
 }
-// Whether a quantised projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
+// Whether a projection back into the residual leaves its sums in shares of K, which the next norm's kernel adds up
 // (pie_hip_shares_rmsnorm), for 5 rows and more: int4 4096 x 14336 and the norm of 16 / 40 / 64 / 96 rows 18.3 / 23.3 / 25.4 / 30.5 us in two launches
 // without shares, 13.4 / 17.5 / 19.9 / 24.2 with them; 4096 x 4096 9.8 / 12.9 / 13.0 / 15.0 and 9.1 / 11.2 / 11.7 / 14.4.  (1e30: not taken, by the products' kernels or the norm's)
 double groups_shares_cost(const Linear& w, int M, size_t ws_bytes) {
     return w.kind == Quant::Int4b8 ? pie_hip_gemm_groups_shares_us(M, w.N, w.K, w.group, ws_bytes) : 1e30;
 }
-double waves_shares_cost(const Linear& w, int M, size_t ws_bytes) { return pie_hip_gemm_waves_us(fmt_code(w.kind), M, w.N, w.K, w.group, ws_bytes, 1); }
+double waves_shares_cost(const Linear& w, int M, size_t ws_bytes) { return pie_hip_gemm_waves_us(fmt_code(w.kind), 1, M, w.N, w.K, w.group, ws_bytes, 1); }
 double shares_cost(const Linear& w, int M, size_t ws_bytes) {
-    if (M < 5 || w.kind == Quant::Bf16 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return 1e30;
+    if (M < 5 || !tile_major(w) || w.N % 8 != 0 || w.N > 16384) return 1e30;
     return std::min(groups_shares_cost(w, M, ws_bytes), waves_shares_cost(w, M, ws_bytes));
 }
 bool in_shares(const Linear& w, int M, size_t ws_bytes) {
@@ -163,13 +171,16 @@ bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     if (M <= 128 && w.shares[M] >= 0) return w.shares[M] == 1;   // (measured at start-up)
     return us < apart_cost(w, M, ws_bytes);
 }
-// The tiled GEMM, up to 128 rows.
-double tiled_cost(const Linear& w, int M) { return 2.0 + w.K / 64 * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, (w.N + 127) / 128 / 512.0); }
+// The tiled GEMM, up to 128 rows (bf16 weights at most as fast as they stream: 24 - 77 rows of 28672 x 4096 53 - 56 us, of 32000 x 4096 58 - 70).
+double tiled_cost(const Linear& w, int M) {
+    const double us = 2.0 + w.K / 64 * (M <= 64 ? 0.60 : 0.68) * std::max(1.0, (w.N + 127) / 128 / 512.0);
+    return w.kind == Quant::Bf16 ? std::max(us, 2.6 + static_cast<double>(w.data_bytes()) / 4.6e6) : us;
+}
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
     const auto [p2, wpasses, wave_form, passes] = skinny_cost(w, M);
     const double waves = in_waves(w, M, ws_bytes) ? waves_cost(w, M, ws_bytes) : 1e30;   // (in the skinny GEMM's place)
-    const double skinny = std::min(w.kind == Quant::Int8 || w.kind == Quant::Fp8 ? passes_cost(w, M) : passes, waves);
+    const double skinny = std::min(w.kind != Quant::Int4b8 ? passes_cost(w, M) : passes, waves);
     const double data = static_cast<double>(w.data_bytes()), groups = groups_cost(w, M, ws_bytes);
     const int steps = w.K / 64;
     if (M > 128) {
@@ -202,6 +213,7 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const int shares = static_cast<int>(need / (static_cast<size_t>(M) * w.N * sizeof(float)));
         const int per = (steps + shares - 1) / shares;
         split = 15.0 + (per + 3) * (M <= 64 ? 1.06 : 1.36) * std::ceil(tiles * shares / 512.0);
+        if (w.kind == Quant::Bf16) split = std::max(split, 8.0 + data / 4.6e6);   // (24 / 64 rows of 32000 x 4096 62 - 66 / 73)
     }
     if (w.kind == Quant::Int4b8) {   // (blocks with fp32 group scales run in the skinny GEMM's place; up to 48 rows of wide outputs that is the wide GEMM's own form)
         if (std::min(waves, groups) < std::min(split, tiled))
@@ -294,8 +306,9 @@ bool linear_fused(const Linear& w, const uint16_t* act, const uint16_t* norm_w, 
                               : tuned == 4 ? GemmPath::Wide
                                            : pick_gemm(w, M, gemm_ws_bytes);   // (forced row limit, GEMV refusal)
         if (path == GemmPath::Skinny && in_waves(w, M, gemm_ws_bytes)) {
-            const int sv = pie_hip_gemm_waves_tiled(fmt, a, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, sbf, w.group, y, M, w.N, w.K, beta, swiglu, glu,
-                                                    gemm_ws, gemm_ws_bytes, s);
+            const int sv = w.data_tiled ? pie_hip_gemm_waves_tiled(fmt, a, w.data_tiled, w.scale_tiled ? w.scale_tiled : w.scale, sbf, w.group, y, M, w.N, w.K, beta,
+                                                                   swiglu, glu, gemm_ws, gemm_ws_bytes, s)
+                                        : pie_hip_gemm_waves_bf16(a, w.data, y, M, w.N, w.K, beta, swiglu, glu, gemm_ws, gemm_ws_bytes, s);
             if (sv == PIE_HIP_OK) return true;
             if (sv != PIE_HIP_ERR_UNSUPPORTED) PIE_KERNEL(sv);
         }

@@ -724,12 +724,12 @@ def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor
 
 def gemm_waves_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
                      workspace: Optional[torch.Tensor] = None, rule: Optional[Glu] = None) -> torch.Tensor:
-    """The GEMM over tile-major int4, int8 or fp8 weights in blocks whose waves take the steps of K in turn (up to 512 rows); with a
+    """The GEMM over tile-major weights (bf16 also row-major) in blocks whose waves take the steps of K in turn (up to 512 rows); with a
     workspace few blocks over a long K run in shares of K."""
     _dev(act, torch.bfloat16, "act")
     M, K = act.shape
-    if K != w.K or not w.kind.endswith("+tiled"):
-        raise KernelError("act K != weight K, or not tile-major weights")
+    if K != w.K or not (w.kind.endswith("+tiled") or w.kind == "bf16"):
+        raise KernelError("act K != weight K, or not weights in an order the kernel reads")
     n_out = w.N // 2 if epilogue == 1 else w.N
     if y is None:
         if beta:
@@ -738,8 +738,13 @@ def gemm_waves_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor]
     _dev(y, torch.bfloat16, "y")
     if tuple(y.shape) != (M, n_out):
         raise KernelError("y shape mismatch")
+    if w.kind == "bf16":
+        _check(kernels().pie_hip_gemm_waves_bf16(_ptr(act), _ptr(w.data), _ptr(y), M, w.N, K, beta, epilogue, None if rule is None else C.byref(rule), _ptr(workspace),
+                                                 C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream()),
+               "pie_hip_gemm_waves_bf16")
+        return y
     _check(kernels().pie_hip_gemm_waves_tiled(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale),
-                                              int(w.scale.dtype == torch.bfloat16), w.group_size, _ptr(y), M, w.N, K, beta, epilogue,
+                                              int(w.scale is not None and w.scale.dtype == torch.bfloat16), w.group_size, _ptr(y), M, w.N, K, beta, epilogue,
                                               None if rule is None else C.byref(rule), _ptr(workspace),
                                               C.c_size_t(0 if workspace is None else workspace.numel() * workspace.element_size()), _stream()),
            "pie_hip_gemm_waves_tiled")
@@ -754,24 +759,24 @@ def gemm_waves_shares_norm(act: torch.Tensor, w: WeightView, x: torch.Tensor, no
     if K != w.K or not w.kind.endswith("+tiled") or tuple(x.shape) != (M, w.N) or norm_weight.numel() != w.N:
         raise KernelError("shape mismatch, or not tile-major weights")
     shares, y = C.c_int(0), torch.empty_like(x)
-    _check(kernels().pie_hip_gemm_waves_shares(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale), int(w.scale.dtype == torch.bfloat16),
-                                               w.group_size, M, w.N, K, _ptr(workspace), C.c_size_t(workspace.numel() * workspace.element_size()),
+    _check(kernels().pie_hip_gemm_waves_shares(FMT[w.kind.removesuffix("+tiled")], _ptr(act), _ptr(w.data), _ptr(w.scale),
+                                               int(w.scale is not None and w.scale.dtype == torch.bfloat16), w.group_size, M, w.N, K, _ptr(workspace), C.c_size_t(workspace.numel() * workspace.element_size()),
                                                C.byref(shares), _stream()), "pie_hip_gemm_waves_shares")
     _check(kernels().pie_hip_shares_rmsnorm(_ptr(workspace), shares, _ptr(x), _ptr(norm_weight), _ptr(y), M, w.N, C.c_float(eps), _stream()),
            "pie_hip_shares_rmsnorm")
     return y, shares.value
 
 
-def gemm_waves_us(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 0, norm: bool = False) -> float:
+def gemm_waves_us(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 0, norm: bool = False, tiled: bool = True) -> float:
     lib = kernels()
     lib.pie_hip_gemm_waves_us.restype = C.c_float
-    return float(lib.pie_hip_gemm_waves_us(FMT[kind], M, N, K, group, C.c_size_t(workspace_bytes), int(norm)))
+    return float(lib.pie_hip_gemm_waves_us(FMT[kind], int(tiled), M, N, K, group, C.c_size_t(workspace_bytes), int(norm)))
 
 
-def gemm_waves_plan(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 0, norm: bool = False) -> Tuple[int, int, int]:
+def gemm_waves_plan(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 0, norm: bool = False, tiled: bool = True) -> Tuple[int, int, int]:
     """Rows and columns of a block and shares of K of `gemm_waves_tiled` (norm: of `gemm_waves_shares_norm`)."""
     rows, cols, shares = C.c_int(0), C.c_int(0), C.c_int(0)
-    _check(kernels().pie_hip_gemm_waves_plan(FMT[kind], M, N, K, group, C.c_size_t(workspace_bytes), int(norm), C.byref(rows), C.byref(cols), C.byref(shares)),
+    _check(kernels().pie_hip_gemm_waves_plan(FMT[kind], int(tiled), M, N, K, group, C.c_size_t(workspace_bytes), int(norm), C.byref(rows), C.byref(cols), C.byref(shares)),
            "pie_hip_gemm_waves_plan")
     return rows.value, cols.value, shares.value
 

@@ -1,4 +1,4 @@
-"""GPU parity: quantised weights in blocks whose waves take the steps of K in turn, against the exact sums in 64 bits and the kernels whose
+"""GPU parity: weights in blocks whose waves take the steps of K in turn, against the exact sums in 64 bits and the kernels whose
 epilogues they share."""
 import numpy as np
 import pytest
@@ -16,7 +16,24 @@ INT4 = {(5, 16, 1152): (16, 16, False), (15, 48, 384): (16, 16, False), (5, 16, 
         (5, 8208, 1152): (16, 64, False), (97, 16, 1152): (32, 16, False), (17, 4112, 1152): (32, 32, False), (161, 144, 4224): (32, 32, True), (32, 8208, 1152): (32, 64, False),
         (230, 16, 1152): (48, 32, False), (230, 16, 3200): (48, 32, True), (33, 12304, 1152): (48, 64, False), (300, 16, 1152): (64, 32, False),
         (300, 16, 2176): (64, 32, True), (97, 6160, 1152): (64, 64, False), (97, 2064, 8320): (64, 64, True), (5, 1024, 128): (16, 16, False)}
-CASES = [(kind, *shape) for kind, table in (("int8", ONE_BYTE), ("fp8", ONE_BYTE), ("int4b8", INT4)) for shape in table]
+BF16 = {(5, 16, 576): (16, 16, False), (15, 48, 192): (16, 16, False), (5, 16, 4160): (16, 16, True), (65, 1040, 576): (16, 32, False), (33, 272, 8256): (16, 32, True),
+        (33, 4112, 576): (16, 64, False), (97, 16, 576): (32, 16, False), (97, 16, 4160): (32, 16, True), (97, 1040, 576): (32, 32, False), (97, 2064, 576): (32, 64, False),
+        (230, 16, 576): (48, 32, False), (230, 16, 2112): (48, 32, True), (230, 2064, 576): (48, 64, False), (300, 16, 576): (64, 32, False), (300, 16, 2112): (64, 32, True),
+        (300, 2064, 576): (64, 64, False), (230, 2064, 1088): (80, 32, False), (230, 4112, 1088): (80, 64, False), (65, 2064, 8256): (80, 64, True), (5, 1024, 64): (16, 16, False)}
+BF16_ROWS = {(5, 16, 576): (16, 16, False), (15, 48, 192): (16, 16, False), (5, 16, 4160): (16, 16, True), (65, 1040, 576): (16, 32, False), (17, 528, 8256): (16, 32, True),
+             (33, 4112, 576): (16, 64, False), (97, 16, 576): (32, 16, False), (97, 16, 4160): (32, 16, True), (97, 1040, 576): (32, 32, False), (97, 2064, 576): (32, 64, False),
+             (17, 2064, 8256): (32, 64, True), (230, 16, 576): (48, 32, False), (230, 16, 2112): (48, 32, True), (130, 4112, 576): (48, 64, False), (300, 16, 576): (64, 32, False),
+             (300, 16, 2112): (64, 32, True), (300, 2064, 576): (64, 64, False), (230, 2064, 576): (80, 32, False), (300, 272, 8256): (80, 32, True),
+             (230, 4112, 576): (80, 64, False), (65, 2064, 8256): (80, 64, True), (5, 1024, 64): (16, 16, False)}
+TABLES = {"int8": ONE_BYTE, "fp8": ONE_BYTE, "int4b8": INT4, "bf16": BF16, "bf16 rows": BF16_ROWS}
+CASES = [(kind, *shape) for kind, table in TABLES.items() for shape in table]
+
+
+def stored(w, kind="bf16"):
+    """The weight in the order the kernel reads: the tile-major copy, or as it is."""
+    from pie_amd import ops
+
+    return w if kind == "bf16 rows" else ops.repack_mfma_tiles(w)
 
 
 def weight_and_sums(kind, M, N, K, seed, gpu, group=128, scale_type=None):
@@ -34,6 +51,11 @@ def weight_and_sums(kind, M, N, K, seed, gpu, group=128, scale_type=None):
         s = scale.double().repeat_interleave(group, dim=1)
         w, size = codes * s, (codes.abs() + 272.0) * s
         view = ops.WeightView("int4b8", data, scale, group, N, K)
+    elif kind.startswith("bf16"):
+        data = (0.03 * torch.randn(N, K, generator=g, device=gpu)).to(torch.bfloat16)
+        w = data.double()
+        size = w.abs()
+        view = ops.WeightView("bf16", data, None, 0, N, K)
     else:
         scale = (0.0005 + 0.001 * torch.rand(N, generator=g, device=gpu)).to(scale_type or torch.bfloat16)
         if kind == "int8":
@@ -52,10 +74,11 @@ def weight_and_sums(kind, M, N, K, seed, gpu, group=128, scale_type=None):
 def test_each_block_is_planned_where_it_is_tested(kind, M, N, K):
     from pie_amd import ops
 
-    rows, cols, shared = (INT4 if kind == "int4b8" else ONE_BYTE)[M, N, K]
-    got = ops.gemm_waves_plan(kind, M, N, K, 128, WORKSPACE)
+    rows, cols, shared = TABLES[kind][M, N, K]
+    kind, tiled = kind.split()[0], not kind.endswith("rows")
+    got = ops.gemm_waves_plan(kind, M, N, K, 128, WORKSPACE, tiled=tiled)
     assert got[:2] == (rows, cols) and (got[2] > 1) == shared
-    assert ops.gemm_waves_plan(kind, M, N, K, 128, 0)[2] == 1   # (no workspace: whole sums)
+    assert ops.gemm_waves_plan(kind, M, N, K, 128, 0, tiled=tiled)[2] == 1   # (no workspace: whole sums)
 
 
 @pytest.mark.gpu
@@ -65,9 +88,9 @@ def test_rows_in_blocks_of_waves(gpu, kind, M, N, K):
     import torch
     from pie_amd import ops
 
-    for scale_type in (torch.bfloat16,) if kind == "int4b8" else (torch.bfloat16, torch.float32):
+    for scale_type in (torch.bfloat16, torch.float32) if kind in ("int8", "fp8") else (torch.bfloat16,):
         act, w, ref, bound = weight_and_sums(kind, M, N, K, 910 + M, gpu, scale_type=scale_type)
-        t = ops.repack_mfma_tiles(w)
+        t = stored(w, kind)
         for work in (None, torch.full((WORKSPACE // 4,), float("nan"), device=gpu)):
             got = ops.gemm_waves_tiled(act, t, workspace=work).double()
             assert torch.isfinite(got).all() and ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + bound).all()
@@ -101,13 +124,13 @@ def test_groups_of_several_steps(gpu, group):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", ["int8", "fp8", "int4b8"])
+@pytest.mark.parametrize("kind", ["int8", "fp8", "int4b8", "bf16", "bf16 rows"])
 def test_as_close_to_the_exact_sums_as_the_passes(gpu, kind):
     import torch
     from pie_amd import ops
 
     act, w, ref, _ = weight_and_sums(kind, 40, 512, 4096, 940, gpu)
-    t, ws = ops.repack_mfma_tiles(w), torch.empty(WORKSPACE // 4, device=gpu)
+    t, ws = stored(w, kind), torch.empty(WORKSPACE // 4, device=gpu)
     err = lambda y: (y.double() - ref).abs().mean()  # noqa: E731
     passes = err(ops.gemm_skinny(act, t))
     assert err(ops.gemm_waves_tiled(act, t)) <= 1.02 * passes and err(ops.gemm_waves_tiled(act, t, workspace=ws)) <= 1.02 * passes
@@ -119,14 +142,16 @@ def test_refusals():
 
     assert ops.gemm_waves_us("int4b8", 32, 128, 256, 64) > 1e29 and ops.gemm_waves_us("int4b8", 32, 128, 192, 64) > 1e29
     assert ops.gemm_waves_us("int8", 32, 128, 96) > 1e29 and ops.gemm_waves_us("int8", 32, 120, 128) > 1e29
-    assert ops.gemm_waves_us("fp8", 513, 128, 128) > 1e29 and ops.gemm_waves_us("bf16", 32, 128, 128) > 1e29
+    assert ops.gemm_waves_us("fp8", 513, 128, 128) > 1e29 and ops.gemm_waves_us("fp8", 32, 128, 128, tiled=False) > 1e29
+    assert ops.gemm_waves_us("bf16", 32, 128, 96) > 1e29 and ops.gemm_waves_us("bf16", 32, 120, 128, tiled=False) > 1e29
     with pytest.raises(ops.KernelError):
         ops.gemm_waves_plan("int8", 600, 128, 128)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,M,hq,hk,d,K,shares", [("int4b8", 18, 4, 2, 16, 256, False), ("int4b8", 37, 32, 8, 128, 4096, True), ("int8", 65, 8, 2, 64, 448, False),
-                                                     ("int8", 24, 4, 1, 128, 8192, True), ("fp8", 131, 6, 2, 128, 1024, False)])
+                                                     ("int8", 24, 4, 1, 128, 8192, True), ("fp8", 131, 6, 2, 128, 1024, False),
+                                                     ("bf16", 77, 32, 8, 64, 2048, False), ("bf16", 19, 4, 2, 64, 8192, True)])
 def test_qkv_rope_epilogue_equals_projection_then_rope_kernel(gpu, oracle, kind, M, hq, hk, d, K, shares):
     import torch
     from pie_amd import ops
@@ -148,7 +173,8 @@ def test_qkv_rope_epilogue_equals_projection_then_rope_kernel(gpu, oracle, kind,
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind,M,N,K", [("int8", 5, 2048, 8192), ("fp8", 40, 528, 4160), ("int4b8", 17, 4096, 4096), ("int4b8", 64, 16384, 1024), ("int8", 130, 1024, 2112)])
+@pytest.mark.parametrize("kind,M,N,K", [("int8", 5, 2048, 8192), ("fp8", 40, 528, 4160), ("int4b8", 17, 4096, 4096), ("int4b8", 64, 16384, 1024), ("int8", 130, 1024, 2112), ("bf16", 40, 2048, 8192),
+                                          ("bf16", 9, 528, 4160)])
 def test_shares_that_meet_in_the_norm(gpu, kind, M, N, K):
     import torch
     from pie_amd import ops
