@@ -29,6 +29,8 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
     __bf16 b = static_cast<__bf16>(f);
     return __builtin_bit_cast(uint16_t, b);
 }
+// (as a conversion back, after which no signalling NaN can be left: a minimum takes it without one more instruction)
+__device__ __forceinline__ float round_bf16(float f) { return static_cast<float>(static_cast<__bf16>(f)); }
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     // one v_cvt_pk_bf16_f32 (round to nearest even, as the scalar conversion)
     typedef __bf16 bf16x2_pk_t __attribute__((ext_vector_type(2)));
@@ -327,7 +329,7 @@ constexpr PieHipGlu kPlainGlu = {nullptr, __builtin_inff(), 1.f, 0.f};
 template <bool F32 = false>
 __device__ __forceinline__ float glu_value(float g, float u, const PieHipGlu& r) {
     g = fminf(g, r.limit);
-    u = fminf(fmaxf(u, -r.limit), r.limit);
+    u = __builtin_amdgcn_fmed3f(u, -r.limit, r.limit);   // (a NaN becomes -limit, as of a maximum and a minimum)
     return (F32 ? g / (1.f + expf(-r.alpha * g)) : silu(g, r.alpha)) * (u + r.shift);
 }
 inline bool glu_ok(const PieHipGlu* r, int epilogue) { return !r || (epilogue == PIE_HIP_EPI_SWIGLU && r->limit >= 0.f); }

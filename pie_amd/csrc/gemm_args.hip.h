@@ -1,6 +1,8 @@
 // What the tiled GEMMs of large batches share: their arguments, and the launch of the wide form.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hip.h"
 
 namespace pie_hip {
@@ -50,23 +52,57 @@ __device__ __forceinline__ void to_lds(const unsigned char* from, u32x4_t* to) {
     __builtin_amdgcn_global_load_lds(from, PIE_LDS_PTR(to), 16, 0, 0);
 }
 
+// What a launch's rows become, so that a block asks once and not every store: gated pairs by the plain rule, by another, values as they are, onto a
+// residual; Any asks for itself (the pointwise functions).  With the questions in every unrolled store a block of 256 x 256 had 23000 instructions in 1900 basic
+// blocks, most of them run once and fetched for it.  256
+// such blocks with K of 1024, before / here: fp8 as they are 51.3 / 46.3 us, gated 50.8 / 48.3, int4 51.1 / 47.7 and 51.0 / 47.9; bf16, 128 columns, 25.7 / 24.1 and 25.2 / 24.4.
+// (Gated stores are bound by their instructions: 133 per four values before, 117 - 143 here.)
+enum class Out { Gated, GatedRule, Plain, Residual, Any };
+template <class Fn>
+__device__ __forceinline__ void by_output(const GemmArgs& a, Fn&& store) {
+    if (a.swiglu) {
+        if (!a.glu.bias && a.glu.limit == __builtin_inff() && a.glu.alpha == 1.f && a.glu.shift == 0.f) store(std::integral_constant<Out, Out::Gated>{});
+        else store(std::integral_constant<Out, Out::GatedRule>{});
+    } else if (a.pointwise) {
+        store(std::integral_constant<Out, Out::Any>{});
+    } else if (a.beta) {
+        store(std::integral_constant<Out, Out::Residual>{});
+    } else {
+        store(std::integral_constant<Out, Out::Plain>{});
+    }
+}
+template <Out O>
+__device__ __forceinline__ bool is_gated(const GemmArgs& a) { return O == Out::Any ? a.swiglu != 0 : O == Out::Gated || O == Out::GatedRule; }
+template <Out O>
+__device__ __forceinline__ bool is_residual(const GemmArgs& a) { return O == Out::Any ? a.beta != 0 : O == Out::Residual; }
+// (the plain rule's limit is opaque: knowing it, the compiler folds the clamp of u into one that makes a NaN plus infinity, not minus)
+template <Out O>
+__device__ __forceinline__ PieHipGlu rule_of(const GemmArgs& a) {
+    if constexpr (O != Out::Gated) return a.glu;
+    float limit = a.glu.limit;
+    asm volatile("" : "+s"(limit));
+    return PieHipGlu{nullptr, limit, 1.f, 0.f};
+}
+
 // The epilogue of row m, columns n .. n + 3 (those below N; n is a multiple of 4): SwiGLU over (gate, up) pairs rounded to
 // bf16 first, or a pointwise function and the residual.
+template <Out O = Out::Any>
 __device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, float* v) {
-    const int N = a.N, nout = a.swiglu ? N / 2 : N;
+    const int N = a.N, nout = is_gated<O>(a) ? N / 2 : N;
     const bool whole = N % 4 == 0 && a.aligned;   // one 8- (SwiGLU: 4-) byte store
-    if (a.swiglu) {
+    if (is_gated<O>(a)) {
+        const PieHipGlu rule = rule_of<O>(a);
         uint16_t o[2];
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             float g = v[2 * r], u = v[2 * r + 1];
-            if (a.glu.bias) {
-                g += a.glu.bias[min(n + 2 * r, N - 1)];
-                u += a.glu.bias[min(n + 2 * r + 1, N - 1)];
+            if (rule.bias) {
+                g += rule.bias[min(n + 2 * r, N - 1)];
+                u += rule.bias[min(n + 2 * r + 1, N - 1)];
             }
-            g = bf16_bits_to_f32(f32_to_bf16_bits(g));
-            u = bf16_bits_to_f32(f32_to_bf16_bits(u));
-            o[r] = f32_to_bf16_bits(glu_value(g, u, a.glu));
+            g = round_bf16(g);
+            u = round_bf16(u);
+            o[r] = f32_to_bf16_bits(glu_value(g, u, rule));
         }
         uint16_t* p = a.y + static_cast<size_t>(m) * nout + n / 2;
         if (whole) {
@@ -78,10 +114,12 @@ __device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, floa
         return;
     }
     uint16_t* p = a.y + static_cast<size_t>(m) * nout + n;
+    if constexpr (O == Out::Any) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = epilogue_pointwise<true>(v[r], a.pointwise);
+        for (int r = 0; r < 4; ++r) v[r] = epilogue_pointwise<true>(v[r], a.pointwise);
+    }
     if (whole) {
-        if (a.beta) {
+        if (is_residual<O>(a)) {
             const u32x2_t old = *reinterpret_cast<const u32x2_t*>(p);
             v[0] += bf16_lo(old.x);
             v[1] += bf16_hi(old.x);
@@ -91,7 +129,7 @@ __device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, floa
         *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     } else {
         for (int r = 0; r < 4 && n + r < N; ++r) {
-            if (a.beta) v[r] += bf16_bits_to_f32(p[r]);
+            if (is_residual<O>(a)) v[r] += bf16_bits_to_f32(p[r]);
             p[r] = f32_to_bf16_bits(v[r]);
         }
     }
@@ -101,9 +139,17 @@ inline int stores_lines(const uint16_t* y, int N) { return N % 32 == 0 && reinte
 // The same for columns n .. n + 3 and n + 16 .. n + 19, n = 32 k + 4 q with q the lane's sixteenth of the wave (a.lines): neighbouring
 // sixteenths swap half of their values, the even ones end with eight columns of the first tile and the odd ones of the second, so that
 // a store is 16 bytes and a row's four lanes fill 64 (SwiGLU: 8 and 32).
-__device__ __forceinline__ void store_pair(const GemmArgs& a, int m, int n, int q, float* v0, float* v1) {
-    const int nout = a.swiglu ? a.N / 2 : a.N, at = q & 1 ? n + 12 : n;
-    if (a.swiglu) {
+// Where store_pair's row m goes; sixteen rows on it is `row_step` values further.
+template <Out O>
+__device__ __forceinline__ uint16_t* pair_place(const GemmArgs& a, int m, int n, int q, int& row_step) {
+    const int nout = is_gated<O>(a) ? a.N / 2 : a.N, at = q & 1 ? n + 12 : n;
+    row_step = 16 * nout;
+    return a.y + static_cast<size_t>(m) * nout + (is_gated<O>(a) ? at / 2 : at);
+}
+template <Out O = Out::Any>
+__device__ __forceinline__ void store_pair(const GemmArgs& a, uint16_t* to, int n, float* v0, float* v1) {
+    if (is_gated<O>(a)) {
+        const PieHipGlu rule = rule_of<O>(a);
         uint32_t o[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -112,27 +158,29 @@ __device__ __forceinline__ void store_pair(const GemmArgs& a, int m, int n, int 
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 float g = v[2 * r], u = v[2 * r + 1];
-                if (a.glu.bias) {
-                    g += a.glu.bias[n + 16 * i + 2 * r];
-                    u += a.glu.bias[n + 16 * i + 2 * r + 1];
+                if (rule.bias) {
+                    g += rule.bias[n + 16 * i + 2 * r];
+                    u += rule.bias[n + 16 * i + 2 * r + 1];
                 }
-                g = bf16_bits_to_f32(f32_to_bf16_bits(g));
-                u = bf16_bits_to_f32(f32_to_bf16_bits(u));
-                w[r] = glu_value(g, u, a.glu);
+                g = round_bf16(g);
+                u = round_bf16(u);
+                w[r] = glu_value(g, u, rule);
             }
             o[i] = pack_bf16x2(w[0], w[1]);
         }
         const auto s = __builtin_amdgcn_permlane16_swap(o[0], o[1], false, false);
-        *reinterpret_cast<u32x2_t*>(a.y + static_cast<size_t>(m) * nout + at / 2) = u32x2_t{s[0], s[1]};
+        *reinterpret_cast<u32x2_t*>(to) = u32x2_t{s[0], s[1]};
         return;
     }
-    u32x4_t* p = reinterpret_cast<u32x4_t*>(a.y + static_cast<size_t>(m) * nout + at);
+    u32x4_t* p = reinterpret_cast<u32x4_t*>(to);
+    if constexpr (O == Out::Any) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        v0[r] = epilogue_pointwise<true>(v0[r], a.pointwise);
-        v1[r] = epilogue_pointwise<true>(v1[r], a.pointwise);
+        for (int r = 0; r < 4; ++r) {
+            v0[r] = epilogue_pointwise<true>(v0[r], a.pointwise);
+            v1[r] = epilogue_pointwise<true>(v1[r], a.pointwise);
+        }
     }
-    if (a.beta) {
+    if (is_residual<O>(a)) {
         const u32x4_t old = *p;
         const auto x = __builtin_amdgcn_permlane16_swap(old[0], old[2], false, false), y = __builtin_amdgcn_permlane16_swap(old[1], old[3], false, false);
         v0[0] += bf16_lo(x[0]);

@@ -190,17 +190,20 @@ __global__ __launch_bounds__(256, 2) void gemm_groups_kernel(const GemmArgs a, c
     if (a.lines && !a.partial && !rot.table) {
         const int n = tile0 * 16 + 4 * q;
         if (n >= N) return;
+        by_output(a, [&](auto out) __attribute__((always_inline)) {
+            int row_step;
+            uint16_t* to = pair_place<decltype(out)::value>(a, m0 + j, n, q, row_step);
 #pragma unroll
-        for (int t = 0; t < RT; ++t) {
-            const int m = m0 + t * 16 + j;
-            if (m >= M) continue;
-            float v[2][4];
+            for (int t = 0; t < RT; ++t, to += row_step) {
+                if (m0 + t * 16 + j >= M) break;   // (no later row is one either)
+                float v[2][4];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[i][r] = acc[t][i][r];
-            store_pair(a, m, n, q, v[0], v[1]);
-        }
+                    for (int r = 0; r < 4; ++r) v[i][r] = acc[t][i][r];
+                store_pair<decltype(out)::value>(a, to, n, v[0], v[1]);
+            }
+        });
         return;
     }
 #pragma unroll

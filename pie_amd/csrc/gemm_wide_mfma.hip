@@ -328,60 +328,64 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void gemm_wide_kernel(const GemmA
     __builtin_amdgcn_s_waitcnt(0x0070);   // (transfers past the last step land before the block ends)
 
     // ---- epilogue: a lane holds four neighbouring columns of one row per tile ----
-    if (a.lines && !a.partial) {
+    float rs[4][4];   // (all asked for at once)
+    if constexpr (F::kRowScale) {
 #pragma unroll
-        for (int nt = 0; nt < 4; nt += 2) {
-            const int n = n0 + wn * 64 + nt * 16 + 4 * q;
-            if (n >= N) continue;
-            float rs[2][4];
-            if constexpr (F::kRowScale) {
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        rs[i][r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[n + 16 * i + r])
-                                                   : reinterpret_cast<const float*>(a.scale)[n + 16 * i + r];
-            }
-#pragma unroll
-            for (int t = 0; t < 4 * AH; ++t) {
-                const int m = m0 + wm * 64 * AH + t * 16 + j;
-                if (m >= M) continue;
-                float v[2][4];
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[i][r] = F::kRowScale ? acc[t][nt + i][r] * rs[i][r] : acc[t][nt + i][r];
-                store_pair(a, m, n, q, v[0], v[1]);
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        const int n = n0 + wn * 64 + nt * 16 + 4 * q;
-        if (n >= N) continue;
-        float rs[4];
-        if constexpr (F::kRowScale) {
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int c = min(n + r, N - 1);
-                rs[r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[c])
-                                        : reinterpret_cast<const float*>(a.scale)[c];
+                const int c = min(n0 + wn * 64 + nt * 16 + 4 * q + r, N - 1);
+                rs[nt][r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[c]) : reinterpret_cast<const float*>(a.scale)[c];
+            }
+        PIE_FENCE();
+    }
+    auto value = [&](int t, int nt, int r) __attribute__((always_inline)) { return F::kRowScale ? acc[t][nt][r] * rs[nt][r] : acc[t][nt][r]; };
+    const int row0 = m0 + wm * 64 * AH + j, col0 = n0 + wn * 64 + 4 * q;
+    if (a.partial) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            const int n = col0 + nt * 16;
+            if (n >= N) continue;
+#pragma unroll
+            for (int t = 0; t < 4 * AH; ++t) {
+                const int m = row0 + t * 16;
+                if (m >= M) continue;
+                float* p = a.partial + (static_cast<size_t>(blockIdx.z) * M + m) * N + n;
+                if (N % 4 == 0) *reinterpret_cast<f32x4_t*>(p) = f32x4_t{value(t, nt, 0), value(t, nt, 1), value(t, nt, 2), value(t, nt, 3)};
+                else
+                    for (int r = 0; r < 4 && n + r < N; ++r) p[r] = value(t, nt, r);
             }
         }
+    } else if (a.lines) {
+        by_output(a, [&](auto out) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < 4 * AH; ++t) {
-            const int m = m0 + wm * 64 * AH + t * 16 + j;
-            if (m >= M) continue;
-            float v[4];
+            for (int nt = 0; nt < 4; nt += 2) {
+                const int n = col0 + nt * 16;
+                if (n >= N) continue;
+                int row_step;
+                uint16_t* to = pair_place<decltype(out)::value>(a, row0, n, q, row_step);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = F::kRowScale ? acc[t][nt][r] * rs[r] : acc[t][nt][r];
-            if (a.partial) {
-                float* p = a.partial + (static_cast<size_t>(blockIdx.z) * M + m) * N + n;
-                if (N % 4 == 0) *reinterpret_cast<f32x4_t*>(p) = f32x4_t{v[0], v[1], v[2], v[3]};
-                else
-                    for (int r = 0; r < 4 && n + r < N; ++r) p[r] = v[r];
-            } else {
+                for (int t = 0; t < 4 * AH; ++t, to += row_step) {
+                    if (row0 + t * 16 >= M) break;   // (no later row is one either)
+                    float v[2][4];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) v[i][r] = value(t, nt + i, r);
+                    store_pair<decltype(out)::value>(a, to, n, v[0], v[1]);
+                }
+            }
+        });
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            const int n = col0 + nt * 16;
+            if (n >= N) continue;
+#pragma unroll
+            for (int t = 0; t < 4 * AH; ++t) {
+                const int m = row0 + t * 16;
+                if (m >= M) continue;
+                float v[4] = {value(t, nt, 0), value(t, nt, 1), value(t, nt, 2), value(t, nt, 3)};
                 wide_store(a, m, n, v);
             }
         }
@@ -578,17 +582,20 @@ __global__ __launch_bounds__(256 * KP, S == 3 ? (RT == 2 ? 6 : 3) : 2) void gemm
                 for (int r = 0; r < 4; ++r)
                     rs[i][r] = a.scale_is_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(scale)[n + 16 * i + r])
                                                : reinterpret_cast<const float*>(scale)[n + 16 * i + r];
+            by_output(a, [&](auto out) __attribute__((always_inline)) {
+                int row_step;
+                uint16_t* to = pair_place<decltype(out)::value>(a, m0 + j, n, q, row_step);
 #pragma unroll
-            for (int t = 0; t < RT; ++t) {
-                const int m = m0 + t * 16 + j;
-                if (m >= M) continue;
-                float v[2][4];
+                for (int t = 0; t < RT; ++t, to += row_step) {
+                    if (m0 + t * 16 + j >= M) break;   // (no later row is one either)
+                    float v[2][4];
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                    for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[i][r] = acc[t][i][r] * rs[i][r];
-                store_pair(a, m, n, q, v[0], v[1]);
-            }
+                        for (int r = 0; r < 4; ++r) v[i][r] = acc[t][i][r] * rs[i][r];
+                    store_pair<decltype(out)::value>(a, to, n, v[0], v[1]);
+                }
+            });
             return;
         }
 #pragma unroll

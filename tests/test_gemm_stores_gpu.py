@@ -148,3 +148,27 @@ def test_blocks_of_routes(gpu, kind, height, counts, N):
 
         assert torch.equal(run(N, 0), sums.bfloat16())
         assert torch.equal(run(N // 2, 1), ops.glu_f32(sums.bfloat16().float().contiguous(), ops.glu()).bfloat16())
+
+
+@pytest.mark.parametrize("kind", ["int4b8", "fp8", "bf16"])
+def test_sums_that_are_no_numbers(gpu, kind):
+    """A NaN is the limit as a gate and minus the limit as a factor; infinities are clamped; both kinds of stores agree."""
+    import torch
+    from pie_amd import ops
+
+    M, N, K = 257, 288, 512
+    act, w, sums = exact_problem(gpu, kind, M, N, K, 980)
+    act, sums = act.clone(), sums.clone()
+    act[3], act[200, 5], act[130] = float("nan"), float("nan"), 3e38   # (the last: sums past the range of bf16, or of fp32)
+    sums[3] = sums[200] = float("nan")
+    for rule, gate, up in ((ops.glu(), float("inf"), float("-inf")), (ops.glu(**RULES), 7.0, -7.0)):
+        got = []
+        for offset in (0, 4):
+            y = torch.empty(M * N // 2 + 8, device=gpu, dtype=torch.bfloat16)[offset:offset + M * N // 2].view(M, N // 2)
+            got.append(ops.gemm_mfma_tiled(act, w, y=y, epilogue=1, rule=rule).clone())
+        assert torch.equal(got[0].isnan(), got[1].isnan()) and torch.equal(got[0].nan_to_num(), got[1].nan_to_num())
+        pair = torch.tensor([[gate, up]], device=gpu)
+        want = ops.glu_f32(pair, rule).bfloat16()
+        assert torch.equal(got[0][3], want.expand(1, N // 2)[0]) and torch.equal(got[0][200], want.expand(1, N // 2)[0])
+        rest = [r for r in range(M) if r not in (3, 130, 200)]
+        assert torch.equal(got[0][rest], ops.glu_f32(sums[rest].bfloat16().float().contiguous(), rule).bfloat16())
