@@ -478,6 +478,7 @@ __global__ __launch_bounds__(256) void moe_topk_shares_kernel(const float* __res
 
 // One block: rank of every route inside its expert, expert offsets, sorted positions.  The first `shared` routes of
 // every token are experts 0 .. shared - 1: their ranks are the tokens.
+template <bool PROMPTS>   // more routes than threads may come
 __device__ __forceinline__ void sort_routes(const int32_t* topk_idx, int32_t* __restrict__ expert_offsets,
                                             int32_t* __restrict__ route_token, int32_t* __restrict__ route_pos, int N, int E,
                                             int K, int shared = 0) {
@@ -487,10 +488,15 @@ __device__ __forceinline__ void sort_routes(const int32_t* topk_idx, int32_t* __
     for (int e = tid; e < E; e += kRouteThreads) cnt[e] = e < shared ? N : 0;
     __syncthreads();
     const int R = N * K;
-    // a prompt's routes stay in registers, their loads in flight together (10552 routes of 1319 tokens: read, counted and
-    // read again one at a time the sort took 15.7 us, so 9.9)
-    constexpr int kKept = 16;
-    const bool kept = R > kRouteThreads && R <= kKept * kRouteThreads;   // (one route per thread: nothing to overlap, 4.6 us either way)
+    // A prompt's routes stay in registers, their loads in flight together, and the tokens of the sorted places meet in LDS, from where they leave in whole lines.
+    // What bounds it: one CU's issue and address unit.  10552 routes of 1319 tokens read, counted and read again one at a time took 15.7 us, kept in registers 9.9; 9896 of 1237 tokens,
+    // kept, with a scattered store and two divisions by K a route 9.2, so 6.9.  (A launch that does next to nothing shows 4.6.)
+    constexpr int kKept = PROMPTS ? 16 : 1;
+    __shared__ uint16_t sorted[PROMPTS ? kKept * kRouteThreads : 1];
+    const bool kept = PROMPTS && R > kRouteThreads && R <= kKept * kRouteThreads;   // (one route per thread: nothing to overlap, 4.6 us either way)
+    const float per_token = 1.f / static_cast<float>(K);
+    // r / K for r < 2^14: the quotient of r + 1/2 is at least 1 / 2K off a whole number, its error at most 2^-23 of it
+    auto token_of = [&](int r) { return static_cast<int>((static_cast<float>(r) + 0.5f) * per_token); };
     int expert[kKept], rank[kKept];
     if (kept) {
 #pragma unroll
@@ -500,8 +506,8 @@ __device__ __forceinline__ void sort_routes(const int32_t* topk_idx, int32_t* __
         }
 #pragma unroll
         for (int i = 0; i < kKept; ++i) {
-            const int r = tid + i * kRouteThreads;
-            if (r < R) rank[i] = r % K < shared ? r / K : atomicAdd(&cnt[expert[i]], 1);
+            const int r = tid + i * kRouteThreads, t = token_of(r);
+            if (r < R) rank[i] = r - t * K < shared ? t : atomicAdd(&cnt[expert[i]], 1);
         }
     } else {
         for (int r = tid; r < R; r += kRouteThreads) route_pos[r] = r % K < shared ? r / K : atomicAdd(&cnt[topk_idx[r]], 1);
@@ -540,9 +546,11 @@ __device__ __forceinline__ void sort_routes(const int32_t* topk_idx, int32_t* __
             if (r < R) {
                 const int pos = base[expert[i]] + rank[i];
                 route_pos[r] = pos;
-                route_token[pos] = r / K;
+                sorted[pos] = static_cast<uint16_t>(token_of(r));
             }
         }
+        __syncthreads();
+        for (int p = tid; p < R; p += kRouteThreads) route_token[p] = sorted[p];
         return;
     }
     for (int r = tid; r < R; r += kRouteThreads) {
@@ -554,7 +562,7 @@ __device__ __forceinline__ void sort_routes(const int32_t* topk_idx, int32_t* __
 __global__ __launch_bounds__(kRouteThreads) void moe_sort_kernel(
     const int32_t* __restrict__ topk_idx, int32_t* __restrict__ expert_offsets,
     int32_t* __restrict__ route_token, int32_t* __restrict__ route_pos, int N, int E, int K, int shared) {
-    sort_routes(topk_idx, expert_offsets, route_token, route_pos, N, E, K, shared);
+    sort_routes<true>(topk_idx, expert_offsets, route_token, route_pos, N, E, K, shared);
 }
 // The choice and the sort in one launch, a wave per token.  us with the logits of 2048 values, in one launch / in two: 1 token of 128 experts 8.9 / 10.3, 16 10.9 / 11.5; 4
 // of 256 11.7 / 13.2, but 16 14.5 / 13.6: the sixteen waves share four SIMDs, and a choice is the longer the more experts there are.
@@ -566,7 +574,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_shares_kernel(const f
     const int t = threadIdx.x / kWave;
     if (t < N) choose_from_shares(part, shares, logits_out, topk_idx, topk_w, N, E, K, renorm, t, threadIdx.x & (kWave - 1));
     __syncthreads();   // (a block's stores are seen by its own threads after the barrier)
-    sort_routes(topk_idx, expert_offsets, route_token, route_pos, N, E, K);
+    sort_routes<false>(topk_idx, expert_offsets, route_token, route_pos, N, E, K);
 }
 
 // fp32 logits and groups of experts: one wave per token, four to a block.
@@ -594,7 +602,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_groups_kernel(const f
         topk_of_token([&](int e) { return row[e]; }, lane, t, topk_idx, topk_w, E, K, 1, groups, best[t]);
     }
     __syncthreads();   // (a block's stores are seen by its own threads after the barrier)
-    sort_routes(topk_idx, expert_offsets, route_token, route_pos, N, E, K);
+    sort_routes<false>(topk_idx, expert_offsets, route_token, route_pos, N, E, K);
 }
 
 // Logistic scores: one wave chooses a token's `top` experts by score + correction; `shared` experts that every
@@ -668,7 +676,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_corrected_kernel(cons
     const int lane = threadIdx.x & (kWave - 1), t = threadIdx.x / kWave;
     if (t < N) corrected_of_token(r, lane, t, topk_idx, topk_w);
     __syncthreads();   // (a block's stores are seen by its own threads after the barrier)
-    sort_routes(topk_idx, expert_offsets, route_token, route_pos, N, r.E + r.shared, r.top + r.shared, r.shared);
+    sort_routes<false>(topk_idx, expert_offsets, route_token, route_pos, N, r.E + r.shared, r.top + r.shared, r.shared);
 }
 
 __global__ __launch_bounds__(256) void moe_combine_kernel(

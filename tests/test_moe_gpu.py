@@ -123,6 +123,27 @@ def test_router_in_shares_of_k(gpu, oracle, T, H, E, K, planes):
             ops.moe_router_route(dev(np.ascontiguousarray(bad[0]), gpu, torch.bfloat16), dev(np.ascontiguousarray(bad[1]), gpu, torch.bfloat16), K, True, bad[2])
 
 
+@pytest.mark.parametrize("T,E,K,shared", [(128, 128, 8, 0), (129, 128, 8, 0), (1025, 1, 1, 0), (147, 64, 7, 0), (2048, 128, 8, 0), (2049, 128, 8, 0),
+                                          (1024, 512, 16, 0), (5461, 6, 3, 0), (256, 300, 61, 3), (257, 300, 61, 3), (93, 40, 10, 1)])
+def test_sort_of_many_routes(gpu, T, E, K, shared):
+    """Routes around 1024 (one per thread) and 16384 (sixteen, kept in registers and sorted in LDS), top_k a power of two or not, with shared experts: the
+    places are a permutation inside the experts' ranges and each place names its route's token."""
+    import torch
+    from pie_amd import ops
+
+    rng = np.random.default_rng(570 + T + E)
+    if shared:
+        lg = torch.from_numpy(rng.standard_normal((T, E + 1)).astype(np.float32)).to(gpu)
+        idx, _, offs, rtok, rpos = ops.moe_route_corrected(lg, torch.zeros(E, device=gpu), K, shared)
+    else:
+        idx, _, offs, rtok, rpos = ops.moe_route(torch.from_numpy(rng.standard_normal((T, E)).astype(np.float32)).to(gpu, torch.bfloat16), K)
+    idx, offs, rtok, rpos = (t.cpu().numpy().reshape(-1) for t in (idx, offs, rtok, rpos))
+    R = T * (K + shared)
+    assert np.array_equal(offs, np.concatenate([[0], np.cumsum(np.bincount(idx, minlength=E + shared))]))
+    assert np.array_equal(np.sort(rpos), np.arange(R)) and np.array_equal(rtok[rpos], np.arange(R) // (K + shared))
+    assert np.all(rpos >= offs[idx]) and np.all(rpos < offs[idx + 1])
+
+
 @pytest.mark.parametrize("T,K,H", [(64, 8, 2048), (3, 2, 512), (130, 6, 8192)])
 def test_combine_with_the_next_norm_equals_the_two_launches(gpu, oracle, T, K, H):
     import torch
