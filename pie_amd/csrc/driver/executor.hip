@@ -1515,7 +1515,7 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
     return model_route(w, M, false, workspace_bytes);
 }
 
-// And in which form that kernel runs, by what a measurement said (0 or 1; -1: by estimate): bit 0 int4 rows in blocks that scale groups in fp32 (in the skinny GEMM's place), bit 1 an int4
+// And in which form that kernel runs, by what a measurement said (0 or 1; -1: by estimate): bit 0 int4 rows in blocks that scale groups in fp32 (in the skinny GEMM's place), bit 1 a
 // projection into the residual in shares of K that meet in the norm's kernel, bit 2 one-byte rows in blocks of 32 to 128 (in the wide GEMM's place), bit 3 rows in
 // blocks whose waves take the steps of K in turn (in the skinny GEMM's place).
 extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, int K, int measured_groups, int measured_shares,

@@ -490,7 +490,7 @@ __device__ __forceinline__ void sort_routes(const int32_t* topk_idx, int32_t* __
     const int R = N * K;
     // A prompt's routes stay in registers, their loads in flight together, and the tokens of the sorted places meet in LDS, from where they leave in whole lines.
     // What bounds it: one CU's issue and address unit.  10552 routes of 1319 tokens read, counted and read again one at a time took 15.7 us, kept in registers 9.9; 9896 of 1237 tokens,
-    // kept, with a scattered store and two divisions by K a route 9.2, so 6.9.  (A launch that does next to nothing shows 4.6.)
+    // kept, with a scattered store and two divisions by K a route 9.2, so 6.3.  (A launch that does next to nothing shows 4.6.)
     constexpr int kKept = PROMPTS ? 16 : 1;
     __shared__ uint16_t sorted[PROMPTS ? kKept * kRouteThreads : 1];
     const bool kept = PROMPTS && R > kRouteThreads && R <= kKept * kRouteThreads;   // (one route per thread: nothing to overlap, 4.6 us either way)
