@@ -329,7 +329,9 @@ constexpr PieHipGlu kPlainGlu = {nullptr, __builtin_inff(), 1.f, 0.f};
 template <bool F32 = false>
 __device__ __forceinline__ float glu_value(float g, float u, const PieHipGlu& r) {
     g = fminf(g, r.limit);
-    u = __builtin_amdgcn_fmed3f(u, -r.limit, r.limit);   // (a NaN becomes -limit, as of a maximum and a minimum)
+    // A NaN becomes -limit.  The median makes that of a quiet NaN only, and sums rounded to bf16 hold no other; fp32 values out of memory may.
+    if constexpr (F32) u = fminf(fmaxf(u, -r.limit), r.limit);
+    else u = __builtin_amdgcn_fmed3f(u, -r.limit, r.limit);
     return (F32 ? g / (1.f + expf(-r.alpha * g)) : silu(g, r.alpha)) * (u + r.shift);
 }
 inline bool glu_ok(const PieHipGlu* r, int epilogue) { return !r || (epilogue == PIE_HIP_EPI_SWIGLU && r->limit >= 0.f); }

@@ -155,6 +155,20 @@ def test_silu_of_every_bf16_gate_is_that_of_expf_and_the_division(gpu, alpha):
     assert there.sum() > 65000 and torch.equal(got[there].view(torch.int32), want[there].view(torch.int32))
 
 
+@pytest.mark.parametrize("nan", [0x7F800001, 0x7FC00000, 0x7FFFFFFF, 0xFF800001, 0xFFC00000])
+def test_a_factor_that_is_no_number_is_minus_the_limit(gpu, nan):
+    """Quiet NaNs and signalling ones, as memory may hold them; as a gate they are the limit."""
+    import torch
+    from pie_amd import ops
+
+    one = 0x3F800000
+    x = dev(np.array([[one, nan], [nan, one]], np.uint32).view(np.int32), gpu).view(torch.float32)
+    for limit in (float("inf"), 7.0):
+        rule = ops.glu(limit=limit, alpha=1.702, shift=1.0)
+        want = ops.glu_f32(torch.tensor([[1.0, -limit], [limit, 1.0]], device=gpu), rule)
+        assert torch.equal(ops.glu_f32(x, rule), want), limit
+
+
 def test_argmax_ties_nan_and_vocab(gpu, oracle):
     import torch
     from pie_amd import ops
