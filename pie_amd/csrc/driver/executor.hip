@@ -131,9 +131,7 @@ double waves_cost(const Linear& w, int M, size_t ws_bytes) {
 double skinny_or_groups(const Linear& w, int M, size_t ws_bytes) { return in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M); }
 bool in_waves(const Linear& w, int M, size_t ws_bytes) {
     const double us = waves_cost(w, M, ws_bytes);
-    if (us > 1e29) return false;
-    if (M <= 128 && w.waves[M] >= 0) return w.waves[M] == 1;   // (measured at start-up)
-    return (M <= 8 && w.kind != Quant::Bf16 ? 1.1 : 1.0) * us < skinny_or_groups(w, M, ws_bytes);   // (of few rows both are short)
+    return us < 1e29 && (M <= 8 && w.kind != Quant::Bf16 ? 1.1 : 1.0) * us < skinny_or_groups(w, M, ws_bytes);   // (of few rows both are short)
 }
 // Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
 // where they are estimated faster.
@@ -170,6 +168,21 @@ bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     if (us > 1e29) return false;
     if (M <= 128 && w.shares[M] >= 0) return w.shares[M] == 1;   // (measured at start-up)
     return us < apart_cost(w, M, ws_bytes);
+}
+bool close(double a, double b) { return std::max(a, b) < 1.2 * std::min(a, b); }
+// Whether a start times the skinny GEMM's passes against the blocks that scale groups: estimates less than a fifth apart.
+bool measures_groups(const Linear& w, int M, size_t ws_bytes) {
+    const double groups = groups_cost(w, M, ws_bytes), passes = passes_cost(w, M);
+    return groups < 1e29 && close(groups, passes);
+}
+// Likewise shares that meet in the norm's kernel against a product and the norm, where blocks that scale groups make the shares.  Blocks whose waves take the steps in
+// turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.2 % on average to the faster of a pair's smallest times (at most 8 %), less than the tenth a
+// measurement needs to overrule an estimate, and of 177 pairs with shares 2 % (12 %).  Timed, they differed from start to start, and with them the
+// kernels' rounding: 40 of the 528 measured row counts in eight starts of each driver, 8 so (19 before there were such blocks).
+bool measures_shares(const Linear& w, int M, size_t ws_bytes, bool routed_as_estimated) {
+    const double us = groups_shares_cost(w, M, ws_bytes);
+    return shares_cost(w, M, ws_bytes) < 1e29 && us < 1e29 && us <= waves_shares_cost(w, M, ws_bytes) && !in_waves(w, M, ws_bytes) &&
+           (!routed_as_estimated || close(us, apart_cost(w, M, ws_bytes)));
 }
 // The tiled GEMM, up to 128 rows (bf16 weights at most as fast as they stream: 24 - 77 rows of 28672 x 4096 53 - 56 us, of 32000 x 4096 58 - 70).
 double tiled_cost(const Linear& w, int M) {
@@ -574,8 +587,6 @@ void Executor::tune_linears() {
     // half a microsecond): candidates that tie keep the model's kernel, so that timing noise
     // does not change which kernel — and with it which rounding — a restart gets.
     auto clearly = [](double us, double than) { return us < 0.9 * than && us + 0.5 < than; };
-    // (int4 forms that the estimates put a fifth apart are not measured: all of them take 55 ms of an 8B driver's start-up, so 20)
-    auto close = [](double a, double b) { return std::max(a, b) < 1.2 * std::min(a, b); };
     const int ladder[] = {2, 3, 4, 17, 24, 32, 33, 40, 48, 56, 64, 65, 72, 80, 88, 96, 97, 104, 112, 120, 128};
     for (const Role& r : roles) {
         const Linear& l0 = model_.layers[0].*(r.lin);
@@ -603,7 +614,7 @@ void Executor::tune_linears() {
             double skinny_t = 1e30;
             if (groups_cost(l0, M, gemm_ws_bytes_) < 1e29) {
                 int form = in_groups(l0, M, gemm_ws_bytes_) ? 1 : 0;
-                if (close(groups_cost(l0, M, gemm_ws_bytes_), passes_cost(l0, M))) {
+                if (measures_groups(l0, M, gemm_ws_bytes_)) {
                     double us[2];
                     for (int f = 0; f < 2; ++f) {
                         set(&Linear::groups, f, M);
@@ -613,22 +624,6 @@ void Executor::tune_linears() {
                     skinny_t = us[form];
                 }
                 set(&Linear::groups, form, lo);
-            }
-            // likewise that or the blocks whose waves take the steps in turn
-            if (waves_cost(l0, M, gemm_ws_bytes_) < 1e29) {
-                int form = in_waves(l0, M, gemm_ws_bytes_) ? 1 : 0;
-                if (close(waves_cost(l0, M, gemm_ws_bytes_), skinny_or_groups(l0, M, gemm_ws_bytes_))) {
-                    double us[2];
-                    for (int f = 0; f < 2; ++f) {
-                        set(&Linear::waves, f, M);
-                        us[f] = time_route(r, M, 1);
-                    }
-                    if (clearly(us[1 - form], us[form])) form = 1 - form;
-                    skinny_t = us[form];
-                } else if (form == 1) {
-                    skinny_t = 1e30;   // (what was measured above does not run)
-                }
-                set(&Linear::waves, form, lo);
             }
             int best = -1;
             double best_t = 1e30, model_t = 1e30;
@@ -656,7 +651,7 @@ void Executor::tune_linears() {
             const double shares = residual ? shares_cost(l0, M, gemm_ws_bytes_) : 1e30;
             if (best >= 0 && shares < 1e29) {
                 int form = in_shares(l0, M, gemm_ws_bytes_) ? 1 : 0;
-                if (close(shares, apart_cost(l0, M, gemm_ws_bytes_)) || best != by_model) {
+                if (measures_shares(l0, M, gemm_ws_bytes_, best == by_model)) {
                     double us[2];
                     us[0] = (best == by_model ? model_t : best_t) + time_us([&](LayerWeights& lw) { return pie_hip_rmsnorm(x_, lw.ffn_norm, xn_, M, H, m.rms_eps, s) == PIE_HIP_OK; });
                     us[1] = time_us([&](LayerWeights& lw) { return project_in_shares(lw.*(r.lin), r.act, lw.ffn_norm, M); });
@@ -1534,6 +1529,22 @@ extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, 
     w.shares.fill(static_cast<int8_t>(measured_shares));
     return (in_groups(w, M, workspace_bytes) ? 1 : 0) | (in_shares(w, M, workspace_bytes) ? 2 : 0) | (in_rows(w, M, workspace_bytes) ? 4 : 0) |
            (in_waves(w, M, workspace_bytes) ? 8 : 0);
+}
+
+// And which pairs of forms the start-up measurement times at a row count of its ladder: bit 0 passes and blocks that scale groups, bit 1 a product with the
+// norm behind it and shares of K that meet in the norm's kernel.
+extern "C" int pie_hip_driver_measured_forms(int format, int group, int M, int N, int K, size_t workspace_bytes) {
+    using namespace pie_hip_driver;
+    if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return -1;
+    constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
+    Linear w;
+    w.kind = kinds[format];
+    w.N = N;
+    w.K = K;
+    w.group = group;
+    int there = 0;
+    w.data_tiled = w.scale_tiled = &there;
+    return (measures_groups(w, M, workspace_bytes) ? 1 : 0) | (measures_shares(w, M, workspace_bytes, true) ? 2 : 0);
 }
 
 // The same for a mixture's experts: whether `routes` over `experts` of a storage format run in blocks of an expert's routes (1)

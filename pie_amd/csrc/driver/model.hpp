@@ -39,9 +39,9 @@ struct Linear {
     // 0 GEMV, 1 skinny GEMM, 2 tiled GEMM, 3 tiled GEMM in K shares, 4 tiled GEMM over the tile-major
     // copy; -1: not measured, the cost model decides
     std::array<int8_t, 129> tuned = [] { std::array<int8_t, 129> t{}; t.fill(-1); return t; }();
-    // likewise for quantised weights, 0 or 1 (-1: by estimate), where the skinny GEMM is chosen: int4 rows in blocks that scale groups in fp32; rows in blocks whose
-    // waves take the steps of K in turn; and the sums of a projection into the residual in shares of K that meet in the norm's kernel
-    std::array<int8_t, 129> groups = tuned, waves = tuned, shares = tuned;
+    // likewise for int4 weights, 0 or 1 (-1: by estimate): blocks that scale groups in fp32 where the skinny GEMM is chosen; the sums of a projection into
+    // the residual in shares of K that meet in the norm's kernel
+    std::array<int8_t, 129> groups = tuned, shares = tuned;
     size_t data_bytes() const {
         const size_t nk = static_cast<size_t>(N) * K;
         switch (kind) {

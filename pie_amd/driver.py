@@ -164,6 +164,8 @@ def lib() -> C.CDLL:
         l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
         l.pie_hip_driver_linear_forms.restype = C.c_int
         l.pie_hip_driver_linear_forms.argtypes = [C.c_int] * 7 + [C.c_size_t]
+        l.pie_hip_driver_measured_forms.restype = C.c_int
+        l.pie_hip_driver_measured_forms.argtypes = [C.c_int] * 5 + [C.c_size_t]
         l.pie_hip_driver_experts_in_blocks.restype = C.c_int
         l.pie_hip_driver_experts_in_blocks.argtypes = [C.c_int, C.c_longlong, C.c_int, C.c_int, C.c_int]
         l.pie_hip_driver_route_form.restype = C.c_int
@@ -489,6 +491,15 @@ def linear_forms(kind: str, M: int, N: int, K: int, group: int = 0, workspace_by
     if bits < 0:
         raise ValueError("linear_forms")
     return {name: bool(bits >> i & 1) for i, name in enumerate(("groups", "shares", "rows", "waves"))}
+
+
+def measured_forms(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 32 << 20) -> dict:
+    """Host-only: the pairs of forms that a driver times at start-up at M rows of tile-major weights: `groups` (passes, or blocks that scale groups), `shares` (a product
+    and the norm, or shares of K that meet in the norm)."""
+    bits = lib().pie_hip_driver_measured_forms(_FORMATS.index(kind), group, M, N, K, workspace_bytes)
+    if bits < 0:
+        raise ValueError("measured_forms")
+    return {name: bool(bits >> i & 1) for i, name in enumerate(("groups", "shares"))}
 
 
 def experts_in_blocks(kind: str, routes: int, experts: int, hidden: int = 0, inner: int = 0) -> bool:

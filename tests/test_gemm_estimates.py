@@ -163,6 +163,27 @@ def test_a_measurement_decides_the_forms_of_up_to_128_int4_rows():
         assert drv.linear_forms("int4b8", 129, 4096, 14336, 128, measured_groups=v, measured_shares=v) == drv.linear_forms("int4b8", 129, 4096, 14336, 128)
 
 
+LADDER = (2, 3, 4, 17, 24, 32, 33, 40, 48, 56, 64, 65, 72, 80, 88, 96, 97, 104, 112, 120, 128)   # (row counts of the start-up measurement)
+
+
+@pytest.mark.parametrize("kind", ["int4b8", "int8", "fp8", "bf16"])
+def test_a_start_measures_the_two_forms_that_it_names(kind):
+    """Where a start times a pair of forms, each setting runs a form of its own, none of them blocks whose waves take the steps of K in turn: those are by
+    estimate alone, so that two starts of one driver run the same ones."""
+    from pie_amd import driver as drv
+
+    group, pairs = 128 if kind == "int4b8" else 0, {"shares": 0}
+    for N, K in ((6144, 4096), (28672, 4096), (4096, 4096), (4096, 14336), (3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (14336, 2048), (8192, 8192)):
+        for M in LADDER:
+            for name, timed in drv.measured_forms(kind, M, N, K, group).items():
+                if not timed or name == "groups":
+                    continue
+                pairs[name] += 1
+                got = [drv.linear_forms(kind, M, N, K, group, **{f"measured_{name}": v}) for v in (0, 1)]
+                assert [f[name] for f in got] == [False, True] and not any(f["waves"] for f in got), (name, M, N, K)
+    assert kind == "int4b8" or pairs["shares"] == 0
+
+
 def test_blocks_of_tile_major_experts_have_the_rows_that_were_asked_for():
     from pie_amd import ops
 
