@@ -170,10 +170,11 @@ bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     return us < apart_cost(w, M, ws_bytes);
 }
 bool close(double a, double b) { return std::max(a, b) < 1.2 * std::min(a, b); }
-// Whether a start times the skinny GEMM's passes against the blocks that scale groups: estimates less than a fifth apart.
+// Whether a start times the skinny GEMM's passes against the blocks that scale groups: estimates less than a fifth apart, and neither gives way to blocks
+// whose waves take the steps in turn, which both settings would then run.
 bool measures_groups(const Linear& w, int M, size_t ws_bytes) {
     const double groups = groups_cost(w, M, ws_bytes), passes = passes_cost(w, M);
-    return groups < 1e29 && close(groups, passes);
+    return groups < 1e29 && close(groups, passes) && waves_cost(w, M, ws_bytes) >= std::max(groups, passes);
 }
 // Likewise shares that meet in the norm's kernel against a product and the norm, where blocks that scale groups make the shares.  Blocks whose waves take the steps in
 // turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.2 % on average to the faster of a pair's smallest times (at most 8 %), less than the tenth a

@@ -172,15 +172,16 @@ def test_a_start_measures_the_two_forms_that_it_names(kind):
     estimate alone, so that two starts of one driver run the same ones."""
     from pie_amd import driver as drv
 
-    group, pairs = 128 if kind == "int4b8" else 0, {"shares": 0}
+    group, pairs = 128 if kind == "int4b8" else 0, {"groups": 0, "shares": 0}
     for N, K in ((6144, 4096), (28672, 4096), (4096, 4096), (4096, 14336), (3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192), (14336, 2048), (8192, 8192)):
         for M in LADDER:
             for name, timed in drv.measured_forms(kind, M, N, K, group).items():
-                if not timed or name == "groups":
+                if not timed:
                     continue
                 pairs[name] += 1
                 got = [drv.linear_forms(kind, M, N, K, group, **{f"measured_{name}": v}) for v in (0, 1)]
                 assert [f[name] for f in got] == [False, True] and not any(f["waves"] for f in got), (name, M, N, K)
+    assert (pairs["groups"] > 0) == (kind == "int4b8")
     assert kind == "int4b8" or pairs["shares"] == 0
 
 
