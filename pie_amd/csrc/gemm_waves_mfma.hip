@@ -305,7 +305,7 @@ int launch(const GemmArgs& a, const Rotation& rot, const Plan& p, hipStream_t st
 // Rows and columns of a block and shares of K.  A block takes `fixed` and, per step of its waves, `step`, of a full chip `full` more (the activations' way to
 // the CUs); blocks past 256 take `again` of that and `start` each round; stores or the shares' sums 0.2 us a MiB.  That and what the weights take at 6 TB/s (int4
 // and row-major bf16 5.5) add up as cubes: either alone where the other is short, a quarter more where they are equal.
-// Shares that meet in a kernel of their own (`norm`: in the norm's) cost what gemm_groups_mfma.hip's do.  Fitted to 20000 launches of 720 products (5 - 512 rows, 15 matrices
+// Shares that meet in a kernel of their own (`norm`: in the norm's) cost what gemm_groups_mfma.hip's do.  Fitted to 20000 launches of 720 products (5 - 480 rows, int4 - 384; 15 matrices
 // of 1024 - 28672 x 1024 - 14336, weights out of HBM and rows that a kernel has just written): 7 - 9 % rms, and the plan taken is within 0.5 % of the fastest on
 // average (the worst 19 %: 160 int8 rows of 2048 x 8192 in four shares 20.7 us, in whole rows 17.4).  Bf16, both orders, over 17 matrices up to 32000 x 4096: 8 - 10 % rms, 0.5 %
 // over the fastest on average (the worst 16 %).
@@ -331,7 +331,9 @@ constexpr Cost kBf16Rows[5][3] = {{{1.00f, 0.56f, 0.00f, 0.91f, 0.00f}, {1.00f, 
                                   {{}, {1.91f, 1.07f, 0.27f, 0.83f, 0.18f}, {2.63f, 1.62f, 0.41f, 0.74f, 3.28f}},
                                   {{}, {2.33f, 1.18f, 0.40f, 0.87f, 1.61f}, {3.24f, 1.73f, 0.65f, 0.72f, 3.54f}},
                                   {{}, {2.87f, 1.46f, 0.33f, 0.82f, 2.44f}, {3.90f, 1.99f, 0.50f, 0.77f, 3.85f}}};
-constexpr int kMostRows = 512;
+// What was measured, and is taken: six blocks of rows, and 1100 blocks in all (70400 columns of up to 80 rows, int4 64: an output head of 128256 is past that).
+constexpr int kRowBlocks = 6, kBlocks = 1100;
+constexpr int most_rows(bool int4) { return kRowBlocks * (int4 ? 64 : 80); }
 enum class Form { Int4, OneByte, Bf16, Bf16Rows };
 Form form_of(int format, bool tiled) {
     return format == PIE_HIP_FMT_INT4B8 ? Form::Int4 : format != PIE_HIP_FMT_BF16 ? Form::OneByte : tiled ? Form::Bf16 : Form::Bf16Rows;
@@ -344,14 +346,14 @@ Plan find_plan(Form form, int M, int N, int K, size_t ws_bytes, bool norm) {
     Plan best;
     for (int mt = 1; mt <= (int4 ? 4 : 5); ++mt) {
         const int rows = (M + mt * 16 - 1) / (mt * 16);
-        if (rows > 6 || (rows > 1 && mt > 1 && rows * mt * 16 > 1.3 * M + 16)) continue;
+        if (rows > kRowBlocks || (rows > 1 && mt > 1 && rows * mt * 16 > 1.3 * M + 16)) continue;
         for (int n = mt <= 2 ? 0 : 1; n < 3; ++n) {   // (16 columns of 48 and more rows are next to never the fastest)
             const Cost& c = costs[mt - 1][n];
             const int tiles = rows * ((N / 16 + (1 << n) - 1) >> n);
             for (int s = norm ? 2 : 1; s <= 8; ++s) {
                 const int per = (steps + s - 1) / s, blocks = tiles * s;
                 const double bytes = 4.0 * s * M * N;
-                if (blocks > (s > 1 ? 520 : 1100)) break;
+                if (blocks > (s > 1 ? 520 : kBlocks)) break;
                 if (s > 1 && (per < 4 || bytes > static_cast<double>(ws_bytes))) break;
                 if ((s - 1) * per >= steps) continue;   // (the last share would be empty)
                 const int turns = (per + kBlockWaves - 1) / kBlockWaves, again = (blocks + 255) / 256 - 1;
@@ -372,7 +374,7 @@ bool fits(int format, int M, int N, int K, int group_size) {
     } else if (format != PIE_HIP_FMT_INT8 && format != PIE_HIP_FMT_FP8 && format != PIE_HIP_FMT_BF16) {
         return false;
     }
-    return M > 0 && M <= kMostRows && N > 0 && N % 16 == 0 && K > 0 && K % (format == PIE_HIP_FMT_INT4B8 ? 128 : 64) == 0 && (format == PIE_HIP_FMT_BF16 ? 2ll : 1ll) * N * K <= 0xFFFFFFFFll &&
+    return M > 0 && M <= most_rows(format == PIE_HIP_FMT_INT4B8) && N > 0 && N % 16 == 0 && K > 0 && K % (format == PIE_HIP_FMT_INT4B8 ? 128 : 64) == 0 && (format == PIE_HIP_FMT_BF16 ? 2ll : 1ll) * N * K <= 0xFFFFFFFFll &&
            2ll * M * K <= 0xFFFFFFFFll;
 }
 // (the same few questions are asked for every layer of a pass: the last answers are kept, per thread)

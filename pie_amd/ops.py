@@ -724,7 +724,7 @@ def gemm_groups_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor
 
 def gemm_waves_tiled(act: torch.Tensor, w: WeightView, y: Optional[torch.Tensor] = None, beta: int = 0, epilogue: int = 0,
                      workspace: Optional[torch.Tensor] = None, rule: Optional[Glu] = None) -> torch.Tensor:
-    """The GEMM over tile-major weights (bf16 also row-major) in blocks whose waves take the steps of K in turn (up to 512 rows); with a
+    """The GEMM over tile-major weights (bf16 also row-major) in blocks whose waves take the steps of K in turn (up to 480 rows, int4 384, and 1100 blocks); with a
     workspace few blocks over a long K run in shares of K."""
     _dev(act, torch.bfloat16, "act")
     M, K = act.shape

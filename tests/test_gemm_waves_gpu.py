@@ -148,6 +148,22 @@ def test_refusals():
         ops.gemm_waves_plan("int8", 600, 128, 128)
 
 
+@pytest.mark.parametrize("kind,tiled,rows,tall", [("int4b8", True, 384, 64), ("int8", True, 480, 80), ("fp8", True, 480, 80), ("bf16", True, 480, 80), ("bf16", False, 480, 80)])
+def test_the_range_ends_where_it_is_said_to(kind, tiled, rows, tall):
+    """The last count of rows and the first that is refused, with and without a workspace, and the last width of one, two and six blocks of rows and the next."""
+    from pie_amd import ops
+
+    us = lambda M, N, **kw: ops.gemm_waves_us(kind, M, N, 1024, 128, tiled=tiled, **kw)  # noqa: E731
+    for ws in (0, WORKSPACE):
+        assert all(us(M, 2048, workspace_bytes=ws) < 1e29 for M in range(1, rows + 1))
+        assert us(rows + 1, 2048, workspace_bytes=ws) > 1e29
+        with pytest.raises(ops.KernelError):
+            ops.gemm_waves_plan(kind, rows + 1, 2048, 1024, 128, ws, tiled=tiled)
+        for blocks, M in ((1, 1), (1, tall), (2, 2 * tall), (6, 6 * tall)):
+            widest = 1100 // blocks * 64
+            assert us(M, widest, workspace_bytes=ws) < 1e29 and us(M, widest + 16, workspace_bytes=ws) > 1e29
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,M,hq,hk,d,K,shares", [("int4b8", 18, 4, 2, 16, 256, False), ("int4b8", 37, 32, 8, 128, 4096, True), ("int8", 65, 8, 2, 64, 448, False),
                                                      ("int8", 24, 4, 1, 128, 8192, True), ("fp8", 131, 6, 2, 128, 1024, False),
