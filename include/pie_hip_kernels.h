@@ -322,7 +322,6 @@ int pie_hip_qkv_rope_groups_tiled(const uint16_t* act_bf16, const void* weight, 
  * tile-major copy: at most 1100 blocks (70400 columns of up to 64 rows of int4b8, 80 of the others; half as many of two blocks of rows, ..), K % 64 == 0 (int4b8: 128,
  * groups a power of two from 128 on), N % 16 == 0, act and weight on 16-byte and int4 scales on 8-byte boundaries.  With a workspace few blocks over a long K run in shares of K,
  * as many as it holds of 4 M N bytes each.  `epilogue` and `glu` as in pie_hip_gemm_mfma_glu; the estimate in microseconds (1e30: not taken). */
- */
 int pie_hip_gemm_waves_tiled(int format, const uint16_t* act_bf16, const void* weight, const void* scale, int scale_is_bf16, int group_size,
                              uint16_t* y_bf16, int M, int N, int K, int beta, int epilogue, const PieHipGlu* glu, void* workspace,
                              size_t workspace_bytes, void* stream);
