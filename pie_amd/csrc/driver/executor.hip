@@ -167,7 +167,9 @@ bool in_shares(const Linear& w, int M, size_t ws_bytes) {
     const double us = shares_cost(w, M, ws_bytes);
     if (us > 1e29) return false;
     if (M <= 128 && w.shares[M] >= 0) return w.shares[M] == 1;   // (measured at start-up)
-    return us < apart_cost(w, M, ws_bytes);
+    // (a product apart reads and writes the residual too: with 0.4 us for that the choice is 0.2 - 1.4 % over the fastest of all on average over 2144 products and norms, without 0.8 - 1.5;
+    // 64 int4 rows of 4096 x 4096 11.3 us in shares, 12.0 apart)
+    return us - 0.4 < apart_cost(w, M, ws_bytes);
 }
 bool close(double a, double b) { return std::max(a, b) < 1.2 * std::min(a, b); }
 // Whether a start times the skinny GEMM's passes against the blocks that scale groups: estimates less than a fifth apart, and neither gives way to blocks
@@ -177,8 +179,8 @@ bool measures_groups(const Linear& w, int M, size_t ws_bytes) {
     return groups < 1e29 && close(groups, passes) && waves_cost(w, M, ws_bytes) >= std::max(groups, passes);
 }
 // Likewise shares that meet in the norm's kernel against a product and the norm, where blocks that scale groups make the shares.  Blocks whose waves take the steps in
-// turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.2 % on average to the faster of a pair's smallest times (at most 8 %), less than the tenth a
-// measurement needs to overrule an estimate, and of 177 pairs with shares 2 % (12 %).  Timed, they differed from start to start, and with them the
+// turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.2 % on average to the faster of a pair's smallest times (at most 8 %), less than the tenth
+// that a measurement needs to overrule an estimate, and of 177 pairs with shares 0.6 % (20 %).  Timed, they differed from start to start, and with them the
 // kernels' rounding: 40 of the 528 measured row counts in eight starts of each driver, 8 so (19 before there were such blocks).
 bool measures_shares(const Linear& w, int M, size_t ws_bytes, bool routed_as_estimated) {
     const double us = groups_shares_cost(w, M, ws_bytes);

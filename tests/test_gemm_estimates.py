@@ -136,6 +136,39 @@ def test_int4_projections_meet_in_the_norm_where_that_is_no_slower(shape):
     assert taken <= 1.06 * apart and taken <= 1.15 * met
 
 
+# (format, rows, N, K): the fastest product with the norm behind it, and in shares of K that meet in the norm's kernel
+NORM_SHARES = {
+    ("int8", 16, 2048, 8192): (12.4, 9.4),
+    ("int8", 24, 4096, 14336): (20.7, 17.7),
+    ("int8", 40, 2048, 2048): (8.2, 8.0),
+    ("int8", 64, 5120, 5120): (19.3, 16.5),
+    ("int8", 96, 4096, 4096): (14.7, 14.6),
+    ("int8", 128, 2048, 8192): (17.4, 15.7),
+    ("int8", 256, 4096, 14336): (46.2, 50.7),
+    ("fp8", 12, 4096, 4096): (11.4, 9.3),
+    ("fp8", 40, 2560, 7168): (15.0, 12.2),
+    ("fp8", 64, 2048, 2048): (8.0, 7.9),
+    ("fp8", 80, 4096, 14336): (28.7, 25.6),
+    ("fp8", 128, 5120, 5120): (21.4, 24.4),
+    ("fp8", 192, 2048, 8192): (20.9, 17.4),
+    ("bf16", 8, 4096, 14336): (27.3, 26.2),
+    ("bf16", 24, 2048, 2048): (8.5, 7.9),
+    ("bf16", 40, 5120, 5120): (24.2, 18.7),
+    ("bf16", 64, 4096, 4096): (16.1, 14.7),
+    ("bf16", 96, 2048, 8192): (19.5, 16.6),
+    ("bf16", 128, 2560, 7168): (23.6, 19.7),
+}
+
+
+@pytest.mark.parametrize("shape", NORM_SHARES, ids=str)
+def test_projections_meet_in_the_norm_where_that_is_no_slower(shape):
+    from pie_amd import driver as drv
+
+    apart, met = NORM_SHARES[shape]
+    taken = met if drv.linear_forms(*shape)["shares"] else apart
+    assert taken <= 1.1 * min(apart, met)
+
+
 @pytest.mark.parametrize("M", [17, 32, 40, 48])
 def test_few_int4_rows_have_one_estimate(M):
     """The wide GEMM runs 17 to 48 rows of int4 weights in the blocks that scale groups in fp32: either way to them costs the same."""
