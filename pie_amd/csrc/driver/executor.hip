@@ -122,16 +122,25 @@ bool in_groups(const Linear& w, int M, size_t ws_bytes) {
     return (M <= 32 ? 1.05 : 1.0) * us < passes_cost(w, M);
 }
 // Microseconds of weights in blocks whose waves take the steps of K in turn (1e30: not taken); they run in the skinny GEMM's place where they
-// are estimated faster than its passes and than blocks that scale groups: over 16 - 320 rows of 15 matrices the choice takes 0.81 of what the others' fastest
-// does for int8, 0.87 for fp8 and 0.90 for int4, 0.4 - 0.6 % more than the fastest of all each time.  Bf16, 5 - 512 rows of 17 matrices: the kernel
-// chosen took 1.26 of what the fastest of all does on average, row-major 1.53, and with these takes 1.01.
+// are estimated faster than its passes and than blocks that scale groups.  Over 5 - 480 rows of 31 matrices, weights out of HBM, what is chosen takes 0.84 of what would be without
+// them for int8, 0.90 for fp8, 0.94 for int4, 0.85 for bf16 and 0.74 for row-major bf16, and 0.8 - 2.6 % more than the fastest of all (row-major 0.1).
 double waves_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 5 && (w.kind == Quant::Bf16 || tile_major(w)) ? pie_hip_gemm_waves_us(fmt_code(w.kind), tile_major(w) ? 1 : 0, M, w.N, w.K, w.group, ws_bytes, 0) : 1e30;
 }
 double skinny_or_groups(const Linear& w, int M, size_t ws_bytes) { return in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M); }
+// They have to be faster by more than what the estimates are off by where that was found to go against them (in graphs, 3559 points of 31 matrices; "before": what runs without this
+// kernel).  Of quantised rows up to 24 both are short (20 int4 / 17 fp8 rows of 2048 x 8192 7.9 / 8.6 us before, 8.9 / 9.8 here); int4 blocks of a short K are
+// estimated up to a fifth low (128 / 80 rows of 6144 x 2048 10.0 / 8.1 before, 11.9 / 9.1 here); row-major bf16 past 320 rows is compared with the passes'
+// bytes alone (480 rows of 128 x 2048 7.1 before, 8.0 here).  With these and those of pick_gemm 20 points are more than 3 % slower than before, the worst by 10 % (48 bf16 rows
+// of 28672 x 1024), where 97 were, the worst by 25 %; the mean gain is what it was, 6 - 26 % by format.
+double waves_margin(const Linear& w, int M, size_t ws_bytes) {
+    if (w.kind == Quant::Bf16) return !tile_major(w) && M > 320 ? 1.25 : 1.0;
+    if (in_groups(w, M, ws_bytes)) return w.K <= 2048 ? 1.2 : 1.0;
+    return M <= 24 ? 1.12 : 1.0;
+}
 bool in_waves(const Linear& w, int M, size_t ws_bytes) {
     const double us = waves_cost(w, M, ws_bytes);
-    return us < 1e29 && (M <= 8 && w.kind != Quant::Bf16 ? 1.1 : 1.0) * us < skinny_or_groups(w, M, ws_bytes);   // (of few rows both are short)
+    return us < 1e29 && waves_margin(w, M, ws_bytes) * us < skinny_or_groups(w, M, ws_bytes);
 }
 // Microseconds of one-byte weights in blocks of 32 to 128 rows (1e30: not taken); they take the place of the blocks of 256 rows
 // where they are estimated faster.
@@ -179,7 +188,7 @@ bool measures_groups(const Linear& w, int M, size_t ws_bytes) {
     return groups < 1e29 && close(groups, passes) && waves_cost(w, M, ws_bytes) >= std::max(groups, passes);
 }
 // Likewise shares that meet in the norm's kernel against a product and the norm, where blocks that scale groups make the shares.  Blocks whose waves take the steps in
-// turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.2 % on average to the faster of a pair's smallest times (at most 8 %), less than the tenth
+// turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.7 % on average to the faster of a pair's smallest times (at most 14 %), about the tenth
 // that a measurement needs to overrule an estimate, and of 177 pairs with shares 0.6 % (20 %).  Timed, they differed from start to start, and with them the
 // kernels' rounding: 40 of the 528 measured row counts in eight starts of each driver, 8 so (19 before there were such blocks).
 bool measures_shares(const Linear& w, int M, size_t ws_bytes, bool routed_as_estimated) {
@@ -195,8 +204,10 @@ double tiled_cost(const Linear& w, int M) {
 GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
     if (w.K % 64 != 0 || M < 17) return GemmPath::Skinny;
     const auto [p2, wpasses, wave_form, passes] = skinny_cost(w, M);
+    const bool one_byte = w.kind == Quant::Int8 || w.kind == Quant::Fp8;
     const double waves = in_waves(w, M, ws_bytes) ? waves_cost(w, M, ws_bytes) : 1e30;   // (in the skinny GEMM's place)
-    const double skinny = std::min(w.kind != Quant::Int4b8 ? passes_cost(w, M) : passes, waves);
+    // (against the blocks of the larger batches: 112 int8 rows of 16384 x 2048 20.1 us in those, 21.9 here)
+    const double skinny = std::min(w.kind != Quant::Int4b8 ? passes_cost(w, M) : passes, (one_byte ? 1.06 : 1.0) * waves);
     const double data = static_cast<double>(w.data_bytes()), groups = groups_cost(w, M, ws_bytes);
     const int steps = w.K / 64;
     if (M > 128) {
@@ -216,9 +227,11 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         const double tiles = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
         const double rows = rows_cost(w, M, ws_bytes), wide = tile_major(w) ? static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes)) : tiles;
         const double blocks = std::min(rows, wide);
+        // (bf16 rows are estimated a fifth low where their blocks come in two rounds, and the tiled GEMM a tenth high: 136 of 16384 x 2048 24.8 us in tiles, 31.1 here; one-byte
+        // rows of a short K likewise: 192 of 8192 x 512 8.0 in blocks of rows, 9.8 here)
+        if ((w.kind == Quant::Bf16 ? 1.12 : one_byte && w.K <= 1024 ? 1.2 : 1.0) * waves < std::min({rows, wide, tiles})) return GemmPath::Skinny;
         // (on narrow outputs blocks of few rows and the passes are close, and the passes' estimate is the one that is too high: 160 rows of 3072 x 4096 and
         // 320 of 2048 x 2048 fp8 13.9 and 13.7 us in passes, 17.0 and 14.7 in blocks)
-        if (waves < std::min({rows, wide, tiles})) return GemmPath::Skinny;
         if (rows_us < std::min(1.12 * rows, wide) || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;
         return blocks < tiles ? GemmPath::Wide : GemmPath::Tiled;
     }
@@ -1517,7 +1530,7 @@ extern "C" int pie_hip_driver_linear_route(int format, int group, int M, int N, 
 // projection into the residual in shares of K that meet in the norm's kernel, bit 2 one-byte rows in blocks of 32 to 128 (in the wide GEMM's place), bit 3 rows in
 // blocks whose waves take the steps of K in turn (in the skinny GEMM's place).
 extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, int K, int measured_groups, int measured_shares,
-                                           size_t workspace_bytes) {
+                                           int tile_major, size_t workspace_bytes) {
     using namespace pie_hip_driver;
     if (format < PIE_HIP_FMT_INT4B8 || format > PIE_HIP_FMT_BF16 || M <= 0 || N <= 0 || K <= 0) return -1;
     constexpr Quant kinds[] = {Quant::Int4b8, Quant::Int8, Quant::Fp8, Quant::Bf16};
@@ -1527,7 +1540,7 @@ extern "C" int pie_hip_driver_linear_forms(int format, int group, int M, int N, 
     w.K = K;
     w.group = group;
     int there = 0;
-    w.data_tiled = w.scale_tiled = &there;
+    if (tile_major) w.data_tiled = w.scale_tiled = &there;
     w.groups.fill(static_cast<int8_t>(measured_groups));
     w.shares.fill(static_cast<int8_t>(measured_shares));
     return (in_groups(w, M, workspace_bytes) ? 1 : 0) | (in_shares(w, M, workspace_bytes) ? 2 : 0) | (in_rows(w, M, workspace_bytes) ? 4 : 0) |

@@ -163,7 +163,7 @@ def lib() -> C.CDLL:
         l.pie_hip_driver_linear_route.restype = C.c_int
         l.pie_hip_driver_linear_route.argtypes = [C.c_int] * 6 + [C.c_size_t]
         l.pie_hip_driver_linear_forms.restype = C.c_int
-        l.pie_hip_driver_linear_forms.argtypes = [C.c_int] * 7 + [C.c_size_t]
+        l.pie_hip_driver_linear_forms.argtypes = [C.c_int] * 8 + [C.c_size_t]
         l.pie_hip_driver_measured_forms.restype = C.c_int
         l.pie_hip_driver_measured_forms.argtypes = [C.c_int] * 5 + [C.c_size_t]
         l.pie_hip_driver_experts_in_blocks.restype = C.c_int
@@ -483,11 +483,11 @@ def linear_route(kind: str, M: int, N: int, K: int, group: int = 0, tile_major: 
 
 
 def linear_forms(kind: str, M: int, N: int, K: int, group: int = 0, workspace_bytes: int = 32 << 20, measured_groups: int = -1,
-                 measured_shares: int = -1) -> dict:
-    """Host-only: the forms the driver's estimates (or measurements: 0, 1) give tile-major weights: `groups` (int4 rows in blocks in the skinny GEMM's place), `shares` (a
+                 measured_shares: int = -1, tile_major: bool = True) -> dict:
+    """Host-only: the forms the driver's estimates (or measurements: 0, 1) give weights with a tile-major copy, or without: `groups` (int4 rows in blocks in the skinny GEMM's place), `shares` (a
     projection into the residual whose sums meet in the norm), `rows` (one-byte rows in blocks in the wide GEMM's place), `waves` (rows in blocks whose waves take the
     steps of K in turn, in the skinny GEMM's place)."""
-    bits = lib().pie_hip_driver_linear_forms(_FORMATS.index(kind), group, M, N, K, measured_groups, measured_shares, workspace_bytes)
+    bits = lib().pie_hip_driver_linear_forms(_FORMATS.index(kind), group, M, N, K, measured_groups, measured_shares, int(tile_major), workspace_bytes)
     if bits < 0:
         raise ValueError("linear_forms")
     return {name: bool(bits >> i & 1) for i, name in enumerate(("groups", "shares", "rows", "waves"))}
