@@ -125,6 +125,44 @@ def test_blocks_of_one_byte_rows(gpu, kind, M, N, K, rows, shares):
     check_stores(gpu, lambda y, beta, epilogue, rule: ops.gemm_rows_tiled(act, w, y=y, beta=beta, epilogue=epilogue, rule=rule, workspace=ws), sums, 940 + M)
 
 
+# (format, rows, N, K, rows and columns of a block, shares of K): rows and columns off a block, steps that do not divide by the waves, one share and several
+WAVES = [(kind, *case) for kind, cases in {
+    "int4b8": [(15, 48, 384, 16, 16, 1), (5, 16, 8320, 16, 16, 5), (17, 4112, 1152, 32, 32, 1), (33, 12304, 1152, 48, 64, 1), (300, 16, 2176, 64, 32, 3), (97, 6160, 1152, 64, 64, 1)],
+    "int8": [(15, 48, 192, 16, 16, 1), (17, 528, 4160, 16, 32, 5), (32, 8208, 576, 32, 64, 1), (230, 16, 4160, 48, 32, 5), (65, 12304, 576, 80, 64, 1)],
+    "fp8": [(16, 4112, 576, 16, 32, 1), (97, 16, 4160, 32, 16, 5), (33, 12304, 576, 48, 64, 1), (300, 16, 2112, 64, 32, 5)],
+    "bf16": [(15, 48, 192, 16, 16, 1), (33, 272, 8256, 16, 32, 6), (97, 2064, 576, 32, 64, 1), (65, 2064, 8256, 80, 64, 6)],
+    "bf16 rows": [(15, 48, 192, 16, 16, 1), (97, 16, 4160, 32, 16, 5), (130, 4112, 576, 48, 64, 1), (300, 272, 8256, 80, 32, 6)]}.items() for case in cases]
+
+
+@pytest.mark.parametrize("kind,M,N,K,rows,cols,shares", WAVES)
+def test_blocks_whose_waves_take_the_steps_of_k_in_turn(gpu, kind, M, N, K, rows, cols, shares):
+    """And a y on two bytes, with the residual and the gated rules."""
+    import torch
+    from pie_amd import ops
+
+    kind, tiled = kind.split()[0], not kind.endswith("rows")
+    ws = torch.full((4 << 20,), float("nan"), device=gpu) if shares > 1 else None
+    act, w, sums = exact_problem(gpu, kind, M, N, K, 1000 + M + N)
+    assert ops.gemm_waves_plan(kind, M, N, K, w.group_size, 0 if ws is None else ws.numel() * 4, tiled=tiled) == (rows, cols, shares)
+    if kind == "bf16" and tiled:
+        w = ops.repack_mfma_tiles(w)
+
+    def call(y, beta, epilogue, rule):
+        return ops.gemm_waves_tiled(act, w, y=y, beta=beta, epilogue=epilogue, rule=rule, workspace=ws)
+
+    check_stores(gpu, call, sums, 1000 + M)
+    g = torch.Generator(device=gpu).manual_seed(1000 + M)
+    y0 = torch.randn(M, N, generator=g, device=gpu).bfloat16()
+    bias = torch.randint(-8, 9, (N,), generator=g, device=gpu).float() / 4
+    off = lambda cols: torch.empty(M * cols + 1, device=gpu, dtype=torch.bfloat16)[1:].view(M, cols)  # noqa: E731
+    assert off(N).data_ptr() % 4 == 2
+    assert torch.equal(call(off(N), 0, 0, None), sums.bfloat16())
+    assert torch.equal(call(off(N).copy_(y0), 1, 0, None), (sums + y0.float()).bfloat16())
+    for rule, add in ((ops.glu(), 0.0), (ops.glu(bias=bias, **RULES), bias)):
+        plain = ops.glu(**RULES) if torch.is_tensor(add) else ops.glu()
+        assert torch.equal(call(off(N // 2), 0, 1, rule), ops.glu_f32((sums + add).bfloat16().float().contiguous(), plain).bfloat16())
+
+
 @pytest.mark.parametrize("kind", ["int8", "fp8"])
 @pytest.mark.parametrize("height,counts", [(32, [0, 1, 31, 33, 7]), (64, [63, 65, 0, 30]), (96, [95, 97, 1, 100]), (128, [127, 129, 1, 257])])
 @pytest.mark.parametrize("N", [288, 272])

@@ -18,6 +18,6 @@ def kernels():
 
 def test_no_gemm_spills_registers():
     """The GEMMs' launch bounds leave each instance the registers it needs: nothing of theirs goes through scratch memory."""
-    gemms = [k for k in kernels() if any(n in k[".name"] for n in ("gemm_columns", "gemm_groups", "gemm_wide", "gemm_mfma"))]
-    assert len(gemms) > 40
+    gemms = [k for k in kernels() if any(n in k[".name"] for n in ("gemm_columns", "gemm_groups", "gemm_waves", "gemm_wide", "gemm_mfma"))]
+    assert len(gemms) > 40 and sum("gemm_waves" in k[".name"] for k in gemms) > 40
     assert not [k[".name"] for k in gemms if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
