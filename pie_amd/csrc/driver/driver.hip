@@ -537,8 +537,8 @@ extern "C" size_t pie_hip_driver_export_tensor(PieHipDriver* d, const char* name
         return sizeof(tab);
     }
     if (nm == "info.tuned_forms") {
-        // what it left of the int4 forms: int8 [2][4 linears][129 row counts], blocks that scale groups in fp32 in the skinny GEMM's place and shares of K that
-        // meet in the norm; 0 or 1, -1 = by estimate
+        // and the forms: int8 [2][4 linears][129 row counts], int4 blocks that scale groups in fp32 in the skinny GEMM's place (where blocks whose waves take the steps
+        // of K in turn, by estimate alone, do not go before) and shares of K that meet in the norm; 0 or 1, -1 = by estimate
         const auto& lw = d->model.layers.at(0);
         const Linear* lins[4] = {&lw.wqkv, &lw.wo, &lw.wgu, &lw.wdown};
         int8_t tab[2][4][129];

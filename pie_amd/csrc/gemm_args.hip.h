@@ -136,16 +136,16 @@ __device__ __forceinline__ void wide_store(const GemmArgs& a, int m, int n, floa
 }
 
 inline int stores_lines(const uint16_t* y, int N) { return N % 32 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0; }
-// The same for columns n .. n + 3 and n + 16 .. n + 19, n = 32 k + 4 q with q the lane's sixteenth of the wave (a.lines): neighbouring
-// sixteenths swap half of their values, the even ones end with eight columns of the first tile and the odd ones of the second, so that
-// a store is 16 bytes and a row's four lanes fill 64 (SwiGLU: 8 and 32).
-// Where store_pair's row m goes; sixteen rows on it is `row_step` values further.
+// Where store_pair's row m goes, q the lane's sixteenth of the wave; sixteen rows on it is `row_step` values further.
 template <Out O>
 __device__ __forceinline__ uint16_t* pair_place(const GemmArgs& a, int m, int n, int q, int& row_step) {
     const int nout = is_gated<O>(a) ? a.N / 2 : a.N, at = q & 1 ? n + 12 : n;
     row_step = 16 * nout;
     return a.y + static_cast<size_t>(m) * nout + (is_gated<O>(a) ? at / 2 : at);
 }
+// wide_store for columns n .. n + 3 and n + 16 .. n + 19, n = 32 k + 4 q (a.lines): neighbouring sixteenths swap half of their values, the even ones end with
+// eight columns of the first tile and the odd ones of the second, so that a store is 16 bytes and a row's four lanes fill 64 (SwiGLU: 8 and 32).
+// `to` is pair_place's for the same O, row, n and sixteenth, and all four lanes of a row call it.
 template <Out O = Out::Any>
 __device__ __forceinline__ void store_pair(const GemmArgs& a, uint16_t* to, int n, float* v0, float* v1) {
     if (is_gated<O>(a)) {
