@@ -122,17 +122,17 @@ bool in_groups(const Linear& w, int M, size_t ws_bytes) {
     return (M <= 32 ? 1.05 : 1.0) * us < passes_cost(w, M);
 }
 // Microseconds of weights in blocks whose waves take the steps of K in turn (1e30: not taken); they run in the skinny GEMM's place where they
-// are estimated faster than its passes and than blocks that scale groups.  Over 5 - 480 rows of 31 matrices, weights out of HBM, what is chosen takes 0.84 of what would be without
-// them for int8, 0.90 for fp8, 0.94 for int4, 0.85 for bf16 and 0.74 for row-major bf16, and 0.8 - 2.6 % more than the fastest of all (row-major 0.1).
+// are estimated faster than its passes and than blocks that scale groups.  Over 5 - 480 rows of 42 matrices, weights out of HBM, what is chosen takes 0.84 of what would be without
+// them for int8, 0.90 for fp8, 0.94 for int4, 0.85 for bf16 and 0.74 for row-major bf16, and 0.8 - 2.6 % more than the fastest of all.
 double waves_cost(const Linear& w, int M, size_t ws_bytes) {
     return M >= 5 && (w.kind == Quant::Bf16 || tile_major(w)) ? pie_hip_gemm_waves_us(fmt_code(w.kind), tile_major(w) ? 1 : 0, M, w.N, w.K, w.group, ws_bytes, 0) : 1e30;
 }
 double skinny_or_groups(const Linear& w, int M, size_t ws_bytes) { return in_groups(w, M, ws_bytes) ? groups_cost(w, M, ws_bytes) : passes_cost(w, M); }
-// They have to be faster by more than what the estimates are off by where that was found to go against them (in graphs, 3559 points of 31 matrices; "before": what runs without this
+// They have to be faster by more than what the estimates are off by where that was found to go against them (in graphs, 4001 points of 42 matrices; "before": what runs without this
 // kernel).  Of quantised rows up to 24 both are short (20 int4 / 17 fp8 rows of 2048 x 8192 7.9 / 8.6 us before, 8.9 / 9.8 here); int4 blocks of a short K are
 // estimated up to a fifth low (128 / 80 rows of 6144 x 2048 10.0 / 8.1 before, 11.9 / 9.1 here); row-major bf16 past 320 rows is compared with the passes'
 // bytes alone (480 rows of 128 x 2048 7.1 before, 8.0 here).  With these and those of pick_gemm 20 points are more than 3 % slower than before, the worst by 10 % (48 bf16 rows
-// of 28672 x 1024), where 97 were, the worst by 25 %; the mean gain is what it was, 6 - 26 % by format.
+// of 28672 x 1024), where 110 were, the worst by 28 %; the mean gain is what it was, 6 - 26 % by format.
 double waves_margin(const Linear& w, int M, size_t ws_bytes) {
     if (w.kind == Quant::Bf16) return !tile_major(w) && M > 320 ? 1.25 : 1.0;
     if (in_groups(w, M, ws_bytes)) return w.K <= 2048 ? 1.2 : 1.0;
@@ -222,14 +222,16 @@ GemmPath pick_gemm(const Linear& w, int M, size_t ws_bytes) {
         // the decoding, not by the weights' width)
         const double bytes = w.kind == Quant::Bf16 ? data : (w.kind == Quant::Int8 ? 0.63 : w.kind == Quant::Fp8 ? 0.57 : 0.5) * w.N * static_cast<double>(w.K);
         const double prompt_form = p2 <= 8 ? wave_form : 1.38 * (1.0 + 0.52 * 7) * 0.9 * (p2 <= 32 ? p2 : wpasses) / 8.0 * (p2 == 32 && wpasses < 32 ? 1.2 : 1.0);
-        const double rows_us = w.data_tiled ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * prompt_form : skinny;
+        const double rows_us = w.data_tiled ? (M > 256 ? 7.0 : 5.0) + bytes / 3.8e6 * prompt_form : w.kind != Quant::Int4b8 ? passes_cost(w, M) : passes;
         const int fmt = fmt_code(w.kind);
         const double tiles = pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 0, ws_bytes);
         const double rows = rows_cost(w, M, ws_bytes), wide = tile_major(w) ? static_cast<double>(pie_hip_gemm_mfma_us(fmt, M, w.N, w.K, w.group, 1, ws_bytes)) : tiles;
         const double blocks = std::min(rows, wide);
-        // (bf16 rows are estimated a fifth low where their blocks come in two rounds, and the tiled GEMM a tenth high: 136 of 16384 x 2048 24.8 us in tiles, 31.1 here; one-byte
-        // rows of a short K likewise: 192 of 8192 x 512 8.0 in blocks of rows, 9.8 here)
-        if ((w.kind == Quant::Bf16 ? 1.12 : one_byte && w.K <= 1024 ? 1.2 : 1.0) * waves < std::min({rows, wide, tiles})) return GemmPath::Skinny;
+        // (bf16 rows are estimated a fifth low where their blocks come in two rounds, and the tiled GEMM a tenth high: 136 of 16384 x 2048 24.8 us in tiles, 31.1 here; more
+        // so of a short K: 352 of 4096 x 512 11.2 and 12.2; not of a long one: 288 of 2048 x 8192 29.7 and 26.0, estimated 29.6; one-byte rows of a short K likewise: 192 of
+        // 8192 x 512 8.0 in blocks of rows, 9.8 here)
+        const double margin = w.kind == Quant::Bf16 ? (w.K <= 768 ? 1.3 : w.K < 8192 ? 1.12 : 1.0) : one_byte && w.K <= 1024 ? 1.2 : 1.0;
+        if (margin * waves < std::min({rows, wide, tiles})) return GemmPath::Skinny;
         // (on narrow outputs blocks of few rows and the passes are close, and the passes' estimate is the one that is too high: 160 rows of 3072 x 4096 and
         // 320 of 2048 x 2048 fp8 13.9 and 13.7 us in passes, 17.0 and 14.7 in blocks)
         if (rows_us < std::min(1.12 * rows, wide) || groups < std::min({skinny, blocks, tiles})) return GemmPath::Skinny;

@@ -189,9 +189,15 @@ FORMS = {
     ("bf16 rows", 128, 5120, 5120): dict(passes=66.1, waves=24.9, tiled=58.3),
     ("bf16 rows", 192, 384, 4096): dict(passes=15.9, waves=8.5, tiled=17.4),
     ("bf16 rows", 288, 2048, 2048): dict(passes=29.9, waves=10.5, tiled=20.7),
+    ("bf16 rows", 136, 16384, 2048): dict(passes=83.5, waves=31.5, tiled=25.0),
+    ("bf16 rows", 288, 8192, 512): dict(passes=46.6, waves=14.4, tiled=11.2),
+    ("bf16 rows", 288, 2048, 8192): dict(passes=96.1, waves=26.0, tiled=29.7),
+    ("bf16 rows", 352, 4096, 512): dict(passes=30.0, waves=12.2, tiled=11.2),
+    ("bf16 rows", 448, 4096, 512): dict(passes=38.4, waves=13.7, tiled=11.0),
+    ("bf16 rows", 224, 6144, 1536): dict(passes=51.7, waves=18.4, tiled=20.4),
     ("bf16 rows", 480, 128, 2048): dict(passes=7.1, waves=8.0, tiled=15.5),
 }
-# (matrices that no estimate was fitted to: over 3588 points of 31 matrices the form taken is 1.01 - 1.03 of the fastest on average by format, 142 are more than a tenth over)
+# (matrices that no estimate was fitted to: over 4030 points of 42 matrices the form taken is 1.01 - 1.03 of the fastest on average by format, 157 are more than a tenth over)
 NOT_FITTED = {(5120, 5120), (9216, 3584), (2560, 7168), (6144, 2048), (10240, 2560), (48000, 2048), (8192, 512), (512, 4096), (384, 4096), (128, 2048)}
 
 
