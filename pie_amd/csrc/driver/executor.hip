@@ -190,7 +190,7 @@ bool measures_groups(const Linear& w, int M, size_t ws_bytes) {
 // Likewise shares that meet in the norm's kernel against a product and the norm, where blocks that scale groups make the shares.  Blocks whose waves take the steps in
 // turn are chosen by estimate alone: over 160 such pairs of seven drivers that loses 0.7 % on average to the faster of a pair's smallest times (at most 14 %), about the tenth
 // that a measurement needs to overrule an estimate, and of 177 pairs with shares 0.6 % (20 %).  Timed, they differed from start to start, and with them the
-// kernels' rounding: 40 of the 528 measured row counts in eight starts of each driver, 8 so (19 before there were such blocks).
+// kernels' rounding: 40 of the 528 measured row counts in eight starts of each driver, 12 so, seven of which run the same kernel either way (19 before there were such blocks).
 bool measures_shares(const Linear& w, int M, size_t ws_bytes, bool routed_as_estimated) {
     const double us = groups_shares_cost(w, M, ws_bytes);
     return shares_cost(w, M, ws_bytes) < 1e29 && us < 1e29 && us <= waves_shares_cost(w, M, ws_bytes) && !in_waves(w, M, ws_bytes) &&
