@@ -108,6 +108,9 @@ double passes_cost(const Linear& w, int M) {
                                  /* row-major */ {{8, 4.80, 6.01e6, 0.191e-3, 0.474e-3}, {16, 5.16, 6.06e6, 0.208e-3, 0.693e-3}, {32, 6.06, 2.93e6, 0.000e-3, 0.160e-3},
                                                   {64, 6.35, 1.97e6, 0.024e-3, 0.449e-3}, {96, 8.00, 1.43e6, 0.000e-3, 0.726e-3}, {128, 8.00, 1.04e6, 0.000e-3, 0.102e-3},
                                                   {192, 8.00, 0.77e6, 0.191e-3, 0.859e-3}, {320, 6.28, 0.46e6, 0.123e-3, 0.209e-3}}};
+    // (parts of a step of K are refused, and the GEMV runs, four rows at a time: 12 / 16 int4 rows of 1536 x 8960 in blocks whose waves take the steps in turn 8.6 / 8.8 us)
+    if (w.K % (w.kind == Quant::Int4b8 ? 512 : w.kind == Quant::Bf16 ? 128 : 256) != 0)
+        return ((M + 3) / 4) * (3.4 + 2.5 * static_cast<double>(w.data_bytes()) / 5.5e6);
     if (w.kind == Quant::Bf16 || tile_major(w))
         for (const Fit& f : kFits[w.kind == Quant::Int4b8 ? 0 : w.kind == Quant::Int8 ? 1 : w.kind == Quant::Fp8 ? 2 : tile_major(w) ? 3 : 4])
             if (M <= f.rows)   // (a list's unused places have no rows)
